@@ -1046,6 +1046,33 @@ int im_newton_solve_dense_tile(const im_newton_args *args, float *H, int32_t *do
 int im_newton_solve_dense_column(const im_newton_args *args, float *H, float *U, int32_t *dof_union, int nv, int nv_pad,
                                  int nM, int32_t *next_world, void *stream);
 
+/* A whole constraint solve in one call: the start point, init_context, the iterations and the
+ * constraint force, in the order of the reference's step
+ * (src/instantmimic/utils/mjw_step_optimized.py:2588-2683), as three launches -- the start
+ * (im_newton_init_context, with qacc = qacc_start and nsolving = nworld), the first factor stage, the
+ * resident loop of im_newton_solve_tree / _sparse / _dense_tile / _dense_column, in which a world
+ * that finishes writes qfrc_constraint itself.  The arrays end as after those calls and
+ * im_qfrc_constraint_from_grad one after the other, bit for bit.  IM_ERR_UNSUPPORTED where the model
+ * has no resident loop: the caller then issues the pieces (which set everything afresh). */
+typedef struct im_newton_start {
+  const float *qacc_start; /* (nworld, ld_start): the warm start, or qacc_smooth */
+  int64_t ld_start;
+  const float *qacc_smooth;
+  int64_t ld_smooth;
+  const float *efc_aref;
+  int64_t ld_aref;
+} im_newton_start;
+typedef struct im_newton_model {
+  const im_tree_plan *tree;     /* the tree stage, or */
+  const im_sparse_plan *sparse; /* the static-pattern stage (U: ctx.hfactor), or neither: the dense stage with */
+  const int32_t *elemid;        /* the (nv, nv) element table of M, */
+  float *H, *U;                 /* ctx.h and ctx.hfactor (nworld, nv_pad, nv_pad), */
+  int32_t *dof_union;           /* (nworld, nv + 1), also of the sparse stage, */
+  int32_t *next_world;          /* one int32 of the caller's */
+  int32_t nv, nv_pad, nM;
+} im_newton_model;
+int im_newton_solve(const im_newton_args *args, const im_newton_start *start, const im_newton_model *model, void *stream);
+
 /* Replaces _init_efc_settling_empty_worlds
  * (src/instantmimic/utils/mjw_kernels/newton_fusion.py:412-428): solver_niter = 0,
  * search_dot = 0, done = (nefc == 0), and a world without constraint rows gets

@@ -87,6 +87,20 @@ class NewtonArgs(C.Structure):
     ]  # fmt: skip
 
 
+class NewtonStart(C.Structure):
+    """im_newton_start"""
+
+    _fields_ = [("qacc_start", C.c_void_p), ("ld_start", C.c_int64), ("qacc_smooth", C.c_void_p), ("ld_smooth", C.c_int64),
+                ("efc_aref", C.c_void_p), ("ld_aref", C.c_int64)]  # fmt: skip
+
+
+class NewtonModel(C.Structure):
+    """im_newton_model"""
+
+    _fields_ = [("tree", C.c_void_p), ("sparse", C.c_void_p), ("elemid", C.c_void_p), ("H", C.c_void_p), ("U", C.c_void_p),
+                ("dof_union", C.c_void_p), ("next_world", C.c_void_p), ("nv", C.c_int32), ("nv_pad", C.c_int32), ("nM", C.c_int32)]  # fmt: skip
+
+
 class RowPairTerm(C.Structure):
     """im_row_pair_term"""
 
@@ -271,6 +285,7 @@ SIGNATURES = {
         _i,
         [_vp, _vp, _vp, _i64, _vp, _i, _vp, _vp, _vp, _i, _vp, _i64, _vp, _i64, _vp, _vp, _i, _i, _vp],
     ),
+    "im_newton_solve": (_i, [C.POINTER(NewtonArgs), C.POINTER(NewtonStart), C.POINTER(NewtonModel), _vp]),
     "im_newton_solve_tree": (_i, [_vp, C.POINTER(NewtonArgs), _vp]),
     "im_newton_solve_dense_tile": (_i, [C.POINTER(NewtonArgs), _vp, _vp, _i, _i, _i, _vp, _vp]),
     "im_newton_solve_dense_column": (_i, [C.POINTER(NewtonArgs), _vp, _vp, _vp, _i, _i, _i, _vp, _vp]),
@@ -316,6 +331,27 @@ def lib():
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+_native = None
+
+
+def native():
+    """``_native.so``: the hot entry points' checks and launches in native code (``csrc/native_calls.cpp``).
+    Its functions return None when they have launched, a library status, or -1 for arguments that the
+    Python caller has to look at itself."""
+    global _native
+    if _native is None:
+        import torch  # noqa: F401  (the module links against torch's libraries)
+
+        lib()
+        path = os.path.join(_HERE, "_native.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python -m instantmimic_amd.build`")
+        from . import _native as module
+
+        _native = module
+    return _native
 
 
 def check(status: int, where: str) -> None:

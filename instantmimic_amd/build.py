@@ -18,8 +18,9 @@ CSRC = os.path.join(HERE, "csrc")
 GEN = os.path.join(CSRC, "gen")
 OBJ = os.path.join(HERE, "_obj")
 LIB = os.path.join(HERE, "libimhip.so")
+NATIVE = os.path.join(HERE, "_native.so")
 
-SOURCES = ["tree_plan.cpp", "sparse_plan.cpp", "tree_kernels.hip", "muscle_kernels.hip", "muscle_geometry.hip", "sparse_kernels.hip", "blocked_kernels.hip", "tile_kernels.hip", "dense_column_kernels.hip", "tree_reduce_kernels.hip", "newton_kernels.hip", "newton_search_kernels.hip", "newton_init_kernels.hip", "implicit_kernels.hip"]
+SOURCES = ["tree_plan.cpp", "sparse_plan.cpp", "tree_kernels.hip", "muscle_kernels.hip", "muscle_geometry.hip", "sparse_kernels.hip", "blocked_kernels.hip", "tile_kernels.hip", "dense_column_kernels.hip", "tree_reduce_kernels.hip", "newton_kernels.hip", "newton_search_kernels.hip", "newton_init_kernels.hip", "newton_solve.hip", "implicit_kernels.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950",
@@ -201,7 +202,30 @@ def build_library(verbose: bool = True) -> str:
     with ThreadPoolExecutor(max_workers=8) as pool:
         objs = list(pool.map(_compile, sources))
     subprocess.run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB], check=True)
+    build_native()
     return LIB
+
+
+def build_native() -> str:
+    """``_native.so``, the CPython module of ``csrc/native_calls.cpp``: host code only, against torch's
+    headers and ``libimhip.so``."""
+    import sysconfig
+
+    import torch
+
+    src = os.path.join(CSRC, "native_calls.cpp")
+    header = os.path.join(HERE, "..", "include", "imhip.h")
+    if os.path.exists(NATIVE) and not os.environ.get("IMHIP_REBUILD") and os.path.getmtime(NATIVE) > max(os.path.getmtime(p) for p in (src, header)):
+        return NATIVE
+    base = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH") or "/opt/rocm"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", f"{base}/include",
+           "-isystem", f"{base}/include/torch/csrc/api/include", "-isystem", f"{rocm}/include",
+           "-isystem", sysconfig.get_paths()["include"], src, "-o", NATIVE, f"-L{base}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python", f"-L{HERE}", "-l:libimhip.so", "-Wl,-rpath,$ORIGIN"]  # fmt: skip
+    subprocess.run(cmd, check=True)
+    return NATIVE
 
 
 if __name__ == "__main__":

@@ -28,6 +28,7 @@
 
 #include "common.h"
 #include "jtdj_wave.h"
+#include "newton_solve.h"
 #include "newton_wave.h"
 #include "pivot.h"
 
@@ -484,7 +485,6 @@ __global__ __launch_bounds__(64 * WAVES, NBLK == 3 ? 3 : 2) void newton_dense_co
   }
 }
 
-__global__ void set_column_counter_kernel(int *counter, int value) { *counter = value; }
 
 struct ColumnVariant {
   int nblk, waves, held;
@@ -496,64 +496,7 @@ struct ColumnVariant {
 
 extern "C" int im_newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32_t *dof_union, int nv,
                                             int nv_pad, int nM, int32_t *next_world, void *stream) {
-  if (!p || !H || !U || !dof_union || !next_world || p->nworld < 0 || nv <= 0 || nv_pad <= nv || nM <= 0) return IM_ERR_ARG;
-  if (nv <= 32 || (nv_pad != 48 && nv_pad != 64)) return IM_ERR_UNSUPPORTED;
-  if (p->nworld == 0) return IM_OK;
-  im::resident::NewtonArgs a{};
-  const int bad = im::resident::convert_args(*p, nv, nM, a);
-  if (bad != IM_OK) return bad;
-  const int njmax = p->njmax;
-#define IM_COLUMN_VARIANT(NBLK, WAVES, HELD) \
-  {NBLK, WAVES, HELD, (const void *)im::newton_dense_column_resident_kernel<NBLK, WAVES, HELD>}
-  // 48 or 64 columns; four or eight worlds per workgroup (a lane holds a whole column: up to 256 registers);
-  // the line search keeps a lane's two rows in registers up to 64 rows and reads them from LDS beyond
-  // (four first: at about 150 registers a lane a CU holds twelve wavefronts, three such workgroups or one of eight)
-  static const im::ColumnVariant variants[] = {IM_COLUMN_VARIANT(3, 4, 2), IM_COLUMN_VARIANT(3, 8, 2), IM_COLUMN_VARIANT(3, 4, 0),
-                                               IM_COLUMN_VARIANT(3, 8, 0), IM_COLUMN_VARIANT(4, 4, 2), IM_COLUMN_VARIANT(4, 8, 2),
-                                               IM_COLUMN_VARIANT(4, 4, 0), IM_COLUMN_VARIANT(4, 8, 0)};
-#undef IM_COLUMN_VARIANT
-  constexpr int kVariants = 8;
-  static bool usable[kVariants] = {};
-  static int regs[kVariants] = {};
-  static bool probed = false;
-  if (!probed) {  // once per process: a variant that spills registers is left out; the large dynamic LDS is asked for
-    for (int i = 0; i < kVariants; ++i) {
-      hipFuncAttributes fa{};
-      // (a variant that parks more than a register or two of its prologue in memory is left out)
-      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
-                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
-      regs[i] = fa.numRegs;
-      (void)hipGetLastError();
-    }
-    probed = true;
-  }
-  const int nblk = nv_pad / 16;
-  for (int i = 0; i < kVariants; ++i) {
-    const im::ColumnVariant &v = variants[i];
-    if (!usable[i] || v.nblk != nblk || v.held != (njmax <= 64 ? 2 : 0)) continue;
-    const int area = nblk == 3 ? im::column_resident_area_words<3>(nv, njmax) : im::column_resident_area_words<4>(nv, njmax);
-    const size_t per_wave = (size_t)area + im::resident::kept_words(nv, njmax, 0);
-    const size_t lds = 4 * ((size_t)im::column_resident_shared_words(p->nterm, nv) + v.waves * per_wave);
-    if (lds > 158 * 1024) continue;
-    static int ncu = 0;
-    if (!ncu) {
-      int dev = 0;
-      IM_HIP_CHECK(hipGetDevice(&dev));
-      IM_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    }
-    // as many workgroups as stay resident at once: by LDS and by registers
-    int per_cu = 0;
-    IM_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, v.fn, 64 * v.waves, lds));
-    per_cu = std::max(1, per_cu);
-    const int needed = (p->nworld + v.waves - 1) / v.waves;
-    const int grid = std::min(needed, std::max(ncu, 1) * per_cu);
-    hipLaunchKernelGGL(im::set_column_counter_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, next_world, grid * v.waves);
-    void *args[] = {&a, &H, &U, &dof_union, &next_world};
-    IM_HIP_CHECK(hipLaunchKernel(v.fn, dim3((unsigned)grid), dim3(64 * v.waves), args, lds, (hipStream_t)stream));
-    return IM_OK;
-  }
-  return IM_ERR_UNSUPPORTED;
+  return im::newton_solve_dense_column(p, H, U, dof_union, nv, nv_pad, nM, next_world, (hipStream_t)stream, nullptr);
 }
 
 extern "C" int im_dense_update_column(const uint8_t *done, const int32_t *state_changes, const int32_t *changes,
@@ -616,3 +559,70 @@ extern "C" int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, co
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
 }
+
+namespace im {
+
+int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32_t *dof_union, int nv, int nv_pad, int nM,
+                              int32_t *next_world, hipStream_t stream, Before *before) {
+  if (!p || !H || !U || !dof_union || !next_world || p->nworld < 0 || nv <= 0 || nv_pad <= nv || nM <= 0) return IM_ERR_ARG;
+  if (nv <= 32 || (nv_pad != 48 && nv_pad != 64)) return IM_ERR_UNSUPPORTED;
+  if (p->nworld == 0) return IM_OK;
+  resident::NewtonArgs a{};
+  const int bad = resident::convert_args(*p, nv, nM, a);
+  if (bad != IM_OK) return bad;
+  const int njmax = p->njmax;
+#define IM_COLUMN_VARIANT(NBLK, WAVES, HELD) \
+  {NBLK, WAVES, HELD, (const void *)newton_dense_column_resident_kernel<NBLK, WAVES, HELD>}
+  // 48 or 64 columns; four or eight worlds per workgroup (a lane holds a whole column: up to 256 registers);
+  // the line search keeps a lane's two rows in registers up to 64 rows and reads them from LDS beyond
+  // (four first: at about 150 registers a lane a CU holds twelve wavefronts, three such workgroups or one of eight)
+  static const ColumnVariant variants[] = {IM_COLUMN_VARIANT(3, 4, 2), IM_COLUMN_VARIANT(3, 8, 2), IM_COLUMN_VARIANT(3, 4, 0),
+                                               IM_COLUMN_VARIANT(3, 8, 0), IM_COLUMN_VARIANT(4, 4, 2), IM_COLUMN_VARIANT(4, 8, 2),
+                                               IM_COLUMN_VARIANT(4, 4, 0), IM_COLUMN_VARIANT(4, 8, 0)};
+#undef IM_COLUMN_VARIANT
+  constexpr int kVariants = 8;
+  static bool usable[kVariants] = {};
+  static int regs[kVariants] = {};
+  static bool probed = false;
+  if (!probed) {  // once per process: a variant that spills registers is left out; the large dynamic LDS is asked for
+    for (int i = 0; i < kVariants; ++i) {
+      hipFuncAttributes fa{};
+      // (a variant that parks more than a register or two of its prologue in memory is left out)
+      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
+                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
+      regs[i] = fa.numRegs;
+      (void)hipGetLastError();
+    }
+    probed = true;
+  }
+  const int nblk = nv_pad / 16;
+  for (int i = 0; i < kVariants; ++i) {
+    const ColumnVariant &v = variants[i];
+    if (!usable[i] || v.nblk != nblk || v.held != (njmax <= 64 ? 2 : 0)) continue;
+    const int area = nblk == 3 ? column_resident_area_words<3>(nv, njmax) : column_resident_area_words<4>(nv, njmax);
+    const size_t per_wave = (size_t)area + resident::kept_words(nv, njmax, 0);
+    const size_t lds = 4 * ((size_t)column_resident_shared_words(p->nterm, nv) + v.waves * per_wave);
+    if (lds > 158 * 1024) continue;
+    int ncu = 0;
+    if (const int st = compute_units(&ncu)) return st;
+    // as many workgroups as stay resident at once: by LDS and by registers
+    int per_cu = 0;
+    if (const int st = resident_per_cu(v.fn, false, 64 * v.waves, lds, &per_cu)) return st;
+    per_cu = std::max(1, per_cu);
+    const int needed = (p->nworld + v.waves - 1) / v.waves;
+    const int grid = std::min(needed, ncu * per_cu);
+    if (before) {
+      a.final_force = 1;
+      if (const int st = (*before)(next_world, grid * v.waves)) return st;
+    } else {
+      set_counter(next_world, grid * v.waves, stream);
+    }
+    void *args[] = {&a, &H, &U, &dof_union, &next_world};
+    IM_HIP_CHECK(hipLaunchKernel(v.fn, dim3((unsigned)grid), dim3(64 * v.waves), args, lds, stream));
+    return IM_OK;
+  }
+  return IM_ERR_UNSUPPORTED;
+}
+
+}  // namespace im

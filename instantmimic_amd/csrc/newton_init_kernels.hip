@@ -11,6 +11,7 @@
 #include <cstdint>
 
 #include "common.h"
+#include "newton_solve.h"
 #include "newton_wave.h"
 
 namespace im {
@@ -21,7 +22,7 @@ __host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return 64
 
 __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::NewtonArgs a, const float *__restrict__ qacc_smooth,
                                                                   int64_t ld_qacc_smooth, const float *__restrict__ aref,
-                                                                  int64_t ld_aref) {
+                                                                  int64_t ld_aref, WholeSolve whole) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -33,6 +34,11 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
   int *rowl = (int *)(f + njmax);
   for (int k = threadIdx.x; k < a.nterm; k += blockDim.x) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
   for (int k = threadIdx.x; k <= nv; k += blockDim.x) radr[k] = a.mulm_rowadr[k];
+  // what the launches behind this one find set: the counter of worlds handed out, the count of worlds still solving
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (whole.counter) *whole.counter = whole.counter_value;
+    if (whole.active && a.nsolving) *a.nsolving = a.nworld;
+  }
   __syncthreads();  // the only workgroup barrier
   const int64_t w = (int64_t)blockIdx.x * 4 + wv;
   if (w >= a.nworld) return;
@@ -46,9 +52,11 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
     a.done[w] = empty ? 1 : 0;
   }
   // a world without constraint rows starts done, at the smooth acceleration
+  // (a whole solve's other worlds start where the caller says; its force without rows is zero)
   for (int k = lane; k < nv; k += 64) {
-    const float q = empty ? qacc_smooth[w * ld_qacc_smooth + k] : a.qacc[w * nv + k];
-    if (empty) a.qacc[w * nv + k] = q;
+    const float q = empty ? qacc_smooth[w * ld_qacc_smooth + k] : whole.start ? whole.start[w * whole.ld_start + k] : a.qacc[w * nv + k];
+    if (empty || whole.start) a.qacc[w * nv + k] = q;
+    if (empty && whole.active) a.qfrc_constraint[w * nv + k] = 0.0f;
     sv[k] = q;
   }
   resident::wave_sync();
@@ -117,23 +125,29 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
 }
 
 }  // namespace
+
+int newton_init_launch(const im_newton_args *p, const float *qacc_smooth, int64_t ld_qacc_smooth, const float *efc_aref,
+                       int64_t ld_aref, int nv, int nM, const WholeSolve &whole, hipStream_t stream) {
+  if (!p || !qacc_smooth || !efc_aref || p->nworld < 0 || nv <= 0 || nM <= 0) return IM_ERR_ARG;
+  if (p->nworld == 0) return IM_OK;
+  resident::NewtonArgs a{};
+  const int bad = resident::convert_args(*p, nv, nM, a);
+  if (bad != IM_OK) return bad;
+  if (ld_qacc_smooth < nv || ld_aref < p->njmax || (whole.start && whole.ld_start < nv)) return IM_ERR_STRIDE;
+  const size_t lds = 4 * ((size_t)p->nterm + nv + 1 + 4 * init_wave_words(nv, p->njmax));
+  if (lds > 160 * 1024) return IM_ERR_UNSUPPORTED;
+  if (lds > 64 * 1024)
+    IM_HIP_CHECK(hipFuncSetAttribute((const void *)newton_init_context_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)lds));
+  hipLaunchKernelGGL(newton_init_context_kernel, dim3((unsigned)((p->nworld + 3) / 4)), dim3(256), lds, stream, a, qacc_smooth,
+                     ld_qacc_smooth, efc_aref, ld_aref, whole);
+  IM_HIP_CHECK(hipGetLastError());
+  return IM_OK;
+}
+
 }  // namespace im
 
 extern "C" int im_newton_init_context(const im_newton_args *p, const float *qacc_smooth, int64_t ld_qacc_smooth,
                                       const float *efc_aref, int64_t ld_aref, int nv, int nM, void *stream) {
-  if (!p || !qacc_smooth || !efc_aref || p->nworld < 0 || nv <= 0 || nM <= 0) return IM_ERR_ARG;
-  if (p->nworld == 0) return IM_OK;
-  im::resident::NewtonArgs a{};
-  const int bad = im::resident::convert_args(*p, nv, nM, a);
-  if (bad != IM_OK) return bad;
-  if (ld_qacc_smooth < nv || ld_aref < p->njmax) return IM_ERR_STRIDE;
-  const size_t lds = 4 * ((size_t)p->nterm + nv + 1 + 4 * im::init_wave_words(nv, p->njmax));
-  if (lds > 160 * 1024) return IM_ERR_UNSUPPORTED;
-  if (lds > 64 * 1024)
-    IM_HIP_CHECK(hipFuncSetAttribute((const void *)im::newton_init_context_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds));
-  hipLaunchKernelGGL(im::newton_init_context_kernel, dim3((unsigned)((p->nworld + 3) / 4)), dim3(256), lds,
-                     (hipStream_t)stream, a, qacc_smooth, ld_qacc_smooth, efc_aref, ld_aref);
-  IM_HIP_CHECK(hipGetLastError());
-  return IM_OK;
+  return im::newton_init_launch(p, qacc_smooth, ld_qacc_smooth, efc_aref, ld_aref, nv, nM, im::WholeSolve{}, (hipStream_t)stream);
 }

@@ -1,0 +1,48 @@
+// What the launches of one whole constraint solve (im_newton_solve) share: the start, the first factor
+// stage and the resident loop, three launches on the caller's stream.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "../../include/imhip.h"
+
+namespace im {
+
+// What the launch of the start also does for a whole solve.
+struct WholeSolve {
+  const float *start = nullptr;  // (nworld, ld_start): where a world with rows starts (null: qacc as it lies there)
+  int64_t ld_start = 0;
+  int *counter = nullptr;  // the resident loop's counter of worlds handed out, set to counter_value
+  int counter_value = 0;
+  int active = 0;  // nsolving = nworld; a world without rows gets a zero constraint force
+};
+int newton_init_launch(const im_newton_args *p, const float *qacc_smooth, int64_t ld_qacc_smooth, const float *efc_aref,
+                       int64_t ld_aref, int nv, int nM, const WholeSolve &whole, hipStream_t stream);
+
+// The resident loops' launchers.  With `before`, it is called once the launch's shape is known (it issues
+// the start, which also sets `counter`, and the first factor stage); without, the counter is set by a
+// launch of its own.  A world then writes its final constraint force itself.
+struct Before {
+  virtual int operator()(int *counter, int value) = 0;
+};
+int newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, hipStream_t stream, Before *before);
+int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, float *hfactor, int32_t *dof_union,
+                        hipStream_t stream, Before *before);
+int newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_union, int nv, int nv_pad, int nM,
+                            int32_t *next_world, hipStream_t stream, Before *before);
+int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32_t *dof_union, int nv, int nv_pad, int nM,
+                              int32_t *next_world, hipStream_t stream, Before *before);
+// the tree stage of a solve's start, without the two sums (the resident loop forms them)
+int newton_tree_first(const im_tree_plan *plan, const im_newton_args *p, hipStream_t stream);
+
+// Workgroups of a kernel that a CU keeps resident, kept per (kernel, threads, LDS) after the first question:
+// the runtime's answer costs as much host time as a launch.
+int resident_per_cu(const void *fn, bool module, int threads, size_t lds, int *per_cu);
+// Compute units of the current device.
+int compute_units(int *ncu);
+// *counter = value, as a launch
+void set_counter(int *counter, int value, hipStream_t stream);
+
+}  // namespace im

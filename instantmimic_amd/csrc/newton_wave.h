@@ -50,6 +50,12 @@ struct NewtonArgs {
   // cooperative loop: whether a wavefront keeps its world's row of M in LDS (1) or reads it from
   // memory in the round's one product with it (0: the LDS saved admits another workgroup per CU)
   int m_lds;
+  // one call for the whole solve: a world that finishes writes its constraint force from the last
+  // gradient (newton_fusion.py:537-555) itself ...
+  int final_force;
+  // ... and (cooperative loop) forms the two sums of the first search direction as it enters, which
+  // a launch of their own would leave in memory
+  int sums_at_enter;
 };
 
 // The public argument block checked and turned into the kernels' (host side).
@@ -86,6 +92,8 @@ inline int convert_args(const im_newton_args &p, int nv, int nM, NewtonArgs &a) 
   a.stage_lds_floats = 0;
   a.next_world = nullptr;
   a.m_lds = 1;
+  a.final_force = 0;
+  a.sums_at_enter = 0;
   return IM_OK;
 }
 
@@ -483,6 +491,11 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
       L.D[r] = a.D[w * njmax + r];
       L.fl[r] = a.frictionloss ? a.frictionloss[w * njmax + r] : 0.0f;
     }
+    if (COOP && a.sums_at_enter) {
+      for (int k = lane_fixed; k < nv; k += 64) L.gl[k] = a.grad[w * a.ld_grad + k];
+      wave_sync();
+      search_sums_world(a, w, L.gl, sc, lane_fixed);
+    }
     wave_sync();
   };
   enter(w_raw);
@@ -647,6 +660,11 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
           if (a.nsolving) atomicAdd(a.nsolving, -1);
         }
       }
+      if (finished && a.final_force)
+        for (int k = lane; k < nv; k += 64) {
+          const float g = sc.grad_scale * a.grad[w * a.ld_grad + k];
+          a.qfrc_constraint[w * nv + k] = L.Ma[k] - a.smooth[w * nv + k] - g;
+        }
       budget -= 1;
       done = finished || budget <= 0;
     }

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "common.h"
+#include "newton_solve.h"
 #include "newton_wave.h"
 #include "sparse_plan.h"
 
@@ -982,7 +983,6 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
   }
 }
 
-__global__ void set_counter_kernel(int *counter, int value) { *counter = value; }
 
 // Per-iteration factor stage: changed rows' dof union, incremental update of packed H,
 // refactor -- or, with no changed row, a forward solve with the stored factor -- then the
@@ -1330,90 +1330,7 @@ int im_sparse_update_factor(const im_sparse_plan *plan, const uint8_t *done, con
 
 int im_newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, float *hfactor, int32_t *dof_union,
                            void *stream) {
-  if (!plan || !p || !hfactor || !dof_union || p->nworld < 0) return IM_ERR_ARG;
-  if (!plan->device_ready || plan->path != IM_SPARSE_FUSED || plan->nv > 64) return IM_ERR_UNSUPPORTED;
-  if (p->nworld == 0) return IM_OK;
-  const int n = plan->nv, njmax = p->njmax;
-  const int nM = plan->nM;
-  if (nM <= 0) return IM_ERR_UNSUPPORTED;
-  im::resident::NewtonArgs a{};
-  const int bad = im::resident::convert_args(*p, n, nM, a);
-  if (bad != IM_OK) return bad;
-  if (p->block != plan->block) return IM_ERR_ARG;
-  im::SparseWave A;
-  for (int i = 0; i < im::NHOST; ++i) A.P.t[i] = plan->t[i];
-  A.P.nv = plan->nv; A.P.nv_pad = plan->nv_pad; A.P.nslots = plan->nslots; A.P.nlevels = plan->nlevels;
-  for (int i = 0; i < im::kStaged; ++i) A.staged[i] = (int)(plan->t[i] - plan->t[0]);
-  const size_t staged = (size_t)(plan->t[im::kStaged] - plan->t[0]);
-  A.staged_words = (int)staged;
-  A.tile_index = nullptr;
-  A.block = plan->block;
-  A.nM = 0;
-  const int32_t *solve_end = plan->t[im::RK] + ((plan->sizes[im::RK] + 3) & ~3);
-  const size_t solve_words = (size_t)(solve_end - plan->t[im::FL]);
-  for (int i = 0; i < 5; ++i) A.solve[i] = (int)(plan->t[im::FL + i] - plan->t[im::FL]);
-  A.solve_words = (int)solve_words;
-  if (staged > 8192 || solve_words > 4096) return IM_ERR_UNSUPPORTED;
-  const size_t shared = staged + solve_words + (size_t)p->nterm + n + 1;
-  auto wave_words = [&](int staged_rows) {
-    return (size_t)im::resident_area_words(plan->nslots, n, plan->block, njmax, staged_rows) + im::resident::kept_words(n, njmax, 0);
-  };
-  // the most worlds per workgroup (one workgroup per CU) that 160 KB of LDS admit and whose kernel
-  // keeps to registers
-  struct Variant {
-    int waves, held;
-    const void *fn;
-  };
-  // the line search keeps a lane's two rows in registers up to 64 rows and reads them from LDS beyond
-  // (four rows a lane up to 128 rows was measured slower here: 997 against 930 us per loop at g1)
-  static const Variant variants[] = {{16, 2, (const void *)im::newton_sparse_resident_kernel<16, 2>},
-                                     {12, 2, (const void *)im::newton_sparse_resident_kernel<12, 2>},
-                                     {8, 2, (const void *)im::newton_sparse_resident_kernel<8, 2>},
-                                     {4, 2, (const void *)im::newton_sparse_resident_kernel<4, 2>},
-                                     {16, 0, (const void *)im::newton_sparse_resident_kernel<16, 0>},
-                                     {12, 0, (const void *)im::newton_sparse_resident_kernel<12, 0>},
-                                     {8, 0, (const void *)im::newton_sparse_resident_kernel<8, 0>},
-                                     {4, 0, (const void *)im::newton_sparse_resident_kernel<4, 0>}};
-  constexpr int kVariants = 8;
-  static bool usable[kVariants] = {};
-  static bool probed = false;
-  if (!probed) {  // once per process: register spills and the grant of the large dynamic LDS
-    for (int i = 0; i < kVariants; ++i) {
-      hipFuncAttributes fa{};
-      // (a variant that parks more than a few values of its prologue in memory is left out)
-      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
-                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
-      (void)hipGetLastError();
-    }
-    probed = true;
-  }
-  for (int i = 0; i < kVariants; ++i) {
-    if (!usable[i] || variants[i].held != (njmax <= 64 ? 2 : 0)) continue;
-    // 32 staged rows where the workgroup still fits with them (they cost a CU no world then), else 16
-    // (snu: 32 rows with eight worlds per CU instead of twelve was measured slower, 1344 against 1283 us per loop)
-    A.staged_rows = 4 * (shared + (size_t)variants[i].waves * wave_words(32)) <= 158 * 1024 ? 32 : 16;
-    const size_t lds = 4 * (shared + (size_t)variants[i].waves * wave_words(A.staged_rows));
-    if (lds > 158 * 1024) continue;
-    const int waves = variants[i].waves;
-    // as many workgroups as stay resident at once (LDS, and sixteen wavefronts of up to 128 registers
-    // per CU); the others' worlds are taken up by the wavefronts that finish
-    static int ncu = 0;
-    if (!ncu) {
-      int dev = 0;
-      IM_HIP_CHECK(hipGetDevice(&dev));
-      IM_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    }
-    const int per_cu = std::max(1, std::min((int)(160 * 1024 / lds), 16 / waves));
-    const int needed = (p->nworld + waves - 1) / waves;
-    const int grid = std::min(needed, std::max(ncu, 1) * per_cu);
-    int *counter = plan->next_world;
-    hipLaunchKernelGGL(im::set_counter_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, counter, grid * waves);
-    void *args[] = {&A, &a, &hfactor, &dof_union, &counter};
-    IM_HIP_CHECK(hipLaunchKernel(variants[i].fn, dim3((unsigned)grid), dim3(64 * waves), args, lds, (hipStream_t)stream));
-    return IM_OK;
-  }
-  return IM_ERR_UNSUPPORTED;
+  return im::newton_solve_sparse(plan, p, hfactor, dof_union, (hipStream_t)stream, nullptr);
 }
 
 int im_sparse_dense_factor(const im_sparse_plan *plan, const uint8_t *done, const float *grad, int ldg,
@@ -1443,3 +1360,96 @@ int im_sparse_dense_factor(const im_sparse_plan *plan, const uint8_t *done, cons
 }
 
 }  // extern "C"
+
+namespace im {
+
+int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, float *hfactor, int32_t *dof_union,
+                        hipStream_t stream, Before *before) {
+  if (!plan || !p || !hfactor || !dof_union || p->nworld < 0) return IM_ERR_ARG;
+  if (!plan->device_ready || plan->path != IM_SPARSE_FUSED || plan->nv > 64) return IM_ERR_UNSUPPORTED;
+  if (p->nworld == 0) return IM_OK;
+  const int n = plan->nv, njmax = p->njmax;
+  const int nM = plan->nM;
+  if (nM <= 0) return IM_ERR_UNSUPPORTED;
+  resident::NewtonArgs a{};
+  const int bad = resident::convert_args(*p, n, nM, a);
+  if (bad != IM_OK) return bad;
+  if (p->block != plan->block) return IM_ERR_ARG;
+  SparseWave A;
+  for (int i = 0; i < NHOST; ++i) A.P.t[i] = plan->t[i];
+  A.P.nv = plan->nv; A.P.nv_pad = plan->nv_pad; A.P.nslots = plan->nslots; A.P.nlevels = plan->nlevels;
+  for (int i = 0; i < kStaged; ++i) A.staged[i] = (int)(plan->t[i] - plan->t[0]);
+  const size_t staged = (size_t)(plan->t[kStaged] - plan->t[0]);
+  A.staged_words = (int)staged;
+  A.tile_index = nullptr;
+  A.block = plan->block;
+  A.nM = 0;
+  const int32_t *solve_end = plan->t[RK] + ((plan->sizes[RK] + 3) & ~3);
+  const size_t solve_words = (size_t)(solve_end - plan->t[FL]);
+  for (int i = 0; i < 5; ++i) A.solve[i] = (int)(plan->t[FL + i] - plan->t[FL]);
+  A.solve_words = (int)solve_words;
+  if (staged > 8192 || solve_words > 4096) return IM_ERR_UNSUPPORTED;
+  const size_t shared = staged + solve_words + (size_t)p->nterm + n + 1;
+  auto wave_words = [&](int staged_rows) {
+    return (size_t)resident_area_words(plan->nslots, n, plan->block, njmax, staged_rows) + resident::kept_words(n, njmax, 0);
+  };
+  // the most worlds per workgroup (one workgroup per CU) that 160 KB of LDS admit and whose kernel
+  // keeps to registers
+  struct Variant {
+    int waves, held;
+    const void *fn;
+  };
+  // the line search keeps a lane's two rows in registers up to 64 rows and reads them from LDS beyond
+  // (four rows a lane up to 128 rows was measured slower here: 997 against 930 us per loop at g1)
+  static const Variant variants[] = {{16, 2, (const void *)newton_sparse_resident_kernel<16, 2>},
+                                     {12, 2, (const void *)newton_sparse_resident_kernel<12, 2>},
+                                     {8, 2, (const void *)newton_sparse_resident_kernel<8, 2>},
+                                     {4, 2, (const void *)newton_sparse_resident_kernel<4, 2>},
+                                     {16, 0, (const void *)newton_sparse_resident_kernel<16, 0>},
+                                     {12, 0, (const void *)newton_sparse_resident_kernel<12, 0>},
+                                     {8, 0, (const void *)newton_sparse_resident_kernel<8, 0>},
+                                     {4, 0, (const void *)newton_sparse_resident_kernel<4, 0>}};
+  constexpr int kVariants = 8;
+  static bool usable[kVariants] = {};
+  static bool probed = false;
+  if (!probed) {  // once per process: register spills and the grant of the large dynamic LDS
+    for (int i = 0; i < kVariants; ++i) {
+      hipFuncAttributes fa{};
+      // (a variant that parks more than a few values of its prologue in memory is left out)
+      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
+                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
+      (void)hipGetLastError();
+    }
+    probed = true;
+  }
+  for (int i = 0; i < kVariants; ++i) {
+    if (!usable[i] || variants[i].held != (njmax <= 64 ? 2 : 0)) continue;
+    // 32 staged rows where the workgroup still fits with them (they cost a CU no world then), else 16
+    // (snu: 32 rows with eight worlds per CU instead of twelve was measured slower, 1344 against 1283 us per loop)
+    A.staged_rows = 4 * (shared + (size_t)variants[i].waves * wave_words(32)) <= 158 * 1024 ? 32 : 16;
+    const size_t lds = 4 * (shared + (size_t)variants[i].waves * wave_words(A.staged_rows));
+    if (lds > 158 * 1024) continue;
+    const int waves = variants[i].waves;
+    // as many workgroups as stay resident at once (LDS, and sixteen wavefronts of up to 128 registers
+    // per CU); the others' worlds are taken up by the wavefronts that finish
+    int ncu = 0;
+    if (const int st = compute_units(&ncu)) return st;
+    const int per_cu = std::max(1, std::min((int)(160 * 1024 / lds), 16 / waves));
+    const int needed = (p->nworld + waves - 1) / waves;
+    const int grid = std::min(needed, ncu * per_cu);
+    int *counter = plan->next_world;
+    if (before) {
+      a.final_force = 1;
+      if (const int st = (*before)(counter, grid * waves)) return st;
+    } else {
+      set_counter(counter, grid * waves, stream);
+    }
+    void *args[] = {&A, &a, &hfactor, &dof_union, &counter};
+    IM_HIP_CHECK(hipLaunchKernel(variants[i].fn, dim3((unsigned)grid), dim3(64 * waves), args, lds, stream));
+    return IM_OK;
+  }
+  return IM_ERR_UNSUPPORTED;
+}
+
+}  // namespace im

@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "jtdj_wave.h"
+#include "newton_solve.h"
 #include "newton_wave.h"
 #include "pivot.h"
 
@@ -515,7 +516,6 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_dense_tile_resi
   }
 }
 
-__global__ void set_dense_counter_kernel(int *counter, int value) { *counter = value; }
 
 template <int NP, int LG>
 int launch_tiles(const float *M, int64_t ld_world, int64_t ld_row, const int32_t *adr, int ntile, int size,
@@ -625,18 +625,27 @@ int im_dense_init_tile(const uint8_t *done, const int32_t *nefc, const float *J,
 
 int im_newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_union, int nv, int nv_pad, int nM,
                                int32_t *next_world, void *stream) {
+  return im::newton_solve_dense_tile(p, H, dof_union, nv, nv_pad, nM, next_world, (hipStream_t)stream, nullptr);
+}
+
+}  // extern "C"
+
+namespace im {
+
+int newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_union, int nv, int nv_pad, int nM,
+                            int32_t *next_world, hipStream_t stream, Before *before) {
   if (!p || !H || !dof_union || !next_world || p->nworld < 0 || nv <= 0 || nv_pad < nv || nM <= 0) return IM_ERR_ARG;
   if (nv > 32) return IM_ERR_UNSUPPORTED;
   if (p->nworld == 0) return IM_OK;
-  im::resident::NewtonArgs a{};
-  const int bad = im::resident::convert_args(*p, nv, nM, a);
+  resident::NewtonArgs a{};
+  const int bad = resident::convert_args(*p, nv, nM, a);
   if (bad != IM_OK) return bad;
   const int njmax = p->njmax;
   struct Variant {
     int np, waves, held;
     const void *fn;
   };
-#define IM_DENSE_VARIANT(NP, WAVES, HELD) {NP, WAVES, HELD, (const void *)im::newton_dense_tile_resident_kernel<NP, WAVES, HELD>}
+#define IM_DENSE_VARIANT(NP, WAVES, HELD) {NP, WAVES, HELD, (const void *)newton_dense_tile_resident_kernel<NP, WAVES, HELD>}
   // tile of 16 or 32 dofs; sixteen or eight worlds per workgroup; the line search keeps a lane's two
   // rows in registers up to 64 rows and reads them from LDS beyond
   static const Variant variants[] = {IM_DENSE_VARIANT(16, 16, 2), IM_DENSE_VARIANT(16, 8, 2), IM_DENSE_VARIANT(16, 16, 0),
@@ -661,26 +670,27 @@ int im_newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_u
   for (int i = 0; i < kVariants; ++i) {
     const Variant &v = variants[i];
     if (!usable[i] || v.np != np || v.held != (njmax <= 64 ? 2 : 0)) continue;
-    const int area = np == 16 ? im::dense_resident_area_words<16>(nv, njmax) : im::dense_resident_area_words<32>(nv, njmax);
-    const size_t per_wave = (size_t)area + im::resident::kept_words(nv, njmax, 0);
-    const size_t lds = 4 * ((size_t)im::dense_resident_shared_words(p->nterm, nv) + v.waves * per_wave);
+    const int area = np == 16 ? dense_resident_area_words<16>(nv, njmax) : dense_resident_area_words<32>(nv, njmax);
+    const size_t per_wave = (size_t)area + resident::kept_words(nv, njmax, 0);
+    const size_t lds = 4 * ((size_t)dense_resident_shared_words(p->nterm, nv) + v.waves * per_wave);
     if (lds > 158 * 1024) continue;
-    static int ncu = 0;
-    if (!ncu) {
-      int dev = 0;
-      IM_HIP_CHECK(hipGetDevice(&dev));
-      IM_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    }
+    int ncu = 0;
+    if (const int st = compute_units(&ncu)) return st;
     // as many workgroups as stay resident at once (LDS, and sixteen wavefronts of up to 128 registers per CU)
     const int per_cu = std::max(1, std::min((int)(160 * 1024 / lds), 16 / v.waves));
     const int needed = (p->nworld + v.waves - 1) / v.waves;
-    const int grid = std::min(needed, std::max(ncu, 1) * per_cu);
-    hipLaunchKernelGGL(im::set_dense_counter_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, next_world, grid * v.waves);
+    const int grid = std::min(needed, ncu * per_cu);
+    if (before) {
+      a.final_force = 1;
+      if (const int st = (*before)(next_world, grid * v.waves)) return st;
+    } else {
+      set_counter(next_world, grid * v.waves, stream);
+    }
     void *args[] = {&a, &H, &dof_union, &nv_pad, &next_world};
-    IM_HIP_CHECK(hipLaunchKernel(v.fn, dim3((unsigned)grid), dim3(64 * v.waves), args, lds, (hipStream_t)stream));
+    IM_HIP_CHECK(hipLaunchKernel(v.fn, dim3((unsigned)grid), dim3(64 * v.waves), args, lds, stream));
     return IM_OK;
   }
   return IM_ERR_UNSUPPORTED;
 }
 
-}  // extern "C"
+}  // namespace im

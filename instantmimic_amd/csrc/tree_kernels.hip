@@ -27,6 +27,7 @@
 #include <cstring>
 
 #include "common.h"
+#include "newton_solve.h"
 #include "tree_row16.h"
 #include <cstdlib>
 #include <vector>
@@ -610,10 +611,6 @@ int tree_plan_upload(im_tree_plan *pl) {
 
 }  // namespace im
 
-namespace im {
-__global__ void set_world_counter_kernel(int *counter, int value) { *counter = value; }
-}  // namespace im
-
 extern "C" {
 
 int im_tree_factor_solve(const im_tree_plan *plan, const float *M, int64_t ldM,
@@ -778,22 +775,35 @@ int im_newton_tree_stage(const im_tree_plan *plan, const uint8_t *skip, const fl
 }
 
 int im_newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, void *stream) {
+  return im::newton_solve_tree(plan, p, (hipStream_t)stream, nullptr);
+}
+
+}  // extern "C"
+
+namespace im {
+
+int newton_tree_first(const im_tree_plan *plan, const im_newton_args *p, hipStream_t stream) {
+  return launch(plan, true, p->M, p->ldM, p->efc_J, p->njmax, p->efc_D, p->efc_state, p->nefc, p->quad, p->grad, p->ld_grad,
+                p->search, plan->nv, nullptr, p->nworld, IM_FLAG_NEGATE, stream, Iterations(), p->search_unchanged);
+}
+
+int newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, hipStream_t stream, Before *before) {
   if (!plan || !p || p->nworld < 0) return IM_ERR_ARG;
   if (!plan->device_ready || !plan->row16) return IM_ERR_UNSUPPORTED;
-  const auto *e = (const im::gen::Row16Entry *)plan->row16;
+  const auto *e = (const gen::Row16Entry *)plan->row16;
   if (!e->newton || !e->newton_long) return IM_ERR_UNSUPPORTED;
   if (p->nworld == 0) return IM_OK;
   const int nv = plan->nv, nM = plan->nM, njmax = p->njmax;
-  im::resident::NewtonArgs a{};
-  const int bad = im::resident::convert_args(*p, nv, nM, a);
+  resident::NewtonArgs a{};
+  const int bad = resident::convert_args(*p, nv, nM, a);
   if (bad != IM_OK) return bad;
   // the factor stage's LDS (its staged tiles and exchange slots plus the four worlds' row lists), or the
   // four wavefronts' staged rows of J where those take more; the loop's own arrays behind it
   const size_t stage_bytes = (size_t)e->lds_bytes + 32 * std::max<size_t>(((size_t)njmax + 15) / 16 * 16, 64);
-  const size_t stage_words = std::max(stage_bytes / 4, im::resident::staged_rows_words(nv));
+  const size_t stage_words = std::max(stage_bytes / 4, resident::staged_rows_words(nv));
   a.stage_lds_floats = (int)stage_words;
-  size_t lds = 4 * (stage_words + im::resident::loop_lds_words(nv, njmax, nM, p->nterm));
-  const size_t lds_lean = 4 * (stage_words + im::resident::loop_lds_words(nv, njmax, 0, p->nterm));
+  size_t lds = 4 * (stage_words + resident::loop_lds_words(nv, njmax, nM, p->nterm));
+  const size_t lds_lean = 4 * (stage_words + resident::loop_lds_words(nv, njmax, 0, p->nterm));
   if (lds_lean > 160 * 1024) return IM_ERR_UNSUPPORTED;
   const bool is_long = njmax > e->short_rows;
   if (!(is_long ? plan->resident_long_ok : plan->resident_ok)) return IM_ERR_UNSUPPORTED;  // the kernel spills registers
@@ -801,13 +811,9 @@ int im_newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, void
   // As many workgroups as the chip keeps resident (registers and LDS); a wavefront whose world is
   // done takes the next world through the plan's counter, so the worlds that need many iterations
   // do not hold three idle wavefronts in place.
-  auto resident_per_cu = [&](size_t bytes, int *per_cu) {
-    if (plan->module) return hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (hipFunction_t)fn, 256, bytes);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, fn, 256, bytes);
-  };
   int per_cu = 0, per_cu_lean = 0;
-  if (lds <= 160 * 1024) IM_HIP_CHECK(resident_per_cu(lds, &per_cu));
-  IM_HIP_CHECK(resident_per_cu(lds_lean, &per_cu_lean));
+  if (lds <= 160 * 1024) if (const int st = resident_per_cu(fn, plan->module != nullptr, 256, lds, &per_cu)) return st;
+  if (const int st = resident_per_cu(fn, plan->module != nullptr, 256, lds_lean, &per_cu_lean)) return st;
   // the worlds' rows of M stay in LDS unless leaving them in memory admits another workgroup per CU
   // (snu: 81 KB a workgroup with them, one per CU; 70 KB without, two)
   if (per_cu_lean > per_cu) {
@@ -815,25 +821,25 @@ int im_newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, void
     lds = lds_lean;
     per_cu = per_cu_lean;
   }
-  static int ncu = 0;
-  if (!ncu) {
-    int dev = 0;
-    IM_HIP_CHECK(hipGetDevice(&dev));
-    IM_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  }
+  int ncu = 0;
+  if (const int st = compute_units(&ncu)) return st;
   const int needed = (p->nworld + 3) / 4;
-  const unsigned grid = (unsigned)std::min(needed, std::max(1, per_cu) * std::max(1, ncu));
-  if ((int)grid < needed) {  // (a batch that is resident all at once has nothing to hand out)
-    a.next_world = plan->next_world;
-    hipLaunchKernelGGL(im::set_world_counter_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, plan->next_world, (int)grid * 4);
+  const unsigned grid = (unsigned)std::min(needed, std::max(1, per_cu) * ncu);
+  // (a batch that is resident all at once has nothing to hand out)
+  if ((int)grid < needed) a.next_world = plan->next_world;
+  if (before) {
+    a.final_force = a.sums_at_enter = 1;
+    if (const int st = (*before)(a.next_world, (int)grid * 4)) return st;
+  } else if (a.next_world) {
+    set_counter(a.next_world, (int)grid * 4, stream);
   }
   void *args[] = {&a};
   if (plan->module)
-    IM_HIP_CHECK(hipModuleLaunchKernel((hipFunction_t)fn, grid, 1, 1, 256, 1, 1, (unsigned)lds, (hipStream_t)stream, args,
+    IM_HIP_CHECK(hipModuleLaunchKernel((hipFunction_t)fn, grid, 1, 1, 256, 1, 1, (unsigned)lds, stream, args,
                                        nullptr));
   else
-    IM_HIP_CHECK(hipLaunchKernel(fn, dim3(grid), dim3(256), args, lds, (hipStream_t)stream));
+    IM_HIP_CHECK(hipLaunchKernel(fn, dim3(grid), dim3(256), args, lds, stream));
   return IM_OK;
 }
 
-}  // extern "C"
+}  // namespace im

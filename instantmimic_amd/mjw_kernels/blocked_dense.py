@@ -102,10 +102,16 @@ def _blocked_dense_factor_solve(
     """x = M^-1 y; the upper factor is left in ``scratch.U`` (or ``factor_workspace``) and, with
     ``factor_out``, copied into the caller's dense-block factor array at ``qLD_block_adr[0]``
     (:958-993)."""
-    import torch
-
     nworld = int(d.nworld)
     workspace = scratch.U if factor_workspace is None else factor_workspace
+    if factor_out is None:
+        status = _lib.native().blocked_factor_solve(nworld, scratch.nv, scratch.pad, scratch.block_size, scratch.nM, scratch.indices, workspace, M, x, y)
+        if status is None:
+            return
+        if status > 0:
+            _lib.check(status, "im_blocked_factor_solve")
+    import torch
+
     for t in (M, x, y, workspace):
         if t.dtype != torch.float32 or not t.is_cuda or t.stride(-1) != 1 or t.device != M.device:
             raise ValueError("blocked factor needs float32 CUDA tensors with contiguous rows on one device")
@@ -388,6 +394,11 @@ def dense_hessian_factor_solve(M_dense, J, D, state, nefc, H, y, x, *, factor=No
     ``H`` (nworld, nv_pad, nv_pad) or None, ``x = H^-1 y`` (nworld, nv), ``factor`` (nworld, pad,
     pad) with ``pad`` = nv rounded up to 16, or None.  Bit for bit what :func:`dense_hessian`
     followed by :func:`_blocked_dense_factor_solve` on the whole H gives."""
+    status = _lib.native().dense_hessian_factor_solve(M_dense, J, D, state, nefc, H, y, x, factor, quad)
+    if status is None:
+        return
+    if status > 0:
+        _lib.check(status, "im_jtdj_factor_solve")
     import torch
 
     nworld, njmax, nv = J.shape

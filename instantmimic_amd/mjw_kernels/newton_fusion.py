@@ -787,12 +787,18 @@ def _resident_args(m, d, ctx, nsolving):
     return a
 
 
-def run_resident(m, d, ctx, nsolving) -> bool:
+def run_resident(m, d, ctx, nsolving, whole: bool = False) -> bool:
     """The whole loop as one resident kernel (a wavefront per world until it is done): for a ``ctx``
     with a fused sparse plan, with the tree stage whose plan carries generated kernels, or for a
     dense model of up to 63 dofs (the single-tile stage up to 32, the blocked stage on a wavefront
     per world for a padded size of 48 or 64).  False when there is no such kernel for
-    this model (the caller then launches the stages one by one)."""
+    this model (the caller then launches the stages one by one).  ``whole``: the start of the solve, the
+    first factor and the constraint force around the loop as well, in one native call."""
+    if whole:
+        status = _lib.native().newton_solve(m, d, ctx, nsolving, DISABLE_WARMSTART, OVERFLOW_LS_ITERATIONS, OVERFLOW_ITERATIONS)
+        if status is not None and status > 0:
+            _lib.check(status, "im_newton_solve")
+        return status is None
     import ctypes as C
 
     import torch
@@ -893,7 +899,11 @@ def solve(m, d, ctx, nsolving, *, mul_m_call=None) -> None:
     """The constraint solve around the fused loop, in the order of ``_solve_monolithic_with_scratch``
     for an eligible model (src/instantmimic/utils/mjw_step_optimized.py:2588-2683): the start point
     (warm start unless disabled), ``init_context``, the loop, the constraint force from the last
-    gradient.  No step reads anything back, so the whole solve can sit in a caller's graph."""
+    gradient.  No step reads anything back, so the whole solve can sit in a caller's graph.  With a
+    resident loop for the model the solve is one native call of three launches (``im_newton_solve``);
+    otherwise the pieces below."""
+    if mul_m_call is None and run_resident(m, d, ctx, nsolving, True):
+        return
     flags = getattr(m.opt, "disableflags", 0)
     warmstart = not (int(flags) & DISABLE_WARMSTART) and getattr(d, "qacc_warmstart", None) is not None
     d.qacc.copy_(d.qacc_warmstart if warmstart else d.qacc_smooth)

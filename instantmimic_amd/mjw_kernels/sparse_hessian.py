@@ -187,6 +187,7 @@ class SparseHessianPlan:
 
     def __init__(self, ptr, on_device: bool):
         self.ptr = ptr
+        self.address = ptr.value
         info = _lib.SparsePlanInfo()
         _lib.check(_lib.lib().im_sparse_plan_get_info(ptr, C.byref(info)), "im_sparse_plan_get_info")
         self.nv, self.nv_pad, self.block = int(info.nv), int(info.nv_pad), int(info.block)

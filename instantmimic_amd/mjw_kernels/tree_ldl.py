@@ -51,6 +51,8 @@ class _PlanHandle:
         )  # fmt: skip
         _lib.check(status, "im_tree_plan_create")
         self.ptr = handle
+        self.address = handle.value  # what the native host path takes, with the plan's sizes beside it
+        self.nv, self.nM = int(rowadr.size), int(colind.size)
         self.structure = tuple(tuple(int(v) for v in a) for a in (rowadr, rownnz, colind))
 
     def __del__(self):
@@ -223,6 +225,12 @@ def _check_against_plan(scratch, M, x, y, others=()) -> int:
 def tree_factor_solve(scratch: TreeFactorSolveScratch, M, x, y) -> None:
     """x = M^-1 y for an M in the model's CSR layout (argument order of the
     reference: scratch, M, x, y)."""
+    plan = scratch.kernel
+    status = _lib.native().tree_factor_solve(plan.address, plan.nv, plan.nM, M, x, y)
+    if status is None:
+        return
+    if status > 0:
+        _lib.check(status, "im_tree_factor_solve")
     import torch
 
     _check_rows(M, x, y)
@@ -248,6 +256,13 @@ def assemble_tree_factor_solve(
     ``J`` (nworld, njmax, nv), ``D``/``state`` (nworld, njmax), ``nefc`` (nworld)
     int32 or ``None``; rows at or beyond ``nefc[w]`` are ignored.
     """
+    if H_out is None:
+        plan = scratch.kernel
+        status = _lib.native().assemble_tree_factor_solve(plan.address, plan.nv, plan.nM, M, J, D, state, nefc, grad, x, negate, quad)
+        if status is None:
+            return
+        if status > 0:
+            _lib.check(status, "im_assemble_tree_ldl_solve")
     import torch
 
     _check_rows(M, x, grad)
