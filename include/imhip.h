@@ -354,8 +354,8 @@ int im_dense_update_factor(const uint8_t *done, const int32_t *state_changes,
                            int nv_pad, int32_t *dof_union, float *search, int64_t ld_search,
                            float *search_dot, float *decrement, int nworld, void *stream);
 
-/* The same stage for nv_pad = 48 or 64 (33 to 63 dofs) on one wavefront per world, a lane per
- * column of the padded matrix: same arguments, same results bit for bit; im_dense_update_factor
+/* The same stage for nv_pad = 48, 64 or 80 (33 to 79 dofs, nv >= nv_pad - 16) on one wavefront per world, in the
+ * wavefront's matrix-core tiles: same arguments, same results bit for bit; im_dense_update_factor
  * hands such shapes here.  IM_ERR_UNSUPPORTED for other paddings. */
 int im_dense_update_column(const uint8_t *done, const int32_t *state_changes, const int32_t *changes,
                            const int32_t *ids, int ld_ids, const float *J, int njmax, const float *D,
@@ -373,7 +373,7 @@ int im_dense_update_column(const uint8_t *done, const int32_t *state_changes, co
  * of a row of M at every pair of dofs, negative outside its pattern (the layout of the reference's
  * m.M_elemid).  nefc may be null (every world has njmax rows).  Same results, bit for bit, as
  * im_dense_from_csr, im_jtdj_mfma and im_dense_update_factor one after the other.  nv <= 32 (any
- * nv_pad that is a multiple of four; U may be null) or nv_pad = 48 or 64; IM_ERR_UNSUPPORTED
+ * nv_pad that is a multiple of four; U may be null) or nv_pad = 48, 64 or 80; IM_ERR_UNSUPPORTED
  * otherwise: the caller then issues the three launches.  H must be 16-byte aligned. */
 int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float *D,
                          const int32_t *state, int quad, const float *M, int64_t ldM, const int32_t *elemid,
@@ -1039,9 +1039,9 @@ int im_newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *arg
 int im_newton_solve_dense_tile(const im_newton_args *args, float *H, int32_t *dof_union, int nv, int nv_pad, int nM,
                                int32_t *next_world, void *stream);
 
-/* The same for a dense model of 33 to 63 dofs with nv_pad = 48 or 64, whose factor stage is the
+/* The same for a dense model of 33 to 79 dofs with nv_pad = 48, 64 or 80, whose factor stage is the
  * augmented blocked Cholesky (newton_stages.py:473-611, 614-742) run as im_dense_update_column
- * runs it, a wavefront per world with a lane per column.  U: ctx.hfactor, (nworld, nv_pad, nv_pad).
+ * runs it, a wavefront per world.  U: ctx.hfactor, (nworld, nv_pad, nv_pad).
  * IM_ERR_UNSUPPORTED for other shapes. */
 int im_newton_solve_dense_column(const im_newton_args *args, float *H, float *U, int32_t *dof_union, int nv, int nv_pad,
                                  int nM, int32_t *next_world, void *stream);

@@ -1,5 +1,5 @@
-// H = M + J' diag(D [state == quad]) J of one world on one wavefront, for up to four 16-column
-// blocks (the first Hessian of a dense Newton solve below 64 dofs), and the store of a lane's share
+// H = M + J' diag(D [state == quad]) J of one world on one wavefront, for up to five 16-column
+// blocks (the first Hessian of a dense Newton solve up to 79 dofs), and the store of a lane's share
 // of a 16 x 16 accumulator tile into H and its mirror image.
 // Reference: upstream's solver._update_gradient as src/instantmimic/utils/mjw_kernels/newton_fusion.py:470
 // calls it (the dense Newton's full assembly ahead of the first factor).
@@ -39,19 +39,20 @@ __device__ __forceinline__ void store_h_mirrored(float *__restrict__ Hw, int nv,
 // of v_mfma_f32_16x16x4_f32 (lane l supplies row 4 q + l / 16, column 16 b + l % 16 of step q: four
 // rows of 64 bytes per load), the next sixteen rows' loads in flight behind the current ones'
 // products; nothing is staged.
-template <int NB>
+// The tiles stay in `acc` (upper block triangle, row by row); STEPS: steps whose operands are in flight.
+template <int NB, int STEPS = 4>
 __device__ __forceinline__ void jtdj_wave(const float *__restrict__ Mw, const int32_t *__restrict__ elemid,
                                           const float *__restrict__ Jw, const float *__restrict__ Dw,
                                           const int32_t *__restrict__ sw, int nefc, int quad, int nv,
-                                          float *__restrict__ Hw, int pad, bool vec, int lane) {
-  constexpr int NT = NB * (NB + 1) / 2;
+                                          float *__restrict__ Hw, int pad, bool vec, int lane,
+                                          float4v (&acc)[NB * (NB + 1) / 2]) {
   const int c = lane & 15, kq = lane >> 4;
   const int nstep = (nefc + 3) >> 2;
-  float u[4][NB], dk[4], un[4][NB], dn[4];
-  // the operands of four steps (sixteen rows): asked for a group ahead of the products that use them
-  auto fetch = [&](int q0, float (&uu)[4][NB], float (&dd)[4]) __attribute__((always_inline)) {
+  float u[STEPS][NB], dk[STEPS], un[STEPS][NB], dn[STEPS];
+  // the operands of STEPS steps (four rows each): asked for a group ahead of the products that use them
+  auto fetch = [&](int q0, float (&uu)[STEPS][NB], float (&dd)[STEPS]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < STEPS; ++s) {
       const int row = 4 * (q0 + s) + kq;
       const bool in = row < nefc;
       const int rowc = in ? row : nefc - 1;
@@ -67,7 +68,6 @@ __device__ __forceinline__ void jtdj_wave(const float *__restrict__ Mw, const in
     }
   };
   if (nstep > 0) fetch(0, u, dk);  // on their way while M is gathered
-  float4v acc[NT];
   {  // the accumulators start from M (a lane holds column j = l % 16 and rows 4 (l / 16) + v of a tile)
     int m = 0;
 #pragma unroll
@@ -84,10 +84,10 @@ __device__ __forceinline__ void jtdj_wave(const float *__restrict__ Mw, const in
         }
       }
   }
-  for (int q0 = 0; q0 < nstep; q0 += 4) {
-    if (q0 + 4 < nstep) fetch(q0 + 4, un, dn);
+  for (int q0 = 0; q0 < nstep; q0 += STEPS) {
+    if (q0 + STEPS < nstep) fetch(q0 + STEPS, un, dn);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < STEPS; ++s) {
       float wt[NB];
 #pragma unroll
       for (int b = 0; b < NB; ++b) wt[b] = u[s][b] * dk[s];
@@ -99,7 +99,7 @@ __device__ __forceinline__ void jtdj_wave(const float *__restrict__ Mw, const in
           acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[bi], u[s][bj], acc[m], 0, 0, 0);
     }
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < STEPS; ++s) {
       dk[s] = dn[s];
 #pragma unroll
       for (int b = 0; b < NB; ++b) u[s][b] = un[s][b];

@@ -434,8 +434,9 @@ __global__ __launch_bounds__(256) void dense_init_tile_kernel(
   nefc = nefc < njmax ? nefc : njmax;
   float *Hw = H_ + w * (int64_t)pad * pad;
   const float *Jw = J + w * (int64_t)njmax * nv;
+  float4v tiles[(NP + 15) / 16 * ((NP + 15) / 16 + 1) / 2];
   jtdj_wave<(NP + 15) / 16>(M + w * ldM, elemid, Jw, D + w * njmax, state + w * njmax, nefc, quad, nv, Hw, pad,
-                            (pad & 3) == 0, lane);
+                            (pad & 3) == 0, lane, tiles);
   if (done && done[w]) return;
   // the lanes read back one another's stores (one CU: its vector cache sees them once they are issued and waited for)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

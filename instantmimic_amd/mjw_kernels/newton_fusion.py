@@ -613,7 +613,7 @@ def _update_gradient(m, d, ctx, *, gradient_done: bool = False) -> None:
         raise RuntimeError("the dense first factor needs attach_scratch(m, d, ctx)")
     if not gradient_done:
         _first_gradient(m, d, ctx)
-    # one launch where the shape has one (up to 63 dofs); IMHIP_NEWTON=stages keeps the three
+    # one launch where the shape has one (up to 79 dofs); IMHIP_NEWTON=stages keeps the three
     if os.environ.get("IMHIP_NEWTON") != "stages" and blocked_dense.dense_init_factor(
             d.M, ctx.newton_elemid, d.efc.J, d.efc.D, d.efc.state, d.nefc, ctx.done, ctx.grad, ctx.h, ctx.hfactor, ctx.search,
             ctx.search_dot, ctx.newton_decrement, ctx.newton_dof_union):  # fmt: skip
@@ -790,8 +790,8 @@ def _resident_args(m, d, ctx, nsolving):
 def run_resident(m, d, ctx, nsolving, whole: bool = False) -> bool:
     """The whole loop as one resident kernel (a wavefront per world until it is done): for a ``ctx``
     with a fused sparse plan, with the tree stage whose plan carries generated kernels, or for a
-    dense model of up to 63 dofs (the single-tile stage up to 32, the blocked stage on a wavefront
-    per world for a padded size of 48 or 64).  False when there is no such kernel for
+    dense model of up to 79 dofs (the single-tile stage up to 32, the blocked stage on a wavefront
+    per world for a padded size of 48, 64 or 80).  False when there is no such kernel for
     this model (the caller then launches the stages one by one).  ``whole``: the start of the solve, the
     first factor and the constraint force around the loop as well, in one native call."""
     if whole:
@@ -806,7 +806,7 @@ def run_resident(m, d, ctx, nsolving, whole: bool = False) -> bool:
     scratch, plan = _tree_scratch(ctx), _fused_plan(ctx)
     dense = scratch is None and plan is None and getattr(ctx, "newton_next_world", None) is not None
     dense_tile = dense and int(m.nv) <= 32
-    dense_column = dense and int(m.nv) > 32 and int(m.nv_pad) in (48, 64)
+    dense_column = dense and int(m.nv) > 32 and int(m.nv_pad) in (48, 64, 80)
     if (scratch is None and plan is None and not (dense_tile or dense_column)) or os.environ.get("IMHIP_NEWTON") == "stages":
         return False
     a = _resident_args(m, d, ctx, nsolving)
