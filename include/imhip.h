@@ -373,7 +373,7 @@ int im_dense_update_column(const uint8_t *done, const int32_t *state_changes, co
  * of a row of M at every pair of dofs, negative outside its pattern (the layout of the reference's
  * m.M_elemid).  nefc may be null (every world has njmax rows).  Same results, bit for bit, as
  * im_dense_from_csr, im_jtdj_mfma and im_dense_update_factor one after the other.  nv <= 32 (any
- * nv_pad that is a multiple of four; U may be null) or nv_pad = 48, 64 or 80; IM_ERR_UNSUPPORTED
+ * nv_pad that is a multiple of four; U may be null) or nv_pad = 48 or 64; IM_ERR_UNSUPPORTED
  * otherwise: the caller then issues the three launches.  H must be 16-byte aligned. */
 int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float *D,
                          const int32_t *state, int quad, const float *M, int64_t ldM, const int32_t *elemid,

@@ -177,11 +177,10 @@ extern "C" int im_dense_init_tile(const uint8_t *done, const int32_t *nefc, cons
                                   float *search, int64_t ld_search, float *search_dot, float *decrement, int nworld,
                                   void *stream);
 
-extern "C" int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float *D,
-                                    const int32_t *state, int quad, const float *M, int64_t ldM, const int32_t *elemid,
-                                    const float *grad, int64_t ldg, float *H, float *U, int nv, int nv_pad,
-                                    int32_t *dof_union, float *search, int64_t ld_search, float *search_dot,
-                                    float *decrement, int nworld, void *stream) {
+static int init_factor(int most, const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float *D,
+                       const int32_t *state, int quad, const float *M, int64_t ldM, const int32_t *elemid, const float
+                       *grad, int64_t ldg, float *H, float *U, int nv, int nv_pad, int32_t *dof_union, float *search,
+                       int64_t ld_search, float *search_dot, float *decrement, int nworld, void *stream) {
   if (nworld < 0 || nv <= 0 || nv_pad < nv || njmax <= 0) return IM_ERR_ARG;
   if (nworld == 0) return IM_OK;
   if (!J || !D || !state || !M || !elemid || !grad || !H || !dof_union || !search || !search_dot || !decrement)
@@ -191,7 +190,7 @@ extern "C" int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, co
     return im_dense_init_tile(done, nefc, J, njmax, D, state, quad, M, ldM, elemid, grad, ldg, H, nv, nv_pad, dof_union,
                               search, ld_search, search_dot, decrement, nworld, stream);
   if (!U) return IM_ERR_ARG;
-  if (!im::wave_shape(nv, nv_pad)) return IM_ERR_UNSUPPORTED;
+  if (!im::wave_shape(nv, nv_pad) || nv_pad > most) return IM_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)((nworld + 3) / 4)), wg(256);
 #define IM_INIT_WAVE(NB)                                                                                                      \
   hipLaunchKernelGGL(im::dense_init_wave_kernel<NB>, grid, wg, 16 * im::wave_stage_words<NB>(), (hipStream_t)stream, done,    \
@@ -205,7 +204,24 @@ extern "C" int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, co
   return IM_OK;
 }
 
+extern "C" int im_dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float
+                                    *D, const int32_t *state, int quad, const float *M, int64_t ldM, const int32_t
+                                    *elemid, const float *grad, int64_t ldg, float *H, float *U, int nv, int nv_pad,
+                                    int32_t *dof_union, float *search, int64_t ld_search, float *search_dot, float
+                                    *decrement, int nworld, void *stream) {
+  return init_factor(64, done, nefc, J, njmax, D, state, quad, M, ldM, elemid, grad, ldg, H, U, nv, nv_pad, dof_union,
+                     search, ld_search, search_dot, decrement, nworld, stream);
+}
+
 namespace im {
+
+int dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float *D, const
+                      int32_t *state, int quad, const float *M, int64_t ldM, const int32_t *elemid, const float *grad,
+                      int64_t ldg, float *H, float *U, int nv, int nv_pad, int32_t *dof_union, float *search, int64_t
+                      ld_search, float *search_dot, float *decrement, int nworld, void *stream) {
+  return init_factor(80, done, nefc, J, njmax, D, state, quad, M, ldM, elemid, grad, ldg, H, U, nv, nv_pad, dof_union,
+                     search, ld_search, search_dot, decrement, nworld, stream);
+}
 
 int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32_t *dof_union, int nv, int nv_pad, int nM,
                               int32_t *next_world, hipStream_t stream, Before *before) {

@@ -34,6 +34,11 @@ int newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_unio
                             int32_t *next_world, hipStream_t stream, Before *before);
 int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32_t *dof_union, int nv, int nv_pad, int nM,
                               int32_t *next_world, hipStream_t stream, Before *before);
+// im_dense_init_factor, and with 80 columns as well, which that entry point leaves to three launches
+int dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, int njmax, const float *D, const
+                      int32_t *state, int quad, const float *M, int64_t ldM, const int32_t *elemid, const float *grad,
+                      int64_t ldg, float *H, float *U, int nv, int nv_pad, int32_t *dof_union, float *search, int64_t
+                      ld_search, float *search_dot, float *decrement, int nworld, void *stream);
 // the tree stage of a solve's start, without the two sums (the resident loop forms them)
 int newton_tree_first(const im_tree_plan *plan, const im_newton_args *p, hipStream_t stream);
 

@@ -74,7 +74,7 @@ struct FirstStage : Before {
       return im_sparse_init_factor(m->sparse, p->done, p->nefc, p->efc_J, p->njmax, p->efc_D, p->efc_state, p->quad, p->M,
                                    (int)p->ldM, p->grad, (int)p->ld_grad, m->U, p->search, p->search_dot, p->newton_decrement,
                                    p->nworld, stream);
-    return im_dense_init_factor(p->done, p->nefc, p->efc_J, p->njmax, p->efc_D, p->efc_state, p->quad, p->M, p->ldM, m->elemid,
+    return dense_init_factor(p->done, p->nefc, p->efc_J, p->njmax, p->efc_D, p->efc_state, p->quad, p->M, p->ldM, m->elemid,
                                 p->grad, p->ld_grad, m->H, m->U, m->nv, m->nv_pad, m->dof_union, p->search, m->nv, p->search_dot,
                                 p->newton_decrement, p->nworld, stream);
   }

@@ -347,13 +347,13 @@ def dense_init_factor(M, elemid, J, D, state, nefc, done, grad, H, U, search, se
     ``elemid`` (nv, nv), then for the worlds that are not ``done`` the dense stage without changed
     rows (factor into ``U`` above 32 dofs, solve for ``grad``, ``search``, ``search_dot``,
     ``decrement``, an empty ``dof_union``).  Returns False, with nothing launched, for a shape
-    the launch does not take (80 dofs and more) or arrays it cannot address; the caller then issues
+    the launch does not take (64 dofs and more) or arrays it cannot address; the caller then issues
     ``dense_from_csr``, :func:`dense_hessian` and the stage."""
     import torch
 
     nworld, njmax, nv = J.shape
     pad = int(H.shape[1])
-    if nv > 32 and pad not in (48, 64, 80):
+    if nv > 32 and pad not in (48, 64):
         return False
     tensors = dict(M=M, J=J, D=D, state=state, grad=grad, H=H, U=U, search=search, search_dot=search_dot, decrement=decrement)
     for name, t in tensors.items():
