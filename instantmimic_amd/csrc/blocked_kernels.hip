@@ -18,6 +18,7 @@
 #include <cstring>
 
 #include "common.h"
+#include "dense_solve.h"
 #include "jtdj_wave.h"
 #include "pivot.h"
 
@@ -655,232 +656,11 @@ __global__ __launch_bounds__(256, 4) void blocked_factor_solve_kernel(
     }
 }
 
-// ---- matrices up to 64 x 64: four worlds per wavefront ----------------------------------------
-// With a wavefront per world most of the factor runs on 8 or 16 of 64 lanes (the pivots of a tile,
-// its triangular solves, the right-hand side), and the SIMDs spend their issue slots on idle
-// lanes.  Here a world has a DPP row of 16 lanes and a wavefront carries four worlds through
-// the same instructions; the only synchronisation is within the wavefront.  U keeps the tiles
-// on or above the diagonal only, tile (bi, bj) at B B (bi nblk - bi (bi - 1) / 2 + bj - bi).
-// Every element sees the operations of blocked_factor_solve_kernel<B> in the same order.
+// LDS written by some lanes of a wavefront, then read by others
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-__host__ __device__ inline int quad_tiles_before(int bi, int nblk) { return bi * nblk - bi * (bi - 1) / 2; }
-// floats of LDS per world: tiles (a block row is updated in place), right-hand side, the
-// diagonal tile's lower factor and reciprocal pivots; rounded so that the four worlds start 8 banks apart
-__host__ __device__ inline int quad_world_floats(int pad, int B) {
-  const int nblk = pad / B;
-  const int need = B * B * quad_tiles_before(nblk, nblk) + pad + B * B + B;
-  return (need + 31) / 32 * 32 + 8;
-}
-
-template <int B>
-__global__ __launch_bounds__(64) void blocked_factor_solve_quad_kernel(
-    const float *__restrict__ M, int64_t ldM, int nM, const int32_t *__restrict__ block_idx,
-    const float *__restrict__ y, int64_t ldy, float *__restrict__ Uout, float *__restrict__ x,
-    int64_t ldx, int nv, int pad, int nworld, const int32_t *__restrict__ active) {
-  extern __shared__ float lds[];
-  constexpr int BB = B * B, PER = BB / 16;  // a lane's elements of a tile: e = l + 16 u
-  const int lane = threadIdx.x, l = lane & 15, q = lane >> 4;
-  const int nblk = pad / B, ntiles = quad_tiles_before(nblk, nblk);
-  const int64_t w_raw = (int64_t)blockIdx.x * 4 + q;
-  // an inactive world rides along like a spare row: computed, nothing stored
-  const bool live = w_raw < nworld && (!active || active[w_raw] != 0);
-  const int64_t w = w_raw < nworld ? w_raw : (int64_t)nworld - 1;  // a spare row repeats the last world and stores nothing
-  const int world_floats = quad_world_floats(pad, B);
-  float *U = lds + q * world_floats;
-  float *rhs = U + BB * ntiles;  // [pad]
-  float *L = rhs + pad;          // [BB + B]
-  auto tile = [&](int bi, int bj) { return U + BB * (quad_tiles_before(bi, nblk) + bj - bi); };
-  const float *Mw = M + w * ldM;
-  {
-    // indexed gather, four tiles in flight
-    int kb = 0, ib = 0;
-    for (int t0 = 0; t0 < ntiles; t0 += 4) {
-      int tk[4], ti[4], idx[4][PER];
-      float v[4][PER];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        tk[g] = kb < nblk ? kb : -1;
-        ti[g] = ib;
-        if (kb < nblk && ++ib == nblk) { ++kb; ib = kb; }
-      }
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-          const int e = l + 16 * u;
-          idx[g][u] = block_idx[tk[g] >= 0 ? (size_t)(tk[g] * nblk + ti[g]) * BB + e : 0];
-          if (tk[g] < 0) idx[g][u] = nM;
-        }
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int u = 0; u < PER; ++u) v[g][u] = Mw[idx[g][u] < nM ? idx[g][u] : 0];
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int u = 0; u < PER; ++u)
-          if (tk[g] >= 0) {
-            const int e = l + 16 * u, r = e / B, c = e % B;
-            float xv = idx[g][u] < nM ? v[g][u] : 0.0f;
-            if (ti[g] == tk[g] && (tk[g] + 1) * B > nv && r == c && (nblk - 1) * B + r >= nv) xv = xv + 1.0f;
-            U[BB * (t0 + g) + e] = xv;
-          }
-    }
-  }
-  for (int i = l; i < pad; i += 16) rhs[i] = (y && i < nv) ? y[w * ldy + i] : 0.0f;
-  wave_sync();
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  typedef float f32x16 __attribute__((ext_vector_type(16)));
-  const int m4 = l & 3, qr = l >> 3, qc = (l >> 2) & 1;  // B = 8: the lane within quadrant (qr, qc) of a tile
-  for (int kb = 0; kb < nblk; ++kb) {
-    const int k = kb * B, ntile = nblk - kb;
-    // The sums over a finished block row on the matrix cores, with instructions that do one
-    // fused multiply-add per element and step: chained from zero over t ascending they are
-    // the scalar sums bit for bit.
-    for (int tb = 0; tb < ntile; ++tb) {
-      const int ib = kb + tb;
-      if constexpr (B == 8) {
-        // v_mfma_f32_4x4x1_16b_f32: sixteen independent 4 x 4 blocks, the four quadrants of one
-        // 8 x 8 tile of each of the four worlds
-        float *Tv = tile(kb, ib) + (4 * qr) * B + 4 * qc + m4;  // rows 4 qr + 0..3 of column 4 qc + m4
-        f32x4 v;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = Tv[u * B];
-        for (int jb = 0; jb < kb; ++jb) {
-          const float *Tk = tile(jb, kb) + 4 * qr + m4, *Ti = tile(jb, ib) + 4 * qc + m4;
-          f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int t = 0; t < B; ++t) sum = __builtin_amdgcn_mfma_f32_4x4x1f32(Tk[t * B], Ti[t * B], sum, 0, 0, 0);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] = v[u] - sum[u];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) Tv[u * B] = v[u];  // in place: nothing else reads this tile before
-      } else {
-        // v_mfma_f32_16x16x1_4b_f32: four independent 16 x 16 blocks, one per world.  Block b takes
-        // its operands from the lanes of world b and leaves its result in registers 4 b .. 4 b + 3
-        // of every lane: rows 4 (lane / 16) + 0..3 of column lane % 16.
-        const int toff = (int)(tile(kb, ib) - U) + (4 * q) * B + l;
-        f32x16 v;
-#pragma unroll
-        for (int wb = 0; wb < 4; ++wb)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[4 * wb + u] = lds[wb * world_floats + toff + u * B];
-        for (int jb = 0; jb < kb; ++jb) {
-          const float *Tk = tile(jb, kb) + l, *Ti = tile(jb, ib) + l;
-          f32x16 sum;
-#pragma unroll
-          for (int u = 0; u < 16; ++u) sum[u] = 0.0f;
-#pragma unroll
-          for (int t = 0; t < B; ++t) sum = __builtin_amdgcn_mfma_f32_16x16x1f32(Tk[t * B], Ti[t * B], sum, 0, 0, 0);
-#pragma unroll
-          for (int u = 0; u < 16; ++u) v[u] = v[u] - sum[u];
-        }
-#pragma unroll
-        for (int wb = 0; wb < 4; ++wb)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) lds[wb * world_floats + toff + u * B] = v[4 * wb + u];
-      }
-    }
-    if (l < B) {
-      float s = rhs[k + l];
-      for (int jb = 0; jb < kb; ++jb) {
-        const float *Tk = tile(jb, kb);
-        float sum = 0.0f;
-#pragma unroll
-        for (int t = 0; t < B; ++t) sum = fma_(Tk[t * B + l], rhs[jb * B + t], sum);
-        s = s - sum;
-      }
-      rhs[k + l] = s;
-    }
-    wave_sync();
-    {
-      // Cholesky of the diagonal tile and the forward solve of the right-hand side, lane i of
-      // the world's row holding row i (see blocked_factor_solve_kernel)
-      const int i = l;
-      float a[B];
-#pragma unroll
-      for (int j = 0; j < B; ++j) a[j] = tile(kb, kb)[(i < B ? i : 0) * B + j];
-      float s = rhs[k + (i < B ? i : 0)];
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        float d, rinv;
-        pivot_sqrt_rcp(row_bcast(a[j], j), true, d, rinv);
-        const float lj = i == j ? d : a[j] * rinv;
-        if (i >= j && i < B) L[i * B + j] = lj;
-        const float z = row_bcast(s, j) * rinv;
-        if (i == j) {
-          rhs[k + j] = z;
-          L[BB + j] = rinv;
-        }
-        s = fma_(-lj, z, s);
-#pragma unroll
-        for (int jj = j + 1; jj < B; ++jj) a[jj] = fma_(-lj, row_bcast(lj, jj), a[jj]);
-      }
-    }
-    wave_sync();
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = l + 16 * u, r = e / B, c = e % B;
-      tile(kb, kb)[e] = c >= r ? L[c * B + r] : 0.0f;
-    }
-    for (int qn = l; qn < (ntile - 1) * B; qn += 16) {
-      const int tb = 1 + qn / B, cc = qn % B;
-      float *Tt = tile(kb, kb + tb);
-      float col[B];
-#pragma unroll
-      for (int r = 0; r < B; ++r) col[r] = Tt[r * B + cc];
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        const float z = col[j] * L[BB + j];
-        col[j] = z;
-#pragma unroll
-        for (int i = j + 1; i < B; ++i) col[i] = fma_(-L[i * B + j], z, col[i]);
-      }
-#pragma unroll
-      for (int r = 0; r < B; ++r) Tt[r * B + cc] = col[r];
-    }
-    wave_sync();
-  }
-  // rhs <- U^-1 rhs, block rows from the bottom
-  for (int ib = nblk - 1; ib >= 0; --ib) {
-    const int i0 = ib * B, r = l < B ? l : 0;
-    const float *Td = tile(ib, ib);
-    float s = rhs[i0 + r];
-    float urow[B];
-#pragma unroll
-    for (int cc = 0; cc < B; ++cc) urow[cc] = Td[r * B + cc];
-    const float rinv = 1.0f / Td[r * B + r];
-    for (int jb = ib + 1; jb < nblk; ++jb) {
-      const float *Tj = tile(ib, jb);
-      float sum = 0.0f;
-#pragma unroll
-      for (int t = 0; t < B; ++t) sum = fma_(Tj[r * B + t], rhs[jb * B + t], sum);
-      s = s - sum;
-    }
-#pragma unroll
-    for (int cc = B - 1; cc >= 0; --cc) {
-      const float xv = row_bcast(s * rinv, cc);
-      if (l == cc) rhs[i0 + cc] = xv;
-      s = fma_(-urow[cc], xv, s);
-    }
-    wave_sync();
-  }
-  if (live) {
-    if (x)
-      for (int i = l; i < nv; i += 16) x[w * ldx + i] = rhs[i];
-    if (Uout) {
-      float4 *dst = (float4 *)(Uout + w * (int64_t)pad * pad);
-      for (int i4 = l; i4 < pad * pad / 4; i4 += 16) {
-        const int row = 4 * i4 / pad, col = 4 * i4 - row * pad, bi = row / B, bj = col / B;
-        if (bj >= bi) dst[i4] = *(const float4 *)(tile(bi, bj) + (row % B) * B + (col % B));  // lower tiles: not written
-      }
-    }
-  }
 }
 
 // Per-iteration factor stage on the dense Hessian: dofs touched by the changed rows,
@@ -1578,56 +1358,6 @@ __global__ __launch_bounds__(256, NVR == 128 ? 4 : 3) void jtdj_mfma_kernel(
   });
 }
 
-// The same assembly followed, in the same workgroup, by the blocked Cholesky of H and the solve:
-// H goes to memory (the per-iteration stage keeps updating it there) and into the factor's LDS
-// array at once, so the factor neither gathers it from memory nor waits for another launch, and
-// on a CU the matrix-core phase of one world runs beside the pivot chains of the others.  The rows
-// of J are staged in the factor's array, which is free until H is complete.  Results are those of
-// im_jtdj_mfma followed by im_blocked_factor_solve (B = 16) bit for bit.
-template <int NVR>
-__global__ __launch_bounds__(256, NVR == 128 ? 4 : 3) void jtdj_factor_solve_kernel(
-    const float *__restrict__ Mdense, const float *__restrict__ J, int njmax, const float *__restrict__ D,
-    const int32_t *__restrict__ state, const int32_t *__restrict__ nefc_p, int quad, float *__restrict__ H, int nv,
-    int nv_pad, const float *__restrict__ y, int64_t ldy, float *__restrict__ Uout, float *__restrict__ x, int64_t ldx,
-    int pad) {
-  constexpr int B = 16;
-  extern __shared__ float lds[];
-  const Stair<B> S{pad};
-  const int nU = S.words();
-  const int nvr = NVR ? NVR : (nv + 31) / 32 * 32, stage_words = 2 * (32 * nvr + 32) + 2 * ((njmax + 3) & ~3);
-  float *U = lds;       // first the staged rows of J (two copies) and the list of contributing rows, then [nU] H, then the factor
-  float *rhs = lds + (nU > stage_words ? nU : stage_words);  // [pad]
-  float *L = rhs + pad;  // [B * B + B]
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int64_t w = blockIdx.x;
-  for (int i = tid; i < pad; i += nt) rhs[i] = (y && i < nv) ? y[w * ldy + i] : 0.0f;
-  float *Hw = H ? H + w * (int64_t)nv_pad * nv_pad : nullptr;
-  // the assembly's last barrier is behind every wavefront when the elements come out, so they can
-  // go where the rows were staged.  The factor reads the upper triangle below nv only (the rest
-  // of a diagonal tile by symmetry, the padding as the identity) and writes every entry of a block
-  // row before anything reads it, so the array needs no clearing.
-  const bool vec = (nv_pad & 3) == 0 && ((uintptr_t)H & 15) == 0;
-  jtdj_tiles<NVR>(Mdense, J, njmax, D, state, nefc_p, quad, nv, lds, [&](int i0, int j, float4v h, bool off) {
-    if (Hw) store_h_mirrored(Hw, nv, nv_pad, vec, i0, j, h, off);
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (i0 + v < nv && j < nv && i0 + v <= j) U[S.at(i0 + v, j)] = h[v];
-  });
-  __syncthreads();
-  const LdsSrc<B> src{U, nv, pad};
-  factor_forward<B>(src, U, rhs, L, pad, tid, nt);
-  backward_solve<B>(U, rhs, pad, tid, nt);
-  if (x)
-    for (int i = tid; i < nv; i += nt) x[w * ldx + i] = rhs[i];
-  if (Uout)
-    for (int i = tid; i < pad * pad / 4; i += nt) {
-      const int r = 4 * i / pad, c = 4 * i - r * pad;
-      // the tiles below the block diagonal are left as the caller has them (the reference's kernel
-      // stores the tiles on and right of the diagonal only, indexed_factor.py:115, 141)
-      if (c >= r / B * B) ((float4 *)(Uout + w * (int64_t)pad * pad))[i] = *(const float4 *)(U + S.at(r, c));
-    }
-}
-
 // Every float whose bit pattern lies in [first, last] and that is in the pivots' range: do the
 // short forms give the bits of sqrtf and of 1.0f / sqrtf?
 __global__ void check_pivot_sqrt_kernel(uint32_t first, uint32_t last, unsigned long long *mismatches) {
@@ -1679,34 +1409,21 @@ static int launch_blocked_factor(const float *M, int64_t ldM, int nM, const int3
                                  int nv, int pad, const float *y, int64_t ldy, float *U, float *x, int64_t ldx,
                                  const int32_t *active, int nworld, void *stream) {
   const int B = block_size;
-  static const bool quad_off = [] {
+  // up to 128 dofs a wavefront holds the matrix in its registers; the workgroup-per-world kernel below serves
+  // the larger ones (IMHIP_BLOCKED_KERNEL=simple: all)
+  static const bool simple = [] {
     const char *e = std::getenv("IMHIP_BLOCKED_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  if (pad <= (B == 8 ? 64 : 48) && !quad_off) {
-    // small matrices: four worlds per wavefront (16 x 16 tiles at pad 64 need 46 KB of LDS per
-    // wavefront, three per CU, and are no faster that way)
-    const size_t quad_bytes = sizeof(float) * 4 * (size_t)im::quad_world_floats(pad, B);
-    auto qfn = B == 8 ? im::blocked_factor_solve_quad_kernel<8> : im::blocked_factor_solve_quad_kernel<16>;
-    hipLaunchKernelGGL(qfn, dim3((unsigned)((nworld + 3) / 4)), dim3(64), quad_bytes, (hipStream_t)stream, M, ldM, nM,
-                       block_idx, y, ldy, U, x, ldx, nv, pad, nworld, active);
-    IM_HIP_CHECK(hipGetLastError());
-    return IM_OK;
-  }
+  if (nv <= 128 && !simple)
+    return im::blocked_solve_wave(M, ldM, nM, block_idx, B, nv, pad, y, ldy, U, x, ldx, active, nworld, (hipStream_t)stream);
   const size_t u_words = B == 8 ? im::Stair<8>{pad}.words() : im::Stair<16>{pad}.words();
   const size_t lds_bytes = sizeof(float) * (u_words + pad + B * B + B);
   if (lds_bytes > 160 * 1024) return IM_ERR_UNSUPPORTED;
   auto fn = B == 8 ? im::blocked_factor_solve_kernel<8> : im::blocked_factor_solve_kernel<16>;
   if (lds_bytes > 64 * 1024)
     IM_HIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-  // The pivots of a tile, the triangular solves and the right-hand side are one wavefront's work
-  // whatever the workgroup size, and the other wavefronts wait at the barriers meanwhile: what
-  // counts is how many worlds are resident on a CU.  Small workgroups leave the registers for more
-  // of them (measured on g1, snu and the 128-dof stress shape: 64 threads up to pad 48, 128 for
-  // 16 x 16 tiles at pad 64, 256 beyond; at pad 128 four workgroups of 38 KB share a CU and the
-  // launch takes 1.30 ms for 16384 worlds where two of 512 threads took 1.90).
-  const int threads = pad <= 48 ? 64 : (pad <= 64 && B == 16) ? 128 : 256;
-  hipLaunchKernelGGL(fn, dim3(nworld), dim3(threads), lds_bytes, (hipStream_t)stream, M, ldM, nM, block_idx, y,
+  hipLaunchKernelGGL(fn, dim3(nworld), dim3(256), lds_bytes, (hipStream_t)stream, M, ldM, nM, block_idx, y,
                      ldy, U, x, ldx, nv, pad, active);
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
@@ -1843,17 +1560,7 @@ int im_jtdj_factor_solve(const float *Mdense, const float *J, int njmax, const f
   if (nv > 128) return IM_ERR_UNSUPPORTED;
   if ((y && ldy < nv) || (x && ldx < nv)) return IM_ERR_STRIDE;
   if (U && ((uintptr_t)U & 15)) return IM_ERR_STRIDE;
-  const int nvr = (nv + 31) / 32 * 32;
-  const size_t stage_words = 2 * (32 * (size_t)nvr + 32) + 2 * (size_t)((njmax + 3) & ~3), u_words = im::Stair<16>{pad}.words();
-  const size_t lds_bytes = sizeof(float) * ((u_words > stage_words ? u_words : stage_words) + pad + 16 * 16 + 16);
-  if (lds_bytes > 160 * 1024) return IM_ERR_UNSUPPORTED;
-  auto fn = nv > 112 ? im::jtdj_factor_solve_kernel<128> : im::jtdj_factor_solve_kernel<0>;
-  if (lds_bytes > 64 * 1024)
-    IM_HIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-  hipLaunchKernelGGL(fn, dim3(nworld), dim3(256), lds_bytes, (hipStream_t)stream, Mdense, J, njmax, D, state, nefc, quad,
-                     H, nv, nv_pad, y, ldy, U, x, ldx, pad);
-  IM_HIP_CHECK(hipGetLastError());
-  return IM_OK;
+  return im::jtdj_solve_wave(Mdense, J, njmax, D, state, nefc, quad, H, nv, nv_pad, y, ldy, U, pad, x, ldx, nworld, (hipStream_t)stream);
 }
 
 int im_dense_update_factor(const uint8_t *done, const int32_t *state_changes, const int32_t *changes,

@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <utility>
 
 #include "jtdj_wave.h"
 #include "newton_wave.h"
@@ -84,8 +85,7 @@ __device__ __forceinline__ unsigned panel_pivots(Panel &k, float a00, float a01,
     if constexpr (FAST) {
       pivot_sqrt_rcp_fast(x, d, inv);
     } else {
-      d = sqrtf(x);
-      inv = 1.0f / d;
+      pivot_sqrt_rcp_any(x, d, inv);
     }
   };
   // distance of the pivots' bit patterns from 2^-96: negative, tiny, infinite and NaN ones lie far out
@@ -107,18 +107,89 @@ __device__ __forceinline__ unsigned panel_pivots(Panel &k, float a00, float a01,
   return m01 > m23 ? m01 : m23;
 }
 
+// f(0) .. f(N - 1) with the index as a constant, whatever the size of the body: an index into the tiles that
+// is left to the compiler's unrolling would put them into scratch memory where it declines.
+template <int... I, class F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F &&f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void each(F &&f) {
+  each_of(std::make_integer_sequence<int, N>{}, f);
+}
+
+// The products of panels P0 .. P1 - 1 of two tiles, one after the other from zero.
+template <int P0, int P1, class A, class C>
+__device__ __forceinline__ float4v block_sum(const A &a, const C &b) {
+  float4v s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int p = P0; p < P1; ++p) s = mfma16(a[p], b[p], s);
+  return s;
+}
+
+// on ? a : b, by one instruction
+__device__ __forceinline__ float pick(bool on, float a, float b) {
+  const float v = on ? a : b;
+  asm("" : : "v"(v));
+  return v;
+}
+
+// The rows of a panel from its pivots: r's rows 4 g + v of lane group p, in panel layout.
+__device__ __forceinline__ float panel_rows(const Panel &q, const float4v &r, int p) {
+  const float f0 = r[0] * q.inv[0];
+  const float f1 = fma_(-q.u01, f0, r[1]) * q.inv[1];
+  const float f2 = fma_(-q.u12, f1, fma_(-q.u02, f0, r[2])) * q.inv[2];
+  const float f3 = fma_(-q.u23, f2, fma_(-q.u13, f1, fma_(-q.u03, f0, r[3]))) * q.inv[3];
+  return p == 0 ? panel_gather<0>(f0, f1, f2, f3) : p == 1 ? panel_gather<1>(f0, f1, f2, f3)
+         : p == 2 ? panel_gather<2>(f0, f1, f2, f3) : panel_gather<3>(f0, f1, f2, f3);
+}
+
+// r -= the sums of the N block rows above, whose solution is in xl; above(k): the tile of block row k in this column
+template <int N, int B, class Above>
+__device__ __forceinline__ void less_sums(float4v &r, const float *xl, int g, Above &&above) {
+  each<N>([&](auto k) __attribute__((always_inline)) {
+    float z[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) z[p] = xl[16 * k + 4 * p + g];
+    if constexpr (B == 8) {
+      r = r - block_sum<0, 2>(above(k), z);
+      r = r - block_sum<2, 4>(above(k), z);
+    } else {
+      r = r - block_sum<0, 4>(above(k), z);
+    }
+  });
+}
+
 // Factor of the tiles in place: U in panel layout (register p of lane (g, c): row 4 p + g, column c), its
 // diagonal in the diagonal tiles, its reciprocals in rd[k] (lane r and 16 + r, ..: row 16 k + r).
-// `last`: whether the last row's pivot counts as 1 (the corner of an augmented matrix).
-template <int NB>
-__device__ __forceinline__ void factor_tiles(float4v (&t)[kTiles<NB>], float (&rd)[NB], bool last, int lane) {
+// `last`: whether the last row's pivot counts as 1 (the corner of an augmented matrix).  Rows at and past nv
+// are rows of the identity (but for the corner), and panels of such rows are not computed.  B: rows of a block of
+// the blocked order, 16 or 8 (then two to a tile row, and a tile row's upper block leaves the lower one by a
+// sum of its own).
+// RHS: also z = U'^-1 rhs, for matrices without a spare column: rhs in xl (16 NB words, zero at and past nv), z in
+// its place.
+template <int NB, int B = 16, bool RHS = false>
+__device__ __forceinline__ void factor_tiles(float4v (&t)[kTiles<NB>], float (&rd)[NB], bool last, float *xl, int nv, int lane) {
   const int g = lane >> 4, c = lane & 15;
-#pragma unroll
-  for (int k = 0; k < NB; ++k) {
+  each<NB>([&](auto block_row) __attribute__((always_inline)) {
+    constexpr int k = block_row;
     float uk[NB][4];  // the finished panels of block row k, tile k + j at [j]
     float rk = 1.0f;
+    float4v r = {0.0f, 0.0f, 0.0f, 0.0f};
+    float zk[4];
+    if constexpr (RHS) {
+      r = *(const float4v *)(xl + 16 * k + 4 * g);
+      less_sums<k, B>(r, xl, g, [&](auto above) __attribute__((always_inline)) { return t[tile_at<NB>(above, k)]; });
+    }
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
+      if (k == NB - 1 && p > 0 && 16 * k + 4 * p >= nv && !(last && p == 3)) {
+        const bool one = c - 4 * p == g;
+        uk[0][p] = one ? 1.0f : 0.0f;
+        rk = c >> 2 == p ? 1.0f : rk;
+        if constexpr (RHS) zk[p] = 0.0f;
+        continue;
+      }
       const float4v dg = t[tile_at<NB>(k, k)];
       const int l0 = 20 * p;  // lane (p, 4 p)
       Panel q;
@@ -128,113 +199,161 @@ __device__ __forceinline__ void factor_tiles(float4v (&t)[kTiles<NB>], float (&r
       float a33 = lane_value(dg[3], l0 + 3);
       // the corner: the gradient column's own row, whose pivot nothing below reads
       const bool corner = last && k == NB - 1 && p == 3;
-      unsigned far = panel_pivots<true>(q, a00, a01, a02, a03, a11, a12, a13, a22, a23, corner ? 0x1p60f : a33);
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)(far >= 0x7f800000u - 0x0f800000u)), 0))
-        (void)panel_pivots<false>(q, a00, a01, a02, a03, a11, a12, a13, a22, a23, corner ? 0x1p60f : a33);
+      // (a branch per panel costs the larger matrices registers, the largest a hundred spilled ones: they take the
+      // forms for every number, which are a twentieth of their work)
+      constexpr bool kBranch = NB < 5;
+      const unsigned far = panel_pivots<kBranch>(q, a00, a01, a02, a03, a11, a12, a13, a22, a23, corner ? 0x1p60f : a33);
+      if constexpr (kBranch)
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)(far >= 0x7f800000u - 0x0f800000u)), 0))
+          (void)panel_pivots<false>(q, a00, a01, a02, a03, a11, a12, a13, a22, a23, corner ? 0x1p60f : a33);
       if (corner) q.d[3] = q.inv[3] = 1.0f;
-      const float dsel = g == 0 ? q.d[0] : g == 1 ? q.d[1] : g == 2 ? q.d[2] : q.d[3];
+      // (one select after another: as a choice among four the compiler makes branches of them)
+      float dsel = pick(g == 0, q.d[0], q.d[3]);
+      dsel = pick(g == 1, q.d[1], dsel);
+      dsel = pick(g == 2, q.d[2], dsel);
       const int at = c - 4 * p;
-      rk = at == 0 ? q.inv[0] : at == 1 ? q.inv[1] : at == 2 ? q.inv[2] : at == 3 ? q.inv[3] : rk;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) rk = pick(at == a, q.inv[a], rk);
 #pragma unroll
       for (int j = k; j < NB; ++j) {
-        const float4v r = t[tile_at<NB>(k, j)];
-        const float f0 = r[0] * q.inv[0];
-        const float f1 = fma_(-q.u01, f0, r[1]) * q.inv[1];
-        const float f2 = fma_(-q.u12, f1, fma_(-q.u02, f0, r[2])) * q.inv[2];
-        const float f3 = fma_(-q.u23, f2, fma_(-q.u13, f1, fma_(-q.u03, f0, r[3]))) * q.inv[3];
-        float u = p == 0 ? panel_gather<0>(f0, f1, f2, f3) : p == 1 ? panel_gather<1>(f0, f1, f2, f3)
-                  : p == 2 ? panel_gather<2>(f0, f1, f2, f3) : panel_gather<3>(f0, f1, f2, f3);
+        if constexpr (NB >= 6)
+          if ((j - k) % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+        float u = panel_rows(q, t[tile_at<NB>(k, j)], p);
         if (j == k) u = at == g ? dsel : u;
         uk[j - k][p] = u;
       }
-      // the rows below, in this block row: groups p + 1 .. (what lands in the finished groups is not read again)
-      if (p < 3) {
+      if constexpr (RHS) {
+        zk[p] = panel_rows(q, r, p);
+        xl[16 * k + 4 * p + g] = zk[p];  // sixteen lanes the same word: cheaper than a branch
+        if (B == 8 && p == 1) {
+          r = r - block_sum<0, 2>(uk[0], zk);
+        } else if (p < 3) {
+          const float4v n = mfma16(-uk[0][p], zk[p], r);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) r[v] = B == 8 && p == 0 && g != 1 ? r[v] : n[v];
+        }
+      }
+      // the rows below, in this block: groups p + 1 .. (what lands in the finished groups is not read again)
+      if (p < 3 && !(B == 8 && p == 1)) {
         const float minus = -uk[0][p];
 #pragma unroll
-        for (int j = k; j < NB; ++j) t[tile_at<NB>(k, j)] = mfma16(minus, uk[j - k][p], t[tile_at<NB>(k, j)]);
+        for (int j = k; j < NB; ++j) {
+          const float4v n = mfma16(minus, uk[j - k][p], t[tile_at<NB>(k, j)]);
+          if (B == 8 && p == 0) {  // the lower block's groups wait for the upper block's whole sum
+#pragma unroll
+            for (int v = 0; v < 4; ++v) t[tile_at<NB>(k, j)][v] = g == 1 ? n[v] : t[tile_at<NB>(k, j)][v];
+          } else {
+            t[tile_at<NB>(k, j)] = n;
+          }
+        }
+      }
+      if (B == 8 && p == 1) {
+#pragma unroll
+        for (int j = k; j < NB; ++j) t[tile_at<NB>(k, j)] = t[tile_at<NB>(k, j)] - block_sum<0, 2>(uk[0], uk[j - k]);
       }
     }
     // the block rows below lose this one's sums
 #pragma unroll
-    for (int i = k + 1; i < NB; ++i)
+    for (int i = k + 1; i < NB; ++i) {
+      // (with many tiles the scheduler would start every one of these sums at once and spill)
+      if constexpr (NB >= 6) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = i; j < NB; ++j) {
-        float4v s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int p = 0; p < 4; ++p) s = mfma16(uk[i - k][p], uk[j - k][p], s);
-        t[tile_at<NB>(i, j)] = t[tile_at<NB>(i, j)] - s;
+        float4v &m = t[tile_at<NB>(i, j)];
+        if constexpr (B == 8) {
+          m = m - block_sum<0, 2>(uk[i - k], uk[j - k]);
+          m = m - block_sum<2, 4>(uk[i - k], uk[j - k]);
+        } else {
+          m = m - block_sum<0, 4>(uk[i - k], uk[j - k]);
+        }
       }
+    }
 #pragma unroll
     for (int j = k; j < NB; ++j) t[tile_at<NB>(k, j)] = float4v{uk[j - k][0], uk[j - k][1], uk[j - k][2], uk[j - k][3]};
     rd[k] = rk;
-  }
+    if constexpr (RHS) wave_sync();
+  });
 }
 
-// z = U'^-1 rhs with a finished factor in panel layout; the right-hand side's block rows as tiles whose
-// columns are all alike.  z into xl.
-template <int NB>
-__device__ __forceinline__ void forward_tiles(const float4v (&t)[kTiles<NB>], const float (&rd)[NB], float4v (&b)[NB], float *xl, int lane) {
+// z = U'^-1 rhs with a finished factor in panel layout: rhs(row) for the 16 NB rows, z into xl.
+template <int NB, class Rhs>
+__device__ __forceinline__ void forward_tiles(const float4v (&t)[kTiles<NB>], const float (&rd)[NB], Rhs &&rhs, float *xl, int nv, int lane) {
   const int g = lane >> 4, c = lane & 15;
+  each<NB>([&](auto tile_row) __attribute__((always_inline)) {
+    constexpr int i = tile_row;
+    float4v r;
 #pragma unroll
-  for (int k = 0; k < NB; ++k) {
-    float zk[4];
-    const float4v dg = t[tile_at<NB>(k, k)];
+    for (int v = 0; v < 4; ++v) r[v] = rhs(16 * i + 4 * g + v);
+    less_sums<i, 16>(r, xl, g, [&](auto above) __attribute__((always_inline)) { return t[tile_at<NB>(above, i)]; });
+    const float4v dg = t[tile_at<NB>(i, i)];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
+      if (i == NB - 1 && p > 0 && 16 * i + 4 * p >= nv) {  // beyond the dofs
+        if (c == 0) xl[16 * i + 4 * p + g] = 0.0f;
+        continue;
+      }
       auto u = [&](int a, int col) { return lane_value(dg[p], 16 * a + 4 * p + col); };
-      auto inv = [&](int a) { return lane_value(rd[k], 4 * p + a); };
-      const float4v r = b[k];
-      const float f0 = r[0] * inv(0);
-      const float f1 = fma_(-u(0, 1), f0, r[1]) * inv(1);
-      const float f2 = fma_(-u(1, 2), f1, fma_(-u(0, 2), f0, r[2])) * inv(2);
-      const float f3 = fma_(-u(2, 3), f2, fma_(-u(1, 3), f1, fma_(-u(0, 3), f0, r[3]))) * inv(3);
-      zk[p] = p == 0 ? panel_gather<0>(f0, f1, f2, f3) : p == 1 ? panel_gather<1>(f0, f1, f2, f3)
-              : p == 2 ? panel_gather<2>(f0, f1, f2, f3) : panel_gather<3>(f0, f1, f2, f3);
-      if (p < 3) b[k] = mfma16(-dg[p], zk[p], b[k]);
-      if (c == 0) xl[16 * k + 4 * p + g] = zk[p];
-    }
+      Panel q;
+      q.u01 = u(0, 1), q.u02 = u(0, 2), q.u03 = u(0, 3), q.u12 = u(1, 2), q.u13 = u(1, 3), q.u23 = u(2, 3);
 #pragma unroll
-    for (int i = k + 1; i < NB; ++i) {
-      float4v s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int p = 0; p < 4; ++p) s = mfma16(t[tile_at<NB>(k, i)][p], zk[p], s);
-      b[i] = b[i] - s;
+      for (int a = 0; a < 4; ++a) q.inv[a] = lane_value(rd[i], 4 * p + a);
+      const float z = panel_rows(q, r, p);
+      if (p < 3) r = mfma16(-dg[p], z, r);
+      if (c == 0) xl[16 * i + 4 * p + g] = z;
     }
-  }
-  wave_sync();
+    wave_sync();
+  });
 }
 
-// U x = z: z in xl (16 NB words), x in its place.  tt: 16 x 17 words.
-template <int NB>
-__device__ __forceinline__ void backward_tiles(const float4v (&t)[kTiles<NB>], const float (&rd)[NB], float *xl, float *tt, int lane) {
+// U x = z: z in xl (16 NB words, zero at and past nv), x in its place.  tt: 16 x 17 words.
+template <int NB, int B = 16>
+__device__ __forceinline__ void backward_tiles(const float4v (&t)[kTiles<NB>], const float (&rd)[NB], float *xl, float *tt, int nv, int lane) {
   const int g = lane >> 4, c = lane & 15;
   float *put = tt + g * 17 + c;          // row 4 p + g: 68 p words on
   const float *take = tt + c * 17 + g;   // row c, column 4 q + g
   const float *last = tt + c * 17 + 3 - g;  // row c, column 4 p + 3 - g
-#pragma unroll
-  for (int ib = NB - 1; ib >= 0; --ib) {
+  each<NB>([&](auto from_below) __attribute__((always_inline)) {
+    constexpr int ib = NB - 1 - from_below;
     float4v r = *(const float4v *)(xl + 16 * ib + 4 * g);
-#pragma unroll
-    for (int j = ib + 1; j < NB; ++j) {
+    // (blocks of 8: the upper block loses the lower one's sum before these, so they are kept)
+    float4v later[B == 8 ? 2 * NB : 1];
+    const float4v z = r;
+    each<NB - 1 - ib>([&](auto right) __attribute__((always_inline)) {
+      constexpr int j = ib + 1 + right;
       const float4v u = t[tile_at<NB>(ib, j)];
 #pragma unroll
       for (int p = 0; p < 4; ++p) put[68 * p] = u[p];
       wave_sync();
-      float4v s = {0.0f, 0.0f, 0.0f, 0.0f};
+      float a[4], x[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) s = mfma16(take[4 * q], xl[16 * j + 4 * q + g], s);
-      r = r - s;
+      for (int q = 0; q < 4; ++q) a[q] = take[4 * q], x[q] = xl[16 * j + 4 * q + g];
+      if constexpr (B == 8) {
+        later[2 * (j - ib - 1)] = block_sum<0, 2>(a, x), later[2 * (j - ib - 1) + 1] = block_sum<2, 4>(a, x);
+        r = r - later[2 * (j - ib - 1)];
+        r = r - later[2 * (j - ib - 1) + 1];
+      } else {
+        r = r - block_sum<0, 4>(a, x);
+      }
       wave_sync();
-    }
+    });
     const float4v dg = t[tile_at<NB>(ib, ib)];
 #pragma unroll
     for (int p = 0; p < 4; ++p) put[68 * p] = dg[p];
     wave_sync();
-    float ad[4];
+    float ad[4], own[4];
 #pragma unroll
     for (int p = 1; p < 4; ++p) ad[p] = -last[4 * p];
+    if constexpr (B == 8) own[2] = take[8], own[3] = take[12];
 #pragma unroll
     for (int p = 3; p >= 0; --p) {
+      if (B == 8 && p == 1) {  // the upper block: less the lower one's sum, then the later blocks'
+        float x[4];
+        x[2] = xl[16 * ib + 8 + g], x[3] = xl[16 * ib + 12 + g];
+        r = z - block_sum<2, 4>(own, x);
+#pragma unroll
+        for (int j = 0; j < 2 * (NB - 1 - ib); ++j) r = r - later[j];
+      }
+      if (ib == NB - 1 && p > 0 && 16 * ib + 4 * p >= nv) continue;
       auto u = [&](int a, int col) { return lane_value(dg[p], 16 * a + 4 * p + col); };
       auto inv = [&](int a) { return lane_value(rd[ib], 4 * p + a); };
       const float x3 = r[3] * inv(3);
@@ -242,13 +361,14 @@ __device__ __forceinline__ void backward_tiles(const float4v (&t)[kTiles<NB>], c
       const float x1 = fma_(-u(1, 2), x2, fma_(-u(1, 3), x3, r[1])) * inv(1);
       const float x0 = fma_(-u(0, 1), x1, fma_(-u(0, 2), x2, fma_(-u(0, 3), x3, r[0]))) * inv(0);
       if (lane == 16 * p) *(float4v *)(xl + 16 * ib + 4 * p) = float4v{x0, x1, x2, x3};
-      if (p > 0) {  // the rows above in this block lose rows 4 p + 3 .. 4 p in that order
+      if (p > 0 && !(B == 8 && p == 2)) {  // the rows above in this block lose rows 4 p + 3 .. 4 p in that order
         const float b = p == 1 ? panel_gather<1>(x3, x2, x1, x0) : p == 2 ? panel_gather<2>(x3, x2, x1, x0) : panel_gather<3>(x3, x2, x1, x0);
         r = mfma16(ad[p], b, r);
       }
+      if (B == 8) wave_sync();
     }
     wave_sync();
-  }
+  });
 }
 
 // The sums over the changed rows of every pair of dofs, from zero in the list's order, as tiles; the dofs
@@ -343,6 +463,10 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
       uni[nv] = 0;
     }
     // H (with its update), the identity beyond the dofs, the gradient in the last column
+    auto beyond = [&](int row, int col, float e) __attribute__((always_inline)) {
+      const bool in = col < nv && row < nv;
+      return in ? e : (c == 15 && row < nv) ? gw[row < nv ? row : 0] : row == col ? 1.0f : 0.0f;
+    };
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -364,14 +488,10 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
             e = d != 0.0f ? h[v] + d : h[v];
             if (d != 0.0f && in && (i < j || row <= col)) Hw[(size_t)row * PAD + col] = e;
           }
-          if (j == NB - 1) {
-            const float beyond = row == col ? 1.0f : 0.0f;
-            e = in ? e : (c == 15 && row < nv) ? gw[row < nv ? row : 0] : beyond;
-          }
-          m[v] = e;
+          m[v] = j == NB - 1 ? beyond(row, col, e) : e;
         }
       }
-    factor_tiles<NB>(t, rd, true, lane);
+    factor_tiles<NB>(t, rd, true, xl, nv, lane);
     // the forward-solved gradient, and the corner of the augmented column: 1e30 less its squares in order,
     // which leaves 1e30 as it is unless one of them comes near half an ulp of it (3.7e22)
     bool large = false;
@@ -407,16 +527,10 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
       }
   } else {
     // the stored factor, the identity in place of its augmented column; forward solve
-    float4v b[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       const float dgv = Uw[(size_t)(16 * i + c) * (PAD + 1)];
       rd[i] = i == NB - 1 && c == 15 ? 1.0f : 1.0f / dgv;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * i + 4 * g + v;
-        b[i][v] = row < nv ? gw[row < nv ? row : 0] : 0.0f;
-      }
 #pragma unroll
       for (int j = i; j < NB; ++j)
 #pragma unroll
@@ -425,9 +539,9 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
           t[tile_at<NB>(i, j)][p] = j == NB - 1 && c == 15 ? (i == j && 4 * p + g == 15 ? 1.0f : 0.0f) : v;
         }
     }
-    forward_tiles<NB>(t, rd, b, xl, lane);
+    forward_tiles<NB>(t, rd, [&](int row) { return row < nv ? gw[row < nv ? row : 0] : 0.0f; }, xl, nv, lane);
   }
-  backward_tiles<NB>(t, rd, xl, tt, lane);
+  backward_tiles<NB>(t, rd, xl, tt, nv, lane);
   // search = -x, x . x and grad . x as 64 lanes striding the dofs sum them
   float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll

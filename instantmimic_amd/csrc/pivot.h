@@ -23,6 +23,17 @@ __device__ __forceinline__ void pivot_sqrt_rcp_fast(float x, float &d, float &ri
   const float r = __builtin_amdgcn_rcpf(d);
   rinv = fma_(fma_(-d, r, 1.0f), r, r);
 }
+// The same for every x, in a few instructions and registers and without a branch: a pivot below the range is
+// moved into it by an even power of two (exact both ways: neither result comes near the denormals), what is not
+// a positive finite number is chosen.
+__device__ __forceinline__ void pivot_sqrt_rcp_any(float x, float &d, float &rinv) {
+  const bool small = x < 0x1p-96f, special = !(x > 0.0f && x < __builtin_inff());
+  pivot_sqrt_rcp_fast(small ? x * 0x1p64f : x, d, rinv);
+  d = small ? d * 0x1p-32f : d;
+  rinv = small ? rinv * 0x1p32f : rinv;
+  d = special ? (x < 0.0f ? __builtin_nanf("") : x) : d;
+  rinv = special ? __builtin_amdgcn_rcpf(d) : rinv;
+}
 // d = sqrtf(x), rinv = 1.0f / d; `checked`: the lanes whose x is a pivot (the others may hold anything)
 __device__ __forceinline__ void pivot_sqrt_rcp(float x, bool checked, float &d, float &rinv) {
   pivot_sqrt_rcp_fast(x, d, rinv);

@@ -1,0 +1,62 @@
+"""The factor and solve of dense matrices on one wavefront's matrix-core tiles at the edges of its block
+rows, with and without a spare column for the right-hand side, with pivots outside the range of the short
+square root, and with contributing rows on both sides of its steps of four, against the CPU restatement."""
+
+import numpy as np
+import pytest
+
+from instantmimic_amd import _lib
+from instantmimic_amd.mjw_kernels import blocked_dense as BD
+from oracle import ref as R
+
+
+def _spd(rng, nworld, nv):
+    a = rng.standard_normal((nworld, nv, nv))
+    M = (a @ a.transpose(0, 2, 1) / nv + np.eye(nv)).astype(np.float32)
+    M[-1] *= np.float32(2.0**-110)  # every pivot below 2^-96
+    return M
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [8, 16])
+@pytest.mark.parametrize("nv", [1, 8, 9, 16, 17, 31, 32, 33, 40, 41, 64, 65, 80, 81, 96, 112, 113, 127, 128])
+def test_gpu_blocked_solve_at_block_edges(device, nv, B):
+    import torch
+
+    rng, nworld = np.random.default_rng(nv), 6
+    M, y = _spd(rng, nworld, nv).reshape(nworld, -1), rng.standard_normal((nworld, nv)).astype(np.float32)
+    pad, layout, _ = BD.block_index_layout(np.arange(nv * nv), nv, nv * nv, B)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    Md, yd, idx, x, U = t(M), t(y), t(layout), torch.full((nworld, nv), np.nan, device=device), torch.zeros((nworld, pad, pad), device=device)
+    st = _lib.lib().im_blocked_factor_solve(Md.data_ptr(), nv * nv, nv * nv, idx.data_ptr(), B, nv, pad, yd.data_ptr(), nv, U.data_ptr(), x.data_ptr(), nv, nworld, None)
+    assert st == 0
+    torch.cuda.synchronize()
+    x_ref, U_ref = R.blocked_factor_solve(M, layout, nv, pad, B, y)
+    np.testing.assert_array_equal(U.cpu().numpy(), U_ref)
+    np.testing.assert_array_equal(x.cpu().numpy(), x_ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv", [1, 15, 16, 17, 33, 48, 64, 79, 80, 96, 112, 127, 128])
+def test_gpu_dense_hessian_solve_at_block_edges(device, nv):
+    import torch
+
+    counts = np.array([0, 1, 3, 4, 5, 8, 63, 64, 65, 130], np.int32)
+    rng, nworld, rows = np.random.default_rng(nv), len(counts), 130
+    pad, hpad = -(-nv // 16) * 16, (nv // 16 + 1) * 16
+    M, y = _spd(rng, nworld, nv), rng.standard_normal((nworld, nv)).astype(np.float32)
+    M[-1] *= np.float32(2.0**110)
+    J = rng.standard_normal((nworld, rows, nv)).astype(np.float32)
+    D = rng.uniform(0.1, 10.0, (nworld, rows)).astype(np.float32)
+    state = (rng.uniform(size=(nworld, rows)) < 0.7).astype(np.int32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    H, x, U = torch.zeros((nworld, hpad, hpad), device=device), torch.zeros((nworld, nv), device=device), torch.zeros((nworld, pad, pad), device=device)
+    BD.dense_hessian_factor_solve(t(M), t(J), t(D), t(state), t(counts), H, t(y), x, factor=U)
+    torch.cuda.synchronize()
+    H_ref = H.cpu().numpy()  # the factor's input: its sums' order is the matrix cores' own
+    assert R.rel_l2(H_ref, R.jtdj_dense(M.reshape(nworld, -1), J, D, state, counts, hpad)) <= 1e-6
+    np.testing.assert_array_equal(H_ref, H_ref.transpose(0, 2, 1))
+    _, layout, _ = BD.block_index_layout(np.arange(nv * nv), nv, nv * nv, 16)
+    x_ref, U_ref = R.blocked_factor_solve(np.ascontiguousarray(H_ref[:, :nv, :nv]).reshape(nworld, -1), layout, nv, pad, 16, y)
+    np.testing.assert_array_equal(U.cpu().numpy(), U_ref)
+    np.testing.assert_array_equal(x.cpu().numpy(), x_ref)
