@@ -23,6 +23,7 @@
 // the same order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 
@@ -233,52 +234,106 @@ __global__ __launch_bounds__(256) void force_velocity_state_kernel(
   out_slope[w * ldo + m] = fv.include_active * active * unit * dmult / velocity_scale;
 }
 
-// The same per world in one workgroup: the world's waypoints, moment entries and velocities come
-// into LDS with coalesced loads (a lane of the kernel above walks a few 12-byte waypoints and a
-// few scattered entries of its own, a cache line per request), then every muscle reads LDS.  Same
-// operations in the same order, so the same bits.  nwords_wp / nentry: what is staged (the
-// arrays' row lengths).
-__global__ __launch_bounds__(256) void force_velocity_state_world_kernel(
-    const float *__restrict__ wp, int64_t ldw, int nwords_wp, const int32_t *__restrict__ waypoint_start,
+// The same with a workgroup per world, resident over worlds.  What bounds it is latency, not
+// traffic: a lane of the kernel above walks a few 12-byte waypoints and a few scattered entries
+// of its own, a cache line per request, and its velocity is a chain of look-ups.  Here a world's
+// waypoints, moment entries and velocities come into LDS with eight coalesced loads in flight
+// per thread; the distances between neighbouring waypoints are taken by all threads side by side
+// (a lane per muscle left the wavefront waiting for its longest muscle's roots); and what does
+// not depend on the world (an entry's dof, a muscle's cos(pennation)) is left in LDS once.  Same
+// operations in the same order, so the same bits.
+// 284 muscles x 4096 worlds: 59.3 us (a workgroup of 256 per world, distances by the muscle's
+// lane) -> 38.9; 256 threads 48.4, 512 threads 52.7.
+constexpr int kFvThreads = 320;
+struct FvLds {
+  int words_wp, nentry, nqvel, nmuscle;  // the longest rows that are staged
+  __host__ __device__ int bytes() const {
+    return 4 * (words_wp + nentry + nqvel + words_wp / 3 + nmuscle) + 2 * ((nentry + 1) & ~1);
+  }
+};
+
+__device__ __forceinline__ void stage_row(float *to, const float *__restrict__ from, int n, int tid) {
+  constexpr int nt = kFvThreads;
+  int i = tid;
+  for (; i + 7 * nt < n; i += 8 * nt) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = from[i + k * nt];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) to[i + k * nt] = v[k];
+  }
+  if (i < n) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = from[min(i + k * nt, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (i + k * nt < n) to[i + k * nt] = v[k];
+  }
+}
+
+__global__ __launch_bounds__(kFvThreads) void force_velocity_state_world_kernel(
+    const float *__restrict__ wp, int64_t ldw, const int32_t *__restrict__ waypoint_start,
     const float *__restrict__ params, int ldpar, const float *__restrict__ rest,
     const float *__restrict__ length_scale, const float *__restrict__ activation, int64_t lda,
-    const float *__restrict__ qvel, int64_t ldq, int nqvel, const float *__restrict__ moment, int64_t ldm, int nentry,
+    const float *__restrict__ qvel, int64_t ldq, const float *__restrict__ moment, int64_t ldm,
     const int32_t *__restrict__ dof_offsets, const int32_t *__restrict__ dof_torque_idx, int root,
-    im_muscle_force_model model, im_muscle_force_velocity_model fv, int nmuscle, float *__restrict__ out_length,
+    im_muscle_force_model model, im_muscle_force_velocity_model fv, FvLds n, float *__restrict__ out_length,
     float *__restrict__ out_activation, float *__restrict__ out_velocity, float *__restrict__ out_multiplier,
-    float *__restrict__ out_slope, int64_t ldo) {
+    float *__restrict__ out_slope, int64_t ldo, int nworld) {
   extern __shared__ float fv_lds[];
-  float *row = fv_lds;            // [nwords_wp]
-  float *mom = row + nwords_wp;   // [nentry]
-  float *qv = mom + nentry;       // [nqvel]
-  const int64_t w = blockIdx.x;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int i = tid; i < nwords_wp; i += nt) row[i] = wp[w * ldw + i];
-  for (int i = tid; i < nentry; i += nt) mom[i] = moment[w * ldm + i];
-  for (int i = tid; i < nqvel; i += nt) qv[i] = qvel[w * ldq + i];
-  __syncthreads();
-  for (int m = tid; m < nmuscle; m += nt) {
-    float len = 0.0f;
-    for (int i = waypoint_start[m]; i < waypoint_start[m + 1] - 1; ++i)
-      len = len + length(sub(ld3(row + 3 * (i + 1)), ld3(row + 3 * i)));
-    float velocity = 0.0f;
-    for (int e = dof_offsets[m]; e < dof_offsets[m + 1]; ++e)
-      velocity = __builtin_fmaf(-mom[e], qv[dof_torque_idx[e] + root], velocity);
-    const float f0 = params[m * ldpar], lm0 = params[m * ldpar + 1], lt0 = params[m * ldpar + 2],
-                pen = params[m * ldpar + 3];
-    const float velocity_scale = fmaxf(length_scale[m] * fv.vmax, 1.0e-6f);
-    float mult, dmult;
-    force_velocity_curve(velocity / velocity_scale, fv.fvmax, &mult, &dmult);
-    float active = activation[w * lda + m];
-    if (fv.clamp_activation != 0.0f) active = fminf(fmaxf(active, 0.0f), 1.0f);
-    const float lm = len / fmaxf(rest[m], 1.0e-6f) - lt0;
-    const float ln = fminf(fmaxf(lm / fmaxf(lm0, 1.0e-6f), model.length_norm_min), model.length_norm_max);
-    const float unit = f0 * active_fl(ln, model.active) * cosf(pen) * model.force_scale;
-    out_length[w * ldo + m] = len;
-    out_activation[w * ldo + m] = active * mult;
-    out_velocity[w * ldo + m] = velocity;
-    out_multiplier[w * ldo + m] = mult;
-    out_slope[w * ldo + m] = fv.include_active * active * unit * dmult / velocity_scale;
+  float *row = fv_lds;                  // the world's waypoints
+  float *mom = row + n.words_wp;        // its moment entries
+  float *qv = mom + n.nentry;           // its velocities
+  float *dist = qv + n.nqvel;           // from every waypoint to the next one
+  float *cosp = dist + n.words_wp / 3;  // [nmuscle]
+  unsigned short *dof = (unsigned short *)(cosp + n.nmuscle);  // [nentry]
+  constexpr int nt = kFvThreads;
+  const int tid = threadIdx.x, nmuscle = n.nmuscle;
+  // what the tables name of a row, which may be a part of a wider array's
+  const int nwp = min(waypoint_start[nmuscle], n.words_wp / 3), ne = min(dof_offsets[nmuscle], n.nentry);
+  for (int e = tid; e < ne; e += nt) dof[e] = (unsigned short)(dof_torque_idx[e] + root);
+  for (int m = tid; m < nmuscle; m += nt) cosp[m] = cosf(params[m * ldpar + 3]);
+  for (int64_t w = blockIdx.x; w < nworld; w += gridDim.x) {
+    __syncthreads();  // the tables are there, the world before is done with
+    stage_row(row, wp + w * ldw, 3 * nwp, tid);
+    stage_row(mom, moment + w * ldm, ne, tid);
+    stage_row(qv, qvel + w * ldq, n.nqvel, tid);
+    __syncthreads();
+    for (int i = tid; i < nwp - 1; i += nt) dist[i] = length(sub(ld3(row + 3 * (i + 1)), ld3(row + 3 * i)));
+    __syncthreads();
+    for (int m = tid; m < nmuscle; m += nt) {
+      float len = 0.0f;
+      for (int i = waypoint_start[m]; i < waypoint_start[m + 1] - 1; ++i) len = len + dist[i];
+      float velocity = 0.0f;
+      const int e1 = dof_offsets[m + 1];
+      int e = dof_offsets[m];
+      for (; e + 4 <= e1; e += 4) {
+        float a[4], v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          a[k] = mom[e + k];
+          v[k] = qv[dof[e + k]];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) velocity = __builtin_fmaf(-a[k], v[k], velocity);
+      }
+      for (; e < e1; ++e) velocity = __builtin_fmaf(-mom[e], qv[dof[e]], velocity);
+      const float f0 = params[m * ldpar], lm0 = params[m * ldpar + 1], lt0 = params[m * ldpar + 2];
+      const float velocity_scale = fmaxf(length_scale[m] * fv.vmax, 1.0e-6f);
+      float mult, dmult;
+      force_velocity_curve(velocity / velocity_scale, fv.fvmax, &mult, &dmult);
+      float active = activation[w * lda + m];
+      if (fv.clamp_activation != 0.0f) active = fminf(fmaxf(active, 0.0f), 1.0f);
+      const float lm = len / fmaxf(rest[m], 1.0e-6f) - lt0;
+      const float ln = fminf(fmaxf(lm / fmaxf(lm0, 1.0e-6f), model.length_norm_min), model.length_norm_max);
+      const float unit = f0 * active_fl(ln, model.active) * cosp[m] * model.force_scale;
+      out_length[w * ldo + m] = len;
+      out_activation[w * ldo + m] = active * mult;
+      out_velocity[w * ldo + m] = velocity;
+      out_multiplier[w * ldo + m] = mult;
+      out_slope[w * ldo + m] = fv.include_active * active * unit * dmult / velocity_scale;
+    }
   }
 }
 
@@ -415,9 +470,7 @@ __global__ __launch_bounds__(256) void torque_bounds_kernel(
   upper[w * ldo + j] = hi;
 }
 
-// ---- one workgroup per world --------------------------------------------------------------
-// One workgroup of 512 threads per world (three of them share a CU at the 553-segment rig's
-// 49 KB of LDS; 384, 640, 768 and 1024 threads measured 2 - 7 % slower there).
+// ---- a workgroup per world, resident over worlds -------------------------------------------
 // The four contractions above visit every applied segment once per (segment, dof) entry and
 // redo its square root and three divisions each time, and they fetch a muscle's force and a
 // dof's motion axis from memory once per entry.  Here a workgroup first leaves in LDS each
@@ -426,6 +479,19 @@ __global__ __launch_bounds__(256) void torque_bounds_kernel(
 // contribution()), and a last pass adds each output's entries in list order, reading them
 // several at a time so that only the additions wait on one another.  Results equal the
 // one-thread-per-output kernels bit for bit.
+//
+// What bounds it is the vector issue rate: 41 instructions of an entry's arithmetic cannot be
+// left out without changing bits, and a launch per world spent as many again on the entry lists
+// (four table reads with their addresses, the entry's row, the products by the LDS records'
+// sizes; 63 - 79 % of the cycles issued a vector instruction).  The lists are the same for every
+// world, so the grid is what the chip holds at once, a workgroup walks over worlds, and a thread
+// keeps its TRIPS entries as LDS addresses and coefficients in registers.  An output's ordered
+// sum runs beside the next world's staging: two barriers per world.
+// 284 muscles (553 segments, 4445 entries) x 4096 worlds, a launch per world with 512 threads ->
+// this: moment 64.6 -> 50.8 us, activation gradient 57.1 -> 52.0, torque 73.9 -> 75 (its longest
+// row's 327 additions are the chain there; its entries issue as in the others, and one form
+// serves all).  512 threads with ten entries each spill 84 bytes a lane at 80 registers (moment
+// 54), 1024 threads with five spill at 64 (moment 49, gradient and torque 10 % slower).
 enum { MW_FORWARD, MW_GRAD, MW_BOUNDS, MW_MOMENT };
 
 struct MwArgs {
@@ -439,50 +505,48 @@ struct MwArgs {
   int64_t ldo;
   int root, nrow, nentry, nseg;
   int ntorque, nmuscle;  // sizes of the staged axes and forces (nmuscle 0 for MW_MOMENT)
+  int nworld;
 };
 
+constexpr int kMwThreads = 768;
 constexpr int kContribPad = 4;  // floats read past the last entry by ordered_sum()
+constexpr int kAxis = 7;        // floats of a dof's record: its cdof and, for MW_GRAD, grad_output
 struct MwLds {
   float *segd;     // [nseg][9]: dir (0 for a degenerate segment), p0 - c0, p1 - c1
   float *contrib;  // [nentry]
-  float *axis;     // [ntorque][6]: the dof's cdof
+  float *axis;     // [ntorque][kAxis]
   float *force;    // [nmuscle]: force of a muscle as the contraction sees it
-  float *gout;     // [ntorque], MW_GRAD only
-  unsigned short *rowid;  // [nentry]
+  unsigned short *rowid;  // [nentry]: an entry's row; in contrib's place where registers keep the entries
 };
-template <int MODE>
 __host__ __device__ inline size_t mw_lds_floats(const MwArgs &a) {
-  return (size_t)9 * a.nseg + (size_t)a.nentry + kContribPad + (size_t)6 * a.ntorque + (size_t)a.nmuscle +
-         (MODE == MW_GRAD ? (size_t)a.ntorque : 0);
+  return (size_t)9 * a.nseg + (size_t)a.nentry + kContribPad + (size_t)kAxis * a.ntorque + (size_t)a.nmuscle;
 }
 
-// What the lists hold about one entry.
+// One entry: word indices of its records in LDS, and its coefficients.
 struct MwEntry {
-  int row, other, seg;
+  unsigned where;  // segment's record | dof's record << 16
+  unsigned force;  // muscle's force
   float a, b;
 };
 template <int MODE>
-__device__ __forceinline__ MwEntry load_entry(const MwArgs &a, const MwLds &l, int e) {
+__device__ __forceinline__ MwEntry load_entry(const MwArgs &a, const MwLds &l, const float *lds, int e) {
+  const int row = l.rowid[e], other = MODE == MW_MOMENT ? 0 : a.e_other[e];
+  const int torque = MODE == MW_GRAD ? other : MODE == MW_MOMENT ? a.row_torque[row] : row;
+  const int muscle = MODE == MW_GRAD ? row : other;
   MwEntry t;
-  t.row = l.rowid[e];
-  t.other = MODE == MW_MOMENT ? 0 : a.e_other[e];
-  t.seg = a.e_seg[e];
+  t.where = (unsigned)(9 * a.e_seg[e]) | (unsigned)(l.axis - lds + kAxis * torque) << 16;
+  t.force = (unsigned)(l.force - lds + muscle);
   t.a = a.e_a[e];
   t.b = a.e_b[e];
   return t;
 }
 
 template <int MODE>
-__device__ __forceinline__ float entry_contribution(const MwArgs &a, const MwLds &l, const MwEntry &t) {
-  int torque, muscle;
-  if (MODE == MW_GRAD) { muscle = t.row; torque = t.other; }
-  else if (MODE == MW_MOMENT) { muscle = 0; torque = a.row_torque[t.row]; }
-  else { torque = t.row; muscle = t.other; }
-  float f = 1.0f;
-  if (MODE != MW_MOMENT) f = l.force[muscle];
-  const float *cd = l.axis + 6 * torque;
+__device__ __forceinline__ float entry_contribution(const float *lds, const MwEntry &t) {
+  const float f = MODE == MW_MOMENT ? 1.0f : lds[t.force];
+  const float *cd = lds + (t.where >> 16);
   const V3 ang = ld3(cd), lin = ld3(cd + 3);
-  const float *sd = l.segd + 9 * t.seg;
+  const float *sd = lds + (t.where & 0xFFFFu);
   const V3 dir = {sd[0], sd[1], sd[2]}, r0 = {sd[3], sd[4], sd[5]}, r1 = {sd[6], sd[7], sd[8]};
   const V3 fv = scale(f, dir);
   const V3 st = add(lin, cross(ang, r0));
@@ -493,11 +557,11 @@ __device__ __forceinline__ float entry_contribution(const MwArgs &a, const MwLds
   asm volatile("" : "+v"(c));
   // an entry whose force is zero is skipped by the reference: it enters the sum as 0
   c = f == 0.0f ? 0.0f : c;
-  if (MODE == MW_GRAD) c = l.gout[torque] * c;
+  if (MODE == MW_GRAD) c = cd[6] * c;
   return c;
 }
 
-// Sum of contrib[e0..e1) in list order from +0.  Whole groups of 16 (LONG) and of 4 entries are
+// Sum of contrib[e0..e1) in list order from +0.  Whole groups of 8 (LONG) and of 4 entries are
 // read with one address and added without a test; the last group reads up to three floats past
 // e1 (contrib is padded for that) and enters them as +0, which leaves every bit of a sum that
 // started at +0 (such a sum is never -0).
@@ -505,14 +569,21 @@ template <bool LONG>
 __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e1) {
   float total = 0.0f;
   int e = e0;
-  if (LONG) {
-    for (; e + 16 <= e1; e += 16) {
-      float c[16];
+  if (LONG && e + 8 <= e1) {  // the next eight are on their way while these are added
+    float c[8];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
+    for (int k = 0; k < 8; ++k) c[k] = contrib[e + k];
+    for (e += 8; e + 8 <= e1; e += 8) {
+      float n[8];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) total = total + c[k];
+      for (int k = 0; k < 8; ++k) n[k] = contrib[e + k];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) total = total + c[k];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) c[k] = n[k];
     }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) total = total + c[k];
   }
   for (; e + 4 <= e1; e += 4) {
     float c[4];
@@ -531,46 +602,21 @@ __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e
   return total;
 }
 
-template <int MODE>
-__global__ __launch_bounds__(1024) void muscle_world_kernel(MwArgs a) {
+// TRIPS: entries that a thread keeps in registers, nentry <= TRIPS * kMwThreads; 0: more
+// entries than that, read from the lists for every world.
+template <int MODE, int TRIPS>
+__global__ __launch_bounds__(kMwThreads, 6) void muscle_world_kernel(MwArgs a) {
   extern __shared__ float lds[];
   MwLds l;
   l.segd = lds;
   l.contrib = l.segd + 9 * a.nseg;
   l.axis = l.contrib + a.nentry + kContribPad;
-  l.force = l.axis + 6 * a.ntorque;
-  l.gout = l.force + a.nmuscle;
-  l.rowid = (unsigned short *)(lds + mw_lds_floats<MODE>(a));
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int64_t w = blockIdx.x;
-  const float *wp = a.g.wp + w * a.g.ldw, *com = a.g.com + w * a.g.ldc, *cdof = a.g.cdof + w * a.g.ldd;
-  for (int sg = tid; sg < a.nseg; sg += nt) {
-    const V3 p0 = ld3(wp + 3 * a.s.p0[sg]), p1 = ld3(wp + 3 * a.s.p1[sg]);
-    const V3 c0 = ld3(com + 3 * a.s.b0[sg]), c1 = ld3(com + 3 * a.s.b1[sg]);
-    const V3 seg = sub(p1, p0);
-    const float len = length(seg);
-    const bool ok = !(len < 1.0e-8f);
-    const V3 r0 = sub(p0, c0), r1 = sub(p1, c1);
-    // a degenerate segment contributes nothing: with a zero direction its entries come out as
-    // +-0, and adding +-0 to a sum that started at +0 leaves every bit of it
-    float *o = l.segd + 9 * sg;
-    o[0] = ok ? seg.x / len : 0.0f;
-    o[1] = ok ? seg.y / len : 0.0f;
-    o[2] = ok ? seg.z / len : 0.0f;
-    o[3] = r0.x; o[4] = r0.y; o[5] = r0.z;
-    o[6] = r1.x; o[7] = r1.y; o[8] = r1.z;
-  }
-  for (int i = tid; i < 6 * a.ntorque; i += nt) l.axis[i] = cdof[6 * a.root + i];
-  for (int m = tid; m < a.nmuscle; m += nt) {
-    float f = a.unit[w * a.ldu + m];
-    if (MODE == MW_FORWARD) {
-      f = f * a.act[w * a.lda + m];
-      if (a.passive) f = f + a.passive[w * a.ldpa + m];
-    }
-    l.force[m] = f;
-  }
-  if (MODE == MW_GRAD)
-    for (int j = tid; j < a.ntorque; j += nt) l.gout[j] = a.gout[w * a.ldg + j];
+  l.force = l.axis + kAxis * a.ntorque;
+  l.rowid = (unsigned short *)(TRIPS ? l.contrib : lds + mw_lds_floats(a));
+  constexpr int nt = kMwThreads;
+  const int tid = threadIdx.x;
+  // staging starts at the last wavefront: the first one's sums of the world before take longest
+  const int rid = nt - 1 - tid;
   if (a.nentry < 32 * a.nrow) {  // short rows: a thread writes its row's
     for (int r = tid; r < a.nrow; r += nt)
       for (int e = a.offsets[r]; e < a.offsets[r + 1]; ++e) l.rowid[e] = (unsigned short)r;
@@ -578,63 +624,115 @@ __global__ __launch_bounds__(1024) void muscle_world_kernel(MwArgs a) {
     for (int r = tid >> 6; r < a.nrow; r += nt >> 6)
       for (int e = a.offsets[r] + (tid & 63); e < a.offsets[r + 1]; e += 64) l.rowid[e] = (unsigned short)r;
   }
-  __syncthreads();
-  // four entries per thread and trip while whole trips remain (all their loads are issued
-  // before the first is needed), then one entry per thread
-  int base = 0;
-  for (; base + 4 * nt <= a.nentry; base += 4 * nt) {
-    MwEntry t[4];
-    float c[4];
+  MwEntry kept[TRIPS ? TRIPS : 1];
+  if (TRIPS) {
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 4; ++k) t[k] = load_entry<MODE>(a, l, base + k * nt + tid);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) c[k] = entry_contribution<MODE>(a, l, t[k]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) l.contrib[base + k * nt + tid] = c[k];
+    for (int k = 0; k < TRIPS; ++k) {
+      kept[k] = load_entry<MODE>(a, l, lds, min(k * nt + tid, a.nentry - 1));
+      if (k % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+    // contrib takes the rows' place only behind the first world's barrier
   }
-  for (int e = base + tid; e < a.nentry; e += nt)
-    l.contrib[e] = entry_contribution<MODE>(a, l, load_entry<MODE>(a, l, e));
-  __syncthreads();
-  const float *contrib = l.contrib;
-  for (int r = tid; r < a.nrow; r += nt) {
-    const int e0 = a.offsets[r], e1 = a.offsets[r + 1];
-    if (MODE == MW_FORWARD) {
-      a.out0[w * a.ldo + r] = ordered_sum<true>(contrib, e0, e1);
-    } else if (MODE == MW_MOMENT) {  // a (muscle, dof) pair has a few segments
-      a.out0[w * a.ldo + r] = ordered_sum<false>(contrib, e0, e1);
-    } else if (MODE == MW_GRAD) {
-      // The one-thread-per-muscle kernel leaves 0 for a muscle without force; its entries are
-      // 0 here as well (gout * 0), but an infinite gout would turn them into NaN
-      a.out0[w * a.ldo + r] = l.force[r] != 0.0f ? ordered_sum<true>(contrib, e0, e1) : 0.0f;
+  for (int64_t w = blockIdx.x; w < a.nworld; w += gridDim.x) {
+    const float *wp = a.g.wp + w * a.g.ldw, *com = a.g.com + w * a.g.ldc, *cdof = a.g.cdof + w * a.g.ldd;
+    for (int sg = rid; sg < a.nseg; sg += nt) {
+      const V3 p0 = ld3(wp + 3 * a.s.p0[sg]), p1 = ld3(wp + 3 * a.s.p1[sg]);
+      const V3 c0 = ld3(com + 3 * a.s.b0[sg]), c1 = ld3(com + 3 * a.s.b1[sg]);
+      const V3 seg = sub(p1, p0);
+      const float len = length(seg);
+      const bool ok = !(len < 1.0e-8f);
+      const V3 r0 = sub(p0, c0), r1 = sub(p1, c1);
+      // a degenerate segment contributes nothing: with a zero direction its entries come out as
+      // +-0, and adding +-0 to a sum that started at +0 leaves every bit of it
+      float *o = l.segd + 9 * sg;
+      o[0] = ok ? seg.x / len : 0.0f;
+      o[1] = ok ? seg.y / len : 0.0f;
+      o[2] = ok ? seg.z / len : 0.0f;
+      o[3] = r0.x; o[4] = r0.y; o[5] = r0.z;
+      o[6] = r1.x; o[7] = r1.y; o[8] = r1.z;
+    }
+    for (int i = rid; i < 6 * a.ntorque; i += nt) l.axis[i + i / 6] = cdof[6 * a.root + i];
+    // MW_GRAD reads force[r] in its sums of the world before: by the thread that overwrites it here
+    for (int m = MODE == MW_GRAD ? tid : rid; m < a.nmuscle; m += nt) {
+      float f = a.unit[w * a.ldu + m];
+      if (MODE == MW_FORWARD) {
+        f = f * a.act[w * a.lda + m];
+        if (a.passive) f = f + a.passive[w * a.ldpa + m];
+      }
+      l.force[m] = f;
+    }
+    if (MODE == MW_GRAD)
+      for (int j = tid; j < a.ntorque; j += nt) l.axis[kAxis * j + 6] = a.gout[w * a.ldg + j];
+    __syncthreads();
+    if (TRIPS) {
+#pragma unroll
+      for (int k = 0; k < TRIPS; ++k) {
+        const float c = entry_contribution<MODE>(lds, kept[k]);
+        if (k * nt + tid < a.nentry) l.contrib[k * nt + tid] = c;
+      }
     } else {
-      int current = -1;
-      float total = 0.0f, lo = 0.0f, hi = 0.0f;
-      for (int e = e0; e < e1; ++e) {
-        const int m = a.e_other[e];
-        if (current >= 0 && m != current) {
+      // four entries per thread and trip while whole trips remain (all their loads are issued
+      // before the first is needed), then one entry per thread
+      int base = 0;
+      for (; base + 4 * nt <= a.nentry; base += 4 * nt) {
+        MwEntry t[4];
+        float c[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[k] = load_entry<MODE>(a, l, lds, base + k * nt + tid);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) c[k] = entry_contribution<MODE>(lds, t[k]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) l.contrib[base + k * nt + tid] = c[k];
+      }
+      for (int e = base + tid; e < a.nentry; e += nt)
+        l.contrib[e] = entry_contribution<MODE>(lds, load_entry<MODE>(a, l, lds, e));
+    }
+    __syncthreads();
+    const float *contrib = l.contrib;
+    for (int r = tid; r < a.nrow; r += nt) {
+      const int e0 = a.offsets[r], e1 = a.offsets[r + 1];
+      if (MODE == MW_FORWARD) {
+        a.out0[w * a.ldo + r] = ordered_sum<true>(contrib, e0, e1);
+      } else if (MODE == MW_MOMENT) {  // a (muscle, dof) pair has a few segments
+        a.out0[w * a.ldo + r] = ordered_sum<false>(contrib, e0, e1);
+      } else if (MODE == MW_GRAD) {
+        // The one-thread-per-muscle kernel leaves 0 for a muscle without force; its entries are
+        // 0 here as well (gout * 0), but an infinite gout would turn them into NaN
+        a.out0[w * a.ldo + r] = l.force[r] != 0.0f ? ordered_sum<true>(contrib, e0, e1) : 0.0f;
+      } else {
+        int current = -1;
+        float total = 0.0f, lo = 0.0f, hi = 0.0f;
+        for (int e = e0; e < e1; ++e) {
+          const int m = a.e_other[e];
+          if (current >= 0 && m != current) {
+            if (total < 0.0f) lo = lo + total;
+            else hi = hi + total;
+            total = 0.0f;
+          }
+          current = m;
+          total = total + contrib[e];
+        }
+        if (current >= 0) {
           if (total < 0.0f) lo = lo + total;
           else hi = hi + total;
-          total = 0.0f;
         }
-        current = m;
-        total = total + contrib[e];
+        a.out0[w * a.ldo + r] = lo;
+        a.out1[w * a.ldo + r] = hi;
       }
-      if (current >= 0) {
-        if (total < 0.0f) lo = lo + total;
-        else hi = hi + total;
-      }
-      a.out0[w * a.ldo + r] = lo;
-      a.out1[w * a.ldo + r] = hi;
     }
   }
 }
 
-// Launches the workgroup-per-world kernel when a world's segments and entries fit in LDS and
-// the entry list states the range of its `other` column; returns false for the caller to use
-// the one-thread-per-output kernel instead.
+// Launches the workgroup-per-world kernel when a world's segments and entries fit in LDS (which
+// also keeps the records' word indices below 16 bits) and the entry list states the range of its
+// `other` column; returns false for the caller to use the one-thread-per-output kernel instead.
 template <int MODE>
-bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
-  const size_t lds_bytes = 4 * mw_lds_floats<MODE>(a) + 2 * (((size_t)a.nentry + 1) & ~(size_t)1);
+bool launch_world(MwArgs a, int nworld, hipStream_t stream) {
+  // six entries per thread are 24 registers beside the evaluation's, what 6 wavefronts per SIMD leave;
+  // more entries (about 295 muscles) are read from the lists by every world
+  const int trips = a.nentry <= 2 * kMwThreads ? 2 : a.nentry <= 4 * kMwThreads ? 4 : a.nentry <= 6 * kMwThreads ? 6 : 0;
+  const size_t lds_bytes = 4 * mw_lds_floats(a) + (trips ? 0 : 2 * (((size_t)a.nentry + 1) & ~(size_t)1));
   static const bool forced_off = [] {
     const char *e = std::getenv("IMHIP_MUSCLE_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
@@ -642,7 +740,12 @@ bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
   if (forced_off || lds_bytes > 64 * 1024 || a.nentry == 0 || a.nseg == 0 || a.nrow > 65535 ||
       a.ntorque <= 0 || (MODE != MW_MOMENT && a.nmuscle <= 0))
     return false;
-  hipLaunchKernelGGL(muscle_world_kernel<MODE>, dim3((unsigned)nworld), dim3(512), lds_bytes, stream, a);
+  a.nworld = nworld;
+  // as many workgroups as are resident at once: 24 wavefronts per CU by registers, or what the LDS holds
+  const int by_lds = (int)(160 * 1024 / ((lds_bytes + 1279) / 1280 * 1280)), resident = 256 * std::min(2, by_lds);
+  auto kernel = trips == 2 ? muscle_world_kernel<MODE, 2> : trips == 4 ? muscle_world_kernel<MODE, 4>
+              : trips == 6 ? muscle_world_kernel<MODE, 6> : muscle_world_kernel<MODE, 0>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(nworld, resident)), dim3(kMwThreads), lds_bytes, stream, a);
   return true;
 }
 
@@ -741,15 +844,19 @@ extern "C" int im_muscle_force_velocity_state(
     const char *e = std::getenv("IMHIP_MUSCLE_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  const int64_t staged_words = ld_waypoints + ld_moment + ld_qvel;
-  if (!forced_off && ld_waypoints > 0 && ld_moment > 0 && ld_qvel > 0 && staged_words * 4 <= 64 * 1024) {
-    const int threads = 256;  // measured at 284 muscles: 45 us; 192 threads (two even passes) 49 us, 320 (one pass) 52 us
-    hipLaunchKernelGGL(force_velocity_state_world_kernel, dim3((unsigned)nworld), dim3(threads), (size_t)staged_words * 4,
-                       (hipStream_t)stream, waypoints, ld_waypoints, (int)ld_waypoints, muscle_waypoint_start,
+  // (beside the distances, the entries' dofs and a cosine per muscle)
+  const FvLds n{(int)std::min<int64_t>(ld_waypoints, 1 << 20), (int)std::min<int64_t>(ld_moment, 1 << 20),
+                (int)std::min<int64_t>(ld_qvel, 1 << 20), nmuscle};
+  if (!forced_off && ld_waypoints > 0 && ld_moment > 0 && ld_qvel > 0 && nmuscle <= 16 * 1024 && n.bytes() <= 128 * 1024) {
+    if (n.bytes() > 64 * 1024)
+      IM_HIP_CHECK(hipFuncSetAttribute((const void *)force_velocity_state_world_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, n.bytes()));
+    const int resident = 256 * std::min(32 / (kFvThreads / 64), 160 * 1024 / ((n.bytes() + 1279) / 1280 * 1280));
+    hipLaunchKernelGGL(force_velocity_state_world_kernel, dim3((unsigned)std::min(nworld, resident)), dim3(kFvThreads),
+                       (size_t)n.bytes(), (hipStream_t)stream, waypoints, ld_waypoints, muscle_waypoint_start,
                        muscle_params, ld_params, muscle_rest_length, force_velocity_length_scale, activation,
-                       ld_activation, qvel, ld_qvel, (int)ld_qvel, moment, ld_moment, (int)ld_moment, muscle_dof_offsets,
-                       muscle_dof_torque_idx, root_dof_count, *model, *fv, nmuscle, muscle_length, effective_activation,
-                       length_velocity, force_velocity_multiplier, force_velocity_slope, ld_out);
+                       ld_activation, qvel, ld_qvel, moment, ld_moment, muscle_dof_offsets, muscle_dof_torque_idx,
+                       root_dof_count, *model, *fv, n, muscle_length, effective_activation, length_velocity,
+                       force_velocity_multiplier, force_velocity_slope, ld_out, nworld);
     IM_HIP_CHECK(hipGetLastError());
     return IM_OK;
   }

@@ -224,3 +224,33 @@ def test_gpu_force_velocity_state(device, active_type):
     np.testing.assert_allclose(outs[4].cpu().numpy(), want[4], rtol=2e-6, atol=1e-6 * np.abs(want[4]).max())
     assert (want[4] == 0).any() and (want[4] != 0).any()
     np.testing.assert_array_equal(outs[4].cpu().numpy() == 0, want[4] == 0)  # the curve's flat parts are exact
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pad", [3, 12001])
+def test_gpu_force_velocity_state_of_many_worlds(device, pad):
+    """More worlds than resident workgroups, and rows that are columns of wider arrays (the last
+    world's row ends with the array; the long stride asks for more than 64 KB of LDS): length, activation, velocity and multiplier bit for bit."""
+    import torch
+
+    n = 2100
+    c = _fv_case(n, active_type=1.0)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+
+    def wide(a):
+        b = torch.full((a.shape[0], a.shape[1] + pad), float("nan"), device=device)
+        b[:, pad:] = t(a)
+        return b[:, pad:]
+
+    outs = [torch.full((n, 37), float("nan"), device=device) for _ in range(5)]
+    Q.eval_muscle_force_velocity_state(
+        t(c["waypoints"]), t(c["wp_start"]), t(c["params"]), t(c["rest"]), t(c["length_scale"]), wide(c["act"]), t(c["qvel"]),
+        wide(c["moment"]), t(c["dof_offsets"]), t(c["dof_torque"]), c["root"], muscle_force_scale=float(c["model"][0]),
+        muscle_length_norm_min=float(c["model"][1]), muscle_length_norm_max=float(c["model"][2]), vmax=1.5, fvmax=1.4,
+        clamp_activation=True, include_active=True, active_force_model_params=c["model"][3:6],
+        muscle_length=outs[0], effective_activation=outs[1], length_velocity=outs[2], force_velocity_multiplier=outs[3],
+        force_velocity_slope=outs[4],
+    )  # fmt: skip
+    want = R.muscle_force_velocity_state(**c)
+    for k in range(4):
+        np.testing.assert_array_equal(outs[k].cpu().numpy(), want[k])

@@ -633,3 +633,29 @@ def test_gpu_entry_lists_without_a_stated_range_take_the_other_kernels():
         e.nother = 0
     for a, b in zip(stated, run()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("muscles", [8, 96, 104, 210, 284, 340])
+def test_gpu_contractions_of_many_worlds_equal_one_world_per_workgroup(muscles):
+    """More worlds than workgroups (a workgroup then takes several, with a remainder), rigs on both
+    sides of the entries a thread keeps (two, four, six; more are read per world): the bits of the
+    one-thread-per-output kernels."""
+    rig = synth.make_muscle_rig(nmuscle=muscles, seed=1003)
+    layer = _gpu_layer(rig)
+    nworld = 1100
+    ctx_d = torch.from_numpy(synth.make_muscle_context(rig, nworld, seed=6)).cuda()
+    act = torch.rand(nworld, rig.muscle_count, device="cuda")
+    act[:, ::7] = 0.0
+    g = torch.randn(nworld, rig.torque_dim, device="cuda")
+
+    def run():
+        mean, _, unit = layer._warp_muscle_dynamics_from_activation_forward(act, ctx_d, include_passive_force=False)
+        lo, hi = layer._compute_activation_torque_bounds_warp(ctx_d, select_active=False)
+        return mean, layer._warp_muscle_dynamics_from_activation_backward(ctx_d, g), layer.eval_muscle_sparse_moment(ctx_d), lo, hi
+
+    kept = run()
+    for e in (layer._torque_entries, layer._muscle_entries, layer._moment_entries):
+        e.nother = 0
+    for a, b in zip(kept, run()):
+        assert torch.equal(a, b)
