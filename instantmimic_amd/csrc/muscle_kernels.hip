@@ -22,31 +22,36 @@ namespace {
 
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-// One workgroup of two wavefronts per world; with 4 nentry + 2 nentry + 4 nmuscle bytes of LDS
-// sixteen and more of them fit a CU, so 4096 worlds are all resident at once.  A and the
-// muscle of every term are first brought into LDS in the order the rows consume them (every
-// lane busy, twelve terms' look-ups in flight per lane), the force row as it is; then lane j of
-// the first wavefront runs row j's chain of fused multiply-adds over consecutive LDS words.
-// Same terms, same order per row as the reference kernel.
-__global__ __launch_bounds__(128) void muscle_project_kernel(
+// One workgroup of four wavefronts per world.  A and the force of every term are first brought
+// into LDS in the order the rows consume them (every lane busy, twelve terms' look-ups in flight
+// per lane); then lane j of the first wavefront runs row j's chain of fused multiply-adds over
+// consecutive LDS words, the next eight terms on their way while these are added.  Same terms,
+// same order per row as the reference kernel.
+// What bounds it is the longest row's chain (hundreds of terms, one after the other) and the
+// staging before it, not the 46 MB: the chain looked a term's muscle up and then its force, two
+// LDS latencies per four terms, and rigs of more than 1536 entries gathered from memory.
+// 2522 entries x 4096 worlds: 36.9 us (two wavefronts, a term's muscle looked up in the chain) -> 23.0.
+constexpr int kProjectThreads = 256;
+__global__ __launch_bounds__(kProjectThreads) void muscle_project_kernel(
     const float *__restrict__ moment, int64_t ldm, const float *__restrict__ force, int64_t ldf,
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ entry_idx,
     const int32_t *__restrict__ entry_muscle, int nentry, int nmuscle, int ntorque, int root,
     float *__restrict__ qfrc, int64_t ldq, int nworld) {
   extern __shared__ float lds[];
-  constexpr int NT = 128, UN = 12;
+  constexpr int NT = kProjectThreads, UN = 12;
   const int tid = threadIdx.x;
   const int64_t w = blockIdx.x;
-  float *av = lds;                                      // [nentry] A[entry_idx[s]]
-  float *fs = av + nentry;                              // [nmuscle] the world's forces
-  unsigned short *ms = (unsigned short *)(fs + nmuscle);  // [nentry] entry_muscle[entry_idx[s]]
+  float *av = lds;           // [nentry] A[entry_idx[s]]
+  float *fv = av + nentry;   // [nentry] the force of its muscle; in between its entry_muscle
+  float *fs = fv + nentry;   // [nmuscle] the world's forces
+  int *ms = (int *)fv;
   const float *mw = moment + w * ldm, *fw = force + w * ldf;
   // Every array is read from memory in its own order (coalesced); the permutation into the
   // rows' order goes through LDS, in place: gather into registers, barrier, write back.
   for (int i = tid; i < nmuscle; i += NT) fs[i] = fw[i];
   if (nentry <= UN * NT) {
     int e[UN], m[UN];
-    float x[UN];
+    float x[UN], f[UN];
 #pragma unroll
     for (int k = 0; k < UN; ++k) {
       const int i = tid + NT * k < nentry ? tid + NT * k : nentry - 1;
@@ -58,23 +63,24 @@ __global__ __launch_bounds__(128) void muscle_project_kernel(
     for (int k = 0; k < UN; ++k)
       if (tid + NT * k < nentry) {
         av[tid + NT * k] = x[k];
-        ms[tid + NT * k] = (unsigned short)m[k];
+        ms[tid + NT * k] = m[k];
       }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < UN; ++k) {
       x[k] = av[e[k]];
-      m[k] = ms[e[k]];
+      f[k] = fs[ms[e[k]]];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < UN; ++k)
       if (tid + NT * k < nentry) {
         av[tid + NT * k] = x[k];
-        ms[tid + NT * k] = (unsigned short)m[k];
+        fv[tid + NT * k] = f[k];
       }
   } else {
     // more entries than one trip holds: gathered from memory, twelve look-ups in flight per lane
+    __syncthreads();
     for (int s0 = tid; s0 < nentry; s0 += UN * NT) {
       int e[UN], m[UN];
       float x[UN];
@@ -89,7 +95,7 @@ __global__ __launch_bounds__(128) void muscle_project_kernel(
       for (int k = 0; k < UN; ++k)
         if (s0 + NT * k < nentry) {
           av[s0 + NT * k] = x[k];
-          ms[s0 + NT * k] = (unsigned short)m[k];
+          fv[s0 + NT * k] = fs[m[k]];
         }
     }
   }
@@ -98,15 +104,23 @@ __global__ __launch_bounds__(128) void muscle_project_kernel(
     float total = 0.0f;
     const int e1 = offsets[j + 1];
     int s = offsets[j];
-    for (; s + 3 < e1; s += 4) {  // four terms' operands read before the first is used
-      const float a0 = av[s], a1 = av[s + 1], a2 = av[s + 2], a3 = av[s + 3];
-      const float f0 = fs[ms[s]], f1 = fs[ms[s + 1]], f2 = fs[ms[s + 2]], f3 = fs[ms[s + 3]];
-      total = fma_(a0, f0, total);
-      total = fma_(a1, f1, total);
-      total = fma_(a2, f2, total);
-      total = fma_(a3, f3, total);
+    if (s + 8 <= e1) {
+      float a[8], f[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) a[k] = av[s + k], f[k] = fv[s + k];
+      for (s += 8; s + 8 <= e1; s += 8) {
+        float an[8], fn[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) an[k] = av[s + k], fn[k] = fv[s + k];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) total = fma_(a[k], f[k], total);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] = an[k], f[k] = fn[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) total = fma_(a[k], f[k], total);
     }
-    for (; s < e1; ++s) total = fma_(av[s], fs[ms[s]], total);
+    for (; s < e1; ++s) total = fma_(av[s], fv[s], total);
     qfrc[w * ldq + root + j] = total;
   }
 }
@@ -183,9 +197,12 @@ int im_muscle_project(const float *moment, int64_t ld_moment, const float *force
   if (!moment || !force || !torque_entry_offsets || !torque_entry_idx || !entry_muscle || !qfrc) return IM_ERR_ARG;
   if (ld_moment < nentry || ld_force < nmuscle || ld_qfrc < root_dof_count + ntorque) return IM_ERR_STRIDE;
   if (nmuscle > 65535) return IM_ERR_UNSUPPORTED;  // muscle ids travel as 16 bits
-  const size_t lds_bytes = sizeof(float) * ((size_t)nentry + nmuscle) + 2 * (((size_t)nentry + 1) & ~(size_t)1);
-  if (lds_bytes > 64 * 1024) return IM_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(im::muscle_project_kernel, dim3(nworld), dim3(128), lds_bytes, (hipStream_t)stream,
+  // the limit is that of a term in six bytes, which a caller has to reckon with; a term takes eight
+  if (sizeof(float) * ((size_t)nentry + nmuscle) + 2 * (((size_t)nentry + 1) & ~(size_t)1) > 64 * 1024) return IM_ERR_UNSUPPORTED;
+  const size_t lds_bytes = sizeof(float) * (2 * (size_t)nentry + nmuscle);
+  if (lds_bytes > 64 * 1024)
+    IM_HIP_CHECK(hipFuncSetAttribute((const void *)im::muscle_project_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+  hipLaunchKernelGGL(im::muscle_project_kernel, dim3(nworld), dim3(im::kProjectThreads), lds_bytes, (hipStream_t)stream,
                      moment, ld_moment, force, ld_force, torque_entry_offsets, torque_entry_idx, entry_muscle,
                      nentry, nmuscle, ntorque, root_dof_count, qfrc, ld_qfrc, nworld);
   IM_HIP_CHECK(hipGetLastError());

@@ -254,3 +254,25 @@ def test_gpu_force_velocity_state_of_many_worlds(device, pad):
     want = R.muscle_force_velocity_state(**c)
     for k in range(4):
         np.testing.assert_array_equal(outs[k].cpu().numpy(), want[k])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("muscles", [30, 690, 1950])
+def test_gpu_projection_staging_sizes(device, muscles):
+    """Rows shorter than eight terms, more than the 3072 entries of one staging trip, and more than
+    64 KB of LDS: bit for bit."""
+    import torch
+
+    nworld = 33
+    mb = synth.make_muscles(nworld, nmuscle=muscles, seed=5)
+    nv = len(synth.csr_from_parents(synth.snu_parents())[0])
+    ent = Q.entries_from_muscle_dofs(mb.muscle_dofs, mb.nmuscle)
+    entries = len(ent.muscle_dof_torque_idx)
+    assert muscles < 600 or entries > 3072
+    assert muscles < 1900 or 4 * (2 * entries + muscles) > 65536 >= 4 * (entries + muscles) + 2 * (entries + 1)
+    offsets, order = Q.torque_sorted_entries(ent.muscle_dof_torque_idx, nv - mb.root_dof_count)
+    t = lambda a, dt=None: torch.from_numpy(np.ascontiguousarray(a if dt is None else a.astype(dt))).to(device)  # noqa: E731
+    qfrc = torch.full((nworld, nv), 7.0, device=device)
+    Q.project_muscle_sparse_moment_qfrc(t(mb.moment), t(mb.force), t(offsets, np.int32), t(order, np.int32), t(ent.muscle_dof_muscle_idx, np.int32), mb.root_dof_count, qfrc)
+    want = R.muscle_project(mb.moment, mb.force, offsets, order, ent.muscle_dof_muscle_idx, mb.root_dof_count, nv)
+    np.testing.assert_array_equal(qfrc.cpu().numpy()[:, mb.root_dof_count :], want[:, mb.root_dof_count :])
