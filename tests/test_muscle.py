@@ -115,8 +115,8 @@ def test_gpu_matches_oracle_bitwise(device, nworld):
 
 @pytest.mark.gpu
 def test_gpu_projection_with_more_entries_than_one_staging_trip(device):
-    """The projection kernel permutes up to 1536 entries through LDS in one trip and gathers
-    larger sets from memory: 420 muscles give about 1900 entries."""
+    """420 muscles give about 1900 entries: several of a thread's twelve places stay empty in the
+    projection kernel's trip through LDS (the sizes beyond one trip are tested below)."""
     import torch
 
     nworld = 97
