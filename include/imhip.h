@@ -1053,7 +1053,8 @@ int im_newton_solve_dense_column(const im_newton_args *args, float *H, float *U,
  * resident loop of im_newton_solve_tree / _sparse / _dense_tile / _dense_column, in which a world
  * that finishes writes qfrc_constraint itself.  The arrays end as after those calls and
  * im_qfrc_constraint_from_grad one after the other, bit for bit.  IM_ERR_UNSUPPORTED where the model
- * has no resident loop: the caller then issues the pieces (which set everything afresh). */
+ * has no resident loop: the caller then issues the pieces (which set everything afresh).  IM_ERR_ARG for a
+ * plan of another model: its dofs must be nv (a sparse plan's padded size nv_pad), its M no longer than nM. */
 typedef struct im_newton_start {
   const float *qacc_start; /* (nworld, ld_start): the warm start, or qacc_smooth */
   int64_t ld_start;

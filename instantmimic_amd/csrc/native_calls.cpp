@@ -198,7 +198,7 @@ PyObject *dense_hessian_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t 
   X(frictionloss) X(aref) X(Ma) X(force) X(state) X(search) X(search_dot) X(mv) X(jv) X(Jaref) X(done) X(alpha)                 \
   X(improvement) X(ls_exhausted) X(quad_changed_ids) X(quad_changed_count) X(state_changed_count) X(search_unchanged) X(grad)   \
   X(grad_dot) X(grad_scale) X(newton_decrement) X(h) X(hfactor) X(newton_tree_scratch) X(sparse_hessian_plan)                   \
-  X(newton_elemid) X(newton_dof_union) X(newton_next_world) X(kernel) X(address) X(path) X(block)
+  X(newton_elemid) X(newton_dof_union) X(newton_next_world) X(kernel) X(address) X(path) X(block) X(nM)
 struct Names {
 #define IM_FIELD(x) PyObject *x = nullptr;
   IM_NAMES(IM_FIELD)
@@ -359,8 +359,10 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   }
   if (tree && plan) return declined();
   if (tree) {
-    k.tree = (const im_tree_plan *)as_address(h.get(h.get(tree, names.kernel), names.address));
-    if (h.missing || !k.tree) return declined();
+    PyObject *kernel = h.get(tree, names.kernel);
+    k.tree = (const im_tree_plan *)as_address(h.get(kernel, names.address));
+    // a plan of another model, or an M shorter than its rows: the Python checks name the error
+    if (h.missing || !k.tree || h.integer(kernel, names.nv) != nv || h.integer(kernel, names.nM) > M->size(1)) return declined();
   } else {
     if (!square(names.hfactor, &k.U) || !rows(ctx, names.newton_dof_union, nv + 1, &k.dof_union)) return declined();
     if (plan) {

@@ -12,6 +12,7 @@
 
 #include "common.h"
 #include "newton_solve.h"
+#include "sparse_plan.h"
 
 namespace im {
 namespace {
@@ -86,6 +87,11 @@ extern "C" int im_newton_solve(const im_newton_args *args, const im_newton_start
                                void *stream) {
   if (!args || !start || !model || !start->qacc_smooth || !start->efc_aref || model->nv <= 0 || model->nM <= 0) return IM_ERR_ARG;
   if (args->iterations <= 0 || (model->tree && model->sparse)) return IM_ERR_ARG;
+  // A plan's kernels take their row lengths from the plan, the start and the arrays from the model: a plan
+  // of other sizes would walk rows of the wrong length.
+  if (model->tree && (model->tree->nv != model->nv || model->tree->nM > model->nM)) return IM_ERR_ARG;
+  if (model->sparse && (model->sparse->nv != model->nv || model->sparse->nv_pad != model->nv_pad || model->sparse->nM > model->nM))
+    return IM_ERR_ARG;
   if (args->nworld == 0) return IM_OK;
   const hipStream_t st = (hipStream_t)stream;
   im::FirstStage first;

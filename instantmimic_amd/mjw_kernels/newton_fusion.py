@@ -529,6 +529,18 @@ def _tree_scratch(ctx):
     return getattr(ctx, "newton_tree_scratch", None) if ctx is not None else None
 
 
+def _check_tree_scratch(m, d, ctx) -> None:
+    """A tree scratch on ``ctx`` against the model and its M, before anything is launched: its kernels
+    take their row lengths from the plan."""
+    scratch = _tree_scratch(ctx)
+    if scratch is None:
+        return
+    if not getattr(scratch, "cuda", False) or scratch.kernel.nv != int(m.nv):
+        raise ValueError("the tree scratch belongs to another model or has no device state")
+    if d.M.dim() != 2 or d.M.shape[1] < scratch.kernel.nM:
+        raise ValueError(f"M must be (nworld, nM) with at least the {scratch.kernel.nM} elements of the tree scratch's plan")
+
+
 def attach_scratch(m, d, ctx, device=None) -> None:
     """Persistent per-world scratch of the fused iteration on ``ctx`` (newton_fusion.py:301-304:
     the dofs the changed rows touch, ``nv`` slots and their count); the dense path's first factor
@@ -630,6 +642,7 @@ def init_context(m, d, ctx, mul_m_call=None) -> None:
     finish at once with ``qacc = qacc_smooth``; ``Jaref = J qacc - aref``; ``Ma = M qacc`` for every
     world; forces and states; the first gradient, Hessian, factor and search direction through the
     sparse plan, the tree stage or the dense path, whichever ``ctx`` carries."""
+    _check_tree_scratch(m, d, ctx)
     first = _init_before_factor(m, d, ctx) if mul_m_call is None else False
     if not first:
         init_empty_worlds(d.nefc, d.qacc_smooth, d.solver_niter, ctx.search_dot, ctx.done, d.qacc)
@@ -803,6 +816,7 @@ def run_resident(m, d, ctx, nsolving, whole: bool = False) -> bool:
 
     import torch
 
+    _check_tree_scratch(m, d, ctx)
     scratch, plan = _tree_scratch(ctx), _fused_plan(ctx)
     dense = scratch is None and plan is None and getattr(ctx, "newton_next_world", None) is not None
     dense_tile = dense and int(m.nv) <= 32
@@ -904,6 +918,7 @@ def solve(m, d, ctx, nsolving, *, mul_m_call=None) -> None:
     otherwise the pieces below."""
     if mul_m_call is None and run_resident(m, d, ctx, nsolving, True):
         return
+    _check_tree_scratch(m, d, ctx)
     flags = getattr(m.opt, "disableflags", 0)
     warmstart = not (int(flags) & DISABLE_WARMSTART) and getattr(d, "qacc_warmstart", None) is not None
     d.qacc.copy_(d.qacc_warmstart if warmstart else d.qacc_smooth)

@@ -213,6 +213,29 @@ def test_init_context_entry_point_checks_its_arguments_before_any_launch():
     assert lib.im_newton_solve_sparse(None, C.byref(_newton_args()), one, one, None) == _lib.IM_ERR_ARG
 
 
+def test_whole_solve_refuses_a_plan_of_another_model():
+    """The tree's or the sparse plan's sizes against the model's, on the host, before the plan's device
+    state is looked at: a plan of other sizes takes rows of another length."""
+    lib = _lib.lib()
+    shapes = {n: synth.csr_from_parents(p) for n, p in (("ant", synth.ant_parents()), ("humanoid", synth.SHAPES["humanoid"].parents))}
+    start, model = _lib.NewtonStart(), _lib.NewtonModel()
+    for name in ("qacc_start", "qacc_smooth", "efc_aref", "H", "U", "elemid", "dof_union", "next_world"):
+        setattr(start if hasattr(start, name) else model, name, 16)
+    start.ld_start, start.ld_smooth, start.ld_aref = 27, 27, 64
+    model.nv, model.nv_pad, model.nM = 27, 32, 243
+    solve = lambda: lib.im_newton_solve(C.byref(_newton_args()), C.byref(start), C.byref(model), None)  # noqa: E731
+    for name, want in (("humanoid", _lib.IM_ERR_UNSUPPORTED), ("ant", _lib.IM_ERR_ARG)):  # (a host-only plan launches nothing)
+        rowadr, rownnz, colind = shapes[name]
+        handle = C.c_void_p()
+        assert lib.im_tree_plan_create(int(rowadr.size), rowadr.ctypes.data, rownnz.ctypes.data, colind.ctypes.data, int(colind.size), 0, 1, C.byref(handle)) == _lib.IM_OK
+        model.tree = handle.value
+        assert solve() == want, name
+        model.nM = 242  # an M shorter than the humanoid plan's rows
+        assert solve() == _lib.IM_ERR_ARG, name
+        model.nM, model.tree = 243, None
+        lib.im_tree_plan_destroy(handle)
+
+
 def test_dense_init_entry_point_checks_its_arguments_before_any_launch():
     lib = _lib.lib()
     one = 16
