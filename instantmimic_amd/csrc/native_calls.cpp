@@ -36,11 +36,15 @@ int unlocked(F &&launch) {
   PyEval_RestoreThread(state);
   return status;
 }
+// Whatever Python exception a declined argument left behind goes: the caller's own checks raise theirs.
+PyObject *declined() {
+  PyErr_Clear();
+  return PyLong_FromLong(-1);
+}
 PyObject *answer(int status) {
   if (status == IM_OK) Py_RETURN_NONE;
-  return PyLong_FromLong(status);
+  return status < 0 ? declined() : PyLong_FromLong(status);
 }
-PyObject *declined() { return PyLong_FromLong(-1); }
 
 // The checks of one call: every tensor on the first one's device, which is the current one.
 struct Call {
@@ -86,10 +90,13 @@ T *ptr(const Tensor *t) { return (T *)t->data_ptr(); }
 template <class T = float>
 T *ptr_or_null(const Tensor *t) { return t ? (T *)t->data_ptr() : nullptr; }
 
-int64_t as_int(PyObject *o) {
-  const int64_t v = PyLong_AsLongLong(o);
-  if (v == -1 && PyErr_Occurred()) PyErr_Clear();
-  return v;
+// An integer, or an object that stands for one (__index__).  False for anything else: a float, say,
+// which the Python callers convert.
+bool as_int(PyObject *o, int64_t *v) {
+  *v = PyLong_AsLongLong(o);
+  if (*v != -1 || !PyErr_Occurred()) return true;
+  PyErr_Clear();
+  return false;
 }
 void *as_address(PyObject *o) {
   void *p = PyLong_AsVoidPtr(o);
@@ -103,7 +110,8 @@ void *as_address(PyObject *o) {
 PyObject *tree_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 6) return declined();
   const auto *plan = (const im_tree_plan *)as_address(a[0]);
-  const int64_t nv = as_int(a[1]), nM = as_int(a[2]);
+  int64_t nv, nM;
+  if (!as_int(a[1], &nv) || !as_int(a[2], &nM)) return declined();
   const Tensor *M = tensor_of(a[3]), *x = tensor_of(a[4]), *y = tensor_of(a[5]);
   Call c;
   if (!plan || !c.rows(M, -1, nM) || !c.rows(x, M->size(0), nv) || !c.rows(y, M->size(0), nv)) return declined();
@@ -117,7 +125,9 @@ PyObject *tree_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *assemble_tree_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 12) return declined();
   const auto *plan = (const im_tree_plan *)as_address(a[0]);
-  const int64_t nv = as_int(a[1]), nM = as_int(a[2]);
+  int64_t nv, nM, quad;
+  const int negate = PyObject_IsTrue(a[10]);
+  if (!as_int(a[1], &nv) || !as_int(a[2], &nM) || negate < 0 || !as_int(a[11], &quad)) return declined();
   const Tensor *M = tensor_of(a[3]), *J = tensor_of(a[4]), *D = tensor_of(a[5]), *state = tensor_of(a[6]), *nefc = tensor_of(a[7]),
                *grad = tensor_of(a[8]), *x = tensor_of(a[9]);
   Call c;
@@ -132,11 +142,10 @@ PyObject *assemble_tree_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t 
       !c.rows(x, nworld, nv))
     return declined();
   void *const stream = c.stream();
-  const int quad = (int)as_int(a[11]);
-  const unsigned flags = PyObject_IsTrue(a[10]) == 1 ? IM_FLAG_NEGATE : 0;
+  const unsigned flags = negate ? IM_FLAG_NEGATE : 0;
   return answer(unlocked([&] {
     return im_assemble_tree_ldl_solve(plan, ptr(M), M->stride(0), ptr(J), (int)njmax, ptr(D), ptr<int32_t>(state),
-                                           ptr_or_null<int32_t>(nefc), quad, ptr(grad), grad->stride(0), ptr(x),
+                                           ptr_or_null<int32_t>(nefc), (int)quad, ptr(grad), grad->stride(0), ptr(x),
                                            x->stride(0), nullptr, (int)nworld, flags, stream);
   }));
 }
@@ -146,7 +155,8 @@ PyObject *assemble_tree_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t 
 // (nworld, nv, pad, block, nM, indices, U, M, x, y)
 PyObject *blocked_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 10) return declined();
-  const int64_t nworld = as_int(a[0]), nv = as_int(a[1]), pad = as_int(a[2]), block = as_int(a[3]), nM = as_int(a[4]);
+  int64_t nworld, nv, pad, block, nM;
+  if (!as_int(a[0], &nworld) || !as_int(a[1], &nv) || !as_int(a[2], &pad) || !as_int(a[3], &block) || !as_int(a[4], &nM)) return declined();
   const Tensor *indices = tensor_of(a[5]), *U = tensor_of(a[6]), *M = tensor_of(a[7]), *x = tensor_of(a[8]), *y = tensor_of(a[9]);
   Call c;
   int64_t ldx = 0, ldy = 0;
@@ -166,7 +176,8 @@ PyObject *dense_hessian_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t 
   const Tensor *M = tensor_of(a[0]), *J = tensor_of(a[1]), *D = tensor_of(a[2]), *state = tensor_of(a[3]), *nefc = tensor_of(a[4]),
                *H = tensor_of(a[5]), *y = tensor_of(a[6]), *x = tensor_of(a[7]), *U = tensor_of(a[8]);
   Call c;
-  if (!c.on(J, at::kFloat) || J->dim() != 3 || !J->is_contiguous() || J->size(1) < 1 || (!nefc && a[4] != Py_None) || (!H && a[5] != Py_None) ||
+  int64_t quad;
+  if (!as_int(a[9], &quad) || !c.on(J, at::kFloat) || J->dim() != 3 || !J->is_contiguous() || J->size(1) < 1 || (!nefc && a[4] != Py_None) || (!H && a[5] != Py_None) ||
       (!U && a[8] != Py_None))
     return declined();
   const int64_t nworld = J->size(0), njmax = J->size(1), nv = J->size(2), pad = (nv + 15) / 16 * 16;
@@ -181,9 +192,8 @@ PyObject *dense_hessian_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t 
   if (H && (H->dim() != 3 || H->size(1) < nv || H->size(1) != H->size(2) || !c.whole(H, at::kFloat, nworld * H->size(1) * H->size(1))))
     return declined();
   void *const stream = c.stream();
-  const int quad = (int)as_int(a[9]);
   return answer(unlocked([&] {
-    return im_jtdj_factor_solve(ptr(M), ptr(J), (int)njmax, ptr(D), ptr<int32_t>(state), ptr_or_null<int32_t>(nefc), quad,
+    return im_jtdj_factor_solve(ptr(M), ptr(J), (int)njmax, ptr(D), ptr<int32_t>(state), ptr_or_null<int32_t>(nefc), (int)quad,
                                      ptr_or_null(H), (int)nv, H ? (int)H->size(1) : 0, ptr(y), ldy, ptr_or_null(U), (int)pad, ptr(x), ldx,
                                      (int)nworld, stream);
   }));
@@ -249,11 +259,8 @@ struct Holder {
   int64_t integer(PyObject *from, PyObject *name, bool optional = false, int64_t otherwise = 0) {
     PyObject *v = get(from, name, optional);
     if (!v) return otherwise;
-    const int64_t i = PyLong_AsLongLong(v);
-    if (i == -1 && PyErr_Occurred()) {
-      PyErr_Clear();
-      missing = true;
-    }
+    int64_t i;
+    if (!as_int(v, &i)) missing = true;
     return i;
   }
 };
@@ -264,6 +271,8 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const char *form = std::getenv("IMHIP_NEWTON");
   if (form && std::strcmp(form, "stages") == 0) return declined();
   PyObject *m = a[0], *d = a[1], *ctx = a[2];
+  int64_t no_warmstart, ls_bit, iterations_bit;
+  if (!as_int(a[4], &no_warmstart) || !as_int(a[5], &ls_bit) || !as_int(a[6], &iterations_bit)) return declined();
   Holder h;
   Call c;
   im_newton_args p{};
@@ -292,7 +301,7 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const int64_t flags = h.integer(opt, names.disableflags, true);
   p.block = 64;
   if (pad < 64) p.block = (int32_t)h.integer(h.get(m, names.block_dim), names.linesearch_iterative);
-  p.quad = 1, p.ls_overflow_bit = (int32_t)as_int(a[5]), p.iterations_overflow_bit = (int32_t)as_int(a[6]);
+  p.quad = 1, p.ls_overflow_bit = (int32_t)ls_bit, p.iterations_overflow_bit = (int32_t)iterations_bit;
   const Tensor *radr = h.tensor(m, names.M_mulm_rowadr), *col = h.tensor(m, names.M_mulm_col), *madr = h.tensor(m, names.M_mulm_madr);
   if (h.missing || p.iterations <= 0 || !c.whole(radr, at::kInt, nv + 1) || !c.whole(col, at::kInt, col->numel()) ||
       !c.whole(madr, at::kInt, col->numel()))
@@ -337,7 +346,7 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   p.nsolving = ptr<int32_t>(left);
   // the start
   const Tensor *smooth = h.tensor(d, names.qacc_smooth), *aref = h.tensor(efc, names.aref);
-  const Tensor *warm = (flags & as_int(a[4])) ? nullptr : h.maybe_tensor(d, names.qacc_warmstart);
+  const Tensor *warm = (flags & no_warmstart) ? nullptr : h.maybe_tensor(d, names.qacc_warmstart);
   if (h.missing || !c.rows(smooth, nworld, nv) || !c.rows(aref, nworld, njmax) || (warm && !c.rows(warm, nworld, nv)) ||
       smooth->size(1) != nv || (warm && warm->size(1) != nv))
     return declined();

@@ -3,8 +3,10 @@ take at once: views with a row stride run, and wrong dtypes, shapes and layouts 
 
 import numpy as np
 import pytest
+import torch
 
 from instantmimic_amd import synth
+from instantmimic_amd.mjw_kernels import blocked_dense as BD
 from instantmimic_amd.mjw_kernels import newton_fusion as NF
 from instantmimic_amd.mjw_kernels import tree_ldl as T
 from oracle import planner as P
@@ -18,8 +20,6 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nworld", [1, 5, 257])
 @pytest.mark.parametrize("layout", ["contiguous", "row stride", "no nefc"])
 def test_gpu_assemble_and_solve_take_any_row_stride(device, nworld, layout):
-    import torch
-
     b = synth.make_batch("humanoid", nworld)
     nv, nM = b.shape.nv, b.colind.size
     sc = T.create_tree_factor_solve_scratch(type("m", (), dict(nv=nv, M_rowadr=b.rowadr, M_rownnz=b.rownnz, M_colind=b.colind)), device)
@@ -42,8 +42,6 @@ def test_gpu_assemble_and_solve_take_any_row_stride(device, nworld, layout):
 
 
 def test_gpu_the_python_checks_still_name_the_error(device):
-    import torch
-
     b = synth.make_batch("humanoid", 8)
     nv = b.shape.nv
     sc = T.create_tree_factor_solve_scratch(type("m", (), dict(nv=nv, M_rowadr=b.rowadr, M_rownnz=b.rownnz, M_colind=b.colind)), device)
@@ -65,14 +63,10 @@ def test_gpu_the_python_checks_still_name_the_error(device):
 
 
 def _snapshot(d, ctx):
-    import torch
-
     return {k: v.clone() for o in (d, d.efc, ctx) for k, v in vars(o).items() if isinstance(v, torch.Tensor)}
 
 
 def _same(before, d, ctx):
-    import torch
-
     return all(torch.equal(torch.nan_to_num(before[k]) if before[k].is_floating_point() else before[k],
                            torch.nan_to_num(v) if v.is_floating_point() else v)
                for o in (d, d.efc, ctx) for k, v in vars(o).items() if isinstance(v, torch.Tensor))  # fmt: skip
@@ -97,3 +91,51 @@ def test_gpu_newton_with_a_tree_scratch_of_another_model(device, call):
     with pytest.raises(ValueError, match="elements"):
         go(m, d, ctx, left)
     assert _same(before, d, ctx) and int(left.item()) == 0
+
+
+def _linear_step(device, nworld=5):
+    b = synth.make_batch("humanoid", nworld)
+    m = type("m", (), dict(nv=b.shape.nv, M_rowadr=b.rowadr, M_rownnz=b.rownnz, M_colind=b.colind))
+    up = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    return T.create_tree_factor_solve_scratch(m, device), [up(a) for a in (b.M, b.J, b.D, b.state[0], b.nefc, b.grad)]
+
+
+def _dense_step(device, nv=35, rows=40, nworld=5, seed=3):
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    a = torch.randn((nworld, nv, nv), generator=g) * 0.2
+    M = (a @ a.transpose(1, 2).contiguous() + torch.eye(nv)).to(device)
+    J, D = torch.randn((nworld, rows, nv), generator=g).to(device), (torch.rand((nworld, rows), generator=g) + 0.5).to(device)
+    state = torch.randint(0, 2, (nworld, rows), generator=g, dtype=torch.int32).to(device)
+    nefc = torch.full((nworld,), rows - 3, dtype=torch.int32, device=device)
+    return [M, J, D, state, nefc, torch.randn((nworld, nv), generator=g).to(device)]
+
+
+@pytest.mark.parametrize("one", [1.0, np.float32(1.0), np.int64(1), True, torch.tensor(1), torch.tensor(1.0)], ids=repr)
+def test_gpu_quad_is_converted_as_int_does(device, one):
+    """``quad`` goes through ``int()``: any number that equals the state selects its rows."""
+    sc, (M, J, D, state, nefc, grad) = _linear_step(device)
+    x, want = torch.zeros_like(grad), torch.zeros_like(grad)
+    T.assemble_tree_factor_solve(sc, M, J, D, state, nefc, grad, want, quad=1)
+    T.assemble_tree_factor_solve(sc, M, J, D, state, nefc, grad, x, quad=one)
+    assert torch.equal(x, want)
+    M, J, D, state, nefc, y = _dense_step(device)
+    x, want = torch.zeros_like(y), torch.zeros_like(y)
+    BD.dense_hessian_factor_solve(M, J, D, state, nefc, None, y, want, quad=1)
+    BD.dense_hessian_factor_solve(M, J, D, state, nefc, None, y, x, quad=one)
+    assert torch.equal(x, want)
+
+
+def test_gpu_arguments_that_are_no_numbers_raise_their_own_error(device):
+    sc, (M, J, D, state, nefc, grad) = _linear_step(device)
+    x = torch.full_like(grad, 7.0)
+    for wrong in ("one", None):
+        with pytest.raises((TypeError, ValueError)):
+            T.assemble_tree_factor_solve(sc, M, J, D, state, nefc, grad, x, quad=wrong)
+
+    class Undecided:
+        def __bool__(self):
+            raise LookupError("neither")
+
+    with pytest.raises(LookupError, match="neither"):
+        T.assemble_tree_factor_solve(sc, M, J, D, state, nefc, grad, x, negate=Undecided())
+    assert bool((x == 7.0).all())
