@@ -246,9 +246,9 @@ __global__ __launch_bounds__(256) void force_velocity_state_kernel(
 // lane) -> 38.9; 256 threads 48.4, 512 threads 52.7.
 constexpr int kFvThreads = 320;
 struct FvLds {
-  int words_wp, nentry, nqvel, nmuscle;  // the longest rows that are staged
+  int words_wp, nentry, nqvel, nmuscle;  // the longest rows that fit; what is read of them is what the tables name
   __host__ __device__ int bytes() const {
-    return 4 * (words_wp + nentry + nqvel + words_wp / 3 + nmuscle) + 2 * ((nentry + 1) & ~1);
+    return 4 * (words_wp + nentry + nqvel + words_wp / 3 + nmuscle + 1) + 2 * ((nentry + 1) & ~1);
   }
 };
 
@@ -287,18 +287,29 @@ __global__ __launch_bounds__(kFvThreads) void force_velocity_state_world_kernel(
   float *qv = mom + n.nentry;           // its velocities
   float *dist = qv + n.nqvel;           // from every waypoint to the next one
   float *cosp = dist + n.words_wp / 3;  // [nmuscle]
-  unsigned short *dof = (unsigned short *)(cosp + n.nmuscle);  // [nentry]
+  int *named = (int *)(cosp + n.nmuscle);  // the velocities up to the last dof that the tables name
+  unsigned short *dof = (unsigned short *)(named + 1);  // [nentry]
   constexpr int nt = kFvThreads;
   const int tid = threadIdx.x, nmuscle = n.nmuscle;
-  // what the tables name of a row, which may be a part of a wider array's
+  // what the tables name of a row, which may be a part of a wider array's: the last world's row ends
+  // with its last named value, wherever the stride would lead
   const int nwp = min(waypoint_start[nmuscle], n.words_wp / 3), ne = min(dof_offsets[nmuscle], n.nentry);
-  for (int e = tid; e < ne; e += nt) dof[e] = (unsigned short)(dof_torque_idx[e] + root);
+  if (tid == 0) *named = 0;
+  __syncthreads();
+  int most = 0;
+  for (int e = tid; e < ne; e += nt) {
+    const int d = dof_torque_idx[e] + root;
+    dof[e] = (unsigned short)d;
+    most = max(most, d + 1);
+  }
+  for (int o = 32; o; o >>= 1) most = max(most, __shfl_xor(most, o));
+  if ((tid & 63) == 0) atomicMax(named, most);
   for (int m = tid; m < nmuscle; m += nt) cosp[m] = cosf(params[m * ldpar + 3]);
   for (int64_t w = blockIdx.x; w < nworld; w += gridDim.x) {
     __syncthreads();  // the tables are there, the world before is done with
     stage_row(row, wp + w * ldw, 3 * nwp, tid);
     stage_row(mom, moment + w * ldm, ne, tid);
-    stage_row(qv, qvel + w * ldq, n.nqvel, tid);
+    stage_row(qv, qvel + w * ldq, min(__builtin_amdgcn_readfirstlane(*named), n.nqvel), tid);
     __syncthreads();
     for (int i = tid; i < nwp - 1; i += nt) dist[i] = length(sub(ld3(row + 3 * (i + 1)), ld3(row + 3 * i)));
     __syncthreads();
@@ -844,10 +855,12 @@ extern "C" int im_muscle_force_velocity_state(
     const char *e = std::getenv("IMHIP_MUSCLE_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  // (beside the distances, the entries' dofs and a cosine per muscle)
+  // Beside the distances, the entries' dofs and a cosine per muscle.  Up to 80 KB, where a CU holds two
+  // workgroups: 4096 worlds of 284 muscles with velocities in rows of 56 / 8000 / 12000 floats (37 / 69 / 85 KB)
+  // take 38.0 / 53.6 / 92.4 us here and 81 - 83 us on the lane-per-muscle kernel.
   const FvLds n{(int)std::min<int64_t>(ld_waypoints, 1 << 20), (int)std::min<int64_t>(ld_moment, 1 << 20),
                 (int)std::min<int64_t>(ld_qvel, 1 << 20), nmuscle};
-  if (!forced_off && ld_waypoints > 0 && ld_moment > 0 && ld_qvel > 0 && nmuscle <= 16 * 1024 && n.bytes() <= 128 * 1024) {
+  if (!forced_off && ld_waypoints > 0 && ld_moment > 0 && ld_qvel > 0 && nmuscle <= 16 * 1024 && n.bytes() <= 80 * 1024) {
     if (n.bytes() > 64 * 1024)
       IM_HIP_CHECK(hipFuncSetAttribute((const void *)force_velocity_state_world_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, n.bytes()));
     const int resident = 256 * std::min(32 / (kFvThreads / 64), 160 * 1024 / ((n.bytes() + 1279) / 1280 * 1280));

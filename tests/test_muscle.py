@@ -257,6 +257,32 @@ def test_gpu_force_velocity_state_of_many_worlds(device, pad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 67])
+@pytest.mark.parametrize("pad", [3, 12001])
+def test_gpu_force_velocity_state_with_velocities_in_a_wider_array(device, n, pad):
+    """The velocities as the last columns of a wider array, so that the last world's row ends with the
+    allocation; poison in front of them: length, activation, velocity and multiplier bit for bit."""
+    import torch
+
+    c = _fv_case(n, active_type=1.0)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    wide = torch.full((n, c["qvel"].shape[1] + pad), float("nan"), device=device)
+    wide[:, pad:] = t(c["qvel"])
+    outs = [torch.full((n, 37), float("nan"), device=device) for _ in range(5)]
+    Q.eval_muscle_force_velocity_state(
+        t(c["waypoints"]), t(c["wp_start"]), t(c["params"]), t(c["rest"]), t(c["length_scale"]), t(c["act"]), wide[:, pad:],
+        t(c["moment"]), t(c["dof_offsets"]), t(c["dof_torque"]), c["root"], muscle_force_scale=float(c["model"][0]),
+        muscle_length_norm_min=float(c["model"][1]), muscle_length_norm_max=float(c["model"][2]), vmax=1.5, fvmax=1.4,
+        clamp_activation=True, include_active=True, active_force_model_params=c["model"][3:6],
+        muscle_length=outs[0], effective_activation=outs[1], length_velocity=outs[2], force_velocity_multiplier=outs[3],
+        force_velocity_slope=outs[4],
+    )  # fmt: skip
+    want = R.muscle_force_velocity_state(**c)
+    for k in range(4):
+        np.testing.assert_array_equal(outs[k].cpu().numpy(), want[k])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("muscles", [30, 690, 1950])
 def test_gpu_projection_staging_sizes(device, muscles):
     """Rows shorter than eight terms, more than the 3072 entries of one staging trip, and more than
