@@ -593,7 +593,8 @@ typedef struct im_muscle_force_velocity_model {
  * entry, in order), and from them effective_activation = a * fv, length_velocity,
  * force_velocity_multiplier = fv and force_velocity_slope = include_active * a * unit_force *
  * fv' / velocity_scale, velocity_scale = max(length_scale[m] * vmax, 1e-6).  The five outputs are
- * (nworld, ld_out >= nmuscle).  Only the active curve of `model` is read. */
+ * (nworld, ld_out >= nmuscle).  Only the active curve of `model` is read.  ld_waypoints, ld_qvel and
+ * ld_moment are taken for the rows' lengths (also with one world) unless one of them is 0. */
 int im_muscle_force_velocity_state(
     const float *waypoints, int64_t ld_waypoints, const int32_t *muscle_waypoint_start,
     const float *muscle_params, int ld_params, const float *muscle_rest_length,

@@ -267,6 +267,15 @@ def project_muscle_sparse_moment_qfrc(
     _lib.check(status, "im_muscle_project")
 
 
+def _rows_apart(t):
+    """``t`` and its row stride, the stride no shorter than a row: the launch takes the strides for the
+    rows' lengths.  A single row has any stride; rows that overlap are copied (stride 0, one row for
+    every world, stays)."""
+    if t.shape[0] > 1 and 0 < t.stride(0) < t.shape[1]:
+        t = t.contiguous()
+    return t, max(t.stride(0), t.shape[1]) if t.shape[0] == 1 else t.stride(0)
+
+
 def eval_muscle_force_velocity_state(
     transformed_waypoints, muscle_waypoint_start, muscle_params, muscle_rest_length, force_velocity_length_scale,
     activation, qvel, moment, muscle_dof_offsets, muscle_dof_torque_idx, root_dof_count: int, *,
@@ -304,12 +313,13 @@ def eval_muscle_force_velocity_state(
     fv = _lib.MuscleForceVelocityModel(float(vmax), float(fvmax), float(bool(clamp_activation)), float(bool(include_active)))
     import ctypes as C
 
+    (wp2, ld_wp), (qvel, ld_qvel), (moment, ld_moment) = (_rows_apart(t) for t in (wp2, qvel, moment))
     with torch.cuda.device(activation.device):
         status = _lib.lib().im_muscle_force_velocity_state(
-            wp2.data_ptr(), wp2.stride(0), muscle_waypoint_start.data_ptr(), muscle_params.data_ptr(),
+            wp2.data_ptr(), ld_wp, muscle_waypoint_start.data_ptr(), muscle_params.data_ptr(),
             muscle_params.stride(0), muscle_rest_length.data_ptr(), force_velocity_length_scale.data_ptr(),
-            activation.data_ptr(), activation.stride(0), qvel.data_ptr(), qvel.stride(0), moment.data_ptr(),
-            moment.stride(0), muscle_dof_offsets.data_ptr(), muscle_dof_torque_idx.data_ptr(), int(root_dof_count),
+            activation.data_ptr(), activation.stride(0), qvel.data_ptr(), ld_qvel, moment.data_ptr(),
+            ld_moment, muscle_dof_offsets.data_ptr(), muscle_dof_torque_idx.data_ptr(), int(root_dof_count),
             C.byref(model), C.byref(fv), nmuscle, *[t.data_ptr() for t in outs], outs[0].stride(0), nworld,
             _stream(activation),
         )  # fmt: skip

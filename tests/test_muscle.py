@@ -283,6 +283,41 @@ def test_gpu_force_velocity_state_with_velocities_in_a_wider_array(device, n, pa
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["column", "overlapping", "one row for all"])
+def test_gpu_force_velocity_state_with_strides_shorter_than_a_row(device, layout):
+    """Velocities and moments whose row stride is no row length: a transposed column (one world, stride
+    1), windows into one array, one row for every world: bit for bit."""
+    import torch
+
+    n = 1 if layout == "column" else 5
+    c = _fv_case(n, active_type=1.0)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+
+    def laid_out(a):
+        if layout == "column":
+            return t(a[0]).as_strided(a.shape, (1, 1))
+        step = 7 if layout == "overlapping" else 0
+        flat = t(np.resize(a, a.shape[1] + step * n))
+        return flat.as_strided((n, a.shape[1]), (step, 1))
+
+    qvel, moment = laid_out(c["qvel"]), laid_out(c["moment"])
+    assert qvel.stride(0) < qvel.shape[1]
+    c["qvel"], c["moment"] = qvel.cpu().numpy().copy(), moment.cpu().numpy().copy()
+    outs = [torch.full((n, 37), float("nan"), device=device) for _ in range(5)]
+    Q.eval_muscle_force_velocity_state(
+        t(c["waypoints"]), t(c["wp_start"]), t(c["params"]), t(c["rest"]), t(c["length_scale"]), t(c["act"]), qvel,
+        moment, t(c["dof_offsets"]), t(c["dof_torque"]), c["root"], muscle_force_scale=float(c["model"][0]),
+        muscle_length_norm_min=float(c["model"][1]), muscle_length_norm_max=float(c["model"][2]), vmax=1.5, fvmax=1.4,
+        clamp_activation=True, include_active=True, active_force_model_params=c["model"][3:6],
+        muscle_length=outs[0], effective_activation=outs[1], length_velocity=outs[2], force_velocity_multiplier=outs[3],
+        force_velocity_slope=outs[4],
+    )  # fmt: skip
+    want = R.muscle_force_velocity_state(**c)
+    for k in range(4):
+        np.testing.assert_array_equal(outs[k].cpu().numpy(), want[k])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("muscles", [30, 690, 1950])
 def test_gpu_projection_staging_sizes(device, muscles):
     """Rows shorter than eight terms, more than the 3072 entries of one staging trip, and more than
