@@ -250,8 +250,10 @@ struct Holder {
     if (!t) missing = true;
     return t;
   }
-  const Tensor *maybe_tensor(PyObject *from, PyObject *name) {
-    PyObject *v = maybe(from, name);
+  // null for None, and for an attribute that is not there where that is allowed (`absent`)
+  const Tensor *maybe_tensor(PyObject *from, PyObject *name, bool absent) {
+    PyObject *v = get(from, name, absent);
+    if (v == Py_None) return nullptr;
     const Tensor *t = tensor_of(v);
     if (v && !t) missing = true;
     return t;
@@ -308,8 +310,9 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return declined();
   p.M_mulm_rowadr = ptr<int32_t>(radr), p.M_mulm_col = ptr<int32_t>(col), p.M_mulm_madr = ptr<int32_t>(madr), p.nterm = (int32_t)col->numel();
   // arrays: (nworld, width) contiguous, or one element per world
-  auto rows = [&](PyObject *from, PyObject *name, int64_t width, auto **out, bool optional = false) {
-    const Tensor *t = optional ? h.maybe_tensor(from, name) : h.tensor(from, name);
+  enum Presence { REQUIRED, MAY_BE_NONE, MAY_BE_ABSENT };
+  auto rows = [&](PyObject *from, PyObject *name, int64_t width, auto **out, Presence presence = REQUIRED) {
+    const Tensor *t = presence == REQUIRED ? h.tensor(from, name) : h.maybe_tensor(from, name, presence == MAY_BE_ABSENT);
     *out = nullptr;
     if (h.missing) return false;
     if (!t) return true;
@@ -325,8 +328,8 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
     *out = (uint8_t *)t->data_ptr();
     return true;
   };
-  if (!rows(d, names.ne, 1, &p.ne, true) || !rows(d, names.nf, 1, &p.nf, true) || !rows(d, names.nefc, 1, &p.nefc) ||
-      !rows(efc, names.D, njmax, &p.efc_D) || !rows(efc, names.frictionloss, njmax, &p.efc_frictionloss, true) ||
+  if (!rows(d, names.ne, 1, &p.ne, MAY_BE_NONE) || !rows(d, names.nf, 1, &p.nf, MAY_BE_NONE) || !rows(d, names.nefc, 1, &p.nefc) ||
+      !rows(efc, names.D, njmax, &p.efc_D) || !rows(efc, names.frictionloss, njmax, &p.efc_frictionloss, MAY_BE_NONE) ||
       !rows(d, names.qfrc_smooth, nv, &p.qfrc_smooth) || !rows(d, names.qacc, nv, &p.qacc) || !rows(efc, names.Ma, nv, &p.efc_Ma) ||
       !rows(efc, names.force, njmax, &p.efc_force) || !rows(efc, names.state, njmax, &p.efc_state) ||
       !rows(ctx, names.Jaref, njmax, &p.Jaref) || !rows(ctx, names.jv, njmax, &p.jv) || !rows(ctx, names.search, nv, &p.search) ||
@@ -335,7 +338,7 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
       !rows(ctx, names.improvement, 1, &p.improvement) || !rows(ctx, names.grad_dot, 1, &p.grad_dot) ||
       !rows(ctx, names.grad_scale, 1, &p.grad_scale) || !rows(ctx, names.newton_decrement, 1, &p.newton_decrement) ||
       !rows(ctx, names.quad_changed_count, 1, &p.quad_changed_count) || !rows(ctx, names.state_changed_count, 1, &p.state_changed_count) ||
-      !rows(d, names.solver_niter, 1, &p.solver_niter) || !rows(d, names.overflow, 1, &p.overflow, true) || !bytes(names.done, &p.done) ||
+      !rows(d, names.solver_niter, 1, &p.solver_niter) || !rows(d, names.overflow, 1, &p.overflow, MAY_BE_ABSENT) || !bytes(names.done, &p.done) ||
       !bytes(names.ls_exhausted, &p.ls_exhausted) || !bytes(names.search_unchanged, &p.search_unchanged))
     return declined();
   const Tensor *grad = h.tensor(ctx, names.grad), *ids = h.tensor(ctx, names.quad_changed_ids), *left = tensor_of(a[3]);
@@ -346,7 +349,7 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   p.nsolving = ptr<int32_t>(left);
   // the start
   const Tensor *smooth = h.tensor(d, names.qacc_smooth), *aref = h.tensor(efc, names.aref);
-  const Tensor *warm = (flags & no_warmstart) ? nullptr : h.maybe_tensor(d, names.qacc_warmstart);
+  const Tensor *warm = (flags & no_warmstart) ? nullptr : h.maybe_tensor(d, names.qacc_warmstart, true);
   if (h.missing || !c.rows(smooth, nworld, nv) || !c.rows(aref, nworld, njmax) || (warm && !c.rows(warm, nworld, nv)) ||
       smooth->size(1) != nv || (warm && warm->size(1) != nv))
     return declined();

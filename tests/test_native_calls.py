@@ -139,3 +139,17 @@ def test_gpu_arguments_that_are_no_numbers_raise_their_own_error(device):
     with pytest.raises(LookupError, match="neither"):
         T.assemble_tree_factor_solve(sc, M, J, D, state, nefc, grad, x, negate=Undecided())
     assert bool((x == 7.0).all())
+
+
+@pytest.mark.parametrize("missing", ["ne", "nf", "frictionloss"])
+def test_gpu_solve_asks_for_every_array_of_the_step(device, missing):
+    """None stands for no equality rows, no friction rows; an attribute that is not there is an error."""
+    p = NC.problem("humanoid", 5, "tree")
+    m, d, ctx, left = NC.device_objects(p, device)
+    delattr(d.efc if missing == "frictionloss" else d, missing)
+    with pytest.raises(AttributeError, match=missing):
+        NF.solve(m, d, ctx, left)
+    m, d, ctx, left = NC.device_objects(p, device)
+    d.ne = d.nf = d.efc.frictionloss = None
+    NF.solve(m, d, ctx, left)
+    assert bool(ctx.done.all()) and bool(torch.isfinite(d.qacc).all())
