@@ -71,6 +71,11 @@ struct Call {
     if (!on(t, type) || !t->is_contiguous() || t->numel() != count) return ok = false;
     return ok;
   }
+  // a contiguous (nworld, pad, pad) float tensor
+  bool squares(const Tensor *t, int64_t nworld, int64_t pad) {
+    if (!on(t, at::kFloat) || t->dim() != 3 || t->size(0) != nworld || t->size(1) != pad || t->size(2) != pad) return ok = false;
+    return ok = ok && t->is_contiguous();
+  }
   // rows of at least `width` floats for `nworld` worlds, given as (nworld, width) with contiguous rows or as any contiguous shape
   bool vectors(const Tensor *t, int64_t nworld, int64_t width, int64_t *ld) {
     if (!on(t, at::kFloat) || t->dim() < 1 || nworld <= 0) return ok = false;
@@ -160,7 +165,7 @@ PyObject *blocked_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const Tensor *indices = tensor_of(a[5]), *U = tensor_of(a[6]), *M = tensor_of(a[7]), *x = tensor_of(a[8]), *y = tensor_of(a[9]);
   Call c;
   int64_t ldx = 0, ldy = 0;
-  if (nworld <= 0 || !c.rows(M, nworld, nM) || !c.whole(U, at::kFloat, nworld * pad * pad) || !c.whole(indices, at::kInt, pad * pad) ||
+  if (nworld <= 0 || !c.rows(M, nworld, nM) || !c.squares(U, nworld, pad) || !c.whole(indices, at::kInt, pad * pad) ||
       !c.vectors(x, nworld, nv, &ldx) || !c.vectors(y, nworld, nv, &ldy))
     return declined();
   void *const stream = c.stream();
@@ -187,9 +192,7 @@ PyObject *dense_hessian_factor_solve(PyObject *, PyObject *const *a, Py_ssize_t 
   };
   if (!c.whole(M, at::kFloat, nworld * nv * nv) || !per_row(D, at::kFloat) || !per_row(state, at::kInt) ||
       (nefc && !c.whole(nefc, at::kInt, nworld)) || !c.vectors(y, nworld, nv, &ldy) || !c.vectors(x, nworld, nv, &ldx) ||
-      (U && (!c.whole(U, at::kFloat, nworld * pad * pad) || U->dim() != 3)))
-    return declined();
-  if (H && (H->dim() != 3 || H->size(1) < nv || H->size(1) != H->size(2) || !c.whole(H, at::kFloat, nworld * H->size(1) * H->size(1))))
+      (U && !c.squares(U, nworld, pad)) || (H && (H->dim() != 3 || H->size(1) < nv || !c.squares(H, nworld, H->size(1)))))
     return declined();
   void *const stream = c.stream();
   return answer(unlocked([&] {
@@ -359,7 +362,7 @@ PyObject *newton_solve(PyObject *, PyObject *const *a, Py_ssize_t n) {
   k.nv = (int32_t)nv, k.nv_pad = (int32_t)pad, k.nM = (int32_t)M->size(1);
   auto square = [&](PyObject *name, float **out) {
     const Tensor *t = h.tensor(ctx, name);
-    if (h.missing || t->dim() != 3 || t->size(1) != pad || !c.whole(t, at::kFloat, nworld * pad * pad)) return false;
+    if (h.missing || !c.squares(t, nworld, pad)) return false;
     *out = ptr(t);
     return true;
   };

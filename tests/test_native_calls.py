@@ -1,6 +1,8 @@
 """The native host path (csrc/native_calls.cpp) hands over to the Python checks what it does not
 take at once: views with a row stride run, and wrong dtypes, shapes and layouts raise as before."""
 
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -153,3 +155,36 @@ def test_gpu_solve_asks_for_every_array_of_the_step(device, missing):
     d.ne = d.nf = d.efc.frictionloss = None
     NF.solve(m, d, ctx, left)
     assert bool(ctx.done.all()) and bool(torch.isfinite(d.qacc).all())
+
+
+def _blocked(device, nworld=5, nv=35, block=8):
+    g = torch.Generator(device="cpu").manual_seed(4)
+    a = torch.randn((nworld, nv, nv), generator=g) * 0.2
+    M = (a @ a.transpose(1, 2).contiguous() + torch.eye(nv)).reshape(nworld, -1).to(device)
+    tile = SimpleNamespace(size=nv, elemid=torch.arange(nv * nv, dtype=torch.int32))
+    d = SimpleNamespace(nworld=nworld, M=M)
+    sc = BD.create_blocked_dense_factor_solve_scratch(SimpleNamespace(nv=nv, M_tiles=[tile]), d, device, block_size=block)
+    return d, M, sc, torch.randn((nworld, nv), generator=g).to(device)
+
+
+@pytest.mark.parametrize("shape", ["rows", "flat", "planes"])
+def test_gpu_a_factor_workspace_has_the_shape_of_the_factor(device, shape):
+    """As many floats in another shape are refused, for the factor of each of the two solves."""
+    d, M, sc, y = _blocked(device)
+    x, n, pad = torch.zeros_like(y), d.nworld, sc.pad
+    shapes = lambda n, pad: dict(rows=(n * pad, pad), flat=(n * pad * pad,), planes=(n, pad // 2, 2 * pad))[shape]  # noqa: E731
+    with pytest.raises(ValueError):
+        BD._blocked_dense_factor_solve(d, M, x, y, sc, factor_workspace=torch.zeros(shapes(n, pad), device=device))
+    M, J, D, state, nefc, y = _dense_step(device)
+    with pytest.raises(ValueError):
+        BD.dense_hessian_factor_solve(M, J, D, state, nefc, None, y, x, factor=torch.zeros(shapes(n, 48), device=device))
+    assert not bool(x.any())
+
+
+@pytest.mark.parametrize("stage,name", [("sparse", "hfactor"), ("dense", "hfactor"), ("dense", "h")])
+def test_gpu_the_solves_squares_have_the_shape_of_the_factor(device, stage, name):
+    p = NC.problem("g1", 6, stage)
+    m, d, ctx, left = NC.device_objects(p, device)
+    setattr(ctx, name, getattr(ctx, name).reshape(3, p.pad, 2 * p.pad))
+    with pytest.raises((TypeError, ValueError)):
+        NF.solve(m, d, ctx, left)
