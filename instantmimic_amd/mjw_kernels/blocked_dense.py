@@ -318,19 +318,43 @@ def blocked_multi_solve(factor, scratch: BlockedDenseFactorSolveScratch, y, acti
     _lib.check(status, "im_blocked_multi_solve")
 
 
+def _check_hessian_inputs(M_dense, J, D, state, nefc) -> None:
+    """What the launches index: contiguous arrays on J's device, of the types and sizes the kernels read."""
+    import torch
+
+    if J.dim() != 3:
+        raise ValueError("J must be (nworld, njmax, nv)")
+    nworld, njmax, nv = J.shape
+    for t in (M_dense, J, D, state, nefc):
+        if t is not None and (not t.is_cuda or t.device != J.device or not t.is_contiguous()):
+            raise ValueError("M_dense, J, D, state and nefc must be contiguous CUDA tensors on one device")
+    if any(t.dtype != torch.float32 for t in (M_dense, J, D)):
+        raise TypeError("M_dense, J and D must be float32")
+    if any(t is not None and t.dtype != torch.int32 for t in (state, nefc)):
+        raise TypeError("state and nefc must be int32")
+    if njmax < 1 or tuple(D.shape) != (nworld, njmax) or tuple(state.shape) != (nworld, njmax) or M_dense.numel() != nworld * nv * nv:
+        raise ValueError("D and state must be (nworld, njmax >= 1) and M_dense (nworld, nv, nv)")
+    if nefc is not None and nefc.numel() != nworld:
+        raise ValueError("nefc needs one element per world")
+
+
+def _check_hessian(H, J) -> None:
+    import torch
+
+    if H.dtype != torch.float32 or H.device != J.device or not H.is_contiguous() or H.dim() != 3 or (
+        H.shape[0] != J.shape[0] or H.shape[1] != H.shape[2] or H.shape[1] < J.shape[2]
+    ):
+        raise ValueError("H must be a contiguous float32 (nworld, nv_pad, nv_pad) tensor on J's device")
+
+
 def dense_hessian(M_dense, J, D, state, nefc, H, *, quad: int = QUADRATIC) -> None:
     """``H[w, :nv, :nv] = M_dense[w] + J[w]' diag(D [state == quad, row < nefc]) J[w]`` on
     fp32 MFMA; ``H`` is (nworld, nv_pad, nv_pad)."""
     import torch
 
+    _check_hessian_inputs(M_dense, J, D, state, nefc)
+    _check_hessian(H, J)
     nworld, njmax, nv = J.shape
-    for t in (M_dense, J, D, state, H):
-        if not t.is_cuda or not t.is_contiguous():
-            raise ValueError("dense_hessian needs contiguous CUDA tensors")
-    if njmax < 1 or tuple(D.shape) != (nworld, njmax) or tuple(state.shape) != (nworld, njmax):
-        raise ValueError("D and state must be (nworld, njmax >= 1)")
-    if H.dim() != 3 or H.shape[0] != nworld or H.shape[1] != H.shape[2] or H.shape[1] < nv or M_dense.numel() != nworld * nv * nv:
-        raise ValueError("H must be (nworld, nv_pad, nv_pad) and M_dense (nworld, nv, nv)")
     with torch.cuda.device(J.device):
         status = _lib.lib().im_jtdj_mfma(
             M_dense.data_ptr(), J.data_ptr(), int(njmax), D.data_ptr(), state.data_ptr(),
@@ -401,18 +425,13 @@ def dense_hessian_factor_solve(M_dense, J, D, state, nefc, H, y, x, *, factor=No
         _lib.check(status, "im_jtdj_factor_solve")
     import torch
 
+    _check_hessian_inputs(M_dense, J, D, state, nefc)
+    if H is not None:
+        _check_hessian(H, J)
     nworld, njmax, nv = J.shape
     pad = -(-nv // 16) * 16
-    for t in (M_dense, J, D, state, y, x):
-        if not t.is_cuda or t.device != J.device:
-            raise ValueError("dense_hessian_factor_solve needs CUDA tensors on one device")
-    for t in (M_dense, J, D, state):
-        if not t.is_contiguous():
-            raise ValueError("M_dense, J, D and state must be contiguous")
-    if njmax < 1 or tuple(D.shape) != (nworld, njmax) or tuple(state.shape) != (nworld, njmax) or M_dense.numel() != nworld * nv * nv:
-        raise ValueError("D and state must be (nworld, njmax >= 1) and M_dense (nworld, nv, nv)")
-    if H is not None and (not H.is_contiguous() or H.dim() != 3 or H.shape[0] != nworld or H.shape[1] != H.shape[2] or H.shape[1] < nv):
-        raise ValueError("H must be a contiguous (nworld, nv_pad, nv_pad) tensor")
+    if any(t is not None and t.device != J.device for t in (y, x, factor)):
+        raise ValueError("y, x and factor must be on J's device")
     y2, x2 = y.reshape(nworld, -1), x.reshape(nworld, -1)
     if y2.shape[1] < nv or x2.shape[1] < nv or y2.stride(1) != 1 or x2.stride(1) != 1 or y.dtype != torch.float32 or x.dtype != torch.float32:
         raise ValueError("y and x must be float32 (nworld, >= nv) tensors with contiguous rows")

@@ -188,3 +188,30 @@ def test_gpu_the_solves_squares_have_the_shape_of_the_factor(device, stage, name
     setattr(ctx, name, getattr(ctx, name).reshape(3, p.pad, 2 * p.pad))
     with pytest.raises((TypeError, ValueError)):
         NF.solve(m, d, ctx, left)
+
+
+_WRONG = {
+    "double": lambda t: t.double() if t.is_floating_point() else t.long(),
+    "half": lambda t: t.half() if t.is_floating_point() else t.short(),
+    "one world less": lambda t: t[:-1],
+    "on the host": lambda t: t.cpu(),
+    "every other column": lambda t: torch.zeros((*t.shape[:-1], 2 * t.shape[-1]), dtype=t.dtype, device=t.device)[..., ::2],
+}
+
+
+@pytest.mark.parametrize("wrong", sorted(_WRONG))
+@pytest.mark.parametrize("call", ["solve", "matrix"])
+def test_gpu_dense_hessian_refuses_what_its_kernels_cannot_read(device, call, wrong):
+    """Each array of the dense J'DJ in turn in another type, length, place or layout: an error, and
+    nothing written."""
+    M, J, D, state, nefc, y = _dense_step(device)
+    x, H, U = torch.full_like(y, 7.0), torch.full((5, 48, 48), 7.0, device=device), torch.full((5, 48, 48), 7.0, device=device)
+    args = dict(M=M, J=J, D=D, state=state, nefc=nefc, H=H, y=y, x=x, U=U)
+    for name in args if call == "solve" else ("M", "J", "D", "state", "nefc", "H"):
+        a = {**args, name: _WRONG[wrong](args[name])}
+        with pytest.raises((TypeError, ValueError)):
+            if call == "solve":
+                BD.dense_hessian_factor_solve(a["M"], a["J"], a["D"], a["state"], a["nefc"], a["H"], a["y"], a["x"], factor=a["U"])
+            else:
+                BD.dense_hessian(a["M"], a["J"], a["D"], a["state"], a["nefc"], a["H"])
+    assert all(bool((t == 7.0).all()) for t in (x, H, U))
