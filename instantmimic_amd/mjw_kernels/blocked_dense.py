@@ -386,6 +386,8 @@ def dense_init_factor(M, elemid, J, D, state, nefc, done, grad, H, U, search, se
     for t in (J, D, state, H, U, search_dot, decrement, elemid, dof_union):
         if not t.is_contiguous():
             return False
+    if any(t is not None and t.device != J.device for t in (elemid, dof_union, nefc, done)):
+        return False
     if M.dim() != 2 or M.shape[0] != nworld or (M.shape[1] > 1 and M.stride(1) != 1) or grad.stride(-1) != 1 or search.stride(-1) != 1:
         return False
     if tuple(H.shape) != (nworld, pad, pad) or tuple(U.shape) != (nworld, pad, pad) or pad % 4 or H.data_ptr() % 16:

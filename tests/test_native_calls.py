@@ -215,3 +215,16 @@ def test_gpu_dense_hessian_refuses_what_its_kernels_cannot_read(device, call, wr
             else:
                 BD.dense_hessian(a["M"], a["J"], a["D"], a["state"], a["nefc"], a["H"])
     assert all(bool((t == 7.0).all()) for t in (x, H, U))
+
+
+@pytest.mark.parametrize("where", ["elemid", "dof_union", "nefc", "done"])
+def test_gpu_first_dense_factor_leaves_arrays_on_the_host(device, where):
+    """The one launch takes no address of host memory: False, with nothing written."""
+    p = NC.problem("g1", 4, "dense")
+    m, d, ctx, _ = NC.device_objects(p, device)
+    a = dict(elemid=ctx.newton_elemid, dof_union=ctx.newton_dof_union, nefc=d.nefc, done=ctx.done)
+    a[where] = a[where].cpu()
+    before = ctx.h.clone()
+    assert not BD.dense_init_factor(d.M, a["elemid"], d.efc.J, d.efc.D, d.efc.state, a["nefc"], a["done"], ctx.grad, ctx.h, ctx.hfactor,
+                                    ctx.search, ctx.search_dot, ctx.newton_decrement, a["dof_union"])  # fmt: skip
+    assert torch.equal(torch.nan_to_num(before), torch.nan_to_num(ctx.h))
