@@ -1200,7 +1200,7 @@ int im_sparse_init_factor(const im_sparse_plan *plan, const uint8_t *done, const
   if (!plan->device_ready || plan->path != IM_SPARSE_FUSED) return IM_ERR_UNSUPPORTED;
   if (nworld == 0) return IM_OK;
   if (!nefc || !J || !D || !state || !M || !grad || !hfactor || !search || !search_dot || !decrement) return IM_ERR_ARG;
-  if (ldg < plan->nv) return IM_ERR_STRIDE;
+  if (ldg < plan->nv || ldM < plan->nM) return IM_ERR_STRIDE;
   im::SparseDev P;
   for (int i = 0; i < im::NHOST; ++i) P.t[i] = plan->t[i];
   P.nv = plan->nv; P.nv_pad = plan->nv_pad; P.nslots = plan->nslots; P.nlevels = plan->nlevels;
@@ -1223,7 +1223,7 @@ int im_sparse_init_factor(const im_sparse_plan *plan, const uint8_t *done, const
     // per world: the factor's arrays and the list of contributing constraint rows (weight and number)
     const size_t per_world = (((size_t)plan->nslots + n + 2 * nw + 3) & ~(size_t)3) + 2 * (((size_t)njmax + 3) & ~(size_t)3);
     const size_t wave_lds = 4 * (((staged + 3) & ~(size_t)3) + 4 * per_world);
-    if (wave_lds <= 64 * 1024 && staged <= 8192 && ldM >= plan->nM) {
+    if (wave_lds <= 64 * 1024 && staged <= 8192) {
       const dim3 grid((unsigned)((nworld + 3) / 4)), wg(256);
       const hipStream_t st = (hipStream_t)stream;
 #define IM_SPARSE_WAVE(NT)                                                                            \

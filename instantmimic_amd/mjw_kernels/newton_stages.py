@@ -17,14 +17,31 @@ from .. import _lib
 from .sparse_hessian import QUADRATIC, SparseHessianPlan
 
 
+_INTEGERS = ("state", "ids", "changes", "state_changes", "nefc", "dof_union")
+_BYTES = ("done", "skip")
+
+
 def _check(tensors, nworld: int) -> None:
+    """Every array as the launch reads it: contiguous, on the first one's device, a row per world, of the
+    kernel's type (the C ABI sees addresses only)."""
+    import torch
+
+    where = next(t for t in tensors.values() if t is not None).device
     for name, t in tensors.items():
         if t is None:
             continue
-        if not t.is_cuda or not t.is_contiguous():
-            raise ValueError(f"{name} must be a contiguous CUDA tensor")
+        if not t.is_cuda or t.device != where or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous CUDA tensor on {where}")
         if t.shape[0] != nworld:
             raise ValueError(f"{name} has {t.shape[0]} worlds, expected {nworld}")
+        types = (torch.int32,) if name in _INTEGERS else (torch.bool, torch.uint8) if name in _BYTES else (torch.float32,)
+        if t.dtype not in types:
+            raise TypeError(f"{name} must be {' or '.join(str(k) for k in types)}")
+
+
+def _check_row_arrays(J, D, state) -> None:
+    if tuple(D.shape) != tuple(J.shape[:2]) or tuple(state.shape) != tuple(J.shape[:2]):
+        raise ValueError("D and state must be (nworld, njmax)")
 
 
 def factor_factory(nv: int, pad: int, sparse_plan: SparseHessianPlan | None = None, *, tree_scratch: Any = None,
@@ -57,8 +74,7 @@ def factor_factory(nv: int, pad: int, sparse_plan: SparseHessianPlan | None = No
                 raise ValueError("J does not match the stage's nv")
             _check(dict(J=J, D=D, state=state, grad=grad, search=search, search_dot=search_dot, decrement=decrement,
                         M=M, skip=skip, nefc=nefc), nworld)  # fmt: skip
-            if skip.dtype not in (torch.bool, torch.uint8):
-                raise TypeError("skip must be a bool tensor")
+            _check_row_arrays(J, D, state)
             if M.dim() != 2 or M.shape[1] < tree_scratch.kernel.info().nM:
                 raise ValueError("M must be (nworld, nM)")
             ldg, lds = grad[0].numel(), search[0].numel()
@@ -87,12 +103,9 @@ def factor_factory(nv: int, pad: int, sparse_plan: SparseHessianPlan | None = No
         _check(dict(J=J, D=D, state=state, ids=ids, changes=changes, state_changes=state_changes, done=done,
                     grad=grad, U=U, search=search, search_dot=search_dot, decrement=decrement,
                     dof_union=dof_union), nworld)  # fmt: skip
+        _check_row_arrays(J, D, state)
         if tuple(U.shape) != (nworld, pad, pad) or tuple(dof_union.shape) != (nworld, nv + 1):
             raise ValueError("U must be (nworld, nv_pad, nv_pad) and dof_union (nworld, nv + 1)")
-        if ids.dtype != torch.int32 or dof_union.dtype != torch.int32 or changes.dtype != torch.int32:
-            raise TypeError("ids, changes and dof_union must be int32")
-        if done is not None and done.dtype not in (torch.bool, torch.uint8):
-            raise TypeError("done must be a bool tensor")
         ldg, lds = grad[0].numel(), search[0].numel()
         stream = int(torch.cuda.current_stream(J.device).cuda_stream)
         done_ptr = None if done is None else done.data_ptr()
@@ -109,7 +122,7 @@ def factor_factory(nv: int, pad: int, sparse_plan: SparseHessianPlan | None = No
                 )  # fmt: skip
                 _lib.check(status, "im_sparse_update_factor")
             else:
-                _check(dict(H=H), nworld)
+                _check(dict(U=U, H=H), nworld)
                 if tuple(H.shape) != (nworld, pad, pad):
                     raise ValueError("H must be (nworld, nv_pad, nv_pad)")
                 status = L.im_dense_update_factor(

@@ -367,6 +367,12 @@ def init_factor_kernel(plan: SparseHessianPlan):
         for t in (J, D, state, M, grad, hfactor, search, search_dot, decrement, nefc):
             if not t.is_cuda or not t.is_contiguous() or t.device != J.device:
                 raise ValueError("arrays must be contiguous CUDA tensors on one device")
+        if any(t.dtype != torch.float32 for t in (J, D, M, grad, hfactor, search, search_dot, decrement)):
+            raise TypeError("J, D, M, grad, hfactor, search, search_dot and decrement must be float32")
+        if state.dtype != torch.int32 or nefc.dtype != torch.int32:
+            raise TypeError("state and nefc must be int32")
+        if search.shape[0] != nworld or search_dot.numel() != nworld or decrement.numel() != nworld:
+            raise ValueError("search, search_dot and decrement need a row per world")
         done_ptr = None
         if done is not None:
             if done.dtype not in (torch.bool, torch.uint8) or done.numel() != nworld:

@@ -228,3 +228,75 @@ def test_gpu_first_dense_factor_leaves_arrays_on_the_host(device, where):
     assert not BD.dense_init_factor(d.M, a["elemid"], d.efc.J, d.efc.D, d.efc.state, a["nefc"], a["done"], ctx.grad, ctx.h, ctx.hfactor,
                                     ctx.search, ctx.search_dot, ctx.newton_decrement, a["dof_union"])  # fmt: skip
     assert torch.equal(torch.nan_to_num(before), torch.nan_to_num(ctx.h))
+
+
+_SOLVE_ARRAYS = {
+    "m": "M_mulm_rowadr M_mulm_col M_mulm_madr", "opt": "tolerance ls_tolerance", "stat": "meaninertia",
+    "d": "M ne nf nefc qfrc_smooth qacc_smooth qacc qfrc_constraint solver_niter overflow",
+    "efc": "J D frictionloss aref Ma force state",
+    "ctx": "search search_dot mv jv Jaref done alpha improvement ls_exhausted quad_changed_ids quad_changed_count "
+           "state_changed_count search_unchanged grad grad_dot grad_scale newton_decrement",
+}  # fmt: skip
+_STAGE_ARRAYS = {"tree": "", "sparse": " hfactor newton_dof_union", "dense": " hfactor newton_dof_union h newton_elemid newton_next_world"}
+
+
+@pytest.mark.parametrize("wrong", sorted(_WRONG))
+@pytest.mark.parametrize("stage,name", [("tree", "humanoid"), ("sparse", "g1"), ("dense", "humanoid"), ("dense", "g1")])
+def test_gpu_solve_refuses_what_its_kernels_cannot_read(device, stage, name, wrong):
+    """Each array of a whole solve in turn in another type, length, place or layout: an error from the
+    Python checks, whichever of them it reaches first."""
+    p = NC.problem(name, 6, stage)
+    m, d, ctx, left = NC.device_objects(p, device)
+    for where, names in _SOLVE_ARRAYS.items():
+        owner = dict(m=m, opt=m.opt, stat=m.stat, d=d, efc=d.efc, ctx=ctx)[where]
+        for attr in (names + (_STAGE_ARRAYS[stage] if where == "ctx" else "")).split():
+            kept = getattr(owner, attr)
+            if wrong == "every other column" and kept.numel() == 1:
+                continue  # (contiguous whatever its stride)
+            setattr(owner, attr, _WRONG[wrong](kept))
+            with pytest.raises((TypeError, ValueError, RuntimeError)):
+                NF.solve(m, d, ctx, left)
+                pytest.fail(f"{where}.{attr} {wrong} was taken")
+            setattr(owner, attr, kept)
+    for bad in (left.long(), left.cpu(), torch.zeros(2, dtype=torch.int32, device=device)):
+        with pytest.raises((TypeError, ValueError, RuntimeError)):
+            NF.solve(m, d, ctx, bad)
+    NF.solve(m, d, ctx, left)
+    NC.compare(p, NC.oracle_solve(p), d, ctx)
+
+
+@pytest.mark.parametrize("wrong", sorted(_WRONG))
+@pytest.mark.parametrize("block", [8, 16])
+def test_gpu_blocked_solve_refuses_what_its_kernels_cannot_read(device, block, wrong):
+    d, M, sc, y = _blocked(device, block=block)
+    args = dict(M=M, x=torch.full_like(y, 7.0), y=y, U=torch.full((d.nworld, sc.pad, sc.pad), 7.0, device=device))
+    for name in args:
+        a = {**args, name: _WRONG[wrong](args[name])}
+        with pytest.raises((TypeError, ValueError)):
+            BD._blocked_dense_factor_solve(d, a["M"], a["x"], a["y"], sc, factor_workspace=a["U"])
+    for short in (dict(M=M[:, :-1]), dict(y=y[:, :-1])):
+        a = {**args, **short}
+        with pytest.raises(ValueError):
+            BD._blocked_dense_factor_solve(d, a["M"], a["x"], a["y"], sc, factor_workspace=a["U"])
+    assert bool((args["x"] == 7.0).all()) and bool((args["U"] == 7.0).all())
+
+
+def test_gpu_views_run_through_the_dense_entry_points(device):
+    """Rows with a stride, and right-hand sides with a third axis, give what plain rows give."""
+    d, M, sc, y = _blocked(device)
+    want, wide = torch.zeros_like(y), torch.zeros((d.nworld, 3 * y.shape[1]), device=device)
+    BD._blocked_dense_factor_solve(d, M, want, y, sc)
+    Mw = torch.zeros((d.nworld, M.shape[1] + 5), device=device)
+    Mw[:, : M.shape[1]] = M
+    view = wide[:, y.shape[1] : 2 * y.shape[1]]
+    BD._blocked_dense_factor_solve(d, Mw[:, : M.shape[1]], view, y, sc)
+    cube = torch.zeros((*y.shape, 1), device=device)
+    BD._blocked_dense_factor_solve(d, M, cube, y[:, :, None].contiguous(), sc)
+    assert torch.equal(view, want) and torch.equal(cube[:, :, 0], want) and bool((wide[:, : y.shape[1]] == 0).all())
+    M, J, D, state, nefc, y = _dense_step(device)
+    BD.dense_hessian_factor_solve(M, J, D, state, nefc, None, y, want)
+    wide.zero_()
+    BD.dense_hessian_factor_solve(M, J, D, state, nefc, None, y, view)
+    cube.zero_()
+    BD.dense_hessian_factor_solve(M, J, D, state, nefc, None, y[:, :, None].contiguous(), cube)
+    assert torch.equal(view, want) and torch.equal(cube[:, :, 0], want) and bool((wide[:, : y.shape[1]] == 0).all())
