@@ -51,7 +51,7 @@ def _host_planner():
     src = os.path.join(CSRC, "tree_plan.cpp")
     os.makedirs(OBJ, exist_ok=True)
     stale = not os.path.exists(PLANNER_LIB) or os.path.getmtime(PLANNER_LIB) < max(
-        os.path.getmtime(p) for p in (src, os.path.join(CSRC, "common.h"), os.path.join(HERE, "..", "include", "imhip.h"))
+        os.path.getmtime(p) for p in (src, os.path.join(CSRC, "common.h"), os.path.join(CSRC, "kept.h"), os.path.join(HERE, "..", "include", "imhip.h"))
     )
     if stale or os.environ.get("IMHIP_REBUILD"):
         cmd = ["hipcc", "--offload-arch=gfx950", "-O1", "-std=c++17", "-fPIC", "-shared", "-DIM_PLANNER_ONLY",

@@ -4,13 +4,18 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <tuple>
 #include <vector>
 
 #include "../../include/imhip.h"
+#include "kept.h"
 
 namespace im {
 
 constexpr int kWave = 64;
+
+// Workgroups of a kernel that a CU keeps resident, by (device, kernel, threads, LDS).
+using Occupancy = Kept<std::tuple<int, const void *, int, size_t>, int>;
 
 void set_hip_error(hipError_t e);
 
@@ -65,6 +70,7 @@ struct im_tree_plan {
   // masks, so such a plan runs on generated kernels only (device_ready, nothing launched before
   // kernels are attached)
   bool table_driven = true;
+  mutable im::Occupancy occupancy;  // of the kernels of `module`
 };
 
 namespace im {

@@ -243,19 +243,9 @@ int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32
                                      IM_WAVE_VARIANT(4, 4, 0), IM_WAVE_VARIANT(5, 4, 2), IM_WAVE_VARIANT(5, 4, 0)};
 #undef IM_WAVE_VARIANT
   constexpr int kVariants = 6;
-  static bool usable[kVariants] = {};
-  static bool probed = false;
-  if (!probed) {  // once per process: a variant that spills registers is left out; the large dynamic LDS is asked for
-    for (int i = 0; i < kVariants; ++i) {
-      hipFuncAttributes fa{};
-      // (a variant that parks more than a register or two of its prologue in memory is left out)
-      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
-                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
-      (void)hipGetLastError();
-    }
-    probed = true;
-  }
+  static Kept<int, std::array<bool, kVariants>> probed;
+  std::array<bool, kVariants> usable;
+  if (const int st = usable_variants(probed, variants, &usable)) return st;
   const int nblk = nv_pad / 16;
   for (int i = 0; i < kVariants; ++i) {
     const Variant &v = variants[i];
@@ -268,7 +258,7 @@ int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32
     if (const int st = compute_units(&ncu)) return st;
     // as many workgroups as stay resident at once: by LDS and by registers
     int per_cu = 0;
-    if (const int st = resident_per_cu(v.fn, false, 64 * v.waves, lds, &per_cu)) return st;
+    if (const int st = resident_per_cu(v.fn, nullptr, 64 * v.waves, lds, &per_cu)) return st;
     per_cu = std::max(1, per_cu);
     const int needed = (p->nworld + v.waves - 1) / v.waves;
     const int grid = std::min(needed, ncu * per_cu);

@@ -4,9 +4,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstdint>
 
 #include "../../include/imhip.h"
+#include "common.h"
 
 namespace im {
 
@@ -42,11 +44,25 @@ int dense_init_factor(const uint8_t *done, const int32_t *nefc, const float *J, 
 // the tree stage of a solve's start, without the two sums (the resident loop forms them)
 int newton_tree_first(const im_tree_plan *plan, const im_newton_args *p, hipStream_t stream);
 
-// Workgroups of a kernel that a CU keeps resident, kept per (kernel, threads, LDS) after the first question:
-// the runtime's answer costs as much host time as a launch.
-int resident_per_cu(const void *fn, bool module, int threads, size_t lds, int *per_cu);
+// Workgroups of a kernel that a CU keeps resident, kept after the first question: the runtime's answer costs as
+// much host time as a launch.  In `plans` for a kernel of a plan's loaded module, null for one of the library's.
+int resident_per_cu(const void *fn, Occupancy *plans, int threads, size_t lds, int *per_cu);
 // Compute units of the current device.
 int compute_units(int *ncu);
+int current_device(int *device);
+// Whether a resident kernel keeps to registers on the current device (one that parks more than a few values of its
+// prologue in memory is left out) and may use a CU's whole LDS, which is asked for.
+bool usable_resident(const void *fn);
+// usable[i] of variants[i].fn on the current device, asked once per device.
+template <class Variant, size_t N>
+int usable_variants(Kept<int, std::array<bool, N>> &kept, const Variant (&variants)[N], std::array<bool, N> *usable) {
+  int device = 0;
+  if (const int st = current_device(&device)) return st;
+  return kept.get(device, [&](std::array<bool, N> &u) {
+    for (size_t i = 0; i < N; ++i) u[i] = usable_resident(variants[i].fn);
+    return (int)IM_OK;
+  }, usable);
+}
 // *counter = value, as a launch
 void set_counter(int *counter, int value, hipStream_t stream);
 

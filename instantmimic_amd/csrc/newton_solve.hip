@@ -6,8 +6,6 @@
 // among them), whose issue took longer than a small batch's work: 117 us per solve of 64 worlds.
 #include <hip/hip_runtime.h>
 
-#include <map>
-#include <mutex>
 #include <tuple>
 
 #include "common.h"
@@ -23,37 +21,41 @@ void set_counter(int *counter, int value, hipStream_t stream) {
   hipLaunchKernelGGL(set_counter_kernel, dim3(1), dim3(1), 0, stream, counter, value);
 }
 
-int resident_per_cu(const void *fn, bool module, int threads, size_t lds, int *per_cu) {
-  static std::mutex lock;
-  static std::map<std::tuple<const void *, int, size_t>, int> known;
-  const std::lock_guard<std::mutex> hold(lock);
-  const auto key = std::make_tuple(fn, threads, lds);
-  const auto it = known.find(key);
-  if (it != known.end()) {
-    *per_cu = it->second;
-    return IM_OK;
-  }
-  int n = 0;
-  if (module)
-    IM_HIP_CHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&n, (hipFunction_t)fn, threads, lds));
-  else
-    IM_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, lds));
-  if (known.size() >= 512) known.clear();  // (models come and go: the answers of unloaded kernels with them)
-  known[key] = n;
-  *per_cu = n;
+int current_device(int *device) {
+  IM_HIP_CHECK(hipGetDevice(device));
   return IM_OK;
 }
 
+int resident_per_cu(const void *fn, Occupancy *plans, int threads, size_t lds, int *per_cu) {
+  static Occupancy library;
+  int device = 0;
+  if (const int st = current_device(&device)) return st;
+  return (plans ? *plans : library).get(std::make_tuple(device, fn, threads, lds), [&](int &n) {
+    if (plans)
+      IM_HIP_CHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&n, (hipFunction_t)fn, threads, lds));
+    else
+      IM_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, lds));
+    return (int)IM_OK;
+  }, per_cu);
+}
+
 int compute_units(int *ncu) {
-  static int known = 0;
-  if (!known) {
-    int dev = 0, n = 0;
-    IM_HIP_CHECK(hipGetDevice(&dev));
-    IM_HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
-    known = n > 0 ? n : 1;
-  }
-  *ncu = known;
-  return IM_OK;
+  static Kept<int, int> known;
+  int device = 0;
+  if (const int st = current_device(&device)) return st;
+  return known.get(device, [&](int &n) {
+    IM_HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device));
+    n = n > 0 ? n : 1;
+    return (int)IM_OK;
+  }, ncu);
+}
+
+bool usable_resident(const void *fn) {
+  hipFuncAttributes fa{};
+  const bool ok = hipFuncGetAttributes(&fa, fn) == hipSuccess && fa.localSizeBytes <= 16 &&
+                  hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
+  (void)hipGetLastError();
+  return ok;
 }
 
 namespace {

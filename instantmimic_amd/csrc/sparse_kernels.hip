@@ -1410,19 +1410,9 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
                                      {8, 0, (const void *)newton_sparse_resident_kernel<8, 0>},
                                      {4, 0, (const void *)newton_sparse_resident_kernel<4, 0>}};
   constexpr int kVariants = 8;
-  static bool usable[kVariants] = {};
-  static bool probed = false;
-  if (!probed) {  // once per process: register spills and the grant of the large dynamic LDS
-    for (int i = 0; i < kVariants; ++i) {
-      hipFuncAttributes fa{};
-      // (a variant that parks more than a few values of its prologue in memory is left out)
-      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
-                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
-      (void)hipGetLastError();
-    }
-    probed = true;
-  }
+  static Kept<int, std::array<bool, kVariants>> probed;
+  std::array<bool, kVariants> usable;
+  if (const int st = usable_variants(probed, variants, &usable)) return st;
   for (int i = 0; i < kVariants; ++i) {
     if (!usable[i] || variants[i].held != (njmax <= 64 ? 2 : 0)) continue;
     // 32 staged rows where the workgroup still fits with them (they cost a CU no world then), else 16

@@ -654,19 +654,9 @@ int newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_unio
                                      IM_DENSE_VARIANT(32, 16, 0), IM_DENSE_VARIANT(32, 8, 0)};
 #undef IM_DENSE_VARIANT
   constexpr int kVariants = 8;
-  static bool usable[kVariants] = {};
-  static bool probed = false;
-  if (!probed) {  // once per process: a variant that spills registers is left out; the large dynamic LDS is asked for
-    for (int i = 0; i < kVariants; ++i) {
-      hipFuncAttributes fa{};
-      // (a variant that parks more than a register or two in memory is left out)
-      usable[i] = hipFuncGetAttributes(&fa, variants[i].fn) == hipSuccess && fa.localSizeBytes <= 16 &&
-                  hipFuncSetAttribute(variants[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
-      (void)hipGetLastError();
-    }
-    probed = true;
-  }
+  static Kept<int, std::array<bool, kVariants>> probed;
+  std::array<bool, kVariants> usable;
+  if (const int st = usable_variants(probed, variants, &usable)) return st;
   const int np = nv <= 16 ? 16 : 32;
   for (int i = 0; i < kVariants; ++i) {
     const Variant &v = variants[i];

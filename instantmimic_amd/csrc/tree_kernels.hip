@@ -812,8 +812,9 @@ int newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, hipStre
   // done takes the next world through the plan's counter, so the worlds that need many iterations
   // do not hold three idle wavefronts in place.
   int per_cu = 0, per_cu_lean = 0;
-  if (lds <= 160 * 1024) if (const int st = resident_per_cu(fn, plan->module != nullptr, 256, lds, &per_cu)) return st;
-  if (const int st = resident_per_cu(fn, plan->module != nullptr, 256, lds_lean, &per_cu_lean)) return st;
+  Occupancy *const plans = plan->module ? &plan->occupancy : nullptr;
+  if (lds <= 160 * 1024) if (const int st = resident_per_cu(fn, plans, 256, lds, &per_cu)) return st;
+  if (const int st = resident_per_cu(fn, plans, 256, lds_lean, &per_cu_lean)) return st;
   // the worlds' rows of M stay in LDS unless leaving them in memory admits another workgroup per CU
   // (snu: 81 KB a workgroup with them, one per CU; 70 KB without, two)
   if (per_cu_lean > per_cu) {
