@@ -29,9 +29,24 @@
 
 #include "../../include/imhip.h"
 #include "common.h"
+#include "newton_solve.h"
 
 namespace im {
 namespace {
+
+// A workgroup per world up to what the chip keeps resident at once (the workgroups walk over worlds: one that
+// does not get in starts when another has done all its worlds).  A CU hands out its LDS in units of 1280
+// bytes, which the runtime's answer does not round up to: 8192 worlds of 250 muscles on a workgroup more per CU
+// than stays resident took 86 us for the force-velocity state instead of 64.
+int resident_grid(const void *fn, int threads, size_t lds, int nworld, unsigned *grid) {
+  int ncu = 0, per_cu = 0;
+  if (const int st = compute_units(&ncu)) return st;
+  if (const int st = resident_per_cu(fn, nullptr, threads, lds, &per_cu)) return st;
+  const size_t unit = 1280, granted = (std::max<size_t>(lds, 1) + unit - 1) / unit * unit;
+  per_cu = std::min(per_cu, (int)(160 * 1024 / granted));
+  *grid = (unsigned)std::min(nworld, ncu * std::max(1, per_cu));
+  return IM_OK;
+}
 
 struct V3 {
   float x, y, z;
@@ -752,11 +767,11 @@ bool launch_world(MwArgs a, int nworld, hipStream_t stream) {
       a.ntorque <= 0 || (MODE != MW_MOMENT && a.nmuscle <= 0))
     return false;
   a.nworld = nworld;
-  // as many workgroups as are resident at once: 24 wavefronts per CU by registers, or what the LDS holds
-  const int by_lds = (int)(160 * 1024 / ((lds_bytes + 1279) / 1280 * 1280)), resident = 256 * std::min(2, by_lds);
   auto kernel = trips == 2 ? muscle_world_kernel<MODE, 2> : trips == 4 ? muscle_world_kernel<MODE, 4>
               : trips == 6 ? muscle_world_kernel<MODE, 6> : muscle_world_kernel<MODE, 0>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(nworld, resident)), dim3(kMwThreads), lds_bytes, stream, a);
+  unsigned grid = 0;
+  if (resident_grid((const void *)kernel, kMwThreads, lds_bytes, nworld, &grid) != IM_OK) return false;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kMwThreads), lds_bytes, stream, a);
   return true;
 }
 
@@ -863,8 +878,9 @@ extern "C" int im_muscle_force_velocity_state(
   if (!forced_off && ld_waypoints > 0 && ld_moment > 0 && ld_qvel > 0 && nmuscle <= 16 * 1024 && n.bytes() <= 80 * 1024) {
     if (n.bytes() > 64 * 1024)
       IM_HIP_CHECK(hipFuncSetAttribute((const void *)force_velocity_state_world_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, n.bytes()));
-    const int resident = 256 * std::min(32 / (kFvThreads / 64), 160 * 1024 / ((n.bytes() + 1279) / 1280 * 1280));
-    hipLaunchKernelGGL(force_velocity_state_world_kernel, dim3((unsigned)std::min(nworld, resident)), dim3(kFvThreads),
+    unsigned grid = 0;
+    if (const int st = resident_grid((const void *)force_velocity_state_world_kernel, kFvThreads, (size_t)n.bytes(), nworld, &grid)) return st;
+    hipLaunchKernelGGL(force_velocity_state_world_kernel, dim3(grid), dim3(kFvThreads),
                        (size_t)n.bytes(), (hipStream_t)stream, waypoints, ld_waypoints, muscle_waypoint_start,
                        muscle_params, ld_params, muscle_rest_length, force_velocity_length_scale, activation,
                        ld_activation, qvel, ld_qvel, moment, ld_moment, muscle_dof_offsets, muscle_dof_torque_idx,

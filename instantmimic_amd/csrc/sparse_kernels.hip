@@ -1292,13 +1292,14 @@ int im_sparse_update_factor(const im_sparse_plan *plan, const uint8_t *done, con
       // (at most 32 wavefronts of 57 registers) is taken, the smallest on a tie and where four
       // per workgroup already hold the whole batch.
       constexpr size_t kCuLds = 160 * 1024;
-      int waves = 4;
+      int waves = 4, ncu = 0;
       int64_t best = 0;
+      if (const int st = im::compute_units(&ncu)) return st;
       for (int cand = 4; cand <= 16; cand *= 2) {
         const size_t bytes = 4 * (staged + solve_words + (size_t)cand * per_world);
         int64_t held = (int64_t)(kCuLds / bytes) * cand;
         held = held < 32 ? held : 32;
-        if (held > best && (cand == 4 || (int64_t)nworld > best * 256)) best = held, waves = cand;
+        if (held > best && (cand == 4 || (int64_t)nworld > best * ncu)) best = held, waves = cand;
       }
       const size_t lds_bytes = 4 * (staged + solve_words + (size_t)waves * per_world);
       const dim3 grid((unsigned)((nworld + waves - 1) / waves)), wg(64 * waves);
