@@ -257,9 +257,10 @@ __global__ __launch_bounds__(256) void force_velocity_state_kernel(
 // (a lane per muscle left the wavefront waiting for its longest muscle's roots); and what does
 // not depend on the world (an entry's dof, a muscle's cos(pennation)) is left in LDS once.  Same
 // operations in the same order, so the same bits.
-// 284 muscles x 4096 worlds: 59.3 us (a workgroup of 256 per world, distances by the muscle's
-// lane) -> 38.9; 256 threads 48.4, 512 threads 52.7.
-constexpr int kFvThreads = 320;
+// As many threads as it takes for a muscle each, 128 to 320: a workgroup's last phase is its muscles'
+// chains, and threads beyond them only take a CU's places from other worlds (8192 worlds of 40 / 100 / 200
+// muscles: 23.5 / 31.3 / 48.7 us, with 320 threads 50 / 59 / 68).  A launch per world with 256 threads,
+// distances by the muscle's lane, took 23.0 / 38.8 / 59.0 us there, and 57.4 at 284 muscles x 4096 worlds, here 38.
 struct FvLds {
   int words_wp, nentry, nqvel, nmuscle;  // the longest rows that fit; what is read of them is what the tables name
   __host__ __device__ int bytes() const {
@@ -267,8 +268,8 @@ struct FvLds {
   }
 };
 
+template <int nt>
 __device__ __forceinline__ void stage_row(float *to, const float *__restrict__ from, int n, int tid) {
-  constexpr int nt = kFvThreads;
   int i = tid;
   for (; i + 7 * nt < n; i += 8 * nt) {
     float v[8];
@@ -287,7 +288,8 @@ __device__ __forceinline__ void stage_row(float *to, const float *__restrict__ f
   }
 }
 
-__global__ __launch_bounds__(kFvThreads) void force_velocity_state_world_kernel(
+template <int nt>
+__global__ __launch_bounds__(nt) void force_velocity_state_world_kernel(
     const float *__restrict__ wp, int64_t ldw, const int32_t *__restrict__ waypoint_start,
     const float *__restrict__ params, int ldpar, const float *__restrict__ rest,
     const float *__restrict__ length_scale, const float *__restrict__ activation, int64_t lda,
@@ -304,7 +306,6 @@ __global__ __launch_bounds__(kFvThreads) void force_velocity_state_world_kernel(
   float *cosp = dist + n.words_wp / 3;  // [nmuscle]
   int *named = (int *)(cosp + n.nmuscle);  // the velocities up to the last dof that the tables name
   unsigned short *dof = (unsigned short *)(named + 1);  // [nentry]
-  constexpr int nt = kFvThreads;
   const int tid = threadIdx.x, nmuscle = n.nmuscle;
   // what the tables name of a row, which may be a part of a wider array's: the last world's row ends
   // with its last named value, wherever the stride would lead
@@ -322,9 +323,9 @@ __global__ __launch_bounds__(kFvThreads) void force_velocity_state_world_kernel(
   for (int m = tid; m < nmuscle; m += nt) cosp[m] = cosf(params[m * ldpar + 3]);
   for (int64_t w = blockIdx.x; w < nworld; w += gridDim.x) {
     __syncthreads();  // the tables are there, the world before is done with
-    stage_row(row, wp + w * ldw, 3 * nwp, tid);
-    stage_row(mom, moment + w * ldm, ne, tid);
-    stage_row(qv, qvel + w * ldq, min(__builtin_amdgcn_readfirstlane(*named), n.nqvel), tid);
+    stage_row<nt>(row, wp + w * ldw, 3 * nwp, tid);
+    stage_row<nt>(mom, moment + w * ldm, ne, tid);
+    stage_row<nt>(qv, qvel + w * ldq, min(__builtin_amdgcn_readfirstlane(*named), n.nqvel), tid);
     __syncthreads();
     for (int i = tid; i < nwp - 1; i += nt) dist[i] = length(sub(ld3(row + 3 * (i + 1)), ld3(row + 3 * i)));
     __syncthreads();
@@ -876,11 +877,20 @@ extern "C" int im_muscle_force_velocity_state(
   const FvLds n{(int)std::min<int64_t>(ld_waypoints, 1 << 20), (int)std::min<int64_t>(ld_moment, 1 << 20),
                 (int)std::min<int64_t>(ld_qvel, 1 << 20), nmuscle};
   if (!forced_off && ld_waypoints > 0 && ld_moment > 0 && ld_qvel > 0 && nmuscle <= 16 * 1024 && n.bytes() <= 80 * 1024) {
+    // (a batch of up to four workgroups per CU, all resident at once, has the threads to spare: 1000 worlds of
+    // 100 muscles 7.7 us with 320 threads, 8.4 with 128)
+    int ncu = 0;
+    if (const int st = compute_units(&ncu)) return st;
+    const int threads = nworld <= 4 * ncu ? 320 : std::min(std::max((nmuscle + 63) / 64 * 64, 128), 320);
+    auto kernel = threads == 128   ? force_velocity_state_world_kernel<128>
+                  : threads == 192 ? force_velocity_state_world_kernel<192>
+                  : threads == 256 ? force_velocity_state_world_kernel<256>
+                                   : force_velocity_state_world_kernel<320>;
     if (n.bytes() > 64 * 1024)
-      IM_HIP_CHECK(hipFuncSetAttribute((const void *)force_velocity_state_world_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, n.bytes()));
+      IM_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, n.bytes()));
     unsigned grid = 0;
-    if (const int st = resident_grid((const void *)force_velocity_state_world_kernel, kFvThreads, (size_t)n.bytes(), nworld, &grid)) return st;
-    hipLaunchKernelGGL(force_velocity_state_world_kernel, dim3(grid), dim3(kFvThreads),
+    if (const int st = resident_grid((const void *)kernel, threads, (size_t)n.bytes(), nworld, &grid)) return st;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads),
                        (size_t)n.bytes(), (hipStream_t)stream, waypoints, ld_waypoints, muscle_waypoint_start,
                        muscle_params, ld_params, muscle_rest_length, force_velocity_length_scale, activation,
                        ld_activation, qvel, ld_qvel, moment, ld_moment, muscle_dof_offsets, muscle_dof_torque_idx,

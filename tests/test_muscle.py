@@ -136,10 +136,10 @@ def test_gpu_projection_with_more_entries_than_one_staging_trip(device):
     assert (got[:, : mb.root_dof_count] == 7.0).all()
 
 
-def _fv_case(nworld, seed=4, active_type=1.0):
+def _fv_case(nworld, seed=4, active_type=1.0, nmuscle=37):
     """Random muscles over random waypoints: every branch of the force-velocity curve is hit."""
     rng = np.random.default_rng(seed)
-    nmuscle, nv, root = 37, 30, 6
+    nv, root = 30, 6
     counts = rng.integers(2, 6, nmuscle)
     wp_start = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
     nwp = int(wp_start[-1])
@@ -246,6 +246,30 @@ def test_gpu_force_velocity_state_of_many_worlds(device, pad):
     Q.eval_muscle_force_velocity_state(
         t(c["waypoints"]), t(c["wp_start"]), t(c["params"]), t(c["rest"]), t(c["length_scale"]), wide(c["act"]), t(c["qvel"]),
         wide(c["moment"]), t(c["dof_offsets"]), t(c["dof_torque"]), c["root"], muscle_force_scale=float(c["model"][0]),
+        muscle_length_norm_min=float(c["model"][1]), muscle_length_norm_max=float(c["model"][2]), vmax=1.5, fvmax=1.4,
+        clamp_activation=True, include_active=True, active_force_model_params=c["model"][3:6],
+        muscle_length=outs[0], effective_activation=outs[1], length_velocity=outs[2], force_velocity_multiplier=outs[3],
+        force_velocity_slope=outs[4],
+    )  # fmt: skip
+    want = R.muscle_force_velocity_state(**c)
+    for k in range(4):
+        np.testing.assert_array_equal(outs[k].cpu().numpy(), want[k])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1030, 3001])
+@pytest.mark.parametrize("nmuscle", [1, 128, 129, 192, 193, 256, 257, 320, 321, 700])
+def test_gpu_force_velocity_state_on_every_workgroup_size(device, nmuscle, n):
+    """Both sides of the muscle counts at which a workgroup gets another 64 threads, more muscles than
+    threads, workgroups that walk over several worlds: bit for bit."""
+    import torch
+
+    c = _fv_case(n, active_type=1.0, nmuscle=nmuscle)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    outs = [torch.full((n, nmuscle), float("nan"), device=device) for _ in range(5)]
+    Q.eval_muscle_force_velocity_state(
+        t(c["waypoints"]), t(c["wp_start"]), t(c["params"]), t(c["rest"]), t(c["length_scale"]), t(c["act"]), t(c["qvel"]),
+        t(c["moment"]), t(c["dof_offsets"]), t(c["dof_torque"]), c["root"], muscle_force_scale=float(c["model"][0]),
         muscle_length_norm_min=float(c["model"][1]), muscle_length_norm_max=float(c["model"][2]), vmax=1.5, fvmax=1.4,
         clamp_activation=True, include_active=True, active_force_model_params=c["model"][3:6],
         muscle_length=outs[0], effective_activation=outs[1], length_velocity=outs[2], force_velocity_multiplier=outs[3],
