@@ -511,14 +511,17 @@ __global__ __launch_bounds__(256) void torque_bounds_kernel(
 // left out without changing bits, and a launch per world spent as many again on the entry lists
 // (four table reads with their addresses, the entry's row, the products by the LDS records'
 // sizes; 63 - 79 % of the cycles issued a vector instruction).  The lists are the same for every
-// world, so the grid is what the chip holds at once, a workgroup walks over worlds, and a thread
-// keeps its TRIPS entries as LDS addresses and coefficients in registers.  An output's ordered
-// sum runs beside the next world's staging: two barriers per world.
-// 284 muscles (553 segments, 4445 entries) x 4096 worlds, a launch per world with 512 threads ->
-// this: moment 64.6 -> 50.8 us, activation gradient 57.1 -> 52.0, torque 73.9 -> 75 (its longest
-// row's 327 additions are the chain there; its entries issue as in the others, and one form
-// serves all).  512 threads with ten entries each spill 84 bytes a lane at 80 registers (moment
-// 54), 1024 threads with five spill at 64 (moment 49, gradient and torque 10 % slower).
+// world, so the grid is what the chip holds at once, a workgroup walks over worlds, and a thread of
+// a small rig keeps its TRIPS entries as LDS addresses and coefficients in registers.  An output's
+// ordered sum runs beside the next world's staging: two barriers per world.
+// Threads by the entries (launch_world).  The kernels alone, torque / gradient / moment, a launch per
+// world with 512 threads -> this:
+//    40 muscles ( 655 entries) x 8192 worlds  41.9 / 36.8 / 29.1 -> 24.8 / 22.0 / 20.3 us
+//   120         (1882)                        70.5 / 53.9 / 51.2 -> 57.0 / 40.1 / 40.5
+//   200         (3145)                        90.7 / 71.9 / 72.0 -> 83.6 / 66.5 / 65.6
+//   284         (4445)                         133 / 98.1 /  108 ->  116 / 86.1 / 87.0
+// 768 threads that keep six entries each, the best for the moment at 284 muscles alone (84.8 us), took
+// 48.7 / 39.0 / 35.6 at 40 muscles and 116 / 78.6 / 75.8 at 200.
 enum { MW_FORWARD, MW_GRAD, MW_BOUNDS, MW_MOMENT };
 
 struct MwArgs {
@@ -535,7 +538,6 @@ struct MwArgs {
   int nworld;
 };
 
-constexpr int kMwThreads = 768;
 constexpr int kContribPad = 4;  // floats read past the last entry by ordered_sum()
 constexpr int kAxis = 7;        // floats of a dof's record: its cdof and, for MW_GRAD, grad_output
 struct MwLds {
@@ -588,29 +590,23 @@ __device__ __forceinline__ float entry_contribution(const float *lds, const MwEn
   return c;
 }
 
-// Sum of contrib[e0..e1) in list order from +0.  Whole groups of 8 (LONG) and of 4 entries are
-// read with one address and added without a test; the last group reads up to three floats past
+// Sum of contrib[e0..e1) in list order from +0.  Whole groups of 16 (LONG) and of 4 entries are
+// read with one address and added without a test (sixteen ahead of their additions: 119.6 -> 111.4 us
+// against eight with the next eight on their way, torque of 284 muscles x 8192 worlds); the last group reads up to three floats past
 // e1 (contrib is padded for that) and enters them as +0, which leaves every bit of a sum that
 // started at +0 (such a sum is never -0).
 template <bool LONG>
 __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e1) {
   float total = 0.0f;
   int e = e0;
-  if (LONG && e + 8 <= e1) {  // the next eight are on their way while these are added
-    float c[8];
+  if (LONG) {
+    for (; e + 16 <= e1; e += 16) {
+      float c[16];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) c[k] = contrib[e + k];
-    for (e += 8; e + 8 <= e1; e += 8) {
-      float n[8];
+      for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) n[k] = contrib[e + k];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) total = total + c[k];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) c[k] = n[k];
+      for (int k = 0; k < 16; ++k) total = total + c[k];
     }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) total = total + c[k];
   }
   for (; e + 4 <= e1; e += 4) {
     float c[4];
@@ -629,10 +625,10 @@ __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e
   return total;
 }
 
-// TRIPS: entries that a thread keeps in registers, nentry <= TRIPS * kMwThreads; 0: more
-// entries than that, read from the lists for every world.
-template <int MODE, int TRIPS>
-__global__ __launch_bounds__(kMwThreads, 6) void muscle_world_kernel(MwArgs a) {
+// TRIPS: entries that a thread keeps in registers, nentry <= TRIPS * NT; 0: they are read from the
+// lists for every world.
+template <int MODE, int NT, int TRIPS>
+__global__ __launch_bounds__(NT, 6) void muscle_world_kernel(MwArgs a) {
   extern __shared__ float lds[];
   MwLds l;
   l.segd = lds;
@@ -640,7 +636,7 @@ __global__ __launch_bounds__(kMwThreads, 6) void muscle_world_kernel(MwArgs a) {
   l.axis = l.contrib + a.nentry + kContribPad;
   l.force = l.axis + kAxis * a.ntorque;
   l.rowid = (unsigned short *)(TRIPS ? l.contrib : lds + mw_lds_floats(a));
-  constexpr int nt = kMwThreads;
+  constexpr int nt = NT;
   const int tid = threadIdx.x;
   // staging starts at the last wavefront: the first one's sums of the world before take longest
   const int rid = nt - 1 - tid;
@@ -730,16 +726,25 @@ __global__ __launch_bounds__(kMwThreads, 6) void muscle_world_kernel(MwArgs a) {
       } else {
         int current = -1;
         float total = 0.0f, lo = 0.0f, hi = 0.0f;
-        for (int e = e0; e < e1; ++e) {
-          const int m = a.e_other[e];
+        auto add = [&](int m, float c) __attribute__((always_inline)) {
           if (current >= 0 && m != current) {
             if (total < 0.0f) lo = lo + total;
             else hi = hi + total;
             total = 0.0f;
           }
           current = m;
-          total = total + contrib[e];
+          total = total + c;
+        };
+        int e = e0;
+        for (; e + 8 <= e1; e += 8) {  // eight entries' muscles on their way at once
+          int m[8];
+          float c[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) m[k] = a.e_other[e + k], c[k] = contrib[e + k];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) add(m[k], c[k]);
         }
+        for (; e < e1; ++e) add(a.e_other[e], contrib[e]);
         if (current >= 0) {
           if (total < 0.0f) lo = lo + total;
           else hi = hi + total;
@@ -754,26 +759,39 @@ __global__ __launch_bounds__(kMwThreads, 6) void muscle_world_kernel(MwArgs a) {
 // Launches the workgroup-per-world kernel when a world's segments and entries fit in LDS (which
 // also keeps the records' word indices below 16 bits) and the entry list states the range of its
 // `other` column; returns false for the caller to use the one-thread-per-output kernel instead.
+template <int MODE, int NT, int TRIPS>
+bool launch_world_on(MwArgs a, bool walk, int nworld, hipStream_t stream) {
+  const size_t lds_bytes = 4 * mw_lds_floats(a) + (TRIPS ? 0 : 2 * (((size_t)a.nentry + 1) & ~(size_t)1));
+  if (lds_bytes > 64 * 1024) return false;
+  unsigned grid = (unsigned)nworld;
+  if (walk && resident_grid((const void *)muscle_world_kernel<MODE, NT, TRIPS>, NT, lds_bytes, nworld, &grid) != IM_OK) return false;
+  a.nworld = nworld;
+  hipLaunchKernelGGL((muscle_world_kernel<MODE, NT, TRIPS>), dim3(grid), dim3(NT), lds_bytes, stream, a);
+  return true;
+}
 template <int MODE>
-bool launch_world(MwArgs a, int nworld, hipStream_t stream) {
-  // six entries per thread are 24 registers beside the evaluation's, what 6 wavefronts per SIMD leave;
-  // more entries (about 295 muscles) are read from the lists by every world
-  const int trips = a.nentry <= 2 * kMwThreads ? 2 : a.nentry <= 4 * kMwThreads ? 4 : a.nentry <= 6 * kMwThreads ? 6 : 0;
-  const size_t lds_bytes = 4 * mw_lds_floats(a) + (trips ? 0 : 2 * (((size_t)a.nentry + 1) & ~(size_t)1));
+bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
   static const bool forced_off = [] {
     const char *e = std::getenv("IMHIP_MUSCLE_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  if (forced_off || lds_bytes > 64 * 1024 || a.nentry == 0 || a.nseg == 0 || a.nrow > 65535 ||
-      a.ntorque <= 0 || (MODE != MW_MOMENT && a.nmuscle <= 0))
-    return false;
-  a.nworld = nworld;
-  auto kernel = trips == 2 ? muscle_world_kernel<MODE, 2> : trips == 4 ? muscle_world_kernel<MODE, 4>
-              : trips == 6 ? muscle_world_kernel<MODE, 6> : muscle_world_kernel<MODE, 0>;
-  unsigned grid = 0;
-  if (resident_grid((const void *)kernel, kMwThreads, lds_bytes, nworld, &grid) != IM_OK) return false;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kMwThreads), lds_bytes, stream, a);
-  return true;
+  if (forced_off || a.nentry == 0 || a.nseg == 0 || a.nrow > 65535 || a.ntorque <= 0 || (MODE != MW_MOMENT && a.nmuscle <= 0)) return false;
+  const bool small = a.nentry <= 6 * 256;
+  // The bounds' rows are long chains of comparisons on a few lanes: a workgroup per world hides them behind other
+  // worlds, one that stays does not (40 / 120 / 200 / 284 muscles x 8192 worlds: 33.6 / 102 / 161 / 274 us; on
+  // workgroups that stay 57 / 124 / 197 / 268; 768 threads with an entry's muscle read at a time 112 / 272 / 426 / 594).
+  if (MODE == MW_BOUNDS)
+    return small ? launch_world_on<MODE, 256, 0>(a, false, nworld, stream) : launch_world_on<MODE, 512, 0>(a, false, nworld, stream);
+  int ncu = 0;
+  if (compute_units(&ncu) != IM_OK) return false;
+  // Entries kept in registers pay from two worlds per workgroup on (seven of 256 threads, three of 512 per CU), and up
+  // to about 2000 entries; beyond, and with 512 threads throughout, reading them from the lists takes as long.
+  if (small && nworld >= 2 * 7 * ncu)
+    return a.nentry <= 2 * 256   ? launch_world_on<MODE, 256, 2>(a, true, nworld, stream)
+           : a.nentry <= 4 * 256 ? launch_world_on<MODE, 256, 4>(a, true, nworld, stream)
+                                 : launch_world_on<MODE, 256, 6>(a, true, nworld, stream);
+  if (!small && a.nentry <= 4 * 512 && nworld >= 2 * 3 * ncu) return launch_world_on<MODE, 512, 4>(a, true, nworld, stream);
+  return launch_world_on<MODE, 512, 0>(a, true, nworld, stream);
 }
 
 bool geo_ok(const im_muscle_geometry *g) {

@@ -659,3 +659,35 @@ def test_gpu_contractions_of_many_worlds_equal_one_world_per_workgroup(muscles):
         e.nother = 0
     for a, b in zip(kept, run()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("muscles", [29, 30, 63, 64, 94, 95, 131, 132])
+def test_gpu_contractions_on_every_workgroup_size(muscles):
+    """Both sides of 512, 1024, 1536 and 2048 entries, where a workgroup's threads and the entries they
+    keep change, in batches below and above those in which workgroups keep any (1536 and 3584 worlds):
+    the bits of the one-thread-per-output kernels."""
+    rig = synth.make_muscle_rig(nmuscle=muscles, seed=1003)
+    layer = _gpu_layer(rig)
+    limit = {29: 512, 63: 1024, 94: 1536, 131: 2048}
+    assert all(layer._torque_entries.nentry <= limit[m] if m in limit else layer._torque_entries.nentry > limit[m - 1] for m in [muscles])
+    entries = (layer._torque_entries, layer._muscle_entries, layer._moment_entries)
+    stated = [e.nother for e in entries]
+    for nworld in (70, 1537, 3601):
+        ctx_d = torch.from_numpy(synth.make_muscle_context(rig, nworld, seed=6)).cuda()
+        act = torch.rand(nworld, rig.muscle_count, device="cuda")
+        act[:, ::7] = 0.0
+        g = torch.randn(nworld, rig.torque_dim, device="cuda")
+
+        def run():
+            mean, _, unit = layer._warp_muscle_dynamics_from_activation_forward(act, ctx_d, include_passive_force=True)
+            lo, hi = layer._compute_activation_torque_bounds_warp(ctx_d, select_active=False)
+            return mean, layer._warp_muscle_dynamics_from_activation_backward(ctx_d, g), layer.eval_muscle_sparse_moment(ctx_d), lo, hi
+
+        got = run()
+        for e in entries:
+            e.nother = 0
+        for a, b in zip(got, run()):
+            assert torch.equal(a, b)
+        for e, n in zip(entries, stated):
+            e.nother = n
