@@ -60,3 +60,61 @@ def test_gpu_dense_hessian_solve_at_block_edges(device, nv):
     x_ref, U_ref = R.blocked_factor_solve(np.ascontiguousarray(H_ref[:, :nv, :nv]).reshape(nworld, -1), layout, nv, pad, 16, y)
     np.testing.assert_array_equal(U.cpu().numpy(), U_ref)
     np.testing.assert_array_equal(x.cpu().numpy(), x_ref)
+
+
+def _hessian_case(nv, rows, counts, seed):
+    rng, nworld = np.random.default_rng(seed), len(counts)
+    M, y = _spd(rng, nworld, nv), rng.standard_normal((nworld, nv)).astype(np.float32)
+    M[-1] *= np.float32(2.0**110)
+    J = rng.standard_normal((nworld, rows, nv)).astype(np.float32)
+    D = rng.uniform(0.1, 10.0, (nworld, rows)).astype(np.float32)
+    state = (rng.uniform(size=(nworld, rows)) < 0.7).astype(np.int32)
+    return M, J, D, state, np.asarray(counts, np.int32), y
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv,hpad,offset", [(9, 9, 0), (15, 15, 0), (17, 18, 0), (33, 35, 0), (48, 48, 1), (64, 67, 0), (79, 80, 3), (127, 127, 0), (128, 128, 2)])
+def test_gpu_dense_hessian_in_rows_that_take_no_wide_store(device, nv, hpad, offset):
+    """H with a row length that is no multiple of four, or off 16 bytes: the bits of an aligned H, nothing
+    written beyond the dofs."""
+    import torch
+
+    c = [torch.from_numpy(np.ascontiguousarray(a)).to(device) for a in _hessian_case(nv, 70, [0, 5, 64, 70, 33], nv)]
+    nworld, apad = 5, -(-nv // 16) * 16
+    x, xa = torch.zeros((nworld, nv), device=device), torch.zeros((nworld, nv), device=device)
+    flat = torch.full((nworld * hpad * hpad + 4,), 7.0, device=device)
+    H = flat[offset : offset + nworld * hpad * hpad].view(nworld, hpad, hpad)
+    aligned = torch.full((nworld, apad, apad), 7.0, device=device)
+    assert (hpad % 4 or H.data_ptr() % 16) and aligned.data_ptr() % 16 == 0
+    BD.dense_hessian_factor_solve(*c[:5], H, c[5], x)
+    BD.dense_hessian_factor_solve(*c[:5], aligned, c[5], xa)
+    assert torch.equal(H[:, :nv, :nv], aligned[:, :nv, :nv]) and torch.equal(x, xa)
+    H[:, :nv, :nv] = 7.0
+    assert bool((flat == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv", [16, 33, 79])
+def test_gpu_dense_hessian_of_long_row_lists(device, nv):
+    """More rows than four worlds' lists fit a workgroup's LDS (a wavefront per workgroup then), and more
+    than one world's list fits a CU's: refused."""
+    import torch
+
+    rows, nworld = 5301, 3
+    M, J, D, state, counts, y = _hessian_case(nv, rows, [rows, 1, 4099], nv)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    pad = -(-nv // 16) * 16
+    H, x, U = torch.zeros((nworld, pad, pad), device=device), torch.zeros((nworld, nv), device=device), torch.zeros((nworld, pad, pad), device=device)
+    BD.dense_hessian_factor_solve(t(M), t(J), t(D), t(state), t(counts), H, t(y), x, factor=U)
+    H_ref = H.cpu().numpy()
+    # 3700 terms an element in another order: about sqrt(3700) half-ulps of 6e-8, 3.6e-6
+    assert R.rel_l2(H_ref, R.jtdj_dense(M.reshape(nworld, -1), J, D, state, counts, pad)) <= 1e-5
+    np.testing.assert_array_equal(H_ref, H_ref.transpose(0, 2, 1))
+    _, layout, _ = BD.block_index_layout(np.arange(nv * nv), nv, nv * nv, 16)
+    x_ref, U_ref = R.blocked_factor_solve(np.ascontiguousarray(H_ref[:, :nv, :nv]).reshape(nworld, -1), layout, nv, pad, 16, y)
+    np.testing.assert_array_equal(U.cpu().numpy(), U_ref)
+    np.testing.assert_array_equal(x.cpu().numpy(), x_ref)
+    many = 20500
+    with pytest.raises(_lib.ImhipError):
+        BD.dense_hessian_factor_solve(t(M[:1]), torch.zeros((1, many, nv), device=device), torch.zeros((1, many), device=device),
+                                      torch.zeros((1, many), dtype=torch.int32, device=device), None, None, t(y[:1]), x[:1])  # fmt: skip
