@@ -342,7 +342,7 @@ def native():
     Python caller has to look at itself."""
     global _native
     if _native is None:
-        import torch  # noqa: F401  (the module links against torch's libraries)
+        import torch  # (the module links against torch's libraries)
 
         lib()
         path = os.path.join(_HERE, "_native.so")
@@ -350,6 +350,9 @@ def native():
             raise RuntimeError(f"{path} is missing: build it with `python -m instantmimic_amd.build`")
         from . import _native as module
 
+        if module.torch_version != torch.__version__:
+            raise RuntimeError(f"{path} was built for torch {module.torch_version}, this is {torch.__version__}: "
+                               "build it again with `python -m instantmimic_amd.build`")  # fmt: skip
         _native = module
     return _native
 

@@ -209,23 +209,31 @@ def build_library(verbose: bool = True) -> str:
 
 def build_native() -> str:
     """``_native.so``, the CPython module of ``csrc/native_calls.cpp``: host code only, against torch's
-    headers and ``libimhip.so``."""
+    headers and ``libimhip.so``.  Built again when its source, the C header, the command or the torch
+    that it was built for has changed (torch's C++ interface differs from release to release)."""
+    import hashlib
     import sysconfig
 
     import torch
 
     src = os.path.join(CSRC, "native_calls.cpp")
     header = os.path.join(HERE, "..", "include", "imhip.h")
-    if os.path.exists(NATIVE) and not os.environ.get("IMHIP_REBUILD") and os.path.getmtime(NATIVE) > max(os.path.getmtime(p) for p in (src, header)):
-        return NATIVE
     base = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH") or "/opt/rocm"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f'-DIM_TORCH_VERSION="{torch.__version__}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", f"{base}/include",
            "-isystem", f"{base}/include/torch/csrc/api/include", "-isystem", f"{rocm}/include",
            "-isystem", sysconfig.get_paths()["include"], src, "-o", NATIVE, f"-L{base}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu",
            "-ltorch_python", f"-L{HERE}", "-l:libimhip.so", "-Wl,-rpath,$ORIGIN"]  # fmt: skip
+    stamp = hashlib.sha256("\n".join([*cmd, str(torch.version.git_version), *(open(p).read() for p in (src, header))]).encode()).hexdigest()
+    note = os.path.join(OBJ, "_native.stamp")
+    if os.path.exists(NATIVE) and os.path.exists(note) and open(note).read() == stamp and not os.environ.get("IMHIP_REBUILD"):
+        return NATIVE
     subprocess.run(cmd, check=True)
+    os.makedirs(OBJ, exist_ok=True)
+    with open(note, "w") as f:
+        f.write(stamp)
     return NATIVE
 
 

@@ -421,5 +421,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Host path of the hot en
 
 PyMODINIT_FUNC PyInit__native(void) {
   if (!names.make()) return nullptr;
-  return PyModule_Create(&module);
+  PyObject *m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", IM_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
 }
