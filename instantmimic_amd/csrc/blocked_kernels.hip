@@ -13,6 +13,7 @@
 //   is applied as a multiplication by 1 / diagonal (the reciprocal is an exact division).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 #include <cstring>
@@ -20,6 +21,7 @@
 #include "common.h"
 #include "dense_solve.h"
 #include "jtdj_wave.h"
+#include "newton_solve.h"
 #include "pivot.h"
 
 namespace im {
@@ -1358,6 +1360,46 @@ __global__ __launch_bounds__(256, NVR == 128 ? 4 : 3) void jtdj_mfma_kernel(
   });
 }
 
+// The same assembly and the blocked Cholesky of H with its solve behind it in one workgroup per world: for
+// batches that leave most of the chip idle with a wavefront per world (dense_solve_kernels.hip), whose
+// tiles one wavefront then forms one after the other (im_jtdj_factor_solve says where the line lies).  H
+// goes into the factor's LDS array at once, where the rows of J were staged; the bits are those of
+// im_jtdj_mfma followed by im_blocked_factor_solve (B = 16).
+__global__ __launch_bounds__(256, 2) void jtdj_factor_solve_kernel(
+    const float *__restrict__ Mdense, const float *__restrict__ J, int njmax, const float *__restrict__ D,
+    const int32_t *__restrict__ state, const int32_t *__restrict__ nefc_p, int quad, float *__restrict__ H, int nv,
+    int nv_pad, const float *__restrict__ y, int64_t ldy, float *__restrict__ Uout, float *__restrict__ x, int64_t ldx,
+    int pad, int rhs_at) {
+  constexpr int B = 16;
+  extern __shared__ float lds[];
+  const Stair<B> S{pad};
+  float *U = lds, *rhs = lds + rhs_at, *L = rhs + pad;  // [rhs_at] the staged rows, then H, then the factor; [pad]; [B * B + B]
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int64_t w = blockIdx.x;
+  for (int i = tid; i < pad; i += nt) rhs[i] = (y && i < nv) ? y[w * ldy + i] : 0.0f;
+  float *Hw = H ? H + w * (int64_t)nv_pad * nv_pad : nullptr;
+  // Every wavefront has passed the assembly's last barrier when the elements come out.  The factor reads
+  // the upper triangle below nv only and writes every entry of a block row before anything reads it.
+  const bool vec = (nv_pad & 3) == 0 && ((uintptr_t)H & 15) == 0;
+  jtdj_tiles<128>(Mdense, J, njmax, D, state, nefc_p, quad, nv, lds, [&](int i0, int j, float4v h, bool off) {
+    if (Hw) store_h_mirrored(Hw, nv, nv_pad, vec, i0, j, h, off);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (i0 + v < nv && j < nv && i0 + v <= j) U[S.at(i0 + v, j)] = h[v];
+  });
+  __syncthreads();
+  const LdsSrc<B> src{U, nv, pad};
+  factor_forward<B>(src, U, rhs, L, pad, tid, nt);
+  backward_solve<B>(U, rhs, pad, tid, nt);
+  if (x)
+    for (int i = tid; i < nv; i += nt) x[w * ldx + i] = rhs[i];
+  if (Uout)
+    for (int i = tid; i < pad * pad / 4; i += nt) {
+      const int r = 4 * i / pad, c = 4 * i - r * pad;
+      if (c >= r / B * B) ((float4 *)(Uout + w * (int64_t)pad * pad))[i] = *(const float4 *)(U + S.at(r, c));  // (tiles on and right of the diagonal)
+    }
+}
+
 // Every float whose bit pattern lies in [first, last] and that is in the pivots' range: do the
 // short forms give the bits of sqrtf and of 1.0f / sqrtf?
 __global__ void check_pivot_sqrt_kernel(uint32_t first, uint32_t last, unsigned long long *mismatches) {
@@ -1410,12 +1452,20 @@ static int launch_blocked_factor(const float *M, int64_t ldM, int nM, const int3
                                  const int32_t *active, int nworld, void *stream) {
   const int B = block_size;
   // up to 128 dofs a wavefront holds the matrix in its registers; the workgroup-per-world kernel below serves
-  // the larger ones (IMHIP_BLOCKED_KERNEL=simple: all)
+  // the larger ones (IMHIP_BLOCKED_KERNEL=simple: all), and in blocks of 16 those from 112 dofs on in batches of
+  // up to a world per CU: 112 / 128 dofs x 256 worlds 34.0 / 39.6 us, a wavefront 36.1 / 44.5 (104 dofs: 34.0
+  // and 32.7, 128 dofs x 257 worlds 46.0 and 44.2)
   static const bool simple = [] {
     const char *e = std::getenv("IMHIP_BLOCKED_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  if (nv <= 128 && !simple)
+  bool wave = nv <= 128 && !simple;
+  if (wave && B == 16 && nv >= 112) {
+    int ncu = 0;
+    if (const int st = im::compute_units(&ncu)) return st;
+    wave = nworld > ncu;
+  }
+  if (wave)
     return im::blocked_solve_wave(M, ldM, nM, block_idx, B, nv, pad, y, ldy, U, x, ldx, active, nworld, (hipStream_t)stream);
   const size_t u_words = B == 8 ? im::Stair<8>{pad}.words() : im::Stair<16>{pad}.words();
   const size_t lds_bytes = sizeof(float) * (u_words + pad + B * B + B);
@@ -1560,6 +1610,25 @@ int im_jtdj_factor_solve(const float *Mdense, const float *J, int njmax, const f
   if (nv > 128) return IM_ERR_UNSUPPORTED;
   if ((y && ldy < nv) || (x && ldx < nv)) return IM_ERR_STRIDE;
   if (U && ((uintptr_t)U & 15)) return IM_ERR_STRIDE;
+  // A wavefront per world, but a workgroup per world for matrices of more than 112 dofs in batches of up to a world
+  // per CU, or two with 192 rows and more: 128 dofs with 96 rows take 45.2 / 47.3 us in 128 / 256 worlds (a wavefront
+  // 52.6 / 56.0), with 256 rows 52.5 / 66.6 in 256 / 512 (71.4 / 73.3); beyond the line 513 worlds take 71.8 with a
+  // wavefront and 77.8 with a workgroup.  112 dofs take a wavefront 38 - 59 us in these batches, a workgroup 41 - 62.
+  int ncu = 0;
+  if (nv > 112)
+    if (const int st = im::compute_units(&ncu)) return st;
+  if (nworld <= (njmax >= 192 ? 2 : 1) * ncu) {
+    const size_t stage_words = 2 * (32 * 128 + 32) + 2 * (((size_t)njmax + 3) & ~(size_t)3), u_words = im::Stair<16>{pad}.words();
+    const size_t rhs_at = std::max(stage_words, u_words), lds_bytes = sizeof(float) * (rhs_at + pad + 16 * 16 + 16);
+    if (lds_bytes <= 160 * 1024) {
+      if (lds_bytes > 64 * 1024)
+        IM_HIP_CHECK(hipFuncSetAttribute((const void *)im::jtdj_factor_solve_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+      hipLaunchKernelGGL(im::jtdj_factor_solve_kernel, dim3(nworld), dim3(256), lds_bytes, (hipStream_t)stream, Mdense, J, njmax, D,
+                         state, nefc, quad, H, nv, nv_pad, y, ldy, U, x, ldx, pad, (int)rhs_at);
+      IM_HIP_CHECK(hipGetLastError());
+      return IM_OK;
+    }
+  }
   return im::jtdj_solve_wave(Mdense, J, njmax, D, state, nefc, quad, H, nv, nv_pad, y, ldy, U, pad, x, ldx, nworld, (hipStream_t)stream);
 }
 

@@ -118,3 +118,47 @@ def test_gpu_dense_hessian_of_long_row_lists(device, nv):
     with pytest.raises(_lib.ImhipError):
         BD.dense_hessian_factor_solve(t(M[:1]), torch.zeros((1, many, nv), device=device), torch.zeros((1, many), device=device),
                                       torch.zeros((1, many), dtype=torch.int32, device=device), None, None, t(y[:1]), x[:1])  # fmt: skip
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv", [111, 112, 113, 121, 128])
+def test_gpu_small_batches_of_large_matrices_equal_the_same_worlds_in_a_large_one(device, nv):
+    """Up to a world per CU (two with 192 rows) a workgroup has a world, beyond that a wavefront: on both
+    sides of the line the same worlds give the same bits, H, factor and solution, with H off 16 bytes and
+    without one."""
+    import torch
+
+    ncu = torch.cuda.get_device_properties(device).multi_processor_count
+    few, pad = 9, -(-nv // 16) * 16
+    for rows, line in ((70, ncu), (191, ncu), (192, 2 * ncu), (215, 2 * ncu)):
+        c = [torch.from_numpy(np.ascontiguousarray(a)).to(device) for a in _hessian_case(nv, rows, [0, 1, 5, 32, 33, 64, 65, 70, rows], nv)]
+
+        def solve(n, offset, with_h):
+            w = [t.repeat(-(-n // few), *[1] * (t.dim() - 1))[:n].contiguous() for t in c]
+            flat = torch.zeros(n * pad * pad + 4, device=device)
+            H = flat[offset : offset + n * pad * pad].view(n, pad, pad) if with_h else None
+            x, U = torch.full((n, nv), 7.0, device=device), torch.full((n, pad, pad), 7.0, device=device)
+            BD.dense_hessian_factor_solve(*w[:5], H, w[5], x, factor=U)
+            return [t[:few] for t in (x, U, *([H[:, :nv, :nv]] if with_h else []))], x, U
+
+        want, x, U = solve(line + 1, 0, True)
+        for n, offset, with_h in ((few, 0, True), (line, 1, True), (line, 0, False)):
+            got, x, U = solve(n, offset, with_h)
+            for a, b in zip(got, want):
+                np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+            reps = n // few
+            for t in (x, U):
+                assert torch.equal(t[: reps * few].view(reps, few, -1).nan_to_num(), t[:few].reshape(1, few, -1).expand(reps, -1, -1).nan_to_num())
+    rng = np.random.default_rng(nv)
+    _, layout, _ = BD.block_index_layout(np.arange(nv * nv), nv, nv * nv, 16)
+    idx = torch.from_numpy(layout).to(device)
+    M, y = _spd(rng, few, nv).reshape(few, -1), rng.standard_normal((few, nv)).astype(np.float32)
+    for n in (ncu, ncu + 1):
+        Md, yd = (torch.from_numpy(a).to(device).repeat(-(-n // few), 1)[:n].contiguous() for a in (M, y))
+        x, U = torch.full((n, nv), np.nan, device=device), torch.zeros((n, pad, pad), device=device)
+        st = _lib.lib().im_blocked_factor_solve(Md.data_ptr(), nv * nv, nv * nv, idx.data_ptr(), 16, nv, pad, yd.data_ptr(), nv, U.data_ptr(), x.data_ptr(), nv, n, None)
+        assert st == 0
+        x_ref, U_ref = R.blocked_factor_solve(M, layout, nv, pad, 16, y)
+        np.testing.assert_array_equal(U[:few].cpu().numpy(), U_ref)
+        np.testing.assert_array_equal(x[:few].cpu().numpy(), x_ref)
+        np.testing.assert_array_equal(x[-few:].cpu().numpy(), np.tile(x_ref, (-(-n // few), 1))[:n][-few:])
