@@ -22,23 +22,25 @@ namespace {
 
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-// One workgroup of four wavefronts per world.  A and the force of every term are first brought
-// into LDS in the order the rows consume them (every lane busy, twelve terms' look-ups in flight
+// One workgroup of NT threads per world.  A and the force of every term are first brought
+// into LDS in the order the rows consume them (every lane busy, UN terms' look-ups in flight
 // per lane); then lane j of the first wavefront runs row j's chain of fused multiply-adds over
 // consecutive LDS words, the next eight terms on their way while these are added.  Same terms,
 // same order per row as the reference kernel.
 // What bounds it is the longest row's chain (hundreds of terms, one after the other) and the
 // staging before it, not the 46 MB: the chain looked a term's muscle up and then its force, two
 // LDS latencies per four terms, and rigs of more than 1536 entries gathered from memory.
-// 2522 entries x 4096 worlds: 36.9 us (two wavefronts, a term's muscle looked up in the chain) -> 23.0.
-constexpr int kProjectThreads = 256;
-__global__ __launch_bounds__(kProjectThreads) void muscle_project_kernel(
+// Two wavefronts with twelve terms a lane that looked a term's muscle up in the chain -> this, with the
+// smallest NT x UN that takes the entries in one trip (places without an entry cost what the others do), x 8192
+// worlds: 355 entries 11.1 -> 7.8 us (256 x 12: 14.1), 743 16.7 -> 14.3 (18.8), 1437 27.7 -> 24.8 (27.1),
+// 2522 59.5 -> 39.3.
+template <int NT, int UN>
+__global__ __launch_bounds__(NT) void muscle_project_kernel(
     const float *__restrict__ moment, int64_t ldm, const float *__restrict__ force, int64_t ldf,
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ entry_idx,
     const int32_t *__restrict__ entry_muscle, int nentry, int nmuscle, int ntorque, int root,
     float *__restrict__ qfrc, int64_t ldq, int nworld) {
   extern __shared__ float lds[];
-  constexpr int NT = kProjectThreads, UN = 12;
   const int tid = threadIdx.x;
   const int64_t w = blockIdx.x;
   float *av = lds;           // [nentry] A[entry_idx[s]]
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(kProjectThreads) void muscle_project_kernel(
         fv[tid + NT * k] = f[k];
       }
   } else {
-    // more entries than one trip holds: gathered from memory, twelve look-ups in flight per lane
+    // more entries than one trip holds: gathered from memory, UN look-ups in flight per lane
     __syncthreads();
     for (int s0 = tid; s0 < nentry; s0 += UN * NT) {
       int e[UN], m[UN];
@@ -200,11 +202,21 @@ int im_muscle_project(const float *moment, int64_t ld_moment, const float *force
   // the limit is that of a term in six bytes, which a caller has to reckon with; a term takes eight
   if (sizeof(float) * ((size_t)nentry + nmuscle) + 2 * (((size_t)nentry + 1) & ~(size_t)1) > 64 * 1024) return IM_ERR_UNSUPPORTED;
   const size_t lds_bytes = sizeof(float) * (2 * (size_t)nentry + nmuscle);
-  if (lds_bytes > 64 * 1024)
-    IM_HIP_CHECK(hipFuncSetAttribute((const void *)im::muscle_project_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-  hipLaunchKernelGGL(im::muscle_project_kernel, dim3(nworld), dim3(im::kProjectThreads), lds_bytes, (hipStream_t)stream,
-                     moment, ld_moment, force, ld_force, torque_entry_offsets, torque_entry_idx, entry_muscle,
-                     nentry, nmuscle, ntorque, root_dof_count, qfrc, ld_qfrc, nworld);
+#define IM_PROJECT(NT, UN)                                                                                                        \
+  do {                                                                                                                            \
+    if (lds_bytes > 64 * 1024)                                                                                                    \
+      IM_HIP_CHECK(hipFuncSetAttribute((const void *)im::muscle_project_kernel<NT, UN>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                       (int)lds_bytes));                                                                          \
+    hipLaunchKernelGGL((im::muscle_project_kernel<NT, UN>), dim3(nworld), dim3(NT), lds_bytes, (hipStream_t)stream, moment,       \
+                       ld_moment, force, ld_force, torque_entry_offsets, torque_entry_idx, entry_muscle, nentry, nmuscle,         \
+                       ntorque, root_dof_count, qfrc, ld_qfrc, nworld);                                                           \
+  } while (0)
+  if (nentry <= 4 * 128) IM_PROJECT(128, 4);
+  else if (nentry <= 8 * 128) IM_PROJECT(128, 8);
+  else if (nentry <= 12 * 128) IM_PROJECT(128, 12);
+  else if (nentry <= 8 * 256) IM_PROJECT(256, 8);
+  else IM_PROJECT(256, 12);
+#undef IM_PROJECT
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
 }

@@ -361,3 +361,26 @@ def test_gpu_projection_staging_sizes(device, muscles):
     Q.project_muscle_sparse_moment_qfrc(t(mb.moment), t(mb.force), t(offsets, np.int32), t(order, np.int32), t(ent.muscle_dof_muscle_idx, np.int32), mb.root_dof_count, qfrc)
     want = R.muscle_project(mb.moment, mb.force, offsets, order, ent.muscle_dof_muscle_idx, mb.root_dof_count, nv)
     np.testing.assert_array_equal(qfrc.cpu().numpy()[:, mb.root_dof_count :], want[:, mb.root_dof_count :])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entries", [511, 512, 513, 1024, 1025, 1536, 1537, 2048, 2049, 3072, 3073])
+def test_gpu_projection_at_the_ends_of_a_trip(device, entries):
+    """Both sides of the entry counts that a workgroup's one trip through LDS holds, with rows without an
+    entry and one with most of them: bit for bit, root dofs and padding untouched."""
+    import torch
+
+    rng = np.random.default_rng(entries)
+    nworld, nmuscle, ntorque, root = 5, 97, 21, 6
+    dof = np.where(rng.uniform(size=entries) < 0.6, 3, rng.integers(0, ntorque, entries))
+    dof[dof == 11] = 12
+    offsets, order = Q.torque_sorted_entries(dof.astype(np.int32), ntorque)
+    muscle = rng.integers(0, nmuscle, entries).astype(np.int32)
+    moment, force = rng.normal(size=(nworld, entries)).astype(np.float32), rng.normal(size=(nworld, nmuscle)).astype(np.float32)
+    t = lambda a, dt=None: torch.from_numpy(np.ascontiguousarray(a if dt is None else a.astype(dt))).to(device)  # noqa: E731
+    qfrc = torch.full((nworld, root + ntorque + 2), 7.0, device=device)
+    Q.project_muscle_sparse_moment_qfrc(t(moment), t(force), t(offsets, np.int32), t(order, np.int32), t(muscle), root, qfrc[:, : root + ntorque])
+    want = R.muscle_project(moment, force, offsets, order, muscle, root, root + ntorque)
+    got = qfrc.cpu().numpy()
+    np.testing.assert_array_equal(got[:, root : root + ntorque], want[:, root:])
+    assert (got[:, :root] == 7.0).all() and (got[:, root + ntorque :] == 7.0).all()
