@@ -35,15 +35,17 @@ namespace im {
 namespace {
 
 // A workgroup per world up to what the chip keeps resident at once (the workgroups walk over worlds: one that
-// does not get in starts when another has done all its worlds).  A CU hands out its LDS in units of 1280
-// bytes, which the runtime's answer does not round up to: 8192 worlds of 250 muscles on a workgroup more per CU
-// than stays resident took 86 us for the force-velocity state instead of 64.
+// does not get in starts when another has done all its worlds, and the launch takes up to twice as long).
+// Less than the runtime's answer in two ways: a CU hands out its LDS in units of 1280 bytes, and these kernels'
+// scalar registers (85 - 106) leave 24 wavefronts to a CU.  Force-velocity state of 8192 worlds by workgroups per
+// CU: 128 threads, 12: 20.1 us, 13: 23.3; 192 threads, 8: 25.6, 9: 32.5; 256 threads, 6: 47.1, 7: 61.1; 320
+// threads, 4: 68.8, 5: 93.3.
 int resident_grid(const void *fn, int threads, size_t lds, int nworld, unsigned *grid) {
   int ncu = 0, per_cu = 0;
   if (const int st = compute_units(&ncu)) return st;
   if (const int st = resident_per_cu(fn, nullptr, threads, lds, &per_cu)) return st;
   const size_t unit = 1280, granted = (std::max<size_t>(lds, 1) + unit - 1) / unit * unit;
-  per_cu = std::min(per_cu, (int)(160 * 1024 / granted));
+  per_cu = std::min({per_cu, (int)(160 * 1024 / granted), 24 * 64 / threads});
   *grid = (unsigned)std::min(nworld, ncu * std::max(1, per_cu));
   return IM_OK;
 }
@@ -259,8 +261,10 @@ __global__ __launch_bounds__(256) void force_velocity_state_kernel(
 // operations in the same order, so the same bits.
 // As many threads as it takes for a muscle each, 128 to 320: a workgroup's last phase is its muscles'
 // chains, and threads beyond them only take a CU's places from other worlds (8192 worlds of 40 / 100 / 200
-// muscles: 23.5 / 31.3 / 48.7 us, with 320 threads 50 / 59 / 68).  A launch per world with 256 threads,
-// distances by the muscle's lane, took 23.0 / 38.8 / 59.0 us there, and 57.4 at 284 muscles x 4096 worlds, here 38.
+// muscles: 20.3 / 31.0 / 47.6 us, with 320 threads 50 / 59 / 68).  A launch per world with 256 threads,
+// distances by the muscle's lane, took 23.1 / 39.2 / 59.1 us there, and 57.5 at 284 muscles x 4096 worlds, here 38.3;
+// it is ahead where the whole batch is resident at once (2048 worlds of 40 / 100 / 200 muscles 6.7 / 9.5 / 17.8 us,
+// here 7.6 / 11.2 / 19.2).
 struct FvLds {
   int words_wp, nentry, nqvel, nmuscle;  // the longest rows that fit; what is read of them is what the tables name
   __host__ __device__ int bytes() const {
@@ -784,9 +788,9 @@ bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
     return small ? launch_world_on<MODE, 256, 0>(a, false, nworld, stream) : launch_world_on<MODE, 512, 0>(a, false, nworld, stream);
   int ncu = 0;
   if (compute_units(&ncu) != IM_OK) return false;
-  // Entries kept in registers pay from two worlds per workgroup on (seven of 256 threads, three of 512 per CU), and up
+  // Entries kept in registers pay from two worlds per workgroup on (six of 256 threads, three of 512 per CU), and up
   // to about 2000 entries; beyond, and with 512 threads throughout, reading them from the lists takes as long.
-  if (small && nworld >= 2 * 7 * ncu)
+  if (small && nworld >= 2 * 6 * ncu)
     return a.nentry <= 2 * 256   ? launch_world_on<MODE, 256, 2>(a, true, nworld, stream)
            : a.nentry <= 4 * 256 ? launch_world_on<MODE, 256, 4>(a, true, nworld, stream)
                                  : launch_world_on<MODE, 256, 6>(a, true, nworld, stream);
