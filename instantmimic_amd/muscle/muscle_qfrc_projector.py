@@ -271,9 +271,16 @@ def _rows_apart(t):
     """``t`` and its row stride, the stride no shorter than a row: the launch takes the strides for the
     rows' lengths.  A single row has any stride; rows that overlap are copied (stride 0, one row for
     every world, stays)."""
-    if t.shape[0] > 1 and 0 < t.stride(0) < t.shape[1]:
+    nrow, row = t.shape
+    stride = t.stride(0)
+    if stride >= row:
+        return t, stride
+    if nrow == 1:
+        return t, row
+    if stride:
         t = t.contiguous()
-    return t, max(t.stride(0), t.shape[1]) if t.shape[0] == 1 else t.stride(0)
+        stride = t.stride(0)
+    return t, stride
 
 
 def eval_muscle_force_velocity_state(
@@ -294,8 +301,9 @@ def eval_muscle_force_velocity_state(
     outs = (muscle_length, effective_activation, length_velocity, force_velocity_multiplier, force_velocity_slope)
     wp2 = transformed_waypoints.reshape(nworld, -1)
     _f32_rows(wp2, activation, qvel, moment, muscle_params, *outs)
+    ld_out = outs[0].stride(0)
     for t in outs:
-        if tuple(t.shape) != (nworld, nmuscle) or t.stride(0) != outs[0].stride(0):
+        if t.shape != (nworld, nmuscle) or t.stride(0) != ld_out:
             raise ValueError("the five outputs must be (nworld, nmuscle) with one row stride")
     for t in (muscle_waypoint_start, muscle_dof_offsets, muscle_dof_torque_idx):
         if t.dtype != torch.int32 or not t.is_cuda or not t.is_contiguous():
@@ -313,14 +321,16 @@ def eval_muscle_force_velocity_state(
     fv = _lib.MuscleForceVelocityModel(float(vmax), float(fvmax), float(bool(clamp_activation)), float(bool(include_active)))
     import ctypes as C
 
-    (wp2, ld_wp), (qvel, ld_qvel), (moment, ld_moment) = (_rows_apart(t) for t in (wp2, qvel, moment))
+    wp2, ld_wp = _rows_apart(wp2)
+    qvel, ld_qvel = _rows_apart(qvel)
+    moment, ld_moment = _rows_apart(moment)
     with torch.cuda.device(activation.device):
         status = _lib.lib().im_muscle_force_velocity_state(
             wp2.data_ptr(), ld_wp, muscle_waypoint_start.data_ptr(), muscle_params.data_ptr(),
             muscle_params.stride(0), muscle_rest_length.data_ptr(), force_velocity_length_scale.data_ptr(),
             activation.data_ptr(), activation.stride(0), qvel.data_ptr(), ld_qvel, moment.data_ptr(),
             ld_moment, muscle_dof_offsets.data_ptr(), muscle_dof_torque_idx.data_ptr(), int(root_dof_count),
-            C.byref(model), C.byref(fv), nmuscle, *[t.data_ptr() for t in outs], outs[0].stride(0), nworld,
+            C.byref(model), C.byref(fv), nmuscle, *[t.data_ptr() for t in outs], ld_out, nworld,
             _stream(activation),
         )  # fmt: skip
     _lib.check(status, "im_muscle_force_velocity_state")
