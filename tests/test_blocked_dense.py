@@ -152,7 +152,7 @@ def test_gpu_dense_hessian_row_counts_and_masks(device):
 
 @pytest.mark.gpu
 def test_gpu_wavefront_per_world_kernel_for_small_tiles_agrees():
-    """Matrices up to 64 x 64 run four worlds per wavefront; the kernel with a
+    """Matrices up to 128 x 128 run a wavefront per world; the kernel with a
     workgroup per world that serves every other shape is forced here in a child process and
     must pass the same oracle comparison."""
     import os
