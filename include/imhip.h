@@ -666,6 +666,38 @@ int im_muscle_sparse_moment(const im_muscle_geometry *geometry,
                             const im_muscle_entries *entry_segments, int root_dof_count,
                             float *moment, int64_t ld_moment, int nworld, void *stream);
 
+/* Torque, activation gradient or sparse moment of a batch in one launch, from the body poses:
+ * what im_muscle_waypoints_forces followed by im_muscle_torque_forward, im_muscle_activation_grad or
+ * im_muscle_sparse_moment leaves in its output, bit for bit, without the waypoints and forces in memory.
+ * Rows of xpos (3 nbody), xquat (4 nbody), subtree_com (3 nbody) and cdof (6 (root + ntorque)), ld* = row
+ * strides in floats.  `offsets` (nrow + 1) are those of the list that the output's rows sum over, `packed`
+ * (npacked, 8-byte aligned) its entries as two words each:
+ *   segment | torque dof << 16,   place in the list | muscle << 16   (muscle 0 for the moment)
+ * ordered by kind: kind_count[0] entries with coefficients (start, end) = (0, 1), then kind_count[1] with
+ * (1, 0), then kind_count[2] with (1, 1); the first two counts are multiples of 64, filled up with entries
+ * (0, place nentry).  Lists with other coefficients have no packed form.
+ * what: IM_MUSCLE_TORQUE: in = activation (nworld, ld_in), passive forces where model.include_passive;
+ * IM_MUSCLE_GRAD: in = grad_output; IM_MUSCLE_MOMENT: in unused.  nworld = 0 only checks the sizes:
+ * IM_ERR_UNSUPPORTED if a world does not fit a workgroup (5120 packed entries; 512 muscles
+ * for torque and gradient; 64 KB of LDS). */
+enum { IM_MUSCLE_TORQUE = 0, IM_MUSCLE_GRAD = 1, IM_MUSCLE_MOMENT = 2 };
+typedef struct im_muscle_context {
+  const float *xpos, *xquat, *subtree_com, *cdof;
+  int64_t ld_xpos, ld_xquat, ld_subtree_com, ld_cdof;
+  const int32_t *waypoint_body;
+  const float *waypoint_local;
+  const int32_t *start_waypoint, *end_waypoint, *start_root_body, *end_root_body;
+  const int32_t *all_segment_start, *all_segment_offsets;
+  const float *params, *rest;
+  const int32_t *offsets;
+  const uint32_t *packed;
+  int32_t ld_params, nbody, nwaypoint, nsegment, ntorque, nmuscle, nrow, nentry, npacked;
+  int32_t kind_count[3];
+  im_muscle_force_model model;
+} im_muscle_context;
+int im_muscle_from_context(const im_muscle_context *context, int what, const float *in, int64_t ld_in,
+                           int root_dof_count, float *out, int64_t ld_out, int nworld, void *stream);
+
 /* ---- steps either side of the solve that walk a world's small trees ------------------- */
 
 /* Replaces the product M v inside the fused Newton kernel

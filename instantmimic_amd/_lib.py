@@ -134,6 +134,22 @@ class MuscleEntries(C.Structure):
     ]  # fmt: skip
 
 
+class MuscleContext(C.Structure):
+    """im_muscle_context"""
+
+    _fields_ = [
+        ("xpos", _vp), ("xquat", _vp), ("subtree_com", _vp), ("cdof", _vp),
+        ("ld_xpos", _i64), ("ld_xquat", _i64), ("ld_subtree_com", _i64), ("ld_cdof", _i64),
+        ("waypoint_body", _vp), ("waypoint_local", _vp),
+        ("start_waypoint", _vp), ("end_waypoint", _vp), ("start_root_body", _vp), ("end_root_body", _vp),
+        ("all_segment_start", _vp), ("all_segment_offsets", _vp), ("params", _vp), ("rest", _vp),
+        ("offsets", _vp), ("packed", _vp),
+        ("ld_params", C.c_int32), ("nbody", C.c_int32), ("nwaypoint", C.c_int32), ("nsegment", C.c_int32), ("ntorque", C.c_int32),
+        ("nmuscle", C.c_int32), ("nrow", C.c_int32), ("nentry", C.c_int32), ("npacked", C.c_int32),
+        ("kind_count", C.c_int32 * 3), ("model", MuscleForceModel),
+    ]  # fmt: skip
+
+
 class BodyWrenches(C.Structure):
     _fields_ = [
         ("body_force", _vp), ("body_torque", _vp), ("xipos", _vp), ("subtree_com", _vp), ("cdof", _vp),
@@ -271,6 +287,7 @@ SIGNATURES = {
     "im_muscle_activation_grad": (_i, [_pgeo, _pseg, _pent, _vp, _i64, _vp, _i64, _i, _vp, _i64, _i, _vp]),
     "im_muscle_torque_bounds": (_i, [_pgeo, _pseg, _pent, _vp, _i64, _i, _vp, _vp, _i64, _i, _vp]),
     "im_muscle_sparse_moment": (_i, [_pgeo, _pseg, _vp, _pent, _i, _vp, _i64, _i, _vp]),
+    "im_muscle_from_context": (_i, [C.POINTER(MuscleContext), _i, _vp, _i64, _i, _vp, _i64, _i, _vp]),
     "im_mul_m_sparse": (_i, [_vp, _i64, _i, _vp, _vp, _vp, _i, _vp, _i64, _vp, _vp, _i64, _i, _i, _vp]),
     "im_tree_accumulate": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp, _i64, _i, _i, _vp]),
     "im_newton_gradient": (

@@ -91,24 +91,32 @@ __device__ __forceinline__ float seg_term(const Geo &g, const Seg &s, int64_t w,
                       ld3(com + 3 * s.b0[seg]), ld3(com + 3 * s.b1[seg]), a, b, force);
 }
 
-// One waypoint in the world frame: the body's position plus its local offset turned by the
-// body's (renormalised) quaternion.  xpos and xquat are one world's rows.
-__device__ __forceinline__ V3 world_waypoint(const float *__restrict__ xpos,
-                                             const float *__restrict__ xquat,
-                                             const int32_t *__restrict__ wp_body,
-                                             const float *__restrict__ wp_local, int i) {
-  const int b = wp_body[i];
-  const float *q = xquat + 4 * b;
+// A body's renormalised quaternion as the rotation uses it: vector part u, s s - u.u and 2 s.
+struct BodyTurn {
+  V3 u;
+  float k, s2;
+};
+__device__ __forceinline__ BodyTurn body_turn(const float *__restrict__ q) {
   const float q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
   // muscle_qfrc_projector.py:91-100
   const float inv = 1.0f / sqrtf(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3 + 1.0e-8f);
   const float s = q0 * inv;
   const V3 u = {q1 * inv, q2 * inv, q3 * inv};
-  const V3 v = ld3(wp_local + 3 * i);
-  // mujoco_warp math.rot_vec_quat: 2 (u.v) u + (s s - u.u) v + 2 s (u x v)
-  V3 r = add(scale(2.0f, scale(dot(u, v), u)), scale(s * s - dot(u, u), v));
-  r = add(r, scale(2.0f * s, cross(u, v)));
-  return add(ld3(xpos + 3 * b), r);
+  return {u, s * s - dot(u, u), 2.0f * s};
+}
+// mujoco_warp math.rot_vec_quat: 2 (u.v) u + (s s - u.u) v + 2 s (u x v)
+__device__ __forceinline__ V3 turned(const BodyTurn &t, V3 v) {
+  const V3 r = add(scale(2.0f, scale(dot(t.u, v), t.u)), scale(t.k, v));
+  return add(r, scale(t.s2, cross(t.u, v)));
+}
+// One waypoint in the world frame: the body's position plus its local offset turned by the
+// body's quaternion.  xpos and xquat are one world's rows.
+__device__ __forceinline__ V3 world_waypoint(const float *__restrict__ xpos,
+                                             const float *__restrict__ xquat,
+                                             const int32_t *__restrict__ wp_body,
+                                             const float *__restrict__ wp_local, int i) {
+  const int b = wp_body[i];
+  return add(ld3(xpos + 3 * b), turned(body_turn(xquat + 4 * b), ld3(wp_local + 3 * i)));
 }
 
 __global__ __launch_bounds__(256) void waypoints_kernel(
@@ -146,12 +154,13 @@ __device__ __forceinline__ float active_fl(float l, const float *m) {
   const float x = (lmax - l) / fmaxf(lmax - hi, 1.0e-8f);
   return 0.5f * x * x;
 }
-__device__ __forceinline__ float passive_fl(float l, const float *m) {
+// (scale: expf(m[1]) - 1, read for the exponential curve only)
+__device__ __forceinline__ float passive_fl(float l, const float *m, float scale) {
   if (m[0] < 0.5f) {
     if (l < 1.0f) return 0.0f;
     float x = m[1] * (l - 1.0f) / m[2];
     x = fminf(fmaxf(x, -80.0f), 80.0f);
-    return (expf(x) - 1.0f) / (expf(m[1]) - 1.0f);
+    return (expf(x) - 1.0f) / scale;
   }
   const float lmax = m[1], fpmax = m[2];
   if (l <= 1.0f) return 0.0f;
@@ -163,6 +172,23 @@ __device__ __forceinline__ float passive_fl(float l, const float *m) {
   return fpmax * (0.5f + (l - mid) / width);
 }
 
+// Force magnitudes of a muscle of length len (par: f0, l_m0, l_t0, ..; c: its pennation's cosine).
+__device__ __forceinline__ void force_of_length(float len, const float *__restrict__ par, float rest, float c, float passive_scale,
+                                                const im_muscle_force_model &model, float *unit, float *passive) {
+  const float f0 = par[0], lm0 = par[1], lt0 = par[2];
+  // muscle_qfrc_projector.py:190-205
+  const float lm = len / fmaxf(rest, 1.0e-6f) - lt0;
+  const float ln =
+      fminf(fmaxf(lm / fmaxf(lm0, 1.0e-6f), model.length_norm_min), model.length_norm_max);
+  *unit = f0 * active_fl(ln, model.active) * c * model.force_scale;
+  if (passive) {
+    float pv = 0.0f;
+    // muscle_qfrc_projector.py:249-277 with include_active 0, include_passive 1
+    if (model.include_passive)
+      pv = f0 * passive_fl(ln, model.passive, passive_scale) * c * model.force_scale;
+    *passive = pv;
+  }
+}
 // Length of muscle m along one world's waypoints and its force magnitudes.
 __device__ __forceinline__ void muscle_force_magnitudes(
     const float *row, const int32_t *__restrict__ seg_start,
@@ -174,21 +200,8 @@ __device__ __forceinline__ void muscle_force_magnitudes(
     const int i = seg_start[s];
     len = len + length(sub(ld3(row + 3 * (i + 1)), ld3(row + 3 * i)));
   }
-  const float f0 = params[m * ldpar], lm0 = params[m * ldpar + 1], lt0 = params[m * ldpar + 2],
-              pen = params[m * ldpar + 3];
-  // muscle_qfrc_projector.py:190-205
-  const float lm = len / fmaxf(rest[m], 1.0e-6f) - lt0;
-  const float ln =
-      fminf(fmaxf(lm / fmaxf(lm0, 1.0e-6f), model.length_norm_min), model.length_norm_max);
-  const float c = cosf(pen);
-  *unit = f0 * active_fl(ln, model.active) * c * model.force_scale;
-  if (passive) {
-    float pv = 0.0f;
-    // muscle_qfrc_projector.py:249-277 with include_active 0, include_passive 1
-    if (model.include_passive)
-      pv = f0 * passive_fl(ln, model.passive) * c * model.force_scale;
-    *passive = pv;
-  }
+  force_of_length(len, params + m * ldpar, rest[m], cosf(params[m * ldpar + 3]),
+                  passive && model.include_passive ? expf(model.passive[1]) - 1.0f : 1.0f, model, unit, passive);
 }
 
 // MuJoCo's force-velocity multiplier and its derivative in the normalised velocity
@@ -798,6 +811,317 @@ bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
   return launch_world_on<MODE, 512, 0>(a, true, nworld, stream);
 }
 
+// ---- a world from its context in one launch --------------------------------------------------
+// Torque, activation gradient and sparse moment straight from body poses: a workgroup takes a world's
+// waypoints, segment records and muscle forces into LDS and contracts them there, so neither waypoints nor
+// forces go to memory (15 KB a world at 284 muscles, written and read back by two launches before).
+//
+// What bounds it is the vector issue rate.  What is left out of a world's instructions, bits unchanged: a
+// body's quaternion is normalised once and not once per waypoint; a muscle's cosine is taken once per
+// workgroup; an entry whose one coefficient is 0 takes the lever of its other end only (0 * finite subtracted from or added to a number
+// leaves it, and a zero's sign does not survive an ordered sum that starts at +0).  The lists come packed, the entries of a
+// kind together, so that a wavefront's entries are of one kind and a thread keeps its entries in two
+// registers each.  A world with a lever or an axis so large that their products may not be finite takes
+// the full expression throughout (0 * inf is NaN there).
+// Four barriers per world: poses and axes, waypoints, segments and forces, contributions; the ordered sums run beside
+// the next world's poses.  4096 worlds of 284 muscles (three workgroups of 512 per CU; the vector ALUs issue in 0.64
+// of the cycles, the LDS is busy in 0.56): torque 80 us where the two launches took 35 + 64, gradient 74 (35 + 49), moment
+// 65 (20 + 58).
+struct CtxArgs {
+  im_muscle_context c;
+  const float *in;  // activation (MW_FORWARD) or grad_output (MW_GRAD)
+  int64_t ldin;
+  float *out;
+  int64_t ldo;
+  int root, nworld;
+  int single_end, single;  // entries before these: end only; end or start only (multiples of 64)
+};
+
+constexpr float kCtxLarge = 1.0e18f;  // two factors below it have a finite product
+constexpr int kCtxTrips = 10;     // packed entries of a thread
+constexpr int kCtxMost = kCtxTrips * 512, kCtxMuscles = 512;
+constexpr int kPose = 8;  // floats of a body's record: u, s s - u.u, 2 s, position
+struct CtxLds {
+  int contrib, segd, axis, force, com, flags, words;
+};
+__host__ __device__ inline CtxLds ctx_lds(const im_muscle_context &c, bool forces) {
+  const int sums = c.nentry + kContribPad, points = 3 * c.nwaypoint, records = 9 * c.nsegment, poses = kPose * c.nbody;
+  CtxLds l;
+  l.contrib = 0;  // the waypoints lie here until the contributions take their place
+  l.segd = sums > points ? sums : points;  // and the bodies' records until the segments' do
+  l.axis = l.segd + (records > poses ? records : poses);
+  l.force = l.axis + kAxis * c.ntorque;
+  l.com = l.force + (forces ? c.nmuscle : 0);
+  l.flags = l.com + 3 * c.nbody;
+  l.words = l.flags + 2;
+  return l;
+}
+
+// An entry with both coefficients 1: contribution() less the products with 1.
+__device__ __forceinline__ float both_ends(const float *cd, const float *sd, float f) {
+  const V3 ang = ld3(cd), lin = ld3(cd + 3), fv = scale(f, ld3(sd));
+  return dot(sub(add(lin, cross(ang, ld3(sd + 3))), add(lin, cross(ang, ld3(sd + 6)))), fv);
+}
+// An entry with one: its end's lever, and the sign bit that the end's term enters with.
+__device__ __forceinline__ float one_end(const float *cd, const float *sd, const float *lever, unsigned sign, float f) {
+  const V3 ang = ld3(cd), lin = ld3(cd + 3), fv = scale(f, ld3(sd));
+  const float v = dot(add(lin, cross(ang, ld3(lever))), fv);
+  return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ sign);
+}
+
+// The kernel's argument block in its argument segment, through a pointer laundered once per phase: held in
+// scalar registers over a world's phases its thirty pointers are spilled.
+__device__ __forceinline__ const CtxArgs &ctx_args() {
+  typedef const CtxArgs __attribute__((address_space(4))) Segment;
+  Segment *p = (Segment *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const CtxArgs *)p;
+}
+
+template <int MODE, int NT, int TRIPS>
+__global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_kernel(CtxArgs) {
+  extern __shared__ float lds[];
+  constexpr int nt = NT;
+  constexpr bool FORCES = MODE != MW_MOMENT;
+  int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) * 64;
+  // a thread's entries: LDS byte offsets of the segment's and the dof's record, the entry's place and the force
+  auto offsets_of = [](const CtxLds &l, uint2 e) __attribute__((always_inline)) {
+    const unsigned seg = 4u * l.segd + 36u * (e.x & 0xFFFFu), axis = 4u * (l.axis + kAxis * (e.x >> 16));
+    return make_uint2(seg | axis << 16, 4u * (e.y & 0xFFFFu) | 4u * (l.force + (e.y >> 16)) << 16);
+  };
+  uint2 kept[TRIPS];
+  float cosine = 1.0f;  // of the pennation of the thread's muscle
+  int turn = 0;
+  {
+    const CtxArgs &a = ctx_args();
+    const im_muscle_context &c = a.c;
+    const CtxLds l = ctx_lds(c, FORCES);
+#pragma unroll
+    for (int k = 0; k < TRIPS; ++k) {
+      const int e = k * nt + tid;
+      kept[k] = offsets_of(l, ((const uint2 *)c.packed)[e < c.npacked ? e : 0]);
+    }
+    if (FORCES) cosine = cosf(c.params[min(tid, c.nmuscle - 1) * c.ld_params + 3]);
+    if (tid < 2) ((int *)(lds + l.flags))[tid] = 0;
+    __syncthreads();
+  }
+  // A phase's table entries are asked for a phase ahead of their use, behind its barrier (up to WT waypoints, ST
+  // segments and a muscle of LT segments a thread; what is beyond is read where it is used).
+  constexpr int WT = 3, ST = 3, LT = 4;
+  for (int64_t w = blockIdx.x; w < ctx_args().nworld; w += gridDim.x, turn ^= 1) {
+    asm volatile("" : "+v"(tid));  // (no address formed from it is kept from world to world)
+    const int rid = nt - 1 - tid;
+    int wp_body[WT];
+    V3 wp_local[WT];
+    {  // poses, centres, axes; activations where the forces will be
+      const CtxArgs &a = ctx_args();
+      const im_muscle_context &c = a.c;
+      const CtxLds l = ctx_lds(c, FORCES);
+#pragma unroll
+      for (int k = 0; k < WT; ++k) {
+        const int i = min(tid + k * nt, c.nwaypoint - 1);
+        wp_body[k] = c.waypoint_body[i];
+        wp_local[k] = ld3(c.waypoint_local + 3 * i);
+      }
+      const float *com = c.subtree_com + w * c.ld_subtree_com, *cdof = c.cdof + w * c.ld_cdof + 6 * a.root;
+      for (int i = rid; i < 6 * c.ntorque; i += nt) {
+        const float v = cdof[i];
+        lds[l.axis + i + i / 6] = v;
+        if (!(fabsf(v) < kCtxLarge)) ((int *)(lds + l.flags))[turn] = 1;
+      }
+      for (int b = rid; b < c.nbody; b += nt) {
+        const float *x = c.xpos + w * c.ld_xpos + 3 * b;
+        const BodyTurn t = body_turn(c.xquat + w * c.ld_xquat + 4 * b);
+        float *o = lds + l.segd + kPose * b;
+        o[0] = t.u.x, o[1] = t.u.y, o[2] = t.u.z, o[3] = t.k, o[4] = t.s2;
+        o[5] = x[0], o[6] = x[1], o[7] = x[2];
+      }
+      for (int i = rid; i < 3 * c.nbody; i += nt) lds[l.com + i] = com[i];
+      if (MODE == MW_FORWARD)
+        for (int m = rid; m < c.nmuscle; m += nt) lds[l.force + m] = a.in[w * a.ldin + m];
+      if (MODE == MW_GRAD)
+        for (int j = rid; j < c.ntorque; j += nt) lds[l.axis + kAxis * j + 6] = a.in[w * a.ldin + j];
+    }
+    __syncthreads();
+    // the segments' wavefronts are the last ones, the muscles' the first: a muscle takes as long as three segments
+    int nseg_threads = nt;
+    int seg_tab[ST][4], length_tab[LT], first_segment = 0, last_segment = 0;
+    float par[3], rest = 0.0f;
+    {
+      const im_muscle_context &c = ctx_args().c;
+      const CtxLds l = ctx_lds(c, FORCES);
+      if (FORCES) nseg_threads = max(nt - ((c.nmuscle + 63) & ~63), nt / 4);
+#pragma unroll
+      for (int k = 0; k < ST; ++k) {
+        const int sg = min(rid + k * nseg_threads, c.nsegment - 1);
+        seg_tab[k][0] = c.start_waypoint[sg], seg_tab[k][1] = c.end_waypoint[sg];
+        seg_tab[k][2] = c.start_root_body[sg], seg_tab[k][3] = c.end_root_body[sg];
+      }
+      if (FORCES) {
+        const int m = min(tid, c.nmuscle - 1);
+        first_segment = c.all_segment_offsets[m], last_segment = c.all_segment_offsets[m + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) par[k] = c.params[m * c.ld_params + k];
+        rest = c.rest[m];
+      }
+      float *wpl = lds + l.contrib;
+      auto waypoint = [&](int i, int body, V3 local) __attribute__((always_inline)) {
+        const float *o = lds + l.segd + kPose * body;
+        const V3 p = add({o[5], o[6], o[7]}, turned({{o[0], o[1], o[2]}, o[3], o[4]}, local));
+        wpl[3 * i] = p.x, wpl[3 * i + 1] = p.y, wpl[3 * i + 2] = p.z;
+      };
+#pragma unroll
+      for (int k = 0; k < WT; ++k)
+        if (tid + k * nt < c.nwaypoint) waypoint(tid + k * nt, wp_body[k], wp_local[k]);
+      for (int i = tid + WT * nt; i < c.nwaypoint; i += nt) waypoint(i, c.waypoint_body[i], ld3(c.waypoint_local + 3 * i));
+      if (tid == 0) ((int *)(lds + l.flags))[turn ^ 1] = 0;
+      if (FORCES)
+#pragma unroll
+        for (int k = 0; k < LT; ++k) length_tab[k] = first_segment + k < last_segment ? c.all_segment_start[first_segment + k] : 0;
+    }
+    __syncthreads();
+    {
+      const CtxArgs &a = ctx_args();
+      const im_muscle_context &c = a.c;
+      const CtxLds l = ctx_lds(c, FORCES);
+      const float *wpl = lds + l.contrib;
+      if (FORCES) {
+        const bool passives = MODE == MW_FORWARD && c.model.include_passive;
+        auto distance = [&](int i) __attribute__((always_inline)) { return length(sub(ld3(wpl + 3 * (i + 1)), ld3(wpl + 3 * i))); };
+        if (tid < c.nmuscle) {
+          float d[LT], len = 0.0f;
+#pragma unroll
+          for (int k = 0; k < LT; ++k) d[k] = distance(length_tab[k]);
+#pragma unroll
+          for (int k = 0; k < LT; ++k) len = first_segment + k < last_segment ? len + d[k] : len;
+          for (int s = first_segment + LT; s < last_segment; ++s) len = len + distance(c.all_segment_start[s]);
+          float unit, passive;
+          force_of_length(len, par, rest, cosine, passives ? expf(c.model.passive[1]) - 1.0f : 1.0f, c.model, &unit,
+                          MODE == MW_FORWARD ? &passive : nullptr);
+          if (MODE == MW_FORWARD) {
+            unit = unit * lds[l.force + tid];
+            if (passives) unit = unit + passive;
+          }
+          lds[l.force + tid] = unit;
+        }
+      }
+      auto segment = [&](int sg, int w0, int w1, int b0, int b1) __attribute__((always_inline)) {
+        const V3 p0 = ld3(wpl + 3 * w0), p1 = ld3(wpl + 3 * w1);
+        const V3 r0 = sub(p0, ld3(lds + l.com + 3 * b0)), r1 = sub(p1, ld3(lds + l.com + 3 * b1));
+        const V3 seg = sub(p1, p0);
+        const float len = length(seg);
+        const bool ok = !(len < 1.0e-8f);  // (as in muscle_world_kernel)
+        float *o = lds + l.segd + 9 * sg;
+        o[0] = ok ? seg.x / len : 0.0f;
+        o[1] = ok ? seg.y / len : 0.0f;
+        o[2] = ok ? seg.z / len : 0.0f;
+        o[3] = r0.x, o[4] = r0.y, o[5] = r0.z;
+        o[6] = r1.x, o[7] = r1.y, o[8] = r1.z;
+        const float all = fabsf(r0.x) + fabsf(r0.y) + fabsf(r0.z) + fabsf(r1.x) + fabsf(r1.y) + fabsf(r1.z);
+        if (!(all < kCtxLarge)) ((int *)(lds + l.flags))[turn] = 1;
+      };
+#pragma unroll
+      for (int k = 0; k < ST; ++k)
+        if (rid < nseg_threads && rid + k * nseg_threads < c.nsegment)
+          segment(rid + k * nseg_threads, seg_tab[k][0], seg_tab[k][1], seg_tab[k][2], seg_tab[k][3]);
+      for (int sg = rid + ST * nseg_threads; rid < nseg_threads && sg < c.nsegment; sg += nseg_threads)
+        segment(sg, c.start_waypoint[sg], c.end_waypoint[sg], c.start_root_body[sg], c.end_root_body[sg]);
+    }
+    __syncthreads();
+    float line = 0.0f;
+    {  // the next world's rows are brought into the L2 beside what follows: a line each 16 floats of a row
+      const CtxArgs &a = ctx_args();
+      const im_muscle_context &c = a.c;
+      const int64_t next = w + gridDim.x < a.nworld ? w + gridDim.x : w;
+      int i = 16 * rid;
+      auto touch = [&](const float *row, int n) __attribute__((always_inline)) {
+        if (i >= 0 && i < n) line = row[i];
+        i -= (n + 15) & ~15;
+      };
+      touch(c.xpos + next * c.ld_xpos, 3 * c.nbody);
+      touch(c.xquat + next * c.ld_xquat, 4 * c.nbody);
+      touch(c.subtree_com + next * c.ld_subtree_com, 3 * c.nbody);
+      touch(c.cdof + next * c.ld_cdof + 6 * a.root, 6 * c.ntorque);
+      if (MODE != MW_MOMENT) touch(a.in + next * a.ldin, MODE == MW_FORWARD ? c.nmuscle : c.ntorque);
+    }
+    {
+      const CtxArgs &a = ctx_args();
+      const int npacked = a.c.npacked, single_end = a.single_end, single = a.single;
+      const char *base = (const char *)lds;
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(((const int *)(lds + ctx_lds(a.c, FORCES).flags))[turn]) == 0, 1)) {
+#pragma unroll
+        for (int k = 0; k < TRIPS; ++k) {
+          const int first = k * nt + wave;  // the wavefront's entries of this trip are of one kind
+          if (first < npacked) {
+            unsigned records = kept[k].x, place = kept[k].y;
+            asm volatile("" : "+v"(records), "+v"(place));  // (their parts are not kept from world to world)
+            const float *sd = (const float *)(base + (records & 0xFFFFu)), *cd = (const float *)(base + (records >> 16));
+            const float f = MODE == MW_MOMENT ? 1.0f : *(const float *)(base + (place >> 16));
+            float v;
+            if (first >= single)
+              v = both_ends(cd, sd, f);
+            else
+              v = one_end(cd, sd, sd + (first < single_end ? 6 : 3), first < single_end ? 0x80000000u : 0u, f);
+            if (MODE != MW_MOMENT) v = f == 0.0f ? 0.0f : v;
+            if (MODE == MW_GRAD) v = cd[6] * v;
+            if (k * nt + tid < npacked) *(float *)((char *)lds + (place & 0xFFFFu)) = v;
+          }
+          if (k % 2) __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        const CtxLds l = ctx_lds(a.c, FORCES);
+        for (int e = tid; e < npacked; e += nt) {
+          const uint2 t = offsets_of(l, ((const uint2 *)a.c.packed)[e]);
+          const float *sd = (const float *)(base + (t.x & 0xFFFFu)), *cd = (const float *)(base + (t.x >> 16));
+          const float f = MODE == MW_MOMENT ? 1.0f : *(const float *)(base + (t.y >> 16));
+          const V3 ang = ld3(cd), lin = ld3(cd + 3), fv = scale(f, ld3(sd));
+          const V3 st = add(lin, cross(ang, ld3(sd + 3))), en = add(lin, cross(ang, ld3(sd + 6)));
+          float v = dot(sub(scale(e < single_end ? 0.0f : 1.0f, st), scale(e >= single_end && e < single ? 0.0f : 1.0f, en)), fv);
+          v = f == 0.0f ? 0.0f : v;
+          if (MODE == MW_GRAD) v = cd[6] * v;
+          *(float *)((char *)lds + (t.y & 0xFFFFu)) = v;
+        }
+      }
+    }
+    asm volatile("" : : "v"(line));
+    __syncthreads();
+    {
+      const CtxArgs &a = ctx_args();
+      for (int r = tid; r < a.c.nrow; r += nt) {
+        const float sum = ordered_sum<MODE != MW_MOMENT>(lds, a.c.offsets[r], a.c.offsets[r + 1]);
+        a.out[w * a.ldo + r] = MODE == MW_GRAD && lds[ctx_lds(a.c, FORCES).force + r] == 0.0f ? 0.0f : sum;
+      }
+    }
+  }
+}
+
+template <int MODE, int NT, int TRIPS>
+int launch_context_on(const CtxArgs &a, hipStream_t stream) {
+  const size_t bytes = 4 * (size_t)ctx_lds(a.c, MODE != MW_MOMENT).words;
+  unsigned grid = 0;
+  if (const int st = resident_grid((const void *)muscle_context_kernel<MODE, NT, TRIPS>, NT, bytes, a.nworld, &grid)) return st;
+  hipLaunchKernelGGL((muscle_context_kernel<MODE, NT, TRIPS>), dim3(grid), dim3(NT), bytes, stream, a);
+  IM_HIP_CHECK(hipGetLastError());
+  return IM_OK;
+}
+// The fewest threads that hold a world at ten entries each, a muscle a thread at most: a world's barriers cost
+// less with fewer wavefronts to wait for, and the CU holds more worlds side by side.  Torque / gradient / moment x 8192
+// worlds by threads, us: 40 muscles (655 entries) 128: 28.2 / 27.5 / 23.2, 256: 39.6 / 38.0 / 30.7, 512: 61.1 / 58.6 /
+// 45.2; 120 (1882) 256: 61.9 / 59.8 / 51.2, 512: 82.9 / 76.9 / 65.6.  Between 2560 and 3584 entries 256 threads with
+// fourteen each where the batch does not fit the chip at once: 200 muscles (3145) x 8192 103 / 99.7 / 76.5 against
+// 112 / 103 / 84.8 with 512, but x 500 15.5 / 14.0 / 11.3 against 14.1 / 12.5 / 10.4.
+template <int MODE>
+int launch_context(const CtxArgs &a, hipStream_t stream) {
+  const int packed = a.c.npacked, muscles = MODE == MW_MOMENT ? 0 : a.c.nmuscle;
+  int ncu = 0;
+  if (const int st = compute_units(&ncu)) return st;
+  if (packed <= kCtxTrips * 128 && muscles <= 128) return launch_context_on<MODE, 128, kCtxTrips>(a, stream);
+  if (packed <= kCtxTrips * 256 && muscles <= 256) return launch_context_on<MODE, 256, kCtxTrips>(a, stream);
+  if (packed <= 14 * 256 && muscles <= 256 && a.nworld > 6 * ncu) return launch_context_on<MODE, 256, 14>(a, stream);
+  return launch_context_on<MODE, 512, kCtxTrips>(a, stream);
+}
+
 bool geo_ok(const im_muscle_geometry *g) {
   return g && g->waypoints && g->subtree_com && g->cdof && g->ld_waypoints >= 0 &&
          g->ld_subtree_com >= 0 && g->ld_cdof >= 0;
@@ -1140,4 +1464,34 @@ extern "C" int im_muscle_torque_bounds(const im_muscle_geometry *geometry,
   }
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
+}
+
+extern "C" int im_muscle_from_context(const im_muscle_context *context, int what, const float *in, int64_t ld_in,
+                                      int root_dof_count, float *out, int64_t ld_out, int nworld, void *stream) {
+  if (!context || nworld < 0 || root_dof_count < 0 || what < 0 || what > 2) return IM_ERR_ARG;
+  const im_muscle_context &c = *context;
+  const int packed = c.kind_count[0] + c.kind_count[1] + c.kind_count[2];
+  if (c.nbody <= 0 || c.nwaypoint <= 0 || c.nsegment <= 0 || c.ntorque <= 0 || c.nmuscle <= 0 || c.nrow <= 0 || c.nentry <= 0 || c.npacked != packed ||
+      c.kind_count[0] < 0 || c.kind_count[1] < 0 || c.kind_count[2] < 0 || c.kind_count[0] % 64 || c.kind_count[1] % 64 || c.ld_params < 4)
+    return IM_ERR_ARG;
+  if (c.npacked > kCtxMost || (what != IM_MUSCLE_MOMENT && c.nmuscle > kCtxMuscles) || 4 * (size_t)c.nentry + 16 * (size_t)c.nwaypoint + 36 * (size_t)c.nsegment + 28 * (size_t)c.ntorque + 8 * (size_t)c.nmuscle > 256 * 1024 ||
+      c.nbody > 65535 || 4 * (size_t)ctx_lds(c, true).words > 64 * 1024)
+    return IM_ERR_UNSUPPORTED;
+  static const bool forced_off = [] {
+    const char *e = std::getenv("IMHIP_MUSCLE_KERNEL");
+    return e && std::strcmp(e, "simple") == 0;
+  }();
+  if (forced_off) return IM_ERR_UNSUPPORTED;
+  if (nworld == 0) return IM_OK;
+  if (!c.xpos || !c.xquat || !c.subtree_com || !c.cdof || !c.waypoint_body || !c.waypoint_local || !c.start_waypoint || !c.end_waypoint ||
+      !c.start_root_body || !c.end_root_body || !c.offsets || !c.packed || ((uintptr_t)c.packed & 7) || !out)
+    return IM_ERR_ARG;
+  if (what != IM_MUSCLE_MOMENT && (!c.all_segment_start || !c.all_segment_offsets || !c.params || !c.rest || !in)) return IM_ERR_ARG;
+  if (c.ld_xpos < 0 || c.ld_xquat < 0 || c.ld_subtree_com < 0 || c.ld_cdof < 0 || ld_in < 0 || ld_out < c.nrow ||
+      (what == IM_MUSCLE_GRAD && c.nrow > c.nmuscle))
+    return IM_ERR_STRIDE;
+  const CtxArgs a{c, in, ld_in, out, ld_out, root_dof_count, nworld, c.kind_count[0], c.kind_count[0] + c.kind_count[1]};
+  return what == IM_MUSCLE_TORQUE ? launch_context<MW_FORWARD>(a, (hipStream_t)stream)
+         : what == IM_MUSCLE_GRAD ? launch_context<MW_GRAD>(a, (hipStream_t)stream)
+                                  : launch_context<MW_MOMENT>(a, (hipStream_t)stream);
 }

@@ -159,6 +159,32 @@ def build_muscle_sparse_torque_entries(
     )
 
 
+# What im_muscle_from_context computes
+_TORQUE, _GRAD, _MOMENT = 0, 1, 2
+
+
+def pack_context_entries(segment, torque, muscle, start_coeff, end_coeff):
+    """A list of (segment, dof) entries in the packed order of im_muscle_from_context: the entries of a
+    kind (end only, start only, both) together, the first two kinds filled up to whole wavefronts.
+    Returns (packed (n, 2) uint32, counts of the kinds), or None where a coefficient is neither 0 nor 1 or
+    a number does not fit 16 bits."""
+    segment, torque, muscle = (np.asarray(a, np.int64) for a in (segment, torque, muscle))
+    a, b, n = np.asarray(start_coeff), np.asarray(end_coeff), len(segment)
+    if n == 0 or n >= 65535 or max(segment.max(), torque.max(), muscle.max()) >= 65536:
+        return None
+    if not (((a == 0) | (a == 1)) & ((b == 0) | (b == 1)) & (a + b > 0)).all():
+        return None
+    words, counts = [], []
+    for kind, on in enumerate(((a == 0) & (b == 1), (a == 1) & (b == 0), (a == 1) & (b == 1))):
+        place = np.flatnonzero(on)
+        place = place[np.lexsort((torque[place], segment[place]))]  # 64 entries: few segments' records, every dof's its own banks
+        block = np.stack([segment[place] | torque[place] << 16, place | muscle[place] << 16], 1)
+        fill = -len(place) % 64 if kind < 2 else 0
+        words += [block, np.tile(np.array([[0, n]], np.int64), (fill, 1))]
+        counts.append(len(place) + fill)
+    return np.concatenate(words).astype(np.uint32), counts
+
+
 @dataclass
 class _Tables:
     keep: list = field(default_factory=list)
@@ -286,6 +312,39 @@ class MuscleDynamicsLayer:
         self._torque_entries = entries(d["tq"], self.torque_dim, self.muscle_count)
         self._muscle_entries = entries(d["ms"], self.muscle_count, self.torque_dim)
         self._moment_entries = entries(d["mom"], len(e.muscle_dof_torque_idx), self.torque_dim, other=False)
+        self._upload_context(up)
+
+    def _upload_context(self, up):
+        """The argument blocks of im_muscle_from_context, one per output; an output whose entry list or
+        sizes it does not take has None and goes by way of waypoints and forces in memory."""
+        d, (tq, ms, e) = self._dev, (self.torque_entries_host, self.muscle_entries_host, self.sparse_entries)
+        ms_muscle = np.repeat(np.arange(self.muscle_count), np.diff(ms[0]))
+        mom_torque = np.repeat(e.muscle_dof_torque_idx, np.diff(e.muscle_dof_segment_offsets))
+        lists = (
+            (d["tq"][0], self.torque_dim, (tq[2], tq[1], tq[3], tq[4], tq[5])),
+            (d["ms"][0], self.muscle_count, (ms[1], ms[2], ms_muscle, ms[3], ms[4])),
+            (d["mom"][0], len(e.muscle_dof_torque_idx), (e.segment_idx, mom_torque, np.zeros_like(mom_torque), e.start_coeff, e.end_coeff)),
+        )
+        self._context = [None, None, None]
+        d["packed"] = []
+        for what, (offsets, nrow, entries) in enumerate(lists):
+            packed = pack_context_entries(*entries)
+            if packed is None:
+                continue
+            words, counts = packed
+            t = up(words.view(np.int32))
+            c = _lib.MuscleContext(
+                waypoint_body=d["wp_body"].data_ptr(), waypoint_local=d["wp_local"].data_ptr(),
+                all_segment_start=d["all_seg_start"].data_ptr(), all_segment_offsets=d["all_seg_off"].data_ptr(),
+                params=d["params"].data_ptr(), rest=d["rest"].data_ptr(), offsets=offsets.data_ptr(), packed=t.data_ptr(),
+                ld_params=self.muscle_params.shape[1], nbody=self.body_count, nwaypoint=self.waypoint_count,
+                nsegment=len(self.segments_host[0]), ntorque=self.torque_dim, nmuscle=self.muscle_count, nrow=nrow,
+                nentry=len(entries[0]), npacked=len(words), kind_count=(C.c_int32 * 3)(*counts), model=self._model,
+            )  # fmt: skip
+            c.start_waypoint, c.end_waypoint, c.start_root_body, c.end_root_body = (s.data_ptr() for s in d["seg"])
+            if _lib.lib().im_muscle_from_context(C.byref(c), what, None, 0, self.root_dof_count, None, nrow, 0, None) == 0:
+                self._context[what] = c
+                d["packed"].append(t)
 
     def _need_gpu(self, *tensors):
         import torch
@@ -340,7 +399,47 @@ class MuscleDynamicsLayer:
         )
         return ws, geo
 
+    def _check_context(self, raw_context):
+        self._need_gpu(raw_context)
+        if raw_context.shape[1] < self.context_dim:
+            raise ValueError(f"raw_context has {raw_context.shape[1]} columns, the layer needs {self.context_dim}")
+
+    def _from_context(self, what: int, raw_context, x, out, include_passive_force: bool = False) -> bool:
+        """One launch from the context to ``out``, where the layer has a packed list for it."""
+        static = self._context[what]
+        # (a list that states no range takes the kernels that need none)
+        if static is None or not (self._torque_entries, self._muscle_entries, self._moment_entries)[what].nother:
+            return False
+        c = _lib.MuscleContext.from_buffer_copy(static)  # a call's own block: calls of several threads do not meet
+        base, ld = raw_context.data_ptr(), raw_context.stride(0)
+        c.xpos, c.xquat = base + 4 * self._xpos_off, base + 4 * self._xquat_off
+        c.subtree_com, c.cdof = base + 4 * self._com_off, base + 4 * self._cdof_off
+        c.ld_xpos = c.ld_xquat = c.ld_subtree_com = c.ld_cdof = ld
+        c.model.include_passive = 1 if include_passive_force else 0
+        _lib.check(
+            _lib.lib().im_muscle_from_context(
+                C.byref(c), what, None if x is None else x.data_ptr(), 0 if x is None else x.stride(0), self.root_dof_count,
+                out.data_ptr(), out.stride(0), raw_context.shape[0], _stream(raw_context),
+            ),
+            "im_muscle_from_context",
+        )  # fmt: skip
+        return True
+
     # ------------------------------------------------------------------ launchers
+    def _torque_from_context(self, activation, raw_context, include_passive_force: bool):
+        """The torque of ``_warp_muscle_dynamics_from_activation_forward`` alone."""
+        import torch
+
+        activation, raw_context = activation.float(), raw_context.float()
+        self._need_gpu(activation, raw_context)
+        if activation.shape != (raw_context.shape[0], self.muscle_count):
+            raise ValueError("activation must be (batch, muscle_count)")
+        self._check_context(raw_context)
+        torque = torch.empty((activation.shape[0], self.torque_dim), device=activation.device)
+        if self._from_context(_TORQUE, raw_context, activation, torque, include_passive_force):
+            return torque
+        return self._warp_muscle_dynamics_from_activation_forward(activation, raw_context, include_passive_force=include_passive_force)[0]
+
     def _warp_muscle_dynamics_from_activation_forward(self, activation, raw_context, *, include_passive_force: bool, mean_out=None):
         """(torque, transformed_waypoints, unit_force_magnitude), as the reference's method of
         this name (muscle_dynamics.py:4958-5009)."""
@@ -373,6 +472,11 @@ class MuscleDynamicsLayer:
         self._need_gpu(raw_context, grad_output, unit_force_magnitude)
         if grad_output.shape != (raw_context.shape[0], self.torque_dim):
             raise ValueError("grad_output must be (batch, torque_dim)")
+        if unit_force_magnitude is None:
+            self._check_context(raw_context)
+            grad = torch.empty((raw_context.shape[0], self.muscle_count), device=raw_context.device)
+            if self._from_context(_GRAD, raw_context, grad_output, grad):
+                return grad
         ws, geo = self._prepare_waypoint_geometry(
             raw_context, include_passive_force_magnitude=False, compute_force_magnitudes=unit_force_magnitude is None
         )
@@ -447,9 +551,13 @@ class MuscleDynamicsLayer:
 
         raw_context = raw_context.float()
         self._need_gpu(raw_context, moment_out)
+        self._check_context(raw_context)
+        if moment_out is None:
+            moment_out = torch.empty((raw_context.shape[0], len(self.sparse_entries.muscle_dof_torque_idx)), device=raw_context.device)
+        if self._from_context(_MOMENT, raw_context, None, moment_out):
+            return moment_out
         ws, geo = self._prepare_waypoint_geometry(raw_context, include_passive_force_magnitude=False, compute_force_magnitudes=False)
-        B, ne = raw_context.shape[0], len(self.sparse_entries.muscle_dof_torque_idx)
-        moment = moment_out if moment_out is not None else torch.empty((B, ne), device=raw_context.device)
+        B, moment = raw_context.shape[0], moment_out
         _lib.check(
             _lib.lib().im_muscle_sparse_moment(
                 C.byref(geo), C.byref(self._segments), self._dev["mom_torque"].data_ptr(), C.byref(self._moment_entries),

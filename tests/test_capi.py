@@ -303,7 +303,7 @@ def test_ctypes_structs_match_the_header(tmp_path):
         "im_tree_plan_info": _lib.TreePlanInfo, "im_sparse_plan_info": _lib.SparsePlanInfo,
         "im_muscle_force_model": _lib.MuscleForceModel, "im_muscle_force_velocity_model": _lib.MuscleForceVelocityModel,
         "im_newton_args": _lib.NewtonArgs, "im_row_pair_term": _lib.RowPairTerm, "im_muscle_geometry": _lib.MuscleGeometry,
-        "im_muscle_segments": _lib.MuscleSegments, "im_muscle_entries": _lib.MuscleEntries,
+        "im_muscle_segments": _lib.MuscleSegments, "im_muscle_entries": _lib.MuscleEntries, "im_muscle_context": _lib.MuscleContext,
         "im_body_wrenches": _lib.BodyWrenches, "im_wrench_topology": _lib.WrenchTopology,
     }  # fmt: skip
     lines = ["#include <stddef.h>", "#include <stdio.h>", '#include "imhip.h"', "int main(void) {"]

@@ -6,6 +6,7 @@ own two-body fixture); GPU tests compare libimhip with the oracle bit for bit wh
 IEEE-exact operations are involved and to 2e-6 where expf/cosf enter.
 """
 
+import dataclasses
 import gc
 
 import numpy as np
@@ -21,6 +22,7 @@ from instantmimic_amd.muscle.muscle_dynamics import (
     build_dof_subtree_mask,
     build_muscle_sparse_torque_entries,
     build_torque_sparse_segment_entries,
+    pack_context_entries,
 )
 from oracle import ref
 
@@ -689,5 +691,64 @@ def test_gpu_contractions_on_every_workgroup_size(muscles):
             e.nother = 0
         for a, b in zip(got, run()):
             assert torch.equal(a, b)
+        for e, n in zip(entries, stated):
+            e.nother = n
+
+
+def test_packed_entries_are_the_list_in_another_order():
+    """Kinds together, the first two in whole wavefronts, every entry once; lists with other coefficients are refused."""
+    layer = MuscleDynamicsLayer((rig := synth.make_muscle_rig(nmuscle=50, seed=3)).topology, **rig.dims(), device="cpu")
+    _, torque, segment, muscle, a, b = layer.torque_entries_host
+    words, counts = pack_context_entries(segment, torque, muscle, a, b)
+    assert counts[0] % 64 == 0 and counts[1] % 64 == 0 and sum(counts) == len(words)
+    place = words[:, 1] & 0xFFFF
+    real = place < len(segment)
+    assert np.array_equal(np.sort(place[real]), np.arange(len(segment))) and (place[~real] == len(segment)).all()
+    at = place[real]
+    assert np.array_equal(words[real, 0], (segment[at] | torque[at] << 16).astype(np.uint32)) and np.array_equal(words[real, 1] >> 16, muscle[at])
+    kind = np.repeat([0, 1, 2], counts)[real]
+    assert np.array_equal(a[at], np.float32([0, 1, 1])[kind]) and np.array_equal(b[at], np.float32([1, 0, 1])[kind])
+    assert pack_context_entries(segment, torque, muscle, a * 0.5, b) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("muscles", [3, 74, 76, 158, 164, 225, 226, 320, 325])
+@pytest.mark.parametrize("swap", [False, True])
+def test_gpu_from_context_equals_waypoints_and_forces_in_memory(muscles, swap):
+    """Torque, gradient and moment in one launch: the bits of the kernels with waypoints and forces in
+    memory, on both sides of 1280, 2560, 3584 and 5120 entries (128, 256 and 512 threads; more than a workgroup keeps), for segments that
+    run up and down the tree, one world and several per workgroup, and with poses, centres and axes that are not finite."""
+    rig = synth.make_muscle_rig(nmuscle=muscles, seed=1003)
+    t = rig.topology
+    if swap:  # the end's body above the start's: entries with a start coefficient alone
+        t = dataclasses.replace(
+            t, apply_segment_start_idx=t.apply_segment_end_idx, apply_segment_end_idx=t.apply_segment_start_idx,
+            apply_segment_body_start_idx=t.apply_segment_body_end_idx, apply_segment_body_end_idx=t.apply_segment_body_start_idx,
+        )  # fmt: skip
+    layer = MuscleDynamicsLayer(t, **rig.dims(), mechanics=MuscleMechanics(), device="cuda")
+    assert (layer._context[0] is None) == (muscles == 325) and (layer._context[1] is None) == (layer._context[2] is None) == (muscles == 325)
+    entries = (layer._torque_entries, layer._muscle_entries, layer._moment_entries)
+    stated = [e.nother for e in entries]
+    for nworld, odd in ((1, False), (1901, False), (67, True)):
+        ctx = synth.make_muscle_context(rig, nworld, seed=6)
+        if odd:
+            for k, v in enumerate((np.inf, -np.inf, np.nan, 3.0e38)):
+                ctx[8 * k + 1, layer._com_off + 3 + k % 3] = v
+                ctx[8 * k + 2, layer._cdof_off + 6 * (layer.root_dof_count + k) + k] = v
+                ctx[8 * k + 3, 3 * (k + 1)] = v
+        ctx_d = torch.from_numpy(np.pad(ctx, ((0, 0), (0, 5)))).cuda()[:, : ctx.shape[1] + 2]
+        act = torch.rand(nworld, rig.muscle_count, device="cuda")
+        act[:, ::7] = 0.0
+        g = torch.randn(nworld, rig.torque_dim, device="cuda")
+
+        def run():
+            return [layer._torque_from_context(act, ctx_d, passive) for passive in (False, True)] + [
+                layer._warp_muscle_dynamics_from_activation_backward(ctx_d, g), layer.eval_muscle_sparse_moment(ctx_d)]  # fmt: skip
+
+        got = run()
+        for e in entries:
+            e.nother = 0
+        for a, b in zip(got, run()):
+            assert torch.equal(torch.nan_to_num(a, 1.0, 2.0, 3.0), torch.nan_to_num(b, 1.0, 2.0, 3.0)) and torch.equal(a.isnan(), b.isnan())
         for e, n in zip(entries, stated):
             e.nother = n
