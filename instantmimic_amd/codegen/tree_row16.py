@@ -915,11 +915,11 @@ def generate(name, rowadr, rownnz, colind, groups, trunk, *, module: bool = Fals
     # rows a lane keeps in registers during the line search: two up to 64 rows, four up to 128 (the
     # same for the whole launch), beyond that the rows are read from LDS at every evaluation
     emit("  if (!LONG)")
-    emit("    im::resident::newton_loop<2, 0, true>(0, L, w, stage);")
+    emit(f"    im::resident::newton_loop<2, {2 if nv > 64 else 1}, true, true>(0, L, w, stage);")
     emit("  else if (a.njmax <= 128)")
-    emit("    im::resident::newton_loop<4, 0, true>(0, L, w, stage);")
+    emit(f"    im::resident::newton_loop<4, {2 if nv > 64 else 1}, true, true>(0, L, w, stage);")
     emit("  else")
-    emit("    im::resident::newton_loop<0, 0, true>(0, L, w, stage);")
+    emit(f"    im::resident::newton_loop<0, {2 if nv > 64 else 1}, true, true>(0, L, w, stage);")
     emit("}")
     if module:
         emit("} }  // namespace im::gen")

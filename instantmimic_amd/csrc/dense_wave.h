@@ -554,14 +554,16 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
       s1 = fma_(gw[i], x, s1);
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    s0 = s0 + __shfl_down(s0, off, 64);
-    s1 = s1 + __shfl_down(s1, off, 64);
-  }
+  // the shuffle-down tree of 64 lanes: the halves, then as for 32 lanes (both sums at once, newton_search.h)
+  float h0 = s0, h1 = s1;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3\n\ts_nop 1" : "+v"(s0), "+v"(h0), "+v"(s1), "+v"(h1));
+  s0 = s0 + h0, s1 = s1 + h1;
+  search::swap_rows(s0, s1);
+  const float s = search::row_sum(s0 + s1);
+  const float dot = search::lane_of(s, 0), descent = search::lane_of(s, 16);
   if (lane == 0) {
-    *search_dot_w = s0;
-    *decrement_w = s1;
+    *search_dot_w = dot;
+    *decrement_w = descent;
   }
 }
 

@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64 * WAVES, NB == 5 ? 3 : 4) void newton_dense_wave
   L.votes = nullptr;
   L.worlds = nullptr;
   L.term = term, L.radr = radr;
-  L.rows = mine;  // the shared area: tile of J, then the gradient's lists, then the stage
+  L.rows = mine;  // the shared area: M's row, the tile of J, then the gradient's lists, then the stage
   L.f = mine;
   L.rowl = (int *)(mine + njmax);
   L.gl = mine + 2 * njmax;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(64 * WAVES, NB == 5 ? 3 : 4) void newton_dense_wave
   // as many wavefronts as the chip keeps resident; one whose world is done takes the next world
   // nobody has started (a counter in memory that only grows: every wavefront reaches the end)
   while (w < nworld) {
-    resident::newton_loop<HELD, -2, false, false>(0, L, w, stage);
+    resident::newton_loop<HELD, NB == 5 ? 2 : 1, NB != 3, false, false>(0, L, w, stage);
     int next = 0;
     if ((threadIdx.x & 63) == 0) next = atomicAdd(next_world, 1);
     w = __builtin_amdgcn_readfirstlane(next);

@@ -17,8 +17,8 @@
 namespace im {
 namespace {
 
-// LDS words of one wavefront: the tile of J, then sv, Ma, gl (nv each), Jaref, f, rowl (njmax each)
-__host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return 64 * 17 + 3 * (size_t)nv + 3 * (size_t)njmax; }
+// LDS words of one wavefront: M's row and the tile of J, then sv, Ma, gl (nv each), Jaref, f, rowl (njmax each)
+__host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return resident::kTileWords + 3 * (size_t)nv + 3 * (size_t)njmax; }
 
 __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::NewtonArgs a, const float *__restrict__ qacc_smooth,
                                                                   int64_t ld_qacc_smooth, const float *__restrict__ aref,
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
   uint32_t *term = (uint32_t *)lds;
   int *radr = (int *)(term + a.nterm);
   float *mine = (float *)(radr + nv + 1) + wv * init_wave_words(nv, njmax);
-  float *tile = mine, *sv = tile + 64 * 17, *Ma_l = sv + nv, *gl = Ma_l + nv, *Jaref_l = gl + nv, *f = Jaref_l + njmax;
+  float *tile = mine, *sv = tile + resident::kTileWords, *Ma_l = sv + nv, *gl = Ma_l + nv, *Jaref_l = gl + nv, *f = Jaref_l + njmax;
   int *rowl = (int *)(f + njmax);
   for (int k = threadIdx.x; k < a.nterm; k += blockDim.x) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
   for (int k = threadIdx.x; k <= nv; k += blockDim.x) radr[k] = a.mulm_rowadr[k];
@@ -59,9 +59,8 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
     if (empty && whole.active) a.qfrc_constraint[w * nv + k] = 0.0f;
     sv[k] = q;
   }
-  resident::wave_sync();
   // Ma = M qacc, for every world
-  resident::mul_m_world(a, term, radr, a.M + w * a.ldM, sv, a.Ma + w * nv, Ma_l, lane);
+  resident::mul_m_world_staged<false, 12>(a, term, radr, a.M + w * a.ldM, sv, a.Ma + w * nv, Ma_l, tile, lane);
   if (empty) {  // what the stages leave of a done world: zero counts and the `unchanged` byte
     if (lane == 0) {
       a.quad_count[w] = 0;
@@ -71,7 +70,11 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
     return;
   }
   const float *Jw = a.J + w * (int64_t)njmax * nv;
-  resident::jv_world_tiled<true, true>(a, Jw, nefc, tile, sv, nullptr, Jaref_l, lane);
+  resident::wave_sync();
+  if (nv > 64)
+    resident::jv_world(a, Jw, nefc, sv, nullptr, Jaref_l, lane, []() {});
+  else
+    resident::jv_world_tiled<true>(a, Jw, nefc, tile, sv, nullptr, Jaref_l, lane, []() {});
   resident::wave_sync();
   // Jaref = J qacc - aref, then force and state of every row (newton_stages.py:385-444 at step 0),
   // the rows whose being quadratic differs from the state that lay there, the rows with a force
@@ -121,7 +124,10 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
   }
   resident::wave_sync();
   resident::Scalars sc{};
-  resident::gradient_world<true>(a, w, Jw, true, cnt, f, rowl, Ma_l, gl, sc, lane);
+  if (nv > 64)
+    resident::gradient_world<2, 4, false>(a, w, Jw, true, cnt, f, rowl, Ma_l, a.smooth + w * nv, gl, sc, lane);
+  else
+    resident::gradient_world<1, 2, false>(a, w, Jw, true, cnt, f, rowl, Ma_l, a.smooth + w * nv, gl, sc, lane);
 }
 
 }  // namespace

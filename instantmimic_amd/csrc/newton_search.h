@@ -32,20 +32,22 @@ __device__ __forceinline__ Pt operator+(Pt a, Pt b) { return {a.c + b.c, a.g + b
 __device__ __forceinline__ float safe_div(float x, float y) { return x / (y != 0.0f ? y : kMinVal); }
 // a quadratic (q0, q1, q2) at alpha
 __device__ __forceinline__ Pt eval_pt(Pt q, float a) { return {a * a * q.h + a * q.g + q.c, 2.0f * a * q.h + q.g, 2.0f * q.h}; }
-__device__ __forceinline__ bool in_bracket(Pt x, Pt y) { return (x.g < y.g && y.g < 0.0f) || (x.g > y.g && y.g > 0.0f); }
+// (not short-circuited: a branch costs more than the comparisons)
+__device__ __forceinline__ bool in_bracket(Pt x, Pt y) { return ((x.g < y.g) & (y.g < 0.0f)) | ((x.g > y.g) & (y.g > 0.0f)); }
 
 // The quadratic a row follows at position x: its own where it is in the quadratic zone, the linear
 // pieces of the friction-loss cost outside, nothing for a satisfied inequality.
 // (rf: the friction row's f / D, which does not change during a search: formed once per row)
 __device__ __forceinline__ Pt row_quad(bool friction, float D, float f, float rf, float jaref, float jv, float x) {
-  const Pt quad = {0.5f * jaref * jaref * D, jv * jaref * D, 0.5f * jv * jv * D};
-  if (friction) {
-    if (x <= -rf) return {f * (-0.5f * rf - jaref), -f * jv, 0.0f};
-    if (x >= rf) return {f * (-0.5f * rf + jaref), f * jv, 0.0f};
-    return quad;
-  }
-  if (x < 0.0f) return quad;
-  return {0.0f, 0.0f, 0.0f};
+  // (every piece formed and one selected: a branch per piece took twice the instructions)
+  const bool below = friction && x <= -rf, above = friction ? x >= rf : !(x < 0.0f);
+  const float c_above = friction ? f * (-0.5f * rf + jaref) : 0.0f, g_above = friction ? f * jv : 0.0f;
+  const float c_below = f * (-0.5f * rf - jaref), g_below = -f * jv;
+  Pt p = {0.5f * jaref * jaref * D, jv * jaref * D, 0.5f * jv * jv * D};
+  p.c = above ? c_above : p.c, p.g = above ? g_above : p.g;
+  p.c = below ? c_below : p.c, p.g = below ? g_below : p.g;
+  p.h = above || below ? 0.0f : p.h;
+  return p;
 }
 // point of a row at alpha, cost relative to alpha 0, with the row's cost at alpha 0 computed beforehand (row_quad(..., jaref).c)
 __device__ __forceinline__ Pt row_point_from(bool friction, float D, float f, float rf, float jaref, float jv, float c0, float alpha) {
@@ -59,51 +61,59 @@ __device__ __forceinline__ Pt row_point_zero(bool friction, float D, float f, fl
   return {q.c, q.g, 2.0f * q.h};
 }
 
-// sum over the 32 lanes of a world: shuffle-down tree, lane 0's value to all, then the +0 of the
+// Sums over the 32 lanes of a world: shuffle-down tree, lane 0's value to all, then the +0 of the
 // later warps' empty partials (newton_stages.py:36-52).  The tree's first step crosses the two
-// rows of 16 lanes of a world (v_permlane16_swap_b32 hands every even row the odd row behind it),
-// the others stay inside a row (DPP shifts); what a lane receives from beyond its row or world
-// never reaches lane 0, whose sum has the association of the 32-lane shuffle-down tree.  Lane 0's
-// (lane 32's) value then goes to its world through a lane read.  A world's 32 lanes are active or
-// inactive together.
+// rows of 16 lanes of a world, the others stay inside a row (DPP shifts); what a lane receives from
+// beyond its row never reaches the row's first lane, whose sum has the association of the 32-lane
+// shuffle-down tree.  v_permlane16_swap_b32 a, b changes the odd rows of a with the even rows of b: with two different
+// sums in a and b, a + b is then the first step of both, a's in the even rows and b's in the odd ones, and the other
+// steps work on both at once.  A world's 32 lanes are active or inactive together.
 template <int N>
 __device__ __forceinline__ float row_shl(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float lanes_sum(float s) {
-  // v_permlane16_swap_b32 a, b: the odd rows of a change places with the even rows of b.  Written
-  // out, with its wait states: the compiler's builtin returns the first result twice when both
-  // operands hold the same value.
-  unsigned upper = __builtin_bit_cast(unsigned, s), lower = upper;
-  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lower), "+v"(upper));
-  s = s + __builtin_bit_cast(float, upper);  // lane i of an even row: lane i + 16
+__device__ __forceinline__ float lane_of(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+// The swap written out, with its wait states: the compiler's builtin returns the first result twice when both
+// operands hold the same value.
+__device__ __forceinline__ void swap_rows(float &a, float &b) {
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void swap_rows(Pt &a, Pt &b) {
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\tv_permlane16_swap_b32 %4, %5\n\ts_nop 1"
+      : "+v"(a.c), "+v"(b.c), "+v"(a.g), "+v"(b.g), "+v"(a.h), "+v"(b.h));
+}
+__device__ __forceinline__ float row_sum(float s) {
   s = s + row_shl<8>(s);
   s = s + row_shl<4>(s);
   s = s + row_shl<2>(s);
-  s = s + row_shl<1>(s);
-  const float first = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 0));
-  const float second = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 32));
-  s = (threadIdx.x & 32) ? second : first;
-  return s + 0.0f;
+  return s + row_shl<1>(s);
 }
-__device__ __forceinline__ Pt lanes_sum(Pt p) { return {lanes_sum(p.c), lanes_sum(p.g), lanes_sum(p.h)}; }
-// The same tree with the sums of both halves of the wavefront handed to every lane: `lower` that of
-// lanes 0 - 31, `upper` that of lanes 32 - 63 (for a wavefront whose halves sum different things).
-__device__ __forceinline__ void lanes_sum_halves(float s, float &lower_sum, float &upper_sum) {
-  unsigned upper = __builtin_bit_cast(unsigned, s), lower = upper;
-  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lower), "+v"(upper));
-  s = s + __builtin_bit_cast(float, upper);
-  s = s + row_shl<8>(s);
-  s = s + row_shl<4>(s);
-  s = s + row_shl<2>(s);
-  s = s + row_shl<1>(s);
-  lower_sum = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 0)) + 0.0f;
-  upper_sum = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 32)) + 0.0f;
+// The sums of a and b of the lane's own world (BOTH: the wavefront's halves hold the same world).
+template <bool BOTH>
+__device__ __forceinline__ void lanes_sum2(float &a, float &b) {
+  swap_rows(a, b);
+  const float s = row_sum(a + b);
+  const bool upper = !BOTH && (threadIdx.x & 32);
+  const float a0 = lane_of(s, 0), b0 = lane_of(s, 16);
+  a = (upper ? lane_of(s, 32) : a0) + 0.0f;
+  b = (upper ? lane_of(s, 48) : b0) + 0.0f;
 }
-__device__ __forceinline__ void lanes_sum_halves(Pt p, Pt &lower_sum, Pt &upper_sum) {
-  lanes_sum_halves(p.c, lower_sum.c, upper_sum.c);
-  lanes_sum_halves(p.g, lower_sum.g, upper_sum.g);
-  lanes_sum_halves(p.h, lower_sum.h, upper_sum.h);
+template <bool BOTH>
+__device__ __forceinline__ Pt lanes_sum(Pt p) {
+  float none = 0.0f;
+  lanes_sum2<BOTH>(p.c, p.g);
+  lanes_sum2<BOTH>(p.h, none);
+  return p;
+}
+// `mine` differs between the wavefront's halves, `same` does not: the sums of both halves' `mine` and of `same`.
+__device__ __forceinline__ void lanes_sum_halves(Pt mine, Pt same, Pt &lower, Pt &upper, Pt &both) {
+  swap_rows(mine, same);
+  const float c = row_sum(mine.c + same.c), g = row_sum(mine.g + same.g), h = row_sum(mine.h + same.h);
+  lower = {lane_of(c, 0) + 0.0f, lane_of(g, 0) + 0.0f, lane_of(h, 0) + 0.0f};
+  upper = {lane_of(c, 32) + 0.0f, lane_of(g, 32) + 0.0f, lane_of(h, 32) + 0.0f};
+  both = {lane_of(c, 16) + 0.0f, lane_of(g, 16) + 0.0f, lane_of(h, 16) + 0.0f};
 }
 
 struct SearchArgs {
@@ -160,7 +170,8 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
     g1 = g1 + jvD * Jaref[r];
     g2 = g2 + 0.5f * jv[r] * jvD;
   }
-  const Pt gauss = {0.0f, lanes_sum(g1), lanes_sum(g2)};
+  lanes_sum2<SPLIT>(g1, g2);
+  const Pt gauss = {0.0f, g1, g2};
   // this lane's rows ne + lane, ne + lane + 32, ...
   constexpr int NH = HELD > 0 ? HELD : 1;
   float hd[NH], hf[NH], hrf[NH], hja[NH], hv[NH], hc0[NH];
@@ -210,11 +221,11 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
   auto rows_at = [&](float alpha) {
     Pt s = {0.0f, 0.0f, 0.0f};
     rows_sum([&](bool fr, float d, float f, float rf, float ja, float v, float c0) { s = s + row_point_from(fr, d, f, rf, ja, v, c0, alpha); });
-    return lanes_sum(s);
+    return lanes_sum<SPLIT>(s);
   };
   Pt z = {0.0f, 0.0f, 0.0f};
   rows_sum([&](bool fr, float d, float f, float rf, float ja, float v, float) { z = z + row_point_zero(fr, d, f, rf, ja, v); });
-  const Pt rows0 = lanes_sum(z);
+  const Pt rows0 = lanes_sum<SPLIT>(z);
   const Pt p0 = {gauss.c + rows0.c, gauss.g + rows0.g, 2.0f * gauss.h + rows0.h};
   const Pt p0_delta = {0.0f, p0.g, p0.h};
   const float q1_abs = sqrtf(2.0f * fmaxf(rows0.c, 0.0f) * fmaxf(rows0.h, 0.0f)) + fabsf(gauss.g);
@@ -237,32 +248,35 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
     Pt lo = lo_less ? lo_in : p0_delta, hi = lo_less ? p0_delta : lo_in;
     float lo_alpha = lo_less ? lo_alpha_in : 0.0f, hi_alpha = lo_less ? 0.0f : lo_alpha_in;
     for (int it = 0; it < wd.ls_iterations; ++it) {
-      const float lo_next_alpha = lo_alpha - safe_div(lo.g, lo.h);
-      const float hi_next_alpha = hi_alpha - safe_div(hi.g, hi.h);
+      float lo_next_alpha, hi_next_alpha;
       const float mid_alpha = 0.5f * (lo_alpha + hi_alpha);
       Pt s_lo = {0.0f, 0.0f, 0.0f}, s_hi = s_lo, s_mid = s_lo;
       Pt lo_next, hi_next, mid;
       if constexpr (SPLIT) {
-        const float mine_alpha = (threadIdx.x & 32) ? hi_next_alpha : lo_next_alpha;
+        // a half's own candidate: one division for both
+        const bool upper = threadIdx.x & 32;
+        const float mine_alpha = (upper ? hi_alpha : lo_alpha) - safe_div(upper ? hi.g : lo.g, upper ? hi.h : lo.h);
+        lo_next_alpha = lane_of(mine_alpha, 0), hi_next_alpha = lane_of(mine_alpha, 32);
         rows_sum([&](bool fr, float d, float f, float rf, float ja, float v, float c0) {
           s_lo = s_lo + row_point_from(fr, d, f, rf, ja, v, c0, mine_alpha);
           s_mid = s_mid + row_point_from(fr, d, f, rf, ja, v, c0, mid_alpha);
         });
-        Pt rows_lo, rows_hi, rows_mid, same;
-        lanes_sum_halves(s_lo, rows_lo, rows_hi);
-        lanes_sum_halves(s_mid, rows_mid, same);
+        Pt rows_lo, rows_hi, rows_mid;
+        lanes_sum_halves(s_lo, s_mid, rows_lo, rows_hi, rows_mid);
         lo_next = eval_pt(gauss, lo_next_alpha) + rows_lo;
         hi_next = eval_pt(gauss, hi_next_alpha) + rows_hi;
         mid = eval_pt(gauss, mid_alpha) + rows_mid;
       } else {
+        lo_next_alpha = lo_alpha - safe_div(lo.g, lo.h);
+        hi_next_alpha = hi_alpha - safe_div(hi.g, hi.h);
         rows_sum([&](bool fr, float d, float f, float rf, float ja, float v, float c0) {
           s_lo = s_lo + row_point_from(fr, d, f, rf, ja, v, c0, lo_next_alpha);
           s_hi = s_hi + row_point_from(fr, d, f, rf, ja, v, c0, hi_next_alpha);
           s_mid = s_mid + row_point_from(fr, d, f, rf, ja, v, c0, mid_alpha);
         });
-        lo_next = eval_pt(gauss, lo_next_alpha) + lanes_sum(s_lo);
-        hi_next = eval_pt(gauss, hi_next_alpha) + lanes_sum(s_hi);
-        mid = eval_pt(gauss, mid_alpha) + lanes_sum(s_mid);
+        lo_next = eval_pt(gauss, lo_next_alpha) + lanes_sum<SPLIT>(s_lo);
+        hi_next = eval_pt(gauss, hi_next_alpha) + lanes_sum<SPLIT>(s_hi);
+        mid = eval_pt(gauss, mid_alpha) + lanes_sum<SPLIT>(s_mid);
       }
       const bool conv_lo = fabsf(lo_next.g) < gtol_accept && lo_next.c < 0.0f;
       const bool conv_hi = fabsf(hi_next.g) < gtol_accept && hi_next.c < 0.0f;
@@ -278,19 +292,18 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
         lo = hi = best;
         lo_alpha = hi_alpha = best_alpha;
       } else {
-        const bool a1 = in_bracket(lo, lo_next);
-        if (a1) lo = lo_next, lo_alpha = lo_next_alpha;
-        const bool a2 = in_bracket(lo, mid);
-        if (a2) lo = mid, lo_alpha = mid_alpha;
-        const bool a3 = in_bracket(lo, hi_next);
-        if (a3) lo = hi_next, lo_alpha = hi_next_alpha;
+        auto take = [](bool on, Pt &to, float &to_alpha, const Pt &from, float from_alpha) __attribute__((always_inline)) {
+          to.c = on ? from.c : to.c, to.g = on ? from.g : to.g, to.h = on ? from.h : to.h;
+          to_alpha = on ? from_alpha : to_alpha;
+          return on;
+        };
+        const bool a1 = take(in_bracket(lo, lo_next), lo, lo_alpha, lo_next, lo_next_alpha);
+        const bool a2 = take(in_bracket(lo, mid), lo, lo_alpha, mid, mid_alpha);
+        const bool a3 = take(in_bracket(lo, hi_next), lo, lo_alpha, hi_next, hi_next_alpha);
         swap_lo = a1 || a2 || a3;
-        const bool b1 = in_bracket(hi, hi_next) || (hi.g < 0.0f && hi_next.g > 0.0f);
-        if (b1) hi = hi_next, hi_alpha = hi_next_alpha;
-        const bool b2 = in_bracket(hi, mid);
-        if (b2) hi = mid, hi_alpha = mid_alpha;
-        const bool b3 = in_bracket(hi, lo_next);
-        if (b3) hi = lo_next, hi_alpha = lo_next_alpha;
+        const bool b1 = take(in_bracket(hi, hi_next) || (hi.g < 0.0f && hi_next.g > 0.0f), hi, hi_alpha, hi_next, hi_next_alpha);
+        const bool b2 = take(in_bracket(hi, mid), hi, hi_alpha, mid, mid_alpha);
+        const bool b3 = take(in_bracket(hi, lo_next), hi, hi_alpha, lo_next, lo_next_alpha);
         swap_hi = b1 || b2 || b3;
       }
       const bool ls_done = conv || (!swap_lo && !swap_hi) || (lo.c < 0.0f && lo.g < 0.0f && lo.g > -gtol) ||

@@ -52,7 +52,7 @@ int compute_units(int *ncu) {
 
 bool usable_resident(const void *fn) {
   hipFuncAttributes fa{};
-  const bool ok = hipFuncGetAttributes(&fa, fn) == hipSuccess && fa.localSizeBytes <= 16 &&
+  const bool ok = hipFuncGetAttributes(&fa, fn) == hipSuccess && fa.localSizeBytes <= 32 &&
                   hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - (int)fa.sharedSizeBytes) == hipSuccess;
   (void)hipGetLastError();
   return ok;

@@ -72,7 +72,7 @@ inline int convert_args(const im_newton_args &p, int nv, int nM, NewtonArgs &a) 
       !p.search_unchanged || (p.nf && !p.efc_frictionloss))
     return IM_ERR_ARG;
   if (p.ldM < nM || p.ld_grad < nv || p.ld_ids < 0) return IM_ERR_STRIDE;
-  if (p.nterm >= 65536 || nM >= 65536 || 64 * (int64_t)nv >= (1 << 20)) return IM_ERR_UNSUPPORTED;
+  if (p.nterm >= 65536 || nM >= 65536 || 64 * (int64_t)nv >= (1 << 20) || (int64_t)njmax * nv >= (1 << 29)) return IM_ERR_UNSUPPORTED;
   a.tolerance = p.opt_tolerance, a.ls_tolerance = p.opt_ls_tolerance, a.meaninertia = p.stat_meaninertia;
   a.ntolerance = p.ntolerance, a.nls_tolerance = p.nls_tolerance, a.nmeaninertia = p.nmeaninertia;
   a.nv = nv, a.njmax = njmax, a.nworld = p.nworld, a.ls_iterations = p.ls_iterations, a.maxiter = p.iterations;
@@ -120,89 +120,100 @@ __device__ __forceinline__ void block_sync() {
 // (one word per term, nv + 1 offsets), then per wavefront the world's row of M, the search
 // direction, Ma, mv, Jaref, jv, D and the friction losses, the gradient's list of rows with a force
 // (value and row number) and its copy of the gradient.  The factor stage's area must also hold four wavefronts'
-// staged tiles of J: 4 x 64 rows x 16 dofs, a row 17 words.
+// rows of M where those are read from memory (kTileWords each).
 // words a wavefront keeps from round to round: M, the search direction, Ma, mv, qacc; Jaref, jv, D, friction losses
 __host__ __device__ inline size_t kept_words(int nv, int njmax, int nM) { return (size_t)nM + 4 * (size_t)nv + 4 * (size_t)njmax; }
 __host__ __device__ inline size_t loop_lds_words(int nv, int njmax, int nM, int nterm) {
   return 8 + (size_t)nterm + nv + 1 + 4 * (kept_words(nv, njmax, nM) + 2 * (size_t)njmax + nv);
 }
-__host__ __device__ inline size_t staged_rows_words(int) { return 4 * 64 * 17; }  // four wavefronts' tiles of J
+constexpr int kTileWords = 64 * 17;
+__host__ __device__ inline size_t staged_rows_words(int) { return 4 * kTileWords; }
 
-// ---- M search (newton_fusion.py:171-176): lane d owns dofs d, d + 64 --------------------------
+// ---- M search (newton_fusion.py:171-176) -------------------------------------------------------
+// WALK: more dofs than lanes.
+template <bool WALK>
 __device__ __forceinline__ void mul_m_world(const NewtonArgs &a, const uint32_t *term, const int *radr, const float *m,
                                             const float *v, float *out, float *out_lds, int lane) {
-  for (int dof = lane; dof < a.nv; dof += 64) {
-    float value = 0.0f;
-    const int end = radr[dof + 1];
-    for (int k = radr[dof]; k < end; k += 4) {  // four terms' operands at a time, a term past the end dropped
-      float x[4], y[4];
+  const int nv = a.nv;
+  if constexpr (!WALK) {
+    for (int dof = lane; dof < nv; dof += 64) {
+      float value = 0.0f;
+      const int end = radr[dof + 1];
+      for (int k = radr[dof]; k < end; k += 8) {  // eight terms' operands at a time, a term past the end dropped
+        float x[8], y[8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t t = term[k + u < end ? k + u : end - 1];
-        x[u] = m[t >> 16];
-        y[u] = v[t & 0xffffu];
+        for (int u = 0; u < 8; ++u) {
+          const uint32_t t = term[k + u < end ? k + u : end - 1];
+          x[u] = m[t >> 16];
+          y[u] = v[t & 0xffffu];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) value = k + u < end ? fma_(x[u], y[u], value) : value;
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) value = k + u < end ? fma_(x[u], y[u], value) : value;
+      out[dof] = value;
+      out_lds[dof] = value;
     }
-    out[dof] = value;
-    out_lds[dof] = value;
+    return;
+  }
+  // a lane takes dof `lane`, then 127 - lane, 128 + lane, ..: one after the other without waiting for the others, so
+  // that the long rows (a free body's dofs, the first ones) have nothing behind them.  Eight terms' operands at a time,
+  // a term past the end dropped; the next terms are read ahead of the current ones' operands.
+  int dof = lane, base = 0;
+  int k = 0, end = 0;
+  if (dof < nv) k = radr[dof], end = radr[dof + 1];
+  uint32_t t[8];
+  auto read = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = term[k + u < end ? k + u : end > 0 ? end - 1 : 0];
+  };
+  if (dof < nv) read(k);
+  float value = 0.0f;
+  while (dof < nv) {
+    float x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      x[u] = m[t[u] >> 16];
+      y[u] = v[t[u] & 0xffffu];
+    }
+    const int k0 = k, last = end;
+    k += 8;
+    int done = -1;
+    if (k >= end) {
+      done = dof;
+      base += 64;
+      dof = base + (base & 64 ? 63 - lane : lane);
+      if (dof < nv) k = radr[dof], end = radr[dof + 1];
+    }
+    if (dof < nv) read(k);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) value = k0 + u < last ? fma_(x[u], y[u], value) : value;
+    if (done >= 0) {
+      out[done] = value;
+      out_lds[done] = value;
+      value = 0.0f;
+    }
   }
 }
-
-// ---- J search (newton_stages.py:157-178): 64 rows at a time through LDS, a lane per row --------
-template <int U>
-__device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, int nefc, float *rows_lds,
-                                         const float *sv, float *jv, float *jv_lds, int lane) {
-  const int nv = a.nv, stride = nv | 1;
-  const float inv_nv = 1.0f / (float)nv;
-  for (int r0 = 0; r0 < nefc; r0 += 64) {
-    const int rows = nefc - r0 < 64 ? nefc - r0 : 64;
-    const float *src = Jw + (int64_t)r0 * nv;
-    const int total = rows * nv;
-    for (int i0 = lane; i0 < total; i0 += U * 64) {
-      float v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = src[i0 + 64 * u < total ? i0 + 64 * u : total - 1];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = i0 + 64 * u;
-        if (i < total) {
-          const int r = (int)(((float)i + 0.5f) * inv_nv);  // i / nv, exact while i stays below 2^20
-          rows_lds[r * stride + (i - r * nv)] = v[u];
-        }
-      }
-    }
+// The same with the world's row of M in memory: it passes through `stage` (kTileWords of LDS) where it fits,
+// LOADS a lane in flight at once.  Read term by term a free body's dofs, whose rows are nv long, waited for memory
+// once per four terms (70 dofs x 2048 worlds: 9 of the 22 us that a round's two products took).
+template <bool WALK, int LOADS>
+__device__ __forceinline__ void mul_m_world_staged(const NewtonArgs &a, const uint32_t *term, const int *radr, const float *m,
+                                                   const float *v, float *out, float *out_lds, float *stage, int lane) {
+  if (a.nM > kTileWords) {
     wave_sync();
-    if (lane < rows) {
-      const float *row = rows_lds + lane * stride;
-      auto chain = [&](int i0, int i1) {
-        float p = 0.0f;
-        int i = i0;
-        for (; i + 8 <= i1; i += 8) {
-          float x[8], y[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            x[u] = row[i + u];
-            y[u] = sv[i + u];
-          }
-#pragma unroll
-          for (int u = 0; u < 8; ++u) p = fma_(x[u], y[u], p);
-        }
-        for (; i < i1; ++i) p = fma_(row[i], sv[i], p);
-        return p;
-      };
-      float acc = 0.0f;
-      if (nv > 50) {
-        for (int start = 0; start < nv; start += 20) acc = acc + chain(start, start + 20 < nv ? start + 20 : nv);
-      } else {
-        acc = chain(0, nv);
-      }
-      jv[r0 + lane] = acc;
-      jv_lds[r0 + lane] = acc;
-    }
-    wave_sync();  // the rows are read before the next 64 overwrite them
+    return mul_m_world<WALK>(a, term, radr, m, v, out, out_lds, lane);
   }
+  for (int k0 = lane; k0 < a.nM; k0 += LOADS * 64) {
+    float x[LOADS];
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) x[u] = m[k0 + 64 * u < a.nM ? k0 + 64 * u : a.nM - 1];
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u)
+      if (k0 + 64 * u < a.nM) stage[k0 + 64 * u] = x[u];
+  }
+  wave_sync();
+  mul_m_world<WALK>(a, term, radr, stage, v, out, out_lds, lane);
 }
 
 // ---- the gradient (newton_stages.py:745-798), a lane per dof ------------------------------------
@@ -215,12 +226,52 @@ struct Scalars {
 // For a world whose states changed: qfrc_constraint = J' force over the listed rows (`cnt` rows with
 // a nonzero force, ascending, in f / rowl), grad = Ma - qfrc_smooth - qfrc_constraint, grad . grad.
 // Otherwise the rescaling of the three scalars.  Returns whether the search direction stays.
-// AHEAD: the next rows' elements are asked for before the current ones are added (ROWS more
-// registers a lane).
-template <bool AHEAD>
+// COLS: dofs of a lane (lane, lane + 64) whose sums run side by side; RING: batches of rows on their way at once.
+// LAZY: a list of one batch asks for no second one.  (Otherwise rows past the list are the last one again: behind a branch
+// every wait would count the youngest batch.)
+template <int COLS, int RING, bool LAZY>
+__device__ __forceinline__ void constraint_force(const float *Jw, int nv, int cnt, const float *f, const int *rowl, int d0, float (&sum)[COLS]) {
+  constexpr int ROWS = 16 / COLS;
+  float v[RING][ROWS][COLS];
+  auto fetch = [&](int p0, float (&v)[ROWS][COLS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      const uint32_t at = (uint32_t)(rowl[p0 + u < cnt ? p0 + u : cnt - 1] * nv);
+#pragma unroll
+      for (int k = 0; k < COLS; ++k) {
+        const int dof = d0 + 64 * k;
+        v[u][k] = *(const float *)((const char *)Jw + 4u * (at + (dof < nv ? dof : nv - 1)));
+      }
+    }
+  };
+  auto add = [&](int p0, float (&v)[ROWS][COLS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      const float fu = f[p0 + u < cnt ? p0 + u : cnt - 1];
+#pragma unroll
+      for (int k = 0; k < COLS; ++k) sum[k] = p0 + u < cnt ? fma_(v[u][k], fu, sum[k]) : sum[k];
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < COLS; ++k) sum[k] = 0.0f;
+  if (cnt <= 0) return;
+  fetch(0, v[0]);
+  if (LAZY && cnt <= ROWS) return add(0, v[0]);
+#pragma unroll
+  for (int b = 1; b < RING; ++b) fetch(b * ROWS, v[b]);
+  for (int p0 = 0; p0 < cnt; p0 += RING * ROWS) {
+#pragma unroll
+    for (int b = 0; b < RING; ++b) {
+      if (p0 + b * ROWS >= cnt) return;
+      add(p0 + b * ROWS, v[b]);
+      fetch(p0 + (b + RING) * ROWS, v[b]);
+    }
+  }
+}
+template <int COLS, int RING, bool LAZY>
 __device__ __forceinline__ bool gradient_world(const NewtonArgs &a, int64_t w, const float *Jw, bool changed, int cnt,
-                                               const float *f, const int *rowl, const float *Ma_l, float *gl, Scalars &sc,
-                                               int lane) {
+                                               const float *f, const int *rowl, const float *Ma_l, const float *smooth, float *gl,
+                                               Scalars &sc, int lane) {
   if (!changed) {
     const float sigma = sc.grad_scale, new_sigma = sigma - sc.alpha;
     float ratio = 0.0f;
@@ -238,34 +289,19 @@ __device__ __forceinline__ bool gradient_world(const NewtonArgs &a, int64_t w, c
     return true;
   }
   const int nv = a.nv;
-#ifndef IM_GRADIENT_ROWS
-#define IM_GRADIENT_ROWS 16
-#endif
-  constexpr int ROWS = IM_GRADIENT_ROWS;
-  for (int dof = lane; dof < nv; dof += 64) {
-    const float ma = Ma_l[dof], sm = a.smooth[w * nv + dof];
-    float sum = 0.0f;
-    // the next ROWS rows' elements are asked for before the current ones are added
-    float jv[ROWS], jn[ROWS];
-    auto fetch = [&](int p0, float (&v)[ROWS]) __attribute__((always_inline)) {
+  for (int d0 = lane; d0 - lane < nv; d0 += 64 * COLS) {
+    float sum[COLS];
+    constraint_force<COLS, RING, LAZY>(Jw, nv, cnt, f, rowl, d0, sum);
 #pragma unroll
-      for (int u = 0; u < ROWS; ++u) v[u] = Jw[(int64_t)rowl[p0 + u < cnt ? p0 + u : cnt - 1] * nv + dof];
-    };
-    if (AHEAD && cnt > 0) fetch(0, jv);
-    for (int p0 = 0; p0 < cnt; p0 += ROWS) {
-      if (!AHEAD) fetch(p0, jv);
-      if (AHEAD && p0 + ROWS < cnt) fetch(p0 + ROWS, jn);
-#pragma unroll
-      for (int u = 0; u < ROWS; ++u) sum = p0 + u < cnt ? fma_(jv[u], f[p0 + u], sum) : sum;
-      if (AHEAD) {
-#pragma unroll
-        for (int u = 0; u < ROWS; ++u) jv[u] = jn[u];
+    for (int k = 0; k < COLS; ++k) {
+      const int dof = d0 + 64 * k;
+      if (dof < nv) {
+        const float g = Ma_l[dof] - smooth[dof] - sum[k];
+        a.qfrc_constraint[w * nv + dof] = sum[k];
+        a.grad[w * a.ld_grad + dof] = g;
+        gl[dof] = g;
       }
     }
-    const float g = ma - sm - sum;
-    a.qfrc_constraint[w * nv + dof] = sum;
-    a.grad[w * a.ld_grad + dof] = g;
-    gl[dof] = g;
   }
   wave_sync();
   // grad . grad as a block of `block` lanes sums it: lane `rank` its dofs rank, rank + block, ..,
@@ -273,9 +309,11 @@ __device__ __forceinline__ bool gradient_world(const NewtonArgs &a, int64_t w, c
   float p = 0.0f;
   if (lane < a.block)
     for (int dof = lane; dof < nv; dof += a.block) p = fma_(gl[dof], gl[dof], p);
-  for (int off = 16; off > 0; off >>= 1) p = p + __shfl_down(p, off, 32);
-  float total = 0.0f + __shfl(p, 0, 64);
-  if (a.block > 32) total = total + __shfl(p, 32, 64);
+  float q = p;
+  search::swap_rows(p, q);  // the even rows of p + q: a row and the one behind it
+  p = search::row_sum(p + q);
+  float total = 0.0f + search::lane_of(p, 0);
+  if (a.block > 32) total = total + search::lane_of(p, 32);
   sc.grad_dot = uniform(total);
   sc.decrement = 0.0f;
   sc.grad_scale = 1.0f;
@@ -289,20 +327,19 @@ __device__ __forceinline__ bool gradient_world(const NewtonArgs &a, int64_t w, c
 }
 
 // ---- search . search and grad . x of a factor stage that leaves only the search direction -----
-__device__ __forceinline__ void search_sums_world(const NewtonArgs &a, int64_t w, const float *gl, Scalars &sc, int lane) {
+// (and the direction itself, for the next round's products)
+__device__ __forceinline__ void search_sums_world(const NewtonArgs &a, int64_t w, const float *gl, float *sv, Scalars &sc, int lane) {
   float s0 = 0.0f, s1 = 0.0f;
   for (int d = lane; d < a.nv && lane < a.block; d += a.block) {
-    const float v = -a.search[w * a.nv + d];
+    const float from = a.search[w * a.nv + d], v = -from;
+    sv[d] = from;
     s0 = fma_(v, v, s0);
     s1 = fma_(gl[d], v, s1);
   }
-  for (int o = 16; o > 0; o >>= 1) {
-    s0 = s0 + __shfl_down(s0, o, 32);
-    s1 = s1 + __shfl_down(s1, o, 32);
-  }
-  const float a1 = __shfl(s0, 32, 64), b1 = __shfl(s1, 32, 64);
-  float ra = 0.0f + __shfl(s0, 0, 64), rb = 0.0f + __shfl(s1, 0, 64);
-  if (a.block > 32) ra = ra + a1, rb = rb + b1;
+  search::swap_rows(s0, s1);  // s0 + s1: the first sum's rows 16 apart in the even rows, the second's in the odd ones
+  const float s = search::row_sum(s0 + s1);
+  float ra = 0.0f + search::lane_of(s, 0), rb = 0.0f + search::lane_of(s, 16);
+  if (a.block > 32) ra = ra + search::lane_of(s, 32), rb = rb + search::lane_of(s, 48);
   sc.search_dot = uniform(ra);
   sc.decrement = uniform(rb);
   if (lane == 0) {
@@ -311,15 +348,130 @@ __device__ __forceinline__ void search_sums_world(const NewtonArgs &a, int64_t w
   }
 }
 
+// ---- J search (newton_stages.py:157-178) beyond 64 dofs, on the matrix cores -------------------------
+// A row's sum is a chain of multiply-adds over the dofs in order, beyond 50 dofs in parts of 20 that are
+// added up.  v_mfma_f32_16x16x4_f32 adds its four products one after the other, so sixteen rows' chains run four
+// dofs per instruction: lane (g, c) = (lane / 16, lane % 16) supplies J[row c][dof 4 q + g] and search[4 q + g]; every
+// column of the result is the rows' sums.  A step is 64 rows x 16 dofs: per sixteen rows a lane loads four neighbouring
+// dofs of a row, which four lane swaps turn into the operands of four instructions.  Four steps are on their way at
+// once (16 registers a lane each): what bounds the product is the trip to memory, J being read once per
+// round.  With the row of M staged (below), M v and J v of a round at 70 dofs x 2048 worlds: 22.4 -> 14 us.
+// `between` runs while the first steps are on their way and leaves the search direction in sv.
+typedef float v4 __attribute__((ext_vector_type(4)));
+typedef v4 v4_words __attribute__((aligned(4)));
+// (the wait states written out: the compiler's builtins return one result twice when both operands hold the same value)
+__device__ __forceinline__ void turn_groups(float &r0, float &r1, float &r2, float &r3) {
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1\n\t"
+      "v_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
+      : "+v"(r0), "+v"(r1), "+v"(r2), "+v"(r3));
+}
+template <class Between>
+__device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, int nefc, const float *sv, float *jv,
+                                         float *jv_lds, int lane, Between &&between) {
+  const int nv = a.nv, g = lane >> 4, c = lane & 15;
+  if (nefc <= 0) return between();
+  const bool split = nv > 50;
+  struct Step {
+    int r0, c0;
+  };
+  // (not behind a branch, the last row's again past the end: a wait for one step's loads counts those of the next)
+  auto fetch = [&](const Step &s, v4 (&v)[4]) __attribute__((always_inline)) {
+    const int col = s.c0 + 4 * g, from = col < nv - 4 ? col : nv - 4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = s.r0 + 16 * t + c;
+      const char *at = (const char *)Jw + 4u * (uint32_t)((row < nefc ? row : nefc - 1) * nv + from);
+      v[t] = *(const v4_words *)at;
+    }
+  };
+  auto advance = [&](Step &s) __attribute__((always_inline)) {
+    s.c0 += 16;
+    if (s.c0 >= nv) s.c0 = 0, s.r0 += 64;
+  };
+  Step now = {0, 0}, ahead = {0, 0};
+  constexpr int DEPTH = 4;
+  v4 v[DEPTH][4];
+#pragma unroll
+  for (int b = 0; b < DEPTH; ++b) fetch(ahead, v[b]), advance(ahead);
+  between();
+  v4 p[4] = {};
+  float sum = 0.0f;  // of the row that this lane puts out: register u of group t of row 16 t + 4 g + u, the same in all
+                     // columns; lane (g, c) takes row 16 (c / 4) + 4 g + c % 4
+  auto take = [&]() __attribute__((always_inline)) {
+    float part = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) part = c == 4 * t + u ? p[t][u] : part;
+      p[t] = v4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    sum = sum + part;
+  };
+  auto work = [&](v4 (&v)[4]) __attribute__((always_inline)) {
+    const int col = now.c0 + 4 * g;
+    float x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = now.c0 + 4 * q + g < nv ? sv[now.c0 + 4 * q + g] : 0.0f;
+    if (now.c0 + 16 > nv) {  // the row's last dofs were loaded from four before its end: moved down, zeros behind them
+      const int by = col + 4 - nv;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (t > 0 && now.r0 + 16 * t >= nefc) continue;
+        v4 m = v[t];
+        m = by >= 1 ? v4{m[1], m[2], m[3], 0.0f} : m;
+        m = by >= 2 ? v4{m[1], m[2], 0.0f, 0.0f} : m;
+        m = by >= 3 ? v4{m[1], 0.0f, 0.0f, 0.0f} : m;
+        v[t] = by >= 4 ? v4{0.0f, 0.0f, 0.0f, 0.0f} : m;
+      }
+    }
+    float e[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (t > 0 && now.r0 + 16 * t >= nefc) continue;
+      e[t][0] = v[t][0], e[t][1] = v[t][1], e[t][2] = v[t][2], e[t][3] = v[t][3];
+      turn_groups(e[t][0], e[t][1], e[t][2], e[t][3]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (split && (now.c0 + 4 * q) % 20 == 0) take();
+      if (q == 0 || now.c0 + 4 * q < nv) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (t == 0 || now.r0 + 16 * t < nefc) p[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[t][q], x[q], p[t], 0, 0, 0);
+      }
+    }
+    if (now.c0 + 16 >= nv) {
+      take();
+      const int row = now.r0 + 16 * (c >> 2) + 4 * g + (c & 3);
+      if (row < nefc) {
+        if (jv) jv[row] = sum;
+        jv_lds[row] = sum;
+      }
+      sum = 0.0f;
+    }
+    advance(now);
+  };
+  for (;;) {
+#pragma unroll
+    for (int b = 0; b < DEPTH; ++b) {
+      work(v[b]);
+      if (now.r0 >= nefc) return;
+      fetch(ahead, v[b]);
+      advance(ahead);
+    }
+  }
+}
+
 // ---- J search through a tile of 64 rows x 16 dofs (4.3 KB of LDS whatever the width of J) ------
-// The same chain per row as jv_world: the dofs in order, the 20-dof partial sums of the reference's
-// rule beyond 50 dofs.  A lane loads 16 elements per tile, four rows of 64 bytes per instruction.
-// AHEAD: the next tile's elements are asked for while the current one is worked on (sixteen more
-// registers a lane).  WIDE: a tile row's operands are read eight at a time ahead of their part of
-// the chain (sixteen more again).
-template <bool AHEAD, bool WIDE>
+// ---- J search up to 64 dofs ------------------------------------------------------------------------
+// The same chains through a tile of 64 rows x 16 dofs in LDS (kTileWords) and on a lane per row: the
+// operands' way into the matrix cores takes more instructions, and where the chip is full of worlds it is the slower
+// form (27 dofs x 4096 worlds 259 us per solve against 250; 56 x 4096 768 against 740).  A lane loads 16 elements per
+// tile, four rows of 64 bytes per instruction; the next tile's elements are asked for while the current one is worked
+// on.  WIDE: a tile row's operands are read eight at a time ahead of their part of the chain (sixteen registers).
+template <bool WIDE, class Between>
 __device__ __forceinline__ void jv_world_tiled(const NewtonArgs &a, const float *Jw, int nefc, float *tile,
-                                               const float *sv, float *jv, float *jv_lds, int lane) {
+                                               const float *sv, float *jv, float *jv_lds, int lane, Between &&between) {
   const int nv = a.nv;
   const int c = lane & 15, rq = lane >> 4;
   const bool split = nv > 50;
@@ -334,19 +486,20 @@ __device__ __forceinline__ void jv_world_tiled(const NewtonArgs &a, const float 
     }
   };
   float v[16];
-  if (AHEAD && nefc > 0) fetch(0, 0, v);
+  if (nefc > 0) fetch(0, 0, v);
+  between();
+  wave_sync();  // (a staged row of M has the tile's place until here)
   for (int r0 = 0; r0 < nefc; r0 += 64) {
     const int rows = nefc - r0 < 64 ? nefc - r0 : 64;
     float acc = 0.0f, p = 0.0f;
     for (int c0 = 0; c0 < nv; c0 += 16) {
       const int cw = nv - c0 < 16 ? nv - c0 : 16;
-      if (!AHEAD) fetch(r0, c0, v);
 #pragma unroll
       for (int k = 0; k < 16; ++k) tile[(rq + 4 * k) * 17 + c] = v[k];
       wave_sync();
       const bool more_columns = c0 + 16 < nv;
       const int next_r0 = more_columns ? r0 : r0 + 64, next_c0 = more_columns ? c0 + 16 : 0;
-      if (AHEAD && next_r0 < nefc) fetch(next_r0, next_c0, v);
+      if (next_r0 < nefc) fetch(next_r0, next_c0, v);
       if (lane < rows) {
         // a tile row's operands are read eight at a time before their part of the chain (two waits
         // per tile, not sixteen)
@@ -359,23 +512,24 @@ __device__ __forceinline__ void jv_world_tiled(const NewtonArgs &a, const float 
             }
             p = fma_(row[i], sv[c0 + i], p);
           }
-        } else
+        } else {
+          // the column, one of every four, ahead of which a part of 20 ends; and columns past the last dof, of which the
+          // products are dropped by a lane's own comparison (as scalars sixteen conditions are more than there is room for)
+          int part = split ? (c0 + 19) / 20 * 20 - c0 : 16, columns = cw;
+          part = c0 + part == 0 || part >= cw ? 16 : part;
+          asm volatile("" : "+v"(columns));
 #pragma unroll
-        for (int h = 0; h < 16; h += 8) {
-          float x[8], y[8];
+          for (int h = 0; h < 16; h += 8) {
+            float x[8], y[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            x[i] = row[h + i];
-            y[i] = sv[c0 + (h + i < cw ? h + i : 0)];
-          }
+            for (int i = 0; i < 8; ++i) x[i] = row[h + i], y[i] = sv[c0 + (h + i < cw ? h + i : 0)];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            if (h + i < cw) {  // the same for every lane
-              if (split && (c0 + h + i) % 20 == 0 && c0 + h + i > 0) {
+            for (int i = 0; i < 8; ++i) {
+              if (i % 4 == 0 && part == h + i) {
                 acc = acc + p;
                 p = 0.0f;
               }
-              p = fma_(x[i], y[i], p);
+              p = h + i < columns ? fma_(x[i], y[i], p) : p;
             }
           }
         }
@@ -406,17 +560,17 @@ struct LoopLds {
   // per wavefront, used within a round (may share one area with the factor stage's own arrays):
   float *f;              // [njmax] forces of the listed rows
   int *rowl;             // [njmax] their numbers
-  float *gl;             // [nv] the gradient (a cooperative stage's loop reads it again after the stage)
-  float *rows;           // staged rows of J: 64 x (nv | 1), or the 64 x 17 tile
+  float *gl;             // [nv] qfrc_smooth, from the products to the gradient; then the gradient (a cooperative stage's loop
+                         // reads it again after the stage)
+  float *rows;           // kTileWords: the world's row of M on its way into the product
 };
 
 // A world's vectors stay in LDS and its scalars in registers from round to round; memory receives
 // every value as it is produced (the arrays end as after the stage launches) and is read again only
 // for what another wavefront or the factor stage has written there.
 // HELD: rows of a world a lane keeps in registers during the line search (0: read from LDS at every
-// evaluation); JU: loads in flight per lane while rows of J are staged, 0 for the tiled staging
-// with the next tile asked for ahead and a tile row's operands read eight at a time, -2 with the
-// first of the two only, -1 with neither (each costs sixteen registers a lane).
+// evaluation).  COLS: dofs of a lane in the gradient (2 beyond 64).  WIDE:
+// registers to spare for operands read ahead.
 // COOP: `stage()` works on the workgroup's four worlds together (every wavefront calls it in step,
 // between two workgroup barriers; it takes the worlds' numbers from L.worlds and skips the worlds
 // whose `unchanged` byte is set).  A wavefront whose world is done takes the next world from the
@@ -441,7 +595,7 @@ __device__ __forceinline__ const NewtonArgs &kernel_args(int kernarg_offset) {
 
 // MLDS: the world's row of M is kept in LDS (where L.m_lds is not null); otherwise `M search` reads it from memory
 // every round, which leaves the LDS to more worlds per CU.
-template <int HELD, int JU, bool COOP, bool MLDS = true, class Stage>
+template <int HELD, int COLS, bool WIDE, bool COOP, bool MLDS = true, class Stage>
 __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L, int64_t w_raw, Stage &&stage) {
   const NewtonArgs &a0 = kernel_args(kernarg_offset);
   const NewtonArgs &a = a0;
@@ -484,6 +638,7 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
       L.Ma[k] = a.Ma[w * nv + k];
       L.mv[k] = a.mv[w * nv + k];
       L.qacc[k] = a.qacc[w * nv + k];
+      L.sv[k] = a.search[w * nv + k];
     }
     for (int r = lane_fixed; r < njmax; r += 64) {
       L.Jaref[r] = a.Jaref[w * njmax + r];
@@ -494,7 +649,7 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
     if (COOP && a.sums_at_enter) {
       for (int k = lane_fixed; k < nv; k += 64) L.gl[k] = a.grad[w * a.ld_grad + k];
       wave_sync();
-      search_sums_world(a, w, L.gl, sc, lane_fixed);
+      search_sums_world(a, w, L.gl, L.sv, sc, lane_fixed);
     }
     wave_sync();
   };
@@ -538,19 +693,36 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
     asm volatile("" : "+v"(lane));
     IM_STAMP(0);
     if (!done) {
+      // qfrc_smooth on its way during the products, which may use its place in LDS
+      float smooth[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) smooth[k] = a.smooth[w * nv + (lane + 64 * k < nv ? lane + 64 * k : 0)];
       if (!unchanged) {
-        for (int k = lane; k < nv; k += 64) L.sv[k] = a.search[w * nv + k];
-        wave_sync();
-        mul_m_world(a, L.term, L.radr, (MLDS && L.m_lds) ? (const float *)L.m_lds : a.M + w * a.ldM, L.sv, a.mv + w * nv, L.mv, lane);
-        if constexpr (JU > 0)
-          jv_world<(JU > 0 ? JU : 1)>(a, Jw, nefc, L.rows, L.sv, a.jv + w * njmax, L.jv, lane);
+        auto m_search = [&]() __attribute__((always_inline)) {
+          if (MLDS && L.m_lds)
+            mul_m_world<COLS == 2>(a, L.term, L.radr, L.m_lds, L.sv, a.mv + w * nv, L.mv, lane);
+          else
+            mul_m_world_staged<COLS == 2, WIDE ? 12 : 8>(a, L.term, L.radr, a.M + w * a.ldM, L.sv, a.mv + w * nv, L.mv, L.rows, lane);
+        };
+        if constexpr (COLS == 2)
+          jv_world(a, Jw, nefc, L.sv, a.jv + w * njmax, L.jv, lane, m_search);
         else
-          jv_world_tiled<(JU == 0 || JU == -2), (JU == 0)>(a, Jw, nefc, L.rows, L.sv, a.jv + w * njmax, L.jv, lane);
+          jv_world_tiled<WIDE>(a, Jw, nefc, L.rows, L.sv, a.jv + w * njmax, L.jv, lane, m_search);
         wave_sync();
       }
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        if (lane + 64 * k < nv) L.gl[lane + 64 * k] = smooth[k];
+      for (int k = lane + 128; k < nv; k += 64) L.gl[k] = a.smooth[w * nv + k];
+      wave_sync();
       IM_STAMP(1);
+      // the rows' states before the step, on their way during the line search
+      constexpr int kBefore = HELD == 2 ? 1 : 2;  // (two held rows a lane: 64 rows)
+      int before[kBefore];
+#pragma unroll
+      for (int k = 0; k < kBefore; ++k) before[k] = a.state[w * njmax + (lane + 64 * k < nefc ? lane + 64 * k : 0)];
       // (the force list and the row list of the gradient are free until the step is taken)
-      const search::LsWorld lw{a.smooth + w * nv, L.D, L.fl, L.Jaref, L.sv, L.mv, L.jv, L.Ma, sc.search_dot, tolerance,
+      const search::LsWorld lw{L.gl, L.D, L.fl, L.Jaref, L.sv, L.mv, L.jv, L.Ma, sc.search_dot, tolerance,
                                ls_tolerance, meaninertia, ne, nf, nefc, nv, a.ls_iterations, L.f, (float *)L.rowl};
       const search::LsResult ls = search::linesearch_rows<HELD, true>(lw, lane & 31);  // both halves on this world
       sc.alpha = uniform(ls.alpha), sc.improvement = uniform(ls.improvement);
@@ -590,7 +762,7 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
           } else if (r >= ne && x >= 0.0f) {
             f = 0.0f, st = 0;
           }
-          const int old = a.state[w * njmax + r];
+          const int old = base == 0 ? before[0] : base < 64 * kBefore ? before[kBefore - 1] : a.state[w * njmax + r];
           a.force[w * njmax + r] = f;
           a.state[w * njmax + r] = st;
           quad_flip = (old == 1) != (st == 1);
@@ -619,7 +791,7 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
       }
       wave_sync();
       IM_STAMP(3);
-      unchanged = gradient_world<(JU == 0 || JU == -2)>(a, w, Jw, nstate != 0, cnt, L.f, L.rowl, L.Ma, L.gl, sc, lane);
+      unchanged = gradient_world<COLS, COLS == 2 ? 4 : 2, COOP>(a, w, Jw, nstate != 0, cnt, L.f, L.rowl, L.Ma, L.gl, L.gl, sc, lane);
       IM_STAMP(4);
     }
     if (COOP) {
@@ -639,10 +811,12 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
       const NewtonArgs &a = kernel_args(kernarg_offset);
       if (!unchanged) {
         if (COOP) {
-          search_sums_world(a, w, L.gl, sc, lane);
-        } else {  // the stage has left the two sums in memory
-          sc.search_dot = uniform(a.search_dot[w]);
-          sc.decrement = uniform(a.decrement[w]);
+          search_sums_world(a, w, L.gl, L.sv, sc, lane);
+        } else {  // the stage has left the direction and the two sums in memory: one trip for all
+          const float dot = a.search_dot[w], decrement = a.decrement[w];
+          for (int k = lane; k < nv; k += 64) L.sv[k] = a.search[w * nv + k];
+          sc.search_dot = uniform(dot);
+          sc.decrement = uniform(decrement);
         }
       }
       // newton_fusion.py:265-296
@@ -701,7 +875,7 @@ __device__ __forceinline__ LoopLds coop_layout(const NewtonArgs &a, float *lds) 
   L.f = L.fl + njmax;
   L.rowl = (int *)(L.f + njmax);
   L.gl = (float *)(L.rowl + njmax);
-  L.rows = lds + wv * (64 * 17);
+  L.rows = lds + wv * kTileWords;
   for (int k = threadIdx.x; k < a.nterm; k += blockDim.x) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
   for (int k = threadIdx.x; k <= nv; k += blockDim.x) radr[k] = a.mulm_rowadr[k];
   return L;

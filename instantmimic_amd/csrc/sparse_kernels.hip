@@ -945,7 +945,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
   resident::LoopLds L;
   L.votes = nullptr;
   L.term = term, L.radr = radr;
-  L.rows = mine;  // the shared area: tile of J, then the gradient's lists, then the stage
+  L.rows = mine;  // the shared area: M's row, the tile of J, then the gradient's lists, then the stage
   L.f = mine;
   L.rowl = (int *)(mine + njmax);
   L.gl = mine + 2 * njmax;
@@ -975,8 +975,8 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
                         (int)b.ld_grad, U_, uni_, b.search, b.search_dot, b.decrement, (int)w, threadIdx.x & 63);
   };
   while (w < nworld) {
-    // HELD: the rows a lane keeps in registers during the line search; the next tile of J is asked for ahead
-    resident::newton_loop<HELD, -2, false, false>(kArgsOffset, L, w, stage);
+    // HELD: the rows a lane keeps in registers during the line search
+    resident::newton_loop<HELD, 1, WAVES == 12 || WAVES == 8 || HELD == 0, false, false>(kArgsOffset, L, w, stage);
     int next = 0;
     if ((threadIdx.x & 63) == 0) next = atomicAdd(next_world, 1);
     w = __builtin_amdgcn_readfirstlane(next);

@@ -478,7 +478,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_dense_tile_resi
   L.votes = nullptr;
   L.worlds = nullptr;
   L.term = term, L.radr = radr;
-  L.rows = mine;  // the shared area: tile of J, then the gradient's lists, then the stage's tile
+  L.rows = mine;  // the shared area: M's row, the tile of J, then the gradient's lists, then the stage's tile
   L.f = mine;
   L.rowl = (int *)(mine + njmax);
   L.gl = mine + 2 * njmax;
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_dense_tile_resi
   // as many wavefronts as the chip keeps resident; one whose world is done takes the next world
   // nobody has started (a counter in memory that only grows: every wavefront reaches the end)
   while (w < nworld) {
-    resident::newton_loop<HELD, -2, false, false>(0, L, w, stage);
+    resident::newton_loop<HELD, 1, true, false, false>(0, L, w, stage);
     int next = 0;
     if ((threadIdx.x & 63) == 0) next = atomicAdd(next_world, 1);
     w = __builtin_amdgcn_readfirstlane(next);
