@@ -910,7 +910,7 @@ def generate(name, rowadr, rownnz, colind, groups, trunk, *, module: bool = Fals
     emit("        (int64_t)a.nv, nullptr, a.nworld, IM_FLAG_NEGATE, 1, 0, 0, 0, a.unchanged, worlds);")
     emit("  };")
     emit("  const im::resident::LoopLds L = im::resident::coop_layout(a, xlds);")
-    emit("  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);")
+    emit("  const int64_t w = im::resident::first_world(a, threadIdx.x >> 6);")
     emit("  im::resident::block_sync();")
     # rows a lane keeps in registers during the line search: two up to 64 rows, four up to 128 (the
     # same for the whole launch), beyond that the rows are read from LDS at every evaluation

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(64 * WAVES, NB == 5 ? 3 : 4) void newton_dense_wave
   for (int k = tid; k < a.nterm; k += 64 * WAVES) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
   for (int k = tid; k <= nv; k += 64 * WAVES) radr[k] = a.mulm_rowadr[k];
   __syncthreads();  // the only workgroup barrier
-  int64_t w = (int64_t)blockIdx.x * WAVES + wv;
+  int64_t w = resident::first_world(a, wv);
   auto stage = [&]() __attribute__((always_inline)) {
     const resident::NewtonArgs &b = resident::kernel_args(0);  // the kernel's first parameter
     int lane = threadIdx.x & 63;
@@ -260,8 +260,7 @@ int newton_solve_dense_column(const im_newton_args *p, float *H, float *U, int32
     int per_cu = 0;
     if (const int st = resident_per_cu(v.fn, nullptr, 64 * v.waves, lds, &per_cu)) return st;
     per_cu = std::max(1, per_cu);
-    const int needed = (p->nworld + v.waves - 1) / v.waves;
-    const int grid = std::min(needed, ncu * per_cu);
+    const int grid = resident_worlds_grid(p->nworld, v.waves, ncu, per_cu, false, &a.group_worlds);
     if (before) {
       a.final_force = 1;
       if (const int st = (*before)(next_world, grid * v.waves)) return st;

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <cstdint>
 
@@ -62,6 +63,29 @@ int usable_variants(Kept<int, std::array<bool, N>> &kept, const Variant (&varian
     for (size_t i = 0; i < N; ++i) u[i] = usable_resident(variants[i].fn);
     return (int)IM_OK;
   }, usable);
+}
+// Workgroups of a resident loop over nworld worlds, up to `waves` of them to a workgroup and `per_cu` workgroups to a CU,
+// and the worlds that each starts with: a batch smaller than the chip is spread over its compute units and SIMDs.
+// Neighbours in a workgroup are worlds next to one another (70 dofs x 2048 worlds with a workgroup's worlds 512 apart,
+// so that their matrices share memory channels: 906 us per solve against 819), and every CU gets as many (683
+// workgroups of three on 256 CUs: 890 us).  `together` (the tree kernels): a workgroup's wavefronts work on its worlds'
+// factors in step, so a second workgroup on a CU does that work twice (35 dofs x 700 worlds, a world each: 217 us
+// against 210): only behind full ones.  Full workgroups always, and now: sparse 35 dofs x 500 worlds 452 -> 420 us,
+// dense 27 x 1000 304 -> 273, tree 27 x 64 174 -> 164.
+inline int resident_worlds_grid(int nworld, int waves, int ncu, int per_cu, bool together, int *group_worlds) {
+  const int each = (int)(((int64_t)nworld + ncu - 1) / ncu);  // worlds of a CU
+  int k = waves;
+  if (together) {
+    k = std::min(waves, each);
+  } else if (each < waves * per_cu) {  // the fewest places for them, in the largest workgroups
+    for (int m = 1, places = waves * per_cu; m <= per_cu; ++m) {
+      const int of_m = (each + m - 1) / m;
+      if (of_m <= waves && of_m * m < places) k = of_m, places = of_m * m;
+    }
+  }
+  k = std::max(1, k);
+  *group_worlds = k;
+  return (int)std::min<int64_t>((int64_t)ncu * per_cu, ((int64_t)nworld + k - 1) / k);
 }
 // *counter = value, as a launch
 void set_counter(int *counter, int value, hipStream_t stream);

@@ -56,6 +56,8 @@ struct NewtonArgs {
   // ... and (cooperative loop) forms the two sums of the first search direction as it enters, which
   // a launch of their own would leave in memory
   int sums_at_enter;
+  // the worlds that a workgroup starts with, its first wavefronts' (resident_worlds_grid)
+  int group_worlds;
 };
 
 // The public argument block checked and turned into the kernels' (host side).
@@ -94,6 +96,7 @@ inline int convert_args(const im_newton_args &p, int nv, int nM, NewtonArgs &a) 
   a.m_lds = 1;
   a.final_force = 0;
   a.sums_at_enter = 0;
+  a.group_worlds = 1;
   return IM_OK;
 }
 
@@ -101,6 +104,11 @@ __device__ __forceinline__ float fma_(float a, float b, float c) { return __buil
 // a value every lane holds alike, as a scalar (so that it occupies no vector register while it waits)
 __device__ __forceinline__ float uniform(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+// the world that a workgroup's wavefront `wv` starts with; nworld: none
+__device__ __forceinline__ int64_t first_world(const NewtonArgs &a, int wv) {
+  return wv < a.group_worlds ? (int64_t)blockIdx.x * a.group_worlds + wv : a.nworld;
 }
 
 // orders this wavefront's writes (LDS and memory) before its later reads: the stages hand their

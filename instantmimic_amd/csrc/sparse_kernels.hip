@@ -965,7 +965,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
   // takes the next world nobody has started (a counter in memory, set to the grid's wavefront count
   // before the launch), so the worlds that need many iterations do not hold idle neighbours in
   // place.  The counter only grows: every wavefront reaches the end of the batch.
-  int64_t w = (int64_t)blockIdx.x * WAVES + wv;
+  int64_t w = resident::first_world(a, wv);
   // NewtonArgs is the kernel's second parameter, behind the plan's block
   constexpr int kArgsOffset = (int)((sizeof(SparseWave) + alignof(resident::NewtonArgs) - 1) / alignof(resident::NewtonArgs) *
                                     alignof(resident::NewtonArgs));
@@ -1427,8 +1427,7 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
     int ncu = 0;
     if (const int st = compute_units(&ncu)) return st;
     const int per_cu = std::max(1, std::min((int)(160 * 1024 / lds), 16 / waves));
-    const int needed = (p->nworld + waves - 1) / waves;
-    const int grid = std::min(needed, ncu * per_cu);
+    const int grid = resident_worlds_grid(p->nworld, waves, ncu, per_cu, false, &a.group_worlds);
     int *counter = plan->next_world;
     if (before) {
       a.final_force = 1;

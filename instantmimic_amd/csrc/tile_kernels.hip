@@ -494,7 +494,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_dense_tile_resi
   for (int k = tid; k < a.nterm; k += 64 * WAVES) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
   for (int k = tid; k <= nv; k += 64 * WAVES) radr[k] = a.mulm_rowadr[k];
   __syncthreads();  // the only workgroup barrier
-  int64_t w = (int64_t)blockIdx.x * WAVES + wv;
+  int64_t w = resident::first_world(a, wv);
   auto stage = [&]() __attribute__((always_inline)) {
     const resident::NewtonArgs &b = resident::kernel_args(0);  // the kernel's first parameter
     int lane = threadIdx.x & 31;
@@ -669,8 +669,7 @@ int newton_solve_dense_tile(const im_newton_args *p, float *H, int32_t *dof_unio
     if (const int st = compute_units(&ncu)) return st;
     // as many workgroups as stay resident at once (LDS, and sixteen wavefronts of up to 128 registers per CU)
     const int per_cu = std::max(1, std::min((int)(160 * 1024 / lds), 16 / v.waves));
-    const int needed = (p->nworld + v.waves - 1) / v.waves;
-    const int grid = std::min(needed, ncu * per_cu);
+    const int grid = resident_worlds_grid(p->nworld, v.waves, ncu, per_cu, false, &a.group_worlds);
     if (before) {
       a.final_force = 1;
       if (const int st = (*before)(next_world, grid * v.waves)) return st;

@@ -824,10 +824,9 @@ int newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, hipStre
   }
   int ncu = 0;
   if (const int st = compute_units(&ncu)) return st;
-  const int needed = (p->nworld + 3) / 4;
-  const unsigned grid = (unsigned)std::min(needed, std::max(1, per_cu) * ncu);
+  const unsigned grid = (unsigned)resident_worlds_grid(p->nworld, 4, ncu, std::max(1, per_cu), true, &a.group_worlds);
   // (a batch that is resident all at once has nothing to hand out)
-  if ((int)grid < needed) a.next_world = plan->next_world;
+  if ((int64_t)grid * 4 < p->nworld) a.next_world = plan->next_world;
   if (before) {
     a.final_force = a.sums_at_enter = 1;
     if (const int st = (*before)(a.next_world, (int)grid * 4)) return st;

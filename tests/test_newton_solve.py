@@ -163,6 +163,19 @@ def test_gpu_solve_from_init_context_matches_the_oracle_chain(device, monkeypatc
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nworld", [1, 5, 257, 514, 1025])
+@pytest.mark.parametrize("name,stage", [("ant", "tree"), ("ant", "dense"), ("g1", "tree"), ("g1", "sparse"), ("g1", "dense")])
+def test_gpu_solve_of_batches_that_do_not_fill_the_chip(device, name, stage, nworld):
+    """A resident loop's workgroups start with as many worlds as spread the batch over the compute units: one world,
+    fewer than units, one and two more than a multiple of them, and more than four a unit."""
+    p = NC.problem(name, nworld, stage, empty_every=13, maxiter=6)
+    s = NC.oracle_solve(p)
+    m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
+    NC.compare(p, s, d, ctx)
+    assert int(nsolving.item()) == int((p.nefc == 0).sum() + ((p.nefc > 0) & (s.done == 0)).sum())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name,nworld,stage", [("humanoid", 301, "tree"), ("g1", 203, "sparse"), ("snu", 131, "tree"), ("ant", 67, "dense"),
                                                ("humanoid", 299, "dense"), ("g1", 201, "dense"), ("snu", 129, "dense")])  # fmt: skip
 def test_gpu_init_context_in_one_launch_leaves_what_the_five_launches_leave(device, monkeypatch, name, nworld, stage):
