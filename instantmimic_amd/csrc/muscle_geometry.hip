@@ -305,7 +305,11 @@ __device__ __forceinline__ void stage_row(float *to, const float *__restrict__ f
   }
 }
 
-template <int nt>
+// AHEAD: a thread holds its share of the next world's rows in registers while it works on this one's (rows of up to 14
+// floats a thread of waypoints, nine of moments, one of velocities: every rig whose muscles have the threads they ask
+// for; wider rows are fetched when the world before is done with).  A workgroup's trip to memory was in front of its
+// two other phases: 4096 worlds of 284 muscles 48.5 -> 43.3 us, implicit terms of 300 muscles x 8192 worlds 315 -> 303.
+template <int nt, bool AHEAD>
 __global__ __launch_bounds__(nt) void force_velocity_state_world_kernel(
     const float *__restrict__ wp, int64_t ldw, const int32_t *__restrict__ waypoint_start,
     const float *__restrict__ params, int ldpar, const float *__restrict__ rest,
@@ -338,11 +342,44 @@ __global__ __launch_bounds__(nt) void force_velocity_state_world_kernel(
   for (int o = 32; o; o >>= 1) most = max(most, __shfl_xor(most, o));
   if ((tid & 63) == 0) atomicMax(named, most);
   for (int m = tid; m < nmuscle; m += nt) cosp[m] = cosf(params[m * ldpar + 3]);
+  constexpr int kPoints = AHEAD ? 14 : 1, kEntries = AHEAD ? 9 : 1;
+  float points[kPoints], entries[kEntries], speed = 0.0f;
+  int nq = 0;
+  auto hold = [&](int64_t w) __attribute__((always_inline)) {
+    int t = tid;
+    asm volatile("" : "+v"(t));  // (no address is kept from world to world)
+    const float *pw = wp + w * ldw, *mw = moment + w * ldm;
+#pragma unroll
+    for (int k = 0; k < kPoints; ++k)
+      if (t + k * nt < 3 * nwp) points[k] = pw[(unsigned)(t + k * nt)];
+#pragma unroll
+    for (int k = 0; k < kEntries; ++k)
+      if (t + k * nt < ne) entries[k] = mw[(unsigned)(t + k * nt)];
+    if (t < nq) speed = qvel[w * ldq + t];
+  };
+  if (AHEAD) {
+    __syncthreads();
+    nq = min(__builtin_amdgcn_readfirstlane(*named), n.nqvel);
+    hold(blockIdx.x);
+  }
   for (int64_t w = blockIdx.x; w < nworld; w += gridDim.x) {
     __syncthreads();  // the tables are there, the world before is done with
-    stage_row<nt>(row, wp + w * ldw, 3 * nwp, tid);
-    stage_row<nt>(mom, moment + w * ldm, ne, tid);
-    stage_row<nt>(qv, qvel + w * ldq, min(__builtin_amdgcn_readfirstlane(*named), n.nqvel), tid);
+    if constexpr (AHEAD) {
+      int t = tid;
+      asm volatile("" : "+v"(t));
+#pragma unroll
+      for (int k = 0; k < kPoints; ++k)
+        if (t + k * nt < 3 * nwp) row[t + k * nt] = points[k];
+#pragma unroll
+      for (int k = 0; k < kEntries; ++k)
+        if (t + k * nt < ne) mom[t + k * nt] = entries[k];
+      if (t < nq) qv[t] = speed;
+      if (w + gridDim.x < nworld) hold(w + gridDim.x);
+    } else {
+      stage_row<nt>(row, wp + w * ldw, 3 * nwp, tid);
+      stage_row<nt>(mom, moment + w * ldm, ne, tid);
+      stage_row<nt>(qv, qvel + w * ldq, min(__builtin_amdgcn_readfirstlane(*named), n.nqvel), tid);
+    }
     __syncthreads();
     for (int i = tid; i < nwp - 1; i += nt) dist[i] = length(sub(ld3(row + 3 * (i + 1)), ld3(row + 3 * i)));
     __syncthreads();
@@ -1228,10 +1265,10 @@ extern "C" int im_muscle_force_velocity_state(
     int ncu = 0;
     if (const int st = compute_units(&ncu)) return st;
     const int threads = nworld <= 4 * ncu ? 320 : std::min(std::max((nmuscle + 63) / 64 * 64, 128), 320);
-    auto kernel = threads == 128   ? force_velocity_state_world_kernel<128>
-                  : threads == 192 ? force_velocity_state_world_kernel<192>
-                  : threads == 256 ? force_velocity_state_world_kernel<256>
-                                   : force_velocity_state_world_kernel<320>;
+    const bool ahead = n.words_wp <= 14 * threads && n.nentry <= 9 * threads && n.nqvel <= threads;
+#define IM_FV(NT) (ahead ? force_velocity_state_world_kernel<NT, true> : force_velocity_state_world_kernel<NT, false>)
+    auto kernel = threads == 128 ? IM_FV(128) : threads == 192 ? IM_FV(192) : threads == 256 ? IM_FV(256) : IM_FV(320);
+#undef IM_FV
     if (n.bytes() > 64 * 1024)
       IM_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, n.bytes()));
     unsigned grid = 0;
