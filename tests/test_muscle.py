@@ -114,6 +114,34 @@ def test_gpu_matches_oracle_bitwise(device, nworld):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nworld", [2047, 2048, 2049])
+@pytest.mark.parametrize("nmuscle", [40, 420, 1100])
+def test_gpu_gather_of_two_worlds_a_workgroup(device, nmuscle, nworld):
+    """Both sides of the batch from which a workgroup takes two worlds, with a world left over, on 256 and on 512 threads and
+    where two worlds do not fit: the oracle's bits, and the columns beside the matrix stay as they are."""
+    import torch
+
+    mb = synth.make_muscles(nworld, nmuscle=nmuscle, seed=5)
+    rowadr, rownnz, colind = synth.csr_from_parents(synth.snu_parents())
+    ent = Q.entries_from_muscle_dofs(mb.muscle_dofs, mb.nmuscle)
+    prepared = Q.prepare_muscle_implicit_qderiv_pairs(
+        pair_entry_i=ent.pair_entry_i, pair_entry_j=ent.pair_entry_j, pair_muscle_idx=ent.pair_muscle_idx,
+        muscle_dof_torque_idx=ent.muscle_dof_torque_idx, matrix_elemid=synth.matrix_elemid(rowadr, rownnz, colind),
+        root_dof_count=mb.root_dof_count,
+    )  # fmt: skip
+    gather = Q.build_muscle_implicit_qderiv_gather(prepared, ent.muscle_dof_muscle_idx, device)
+    q0 = np.random.default_rng(3).normal(size=(nworld, len(colind))).astype(np.float32)
+    wide = torch.full((nworld, len(colind) + 3), 7.0, device=device)
+    wide[:, :-3] = torch.from_numpy(q0).to(device)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    Q.apply_muscle_implicit_qderiv_gather(gather, t(mb.moment), t(mb.slope), mb.timestep, wide[:, :-3])
+    tables = Q.gather_tables(prepared, ent.muscle_dof_muscle_idx)
+    want = R.muscle_implicit_gather(mb.moment, mb.slope, ent.muscle_dof_muscle_idx, tables[0], tables[1], tables[2], tables[4], mb.timestep, q0)
+    np.testing.assert_array_equal(wide[:, :-3].cpu().numpy(), want)
+    assert (wide[:, -3:] == 7.0).all()
+
+
+@pytest.mark.gpu
 def test_gpu_projection_with_more_entries_than_one_staging_trip(device):
     """420 muscles give about 1900 entries: several of a thread's twelve places stay empty in the
     projection kernel's trip through LDS (the sizes beyond one trip are tested below)."""
