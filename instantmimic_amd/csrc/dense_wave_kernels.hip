@@ -38,8 +38,110 @@ __global__ __launch_bounds__(256, NB == 5 ? 3 : 4) void dense_update_wave_kernel
                               decrement + w, nv, lane);
 }
 
+// H = M + J' D_act J of one world, as jtdj_wave (jtdj_wave.h) forms it, over the rows that contribute: their numbers
+// are listed in LDS (ascending, by ballot, kListedRows rows of J at a time) while nothing else uses the area, and only
+// they are read.  A row with weight zero leaves every chain as it is, but costs its trip to memory: at two wavefronts
+// per SIMD the launch is a chain of such trips, a fetch of STEPS steps of four rows each.
+// Whole solves, all rows read (and at 80 columns two steps in flight) -> now: 70 dofs x 2048 with 192 rows 873 -> 840 us, 56 x
+// 4096 with 128 rows 705 -> 691, 35 x 8192 with 96 rows 694 -> 676, 62 x 2000 521 -> 511.
+constexpr int kListedRows = 256;
+
+template <int NB, int STEPS>
+__device__ __forceinline__ void jtdj_listed(const float *__restrict__ Mw, const int32_t *__restrict__ elemid,
+                                            const float *__restrict__ Jw, const float *__restrict__ Dw,
+                                            const int32_t *__restrict__ sw, int nefc, int quad, int nv,
+                                            float *__restrict__ Hw, int *list, int lane, float4v (&acc)[kTiles<NB>]) {
+  static_assert(kListedRows <= wave_stage_words<NB>(), "the list lies in the stage's area");
+  const int c = lane & 15, kq = lane >> 4;
+  float u[STEPS][NB], dk[STEPS], un[STEPS][NB], dn[STEPS];
+  int cnt = 0;
+  auto list_rows = [&](int r0) __attribute__((always_inline)) {
+    const int end = nefc - r0 < kListedRows ? nefc : r0 + kListedRows;
+    cnt = 0;
+    for (int base = r0; base < end; base += 64) {
+      const int r = base + lane;
+      const bool on = r < end && sw[r < end ? r : end - 1] == quad;
+      const unsigned long long m = __ballot(on);
+      if (on) list[cnt + __popcll(m & ((1ull << lane) - 1ull))] = r;
+      cnt += __popcll(m);
+    }
+    wave_sync();
+  };
+  // the operands of STEPS steps (four rows each): asked for a group ahead of the products that use them
+  auto fetch = [&](int q0, float (&uu)[STEPS][NB], float (&dd)[STEPS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const int at = 4 * (q0 + s) + kq;
+      const bool in = at < cnt;
+      const int row = list[in ? at : cnt - 1];
+      const float dv = Dw[row];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int col = 16 * b + c;
+        const float jv = Jw[(int64_t)row * nv + (col < nv ? col : nv - 1)];
+        uu[s][b] = (in && col < nv) ? jv : 0.0f;
+      }
+      dd[s] = in ? dv : 0.0f;
+    }
+  };
+  if (nefc > 0) list_rows(0);
+  if (cnt > 0) fetch(0, u, dk);  // on their way while M is gathered
+  int m = 0;
+  // the accumulators start from M (a lane holds column j = l % 16 and rows 4 (l / 16) + v of a tile)
+#pragma unroll
+  for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+    for (int bj = bi; bj < NB; ++bj, ++m) {
+      const int j = 16 * bj + c, jc = j < nv ? j : nv - 1;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 16 * bi + 4 * kq + v, ic = i < nv ? i : nv - 1;
+        const int id = elemid[ic * nv + jc];
+        const float mv = Mw[id < 0 ? 0 : id];
+        acc[m][v] = (i < nv && j < nv && id >= 0) ? mv : 0.0f;
+      }
+    }
+  for (int r0 = 0; r0 < nefc;) {
+    const int nstep = (cnt + 3) >> 2;
+    for (int q0 = 0; q0 < nstep; q0 += STEPS) {
+      if (q0 + STEPS < nstep) fetch(q0 + STEPS, un, dn);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        float wt[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) wt[b] = u[s][b] * dk[s];
+        int t = 0;
+#pragma unroll
+        for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+          for (int bj = bi; bj < NB; ++bj, ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[bi], u[s][bj], acc[t], 0, 0, 0);
+      }
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        dk[s] = dn[s];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) u[s][b] = un[s][b];
+      }
+    }
+    r0 += kListedRows;
+    if (r0 < nefc) {
+      wave_sync();
+      list_rows(r0);
+      if (cnt > 0) fetch(0, u, dk);
+    }
+  }
+  wave_sync();  // the stage takes the list's area
+  m = 0;
+#pragma unroll
+  for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+    for (int bj = bi; bj < NB; ++bj, ++m)
+      store_h_mirrored(Hw, nv, 16 * NB, true, 16 * bi + 4 * kq, 16 * bj + c, acc[m], bi != bj);
+}
+
 // The first Hessian and its factor in one launch: H = M + J' D_act J of every world on the matrix
-// cores of its wavefront (jtdj_wave.h), stored, and for the worlds that are not done factored where it lies: in
+// cores of its wavefront (jtdj_listed), stored, and for the worlds that are not done factored where it lies: in
 // the accumulators.
 template <int NB>
 __global__ __launch_bounds__(256, NB == 3 ? 3 : 2) void dense_init_wave_kernel(
@@ -59,9 +161,11 @@ __global__ __launch_bounds__(256, NB == 3 ? 3 : 2) void dense_init_wave_kernel(
   float *Hw = H_ + w * (int64_t)PAD * PAD;
   const float *Jw = J + w * (int64_t)njmax * nv;
   float4v t[kTiles<NB>];
-  jtdj_wave<NB, NB == 5 ? 2 : 4>(M + w * ldM, elemid, Jw, D + w * njmax, state + w * njmax, nefc, quad, nv, Hw, PAD, true, lane, t);
+  nefc = __builtin_amdgcn_readfirstlane(nefc);
+  float *area = lds + wv * wave_stage_words<NB>();
+  jtdj_listed<NB, 4>(M + w * ldM, elemid, Jw, D + w * njmax, state + w * njmax, nefc, quad, nv, Hw, (int *)area, lane, t);
   if (done && done[w]) return;
-  dense_wave_world<NB, true>(t, lds + wv * wave_stage_words<NB>(), Hw, U_ + w * (int64_t)PAD * PAD, Jw, D + w * njmax,
+  dense_wave_world<NB, true>(t, area, Hw, U_ + w * (int64_t)PAD * PAD, Jw, D + w * njmax,
                              grad + w * ldg, state + w * njmax, nullptr, -1, 0, quad, uni_ + w * (nv + 1),
                              search + w * ld_search, search_dot + w, decrement + w, nv, lane);
 }
