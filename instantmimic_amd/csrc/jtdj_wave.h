@@ -1,6 +1,7 @@
-// H = M + J' diag(D [state == quad]) J of one world on one wavefront, for up to five 16-column
-// blocks (the first Hessian of a dense Newton solve up to 79 dofs), and the store of a lane's share
-// of a 16 x 16 accumulator tile into H and its mirror image.
+// H = M + J' diag(D [state == quad]) J of one world on one wavefront, for one or two 16-column
+// blocks (the first Hessian of a dense Newton solve up to 32 dofs; with more the contributing rows are
+// listed first, jtdj_listed), and the store of a lane's share of a 16 x 16 accumulator tile into H
+// and its mirror image.
 // Reference: upstream's solver._update_gradient as src/instantmimic/utils/mjw_kernels/newton_fusion.py:470
 // calls it (the dense Newton's full assembly ahead of the first factor).
 // An element's sum is the chain fma(J[r][i] * Dc[r], J[r][j], .) over the rows in order, from M:
@@ -39,13 +40,14 @@ __device__ __forceinline__ void store_h_mirrored(float *__restrict__ Hw, int nv,
 // of v_mfma_f32_16x16x4_f32 (lane l supplies row 4 q + l / 16, column 16 b + l % 16 of step q: four
 // rows of 64 bytes per load), the next sixteen rows' loads in flight behind the current ones'
 // products; nothing is staged.
-// The tiles stay in `acc` (upper block triangle, row by row); STEPS: steps whose operands are in flight.
-template <int NB, int STEPS = 4>
+// The tiles stay in `acc` (upper block triangle, row by row).
+template <int NB>
 __device__ __forceinline__ void jtdj_wave(const float *__restrict__ Mw, const int32_t *__restrict__ elemid,
                                           const float *__restrict__ Jw, const float *__restrict__ Dw,
                                           const int32_t *__restrict__ sw, int nefc, int quad, int nv,
                                           float *__restrict__ Hw, int pad, bool vec, int lane,
                                           float4v (&acc)[NB * (NB + 1) / 2]) {
+  constexpr int STEPS = 4;  // steps whose operands are in flight
   const int c = lane & 15, kq = lane >> 4;
   const int nstep = (nefc + 3) >> 2;
   float u[STEPS][NB], dk[STEPS], un[STEPS][NB], dn[STEPS];
