@@ -20,6 +20,10 @@ namespace {
 // LDS words of one wavefront: M's row and the tile of J, then sv, Ma, gl (nv each), Jaref, f, rowl (njmax each)
 __host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return resident::kTileWords + 3 * (size_t)nv + 3 * (size_t)njmax; }
 
+// WIDE: more than 64 dofs (the product on the matrix cores, two dofs a lane in the gradient): 124 registers a lane against
+// 72.  What bounds the launch is J's trip from memory, hidden by other wavefronts, and one kernel of both forms gives every
+// model the wide form's four per SIMD: 27 dofs x 8192 worlds with 64 rows 33.1 -> 29.9 us, 35 x 8192 with 96 rows 47.9 -> 43.1.
+template <bool WIDE>
 __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::NewtonArgs a, const float *__restrict__ qacc_smooth,
                                                                   int64_t ld_qacc_smooth, const float *__restrict__ aref,
                                                                   int64_t ld_aref, WholeSolve whole) {
@@ -71,7 +75,7 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
   }
   const float *Jw = a.J + w * (int64_t)njmax * nv;
   resident::wave_sync();
-  if (nv > 64)
+  if constexpr (WIDE)
     resident::jv_world(a, Jw, nefc, sv, nullptr, Jaref_l, lane, []() {});
   else
     resident::jv_world_tiled<true>(a, Jw, nefc, tile, sv, nullptr, Jaref_l, lane, []() {});
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
   }
   resident::wave_sync();
   resident::Scalars sc{};
-  if (nv > 64)
+  if constexpr (WIDE)
     resident::gradient_world<2, 4, false>(a, w, Jw, true, cnt, f, rowl, Ma_l, a.smooth + w * nv, gl, sc, lane);
   else
     resident::gradient_world<1, 2, false>(a, w, Jw, true, cnt, f, rowl, Ma_l, a.smooth + w * nv, gl, sc, lane);
@@ -142,10 +146,10 @@ int newton_init_launch(const im_newton_args *p, const float *qacc_smooth, int64_
   if (ld_qacc_smooth < nv || ld_aref < p->njmax || (whole.start && whole.ld_start < nv)) return IM_ERR_STRIDE;
   const size_t lds = 4 * ((size_t)p->nterm + nv + 1 + 4 * init_wave_words(nv, p->njmax));
   if (lds > 160 * 1024) return IM_ERR_UNSUPPORTED;
+  auto kernel = nv > 64 ? newton_init_context_kernel<true> : newton_init_context_kernel<false>;
   if (lds > 64 * 1024)
-    IM_HIP_CHECK(hipFuncSetAttribute((const void *)newton_init_context_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds));
-  hipLaunchKernelGGL(newton_init_context_kernel, dim3((unsigned)((p->nworld + 3) / 4)), dim3(256), lds, stream, a, qacc_smooth,
+    IM_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((p->nworld + 3) / 4)), dim3(256), lds, stream, a, qacc_smooth,
                      ld_qacc_smooth, efc_aref, ld_aref, whole);
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;

@@ -1,0 +1,53 @@
+"""What the compiler gave the kernels of ``libimhip.so``, from the metadata of its code objects: registers and
+private memory decide how many wavefronts a SIMD holds, and neither shows in a result."""
+
+import struct
+
+import pytest
+
+from instantmimic_amd import build
+
+msgpack = pytest.importorskip("msgpack")
+
+_MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+_NOTES, _AMDGPU_METADATA = 7, 32  # section and note types
+
+
+def _kernels_of(elf: bytes):
+    sections, (size, count) = struct.unpack_from("<Q", elf, 40)[0], struct.unpack_from("<HH", elf, 58)
+    for i in range(count):
+        _, kind, _, _, at, _ = struct.unpack_from("<IIQQQQ", elf, sections + i * size)
+        if kind == _NOTES:
+            name, words, note = struct.unpack_from("<III", elf, at)
+            if note == _AMDGPU_METADATA:
+                start = at + 12 + -(-name // 4) * 4
+                yield from msgpack.unpackb(elf[start : start + words], strict_map_key=False)["amdhsa.kernels"]
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    """{mangled name: metadata} of the library's gfx950 kernels."""
+    with open(build.LIB, "rb") as f:
+        lib = f.read()
+    found, at = {}, lib.find(_MAGIC)
+    while at >= 0:
+        entry = at + 32
+        for _ in range(struct.unpack_from("<Q", lib, at + 24)[0]):
+            offset, size, length = struct.unpack_from("<QQQ", lib, entry)
+            if size and b"gfx950" in lib[entry + 24 : entry + 24 + length]:
+                found.update((k[".name"], k) for k in _kernels_of(lib[at + offset : at + offset + size]))
+            entry += 24 + length
+        at = lib.find(_MAGIC, at + 1)
+    return found
+
+
+def _wavefronts(kernel) -> int:
+    """Wavefronts that a SIMD's 512 registers a lane hold, handed out by eights."""
+    return 512 // (-(-kernel[".vgpr_count"] // 8) * 8)
+
+
+def test_start_of_a_solve_does_not_pay_for_the_wide_form(kernels):
+    """Up to 64 dofs the launch needs 72 registers a lane, beyond 124: in one kernel every model had the four
+    wavefronts per SIMD of the wide form."""
+    starts = [k for n, k in kernels.items() if "newton_init_context_kernel" in n]
+    assert max(map(_wavefronts, starts)) >= 5 and all(k[".private_segment_fixed_size"] == 0 for k in starts)
