@@ -1,6 +1,8 @@
 """What the compiler gave the kernels of ``libimhip.so``, from the metadata of its code objects: registers and
 private memory decide how many wavefronts a SIMD holds, and neither shows in a result."""
 
+import os
+import re
 import struct
 
 import pytest
@@ -51,3 +53,11 @@ def test_start_of_a_solve_does_not_pay_for_the_wide_form(kernels):
     wavefronts per SIMD of the wide form."""
     starts = [k for n, k in kernels.items() if "newton_init_context_kernel" in n]
     assert max(map(_wavefronts, starts)) >= 5 and all(k[".private_segment_fixed_size"] == 0 for k in starts)
+
+
+def test_resident_loops_stay_within_the_private_memory_they_are_admitted_with(kernels):
+    """A resident kernel beyond the limit is left out at run time without a word, and its batches take a slower one."""
+    with open(os.path.join(build.CSRC, "newton_solve.hip")) as f:
+        limit = int(re.search(r"kResidentPrivate = (\d+);", f.read())[1])
+    private = {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if re.search(r"newton_(sparse|dense_tile|dense_wave)_resident_kernel", n)}
+    assert len(private) == 22 and max(private.values()) <= limit <= 2 * max(private.values())
