@@ -497,6 +497,8 @@ int tree_plan_upload(im_tree_plan *pl) {
     pl->table_driven = false;
     pl->row16 = nullptr;
     IM_HIP_CHECK(hipGetDevice(&pl->device));
+    IM_HIP_CHECK(hipMalloc(&pl->dev_blob, 16));
+    pl->next_world = (int *)pl->dev_blob;
     pl->device_ready = true;
     return IM_OK;
   }
@@ -826,7 +828,10 @@ int newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, hipStre
   if (const int st = compute_units(&ncu)) return st;
   const unsigned grid = (unsigned)resident_worlds_grid(p->nworld, 4, ncu, std::max(1, per_cu), true, &a.group_worlds);
   // (a batch that is resident all at once has nothing to hand out)
-  if ((int64_t)grid * 4 < p->nworld) a.next_world = plan->next_world;
+  if ((int64_t)grid * 4 < p->nworld) {
+    if (!plan->next_world) return IM_ERR_UNSUPPORTED;  // worlds behind the first ones would be left as they are
+    a.next_world = plan->next_world;
+  }
   if (before) {
     a.final_force = a.sums_at_enter = 1;
     if (const int st = (*before)(a.next_world, (int)grid * 4)) return st;

@@ -3,6 +3,8 @@ and the force recovery (src/instantmimic/utils/mjw_step_optimized.py:2588-2683,
 src/instantmimic/utils/mjw_kernels/newton_fusion.py:330-539), started from poisoned solver state,
 captured in a graph without any read-back, against the oracle's pieces chained in the same order."""
 
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -173,6 +175,32 @@ def test_gpu_solve_of_batches_that_do_not_fill_the_chip(device, name, stage, nwo
     m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
     NC.compare(p, s, d, ctx)
     assert int(nsolving.item()) == int((p.nefc == 0).sum() + ((p.nefc > 0) & (s.done == 0)).sum())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv,stage,chains,rows", [(65, "dense", 1, 64), (67, "dense", 1, 520), (69, "dense", 1, 130), (77, "dense", 1, 80),
+                                                     (70, "tree", 4, 130), (66, "sparse", 4, 130)])  # fmt: skip
+def test_gpu_solve_beyond_64_dofs(device, monkeypatch, nv, stage, chains, rows):
+    """Every remainder of four dofs, rows on both sides of the 64 that a product takes at once and of the 256 that the first
+    Hessian lists at once; and the batch's worlds again and again, more of them than the chip keeps resident: the same bits in
+    every copy."""
+    import torch
+
+    name = f"wide{nv}x{rows}"
+    monkeypatch.setitem(synth.SHAPES, name, synth.Shape(name, _floating_chain(nv, chains), rows, 64, (0.5, 8.0), 0.02, (-4.0, 4.0), 0.6, 1, 1300 + nv))
+    p = NC.problem(name, 23, stage, empty_every=9, maxiter=4)
+    s = NC.oracle_solve(p)
+    m, d, ctx, _ = _solve_on_gpu(p, device, graph=False)
+    NC.compare(p, s, d, ctx)
+    index = np.arange(12 * torch.cuda.get_device_properties(0).multi_processor_count + 9) % p.nworld
+    p.b = SimpleNamespace(M=p.b.M)
+    for ns in (p, p.b, s):
+        for k, v in vars(ns).items():
+            if isinstance(v, np.ndarray) and v.ndim and len(v) == 23:
+                setattr(ns, k, v[index])
+    p.nworld = len(index)
+    m, d, ctx, _ = _solve_on_gpu(p, device, graph=False)
+    NC.compare(p, s, d, ctx)
 
 
 @pytest.mark.gpu
