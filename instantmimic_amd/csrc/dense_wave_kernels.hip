@@ -40,8 +40,8 @@ __global__ __launch_bounds__(256, NB == 5 ? 3 : 4) void dense_update_wave_kernel
 
 // H = M + J' D_act J of one world, as jtdj_wave (jtdj_wave.h) forms it, over the rows that contribute: their numbers
 // are listed in LDS (ascending, by ballot, kListedRows rows of J at a time) while nothing else uses the area, and only
-// they are read.  A row with weight zero leaves every chain as it is, but costs its trip to memory: at two wavefronts
-// per SIMD the launch is a chain of such trips, a fetch of STEPS steps of four rows each.
+// they are read.  A row with weight zero leaves every chain as it is, but costs its trip to memory: with two wavefronts
+// per SIMD (2048 worlds) the launch is a chain of such trips, a fetch of STEPS steps of four rows each.
 // Whole solves, all rows read (and at 80 columns two steps in flight) -> now: 70 dofs x 2048 with 192 rows 873 -> 840 us, 56 x
 // 4096 with 128 rows 705 -> 691, 35 x 8192 with 96 rows 694 -> 676, 62 x 2000 521 -> 511.
 constexpr int kListedRows = 256;
@@ -143,8 +143,13 @@ __device__ __forceinline__ void jtdj_listed(const float *__restrict__ Mw, const 
 // The first Hessian and its factor in one launch: H = M + J' D_act J of every world on the matrix
 // cores of its wavefront (jtdj_listed), stored, and for the worlds that are not done factored where it lies: in
 // the accumulators.
-template <int NB>
-__global__ __launch_bounds__(256, NB == 3 ? 3 : 2) void dense_init_wave_kernel(
+// STEPS 2 (with 80 columns): four wavefronts per SIMD of 128 registers, where four steps take 162 and leave three.  The
+// batches that three hold gain nothing by it and have fewer loads on their way; beyond, a fourth spares them a second turn
+// on the chip.  70 dofs with 157 rows, four steps / two, us: x 300 47.7 / 48.5, x 1024 54.1 / 56.7, x 2048 71.8 / 73.4, x
+// 3072 86.7 / 87.0, x 4096 139.4 / 107.4, x 6144 185.2 / 183.6, x 8192 266.6 / 235.4 (all rows read, two steps, x 4096:
+// 132.7).
+template <int NB, int STEPS>
+__global__ __launch_bounds__(256, NB == 3 ? 3 : STEPS == 2 ? 4 : 2) void dense_init_wave_kernel(
     const uint8_t *__restrict__ done, const int32_t *__restrict__ nefc_p, const float *__restrict__ J, int njmax,
     const float *__restrict__ D, const int32_t *__restrict__ state, int quad, const float *__restrict__ M, int64_t ldM,
     const int32_t *__restrict__ elemid, const float *__restrict__ grad, int64_t ldg, float *H_, float *U_,
@@ -163,7 +168,7 @@ __global__ __launch_bounds__(256, NB == 3 ? 3 : 2) void dense_init_wave_kernel(
   float4v t[kTiles<NB>];
   nefc = __builtin_amdgcn_readfirstlane(nefc);
   float *area = lds + wv * wave_stage_words<NB>();
-  jtdj_listed<NB, 4>(M + w * ldM, elemid, Jw, D + w * njmax, state + w * njmax, nefc, quad, nv, Hw, (int *)area, lane, t);
+  jtdj_listed<NB, STEPS>(M + w * ldM, elemid, Jw, D + w * njmax, state + w * njmax, nefc, quad, nv, Hw, (int *)area, lane, t);
   if (done && done[w]) return;
   dense_wave_world<NB, true>(t, area, Hw, U_ + w * (int64_t)PAD * PAD, Jw, D + w * njmax,
                              grad + w * ldg, state + w * njmax, nullptr, -1, 0, quad, uni_ + w * (nv + 1),
@@ -296,13 +301,20 @@ static int init_factor(int most, const uint8_t *done, const int32_t *nefc, const
   if (!U) return IM_ERR_ARG;
   if (!im::wave_shape(nv, nv_pad) || nv_pad > most) return IM_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)((nworld + 3) / 4)), wg(256);
-#define IM_INIT_WAVE(NB)                                                                                                      \
-  hipLaunchKernelGGL(im::dense_init_wave_kernel<NB>, grid, wg, 16 * im::wave_stage_words<NB>(), (hipStream_t)stream, done,    \
-                     nefc, J, njmax, D, state, quad, M, ldM, elemid, grad, ldg, H, U, dof_union, search, ld_search,           \
+#define IM_INIT_WAVE(NB, STEPS)                                                                                               \
+  hipLaunchKernelGGL((im::dense_init_wave_kernel<NB, STEPS>), grid, wg, 16 * im::wave_stage_words<NB>(), (hipStream_t)stream, \
+                     done, nefc, J, njmax, D, state, quad, M, ldM, elemid, grad, ldg, H, U, dof_union, search, ld_search,     \
                      search_dot, decrement, nv, nworld)
-  if (nv_pad == 48) IM_INIT_WAVE(3);
-  else if (nv_pad == 64) IM_INIT_WAVE(4);
-  else IM_INIT_WAVE(5);
+  if (nv_pad == 48) {
+    IM_INIT_WAVE(3, 4);
+  } else if (nv_pad == 64) {
+    IM_INIT_WAVE(4, 4);
+  } else {
+    int ncu = 0;
+    if (const int st = im::compute_units(&ncu)) return st;
+    if (nworld <= 12 * ncu) IM_INIT_WAVE(5, 4);
+    else IM_INIT_WAVE(5, 2);
+  }
 #undef IM_INIT_WAVE
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
