@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "common.h"
+#include "newton_solve.h"
 
 namespace im {
 namespace {
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(NT) void muscle_project_kernel(
   }
 }
 
-// One workgroup of 256 for W worlds side by side, a value of each next to one another in LDS: a chunk's sixteen packed
+// One workgroup (of 256 threads, or 512 where its LDS is large) for W worlds side by side, a value of each next to one another in LDS: a chunk's sixteen packed
 // pairs (64 KB of tables at 284 muscles, more than a CU's cache holds beside the worlds') are read and taken apart once
 // for W products.
 template <int W>
@@ -286,10 +287,15 @@ int im_muscle_implicit_gather(const float *moment, int64_t ld_moment, const floa
   if (ld_moment < nentry) return IM_ERR_STRIDE;
   const size_t lds_bytes = sizeof(float) * (2 * ((size_t)nentry + 1) + chunk_count);
   if (lds_bytes > 64 * 1024) return IM_ERR_UNSUPPORTED;
-  // Two worlds where both fit beside one another and the batch has eight for every CU; 512 threads where their LDS leaves a
-  // CU three workgroups.  4096 worlds of 2522 entries, 1038 chunks: a world 34.2 us, two 32.0, two on 512 threads 23.8; the
-  // implicit step's terms of 355 entries x 8192 worlds 94 -> 85 us.
-  const bool two = nworld >= 2048 && 2 * lds_bytes <= 80 * 1024;
+  // Two worlds where a CU holds two such workgroups and the batch has two worlds for every CU; 512 threads where their LDS
+  // leaves a CU three workgroups.  4096 worlds of 2522 entries, 1038 chunks: a world 34.2 us, two 32.0, two on 512 threads
+  // 23.8.  A world / two by batch (256 CUs), us: 355 entries x 256 5.1 / 5.3, x 512 5.8 / 5.3, x 2047 9.1 / 7.5, x 8192
+  // 26.4 / 17.1; 1077 entries x 256 5.6 / 6.2, x 512 6.5 / 6.5, x 1024 8.2 / 7.8; 2522 x 512 9.1 / 6.9, x 1024 12.2 / 8.7.
+  // By LDS, x 4096: two of 61 KB 42.9 / 32.6, 72 KB 48.2 / 34.4, 78 KB 53.7 / 37.5; beyond, one to a CU, 85 KB 67.7 / 59.5
+  // but 87 KB with fewer chunks 56.9 / 57.9.
+  int ncu = 0;
+  if (const int st = im::compute_units(&ncu)) return st;
+  const bool two = nworld >= 2 * ncu && 2 * lds_bytes <= 80 * 1024;
   auto kernel = two ? im::muscle_gather_kernel<2> : im::muscle_gather_kernel<1>;
   const size_t bytes = two ? 2 * lds_bytes : lds_bytes;
   if (bytes > 64 * 1024) IM_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));

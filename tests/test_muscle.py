@@ -114,11 +114,12 @@ def test_gpu_matches_oracle_bitwise(device, nworld):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("nworld", [2047, 2048, 2049])
-@pytest.mark.parametrize("nmuscle", [40, 420, 1100])
+@pytest.mark.parametrize("nworld", [511, 512, 513, 2047, 2048, 2049])
+@pytest.mark.parametrize("nmuscle", [20, 40, 420, 1100])
 def test_gpu_gather_of_two_worlds_a_workgroup(device, nmuscle, nworld):
-    """Both sides of the batch from which a workgroup takes two worlds, with a world left over, on 256 and on 512 threads and
-    where two worlds do not fit: the oracle's bits, and the columns beside the matrix stay as they are."""
+    """Both sides of the batch from which a workgroup takes two worlds (two for every compute unit), with a world left over,
+    on 256 threads (20 muscles) and on 512, and where a unit does not hold two such workgroups (1100): the oracle's bits, and
+    the columns beside the matrix stay as they are."""
     import torch
 
     mb = synth.make_muscles(nworld, nmuscle=nmuscle, seed=5)
