@@ -15,10 +15,9 @@
 //   contribution      = dot(a (lin + ang x (p0 - c0)) - b (lin + ang x (p1 - c1)), f dir)
 //     reference: muscle_qfrc_projector.py:280-304
 //
-// All five are gathers over a world's row of poses (a few KB, L1/L2 resident after the
-// first touch) and write one float per thread; none of them reuses data across worlds, so
-// they are HBM bound on the pose rows.  Threads are laid out output-major inside a world
-// so that a wavefront's writes coalesce.  Arithmetic is written out operation by operation
+// All five are gathers over a world's row of poses (a few KB) and reuse nothing across worlds.  Their bytes would
+// pass in a tenth of the time: what bounds each is instructions or the trips within a world, and stands at its
+// kernel.  Threads are laid out output-major inside a world so that a wavefront's writes coalesce.  Arithmetic is written out operation by operation
 // (this file is compiled without floating-point contraction) and the CPU checker follows
 // the same order.
 #include <hip/hip_runtime.h>

@@ -470,9 +470,8 @@ __device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, i
   }
 }
 
-// ---- J search through a tile of 64 rows x 16 dofs (4.3 KB of LDS whatever the width of J) ------
-// ---- J search up to 64 dofs ------------------------------------------------------------------------
-// The same chains through a tile of 64 rows x 16 dofs in LDS (kTileWords) and on a lane per row: the
+// ---- J search through a tile of 64 rows x 16 dofs (kTileWords of LDS whatever the width of J) -------
+// Up to 64 dofs, the same chains through the tile and on a lane per row: the
 // operands' way into the matrix cores takes more instructions, and where the chip is full of worlds it is the slower
 // form (27 dofs x 4096 worlds 259 us per solve against 250; 56 x 4096 768 against 740).  A lane loads 16 elements per
 // tile, four rows of 64 bytes per instruction; the next tile's elements are asked for while the current one is worked
