@@ -713,19 +713,25 @@ def test_packed_entries_are_the_list_in_another_order():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("muscles", [3, 74, 76, 158, 164, 225, 226, 320, 325])
-@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("swap", [False, True, "some"])
 def test_gpu_from_context_equals_waypoints_and_forces_in_memory(muscles, swap):
     """Torque, gradient and moment in one launch: the bits of the kernels with waypoints and forces in
     memory, on both sides of 1280, 2560, 3584 and 5120 entries (128, 256 and 512 threads; more than a workgroup keeps), for segments that
-    run up and down the tree, one world and several per workgroup, and with poses, centres and axes that are not finite."""
+    run up the tree, down it and, in one list, both, one world and several per workgroup, and with poses, centres and axes that are not finite."""
     rig = synth.make_muscle_rig(nmuscle=muscles, seed=1003)
     t = rig.topology
     if swap:  # the end's body above the start's: entries with a start coefficient alone
+        on = np.arange(len(t.apply_segment_start_idx)) % 3 != 0 if swap == "some" else True
+        pick = lambda a, b: np.where(on, np.asarray(b), np.asarray(a))  # noqa: E731
         t = dataclasses.replace(
-            t, apply_segment_start_idx=t.apply_segment_end_idx, apply_segment_end_idx=t.apply_segment_start_idx,
-            apply_segment_body_start_idx=t.apply_segment_body_end_idx, apply_segment_body_end_idx=t.apply_segment_body_start_idx,
+            t, apply_segment_start_idx=pick(t.apply_segment_start_idx, t.apply_segment_end_idx),
+            apply_segment_end_idx=pick(t.apply_segment_end_idx, t.apply_segment_start_idx),
+            apply_segment_body_start_idx=pick(t.apply_segment_body_start_idx, t.apply_segment_body_end_idx),
+            apply_segment_body_end_idx=pick(t.apply_segment_body_end_idx, t.apply_segment_body_start_idx),
         )  # fmt: skip
     layer = MuscleDynamicsLayer(t, **rig.dims(), mechanics=MuscleMechanics(), device="cuda")
+    kinds = [c.kind_count[:2] for c in layer._context if c is not None]
+    assert all((k[0] > 0) == (swap is not True) and (k[1] > 0) == bool(swap) for k in kinds)
     assert (layer._context[0] is None) == (muscles == 325) and (layer._context[1] is None) == (layer._context[2] is None) == (muscles == 325)
     entries = (layer._torque_entries, layer._muscle_entries, layer._moment_entries)
     stated = [e.nother for e in entries]
