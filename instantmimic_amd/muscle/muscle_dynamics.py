@@ -367,8 +367,7 @@ class MuscleDynamicsLayer:
         import torch
 
         self._need_gpu(raw_context)
-        if raw_context.shape[1] < self.context_dim:
-            raise ValueError(f"raw_context has {raw_context.shape[1]} columns, the layer needs {self.context_dim}")
+        self._check_context(raw_context)
         B, ld = raw_context.shape[0], raw_context.stride(0)
         base, d, s = raw_context.data_ptr(), self._dev, _stream(raw_context)
         ws = {"transformed_waypoints": torch.empty((B, 3 * self.waypoint_count), device=raw_context.device)}
@@ -400,7 +399,7 @@ class MuscleDynamicsLayer:
         return ws, geo
 
     def _check_context(self, raw_context):
-        self._need_gpu(raw_context)
+        """The context's columns; its type, device and rows are ``_need_gpu``'s, which goes before."""
         if raw_context.shape[1] < self.context_dim:
             raise ValueError(f"raw_context has {raw_context.shape[1]} columns, the layer needs {self.context_dim}")
 
