@@ -128,9 +128,9 @@ __global__ __launch_bounds__(NT) void muscle_project_kernel(
   }
 }
 
-// One workgroup (of 256 threads, or 512 where its LDS is large) for W worlds side by side, a value of each next to one another in LDS: a chunk's sixteen packed
-// pairs (64 KB of tables at 284 muscles, more than a CU's cache holds beside the worlds') are read and taken apart once
-// for W products.
+// One workgroup (of 256 threads, or 512 where its LDS is large) for W worlds side by side, a value of each next to one
+// another in LDS: a chunk's sixteen packed pairs (64 KB of tables at 284 muscles, more than a CU's cache holds beside the
+// worlds') are read and taken apart once for W products.
 template <int W>
 __global__ __launch_bounds__(512) void muscle_gather_kernel(
     const float *__restrict__ moment, int64_t ldm, const float *__restrict__ slope, int64_t lds_,

@@ -128,14 +128,14 @@ __device__ __forceinline__ void block_sync() {
 // (one word per term, nv + 1 offsets), then per wavefront the world's row of M, the search
 // direction, Ma, mv, Jaref, jv, D and the friction losses, the gradient's list of rows with a force
 // (value and row number) and its copy of the gradient.  The factor stage's area must also hold four wavefronts'
-// rows of M where those are read from memory (kTileWords each).
+// rows of M where those are read from memory, and their tiles of J (kTileWords each).
 // words a wavefront keeps from round to round: M, the search direction, Ma, mv, qacc; Jaref, jv, D, friction losses
 __host__ __device__ inline size_t kept_words(int nv, int njmax, int nM) { return (size_t)nM + 4 * (size_t)nv + 4 * (size_t)njmax; }
 __host__ __device__ inline size_t loop_lds_words(int nv, int njmax, int nM, int nterm) {
   return 8 + (size_t)nterm + nv + 1 + 4 * (kept_words(nv, njmax, nM) + 2 * (size_t)njmax + nv);
 }
 constexpr int kTileWords = 64 * 17;
-__host__ __device__ inline size_t staged_rows_words(int) { return 4 * kTileWords; }
+constexpr size_t kStagedWords = 4 * kTileWords;
 
 // ---- M search (newton_fusion.py:171-176) -------------------------------------------------------
 // WALK: more dofs than lanes.
@@ -569,7 +569,7 @@ struct LoopLds {
   int *rowl;             // [njmax] their numbers
   float *gl;             // [nv] qfrc_smooth, from the products to the gradient; then the gradient (a cooperative stage's loop
                          // reads it again after the stage)
-  float *rows;           // kTileWords: the world's row of M on its way into the product
+  float *rows;           // kTileWords: the world's row of M on its way into the product, then the tile of J
 };
 
 // A world's vectors stay in LDS and its scalars in registers from round to round; memory receives

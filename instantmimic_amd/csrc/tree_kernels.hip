@@ -800,9 +800,9 @@ int newton_solve_tree(const im_tree_plan *plan, const im_newton_args *p, hipStre
   const int bad = resident::convert_args(*p, nv, nM, a);
   if (bad != IM_OK) return bad;
   // the factor stage's LDS (its staged tiles and exchange slots plus the four worlds' row lists), or the
-  // four wavefronts' staged rows of J where those take more; the loop's own arrays behind it
+  // four wavefronts' rows of M and tiles of J where those take more; the loop's own arrays behind it
   const size_t stage_bytes = (size_t)e->lds_bytes + 32 * std::max<size_t>(((size_t)njmax + 15) / 16 * 16, 64);
-  const size_t stage_words = std::max(stage_bytes / 4, resident::staged_rows_words(nv));
+  const size_t stage_words = std::max(stage_bytes / 4, resident::kStagedWords);
   a.stage_lds_floats = (int)stage_words;
   size_t lds = 4 * (stage_words + resident::loop_lds_words(nv, njmax, nM, p->nterm));
   const size_t lds_lean = 4 * (stage_words + resident::loop_lds_words(nv, njmax, 0, p->nterm));
