@@ -179,16 +179,26 @@ def test_gpu_solve_of_batches_that_do_not_fill_the_chip(device, name, stage, nwo
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("nv,stage,chains,rows", [(65, "dense", 1, 64), (67, "dense", 1, 520), (69, "dense", 1, 130), (77, "dense", 1, 80),
-                                                     (70, "tree", 4, 130), (66, "sparse", 4, 130)])  # fmt: skip
+                                                     (79, "dense", 1, 520), (70, "tree", 4, 130), (66, "sparse", 4, 130)])  # fmt: skip
 def test_gpu_solve_beyond_64_dofs(device, monkeypatch, nv, stage, chains, rows):
     """Every remainder of four dofs, rows on both sides of the 64 that a product takes at once and of the 256 that the first
-    Hessian lists at once; and the batch's worlds again and again, more of them than the chip keeps resident: the same bits in
-    every copy."""
+    Hessian lists at once, with quadratic rows in the first listing only, in the last only and in none; and the batch's worlds
+    again and again, more of them than the chip keeps resident: the same bits in every copy."""
     import torch
 
+    taken = []
+    inner = NF.run_resident
+    monkeypatch.setattr(NF, "run_resident", lambda *a: taken.append(inner(*a)) or taken[-1])
     name = f"wide{nv}x{rows}"
     monkeypatch.setitem(synth.SHAPES, name, synth.Shape(name, _floating_chain(nv, chains), rows, 64, (0.5, 8.0), 0.02, (-4.0, 4.0), 0.6, 1, 1300 + nv))
     p = NC.problem(name, 23, stage, empty_every=9, maxiter=4)
+    if rows > 512:
+        for w, (first, last) in enumerate(((0, 256), (512, rows), (0, 0), (256, 512))):  # the rows that may be quadratic
+            w = 4 + w
+            p.nefc[w], p.ne[w], p.nf[w] = rows, 0, 0
+            p.aref[w, :first] = p.aref[w, last:] = -500.0  # satisfied by far
+            quad = np.flatnonzero(NC.oracle_init(p).state[w] == synth.QUADRATIC)
+            assert all(first <= r < last for r in quad) and (len(quad) > 0) == (last > first)
     s = NC.oracle_solve(p)
     m, d, ctx, _ = _solve_on_gpu(p, device, graph=False)
     NC.compare(p, s, d, ctx)
@@ -201,6 +211,7 @@ def test_gpu_solve_beyond_64_dofs(device, monkeypatch, nv, stage, chains, rows):
     p.nworld = len(index)
     m, d, ctx, _ = _solve_on_gpu(p, device, graph=False)
     NC.compare(p, s, d, ctx)
+    assert len(taken) >= 2 and all(taken) == (stage != "sparse")  # (the sparse stage beyond 64 dofs is a workgroup per world)
 
 
 @pytest.mark.gpu
