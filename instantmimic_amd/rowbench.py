@@ -454,14 +454,15 @@ def run(launches: int = 32, only: str | None = None) -> None:
               f"segments, {len(layer.torque_entries_host[2])} torque entries x {nworld} worlds")  # fmt: skip
         cbytes = 4 * layer.context_dim
         sec = _timeit(torch, lambda i: layer._warp_muscle_dynamics_from_activation_forward(act, ctx[i], include_passive_force=True), 4, launches)
-        _line("torque_forward (waypoints + force magnitudes + im_muscle_torque_forward)", wl, sec,
+        _line("torque_forward (im_muscle_waypoints_forces + im_muscle_torque_forward)", wl, sec,
               bytes_=nworld * (cbytes + 4 * (3 * layer.waypoint_count * 2 + 3 * rig.muscle_count + rig.muscle_count + rig.torque_dim)), nworld=nworld)  # fmt: skip
-        sec = _timeit(torch, lambda i: layer._warp_muscle_dynamics_from_activation_backward(ctx[i], gout), 4, launches)
-        _line("torque_backward (waypoints + force magnitudes + im_muscle_activation_grad)", wl, sec,
-              bytes_=nworld * (cbytes + 4 * (3 * layer.waypoint_count * 2 + 2 * rig.muscle_count + rig.muscle_count + rig.torque_dim)), nworld=nworld)  # fmt: skip
-        sec = _timeit(torch, lambda i: layer.eval_muscle_sparse_moment(ctx[i]), 4, launches)
-        _line("eval_muscle_sparse_moment (waypoints + im_muscle_sparse_moment)", wl, sec,
-              bytes_=nworld * (cbytes + 4 * (3 * layer.waypoint_count * 2 + len(layer.sparse_entries.muscle_dof_torque_idx))), nworld=nworld)  # fmt: skip
+        for name, fn, words in (
+            ("torque", lambda i: layer._torque_from_context(act, ctx[i], True), rig.muscle_count + rig.torque_dim),
+            ("activation gradient", lambda i: layer._warp_muscle_dynamics_from_activation_backward(ctx[i], gout), rig.torque_dim + rig.muscle_count),
+            ("sparse moment", lambda i: layer.eval_muscle_sparse_moment(ctx[i]), len(layer.sparse_entries.muscle_dof_torque_idx)),
+        ):
+            sec = _timeit(torch, fn, 4, launches)
+            _line(f"im_muscle_from_context ({name})", wl, sec, bytes_=nworld * (cbytes + 4 * words), nworld=nworld)
 
     # ---- the tree walks either side of the solve
     if section("walks"):
