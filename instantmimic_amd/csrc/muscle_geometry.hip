@@ -860,9 +860,9 @@ bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
 // registers each.  A world with a lever or an axis so large that their products may not be finite takes
 // the full expression throughout (0 * inf is NaN there).
 // Four barriers per world: poses and axes, waypoints, segments and forces, contributions; the ordered sums run beside
-// the next world's poses.  4096 worlds of 284 muscles (three workgroups of 512 per CU; the vector ALUs issue in 0.64
-// of the cycles, the LDS is busy in 0.56): torque 80 us where the two launches took 35 + 64, gradient 74 (35 + 49), moment
-// 65 (20 + 58).
+// the next world's poses.  4096 worlds of 284 muscles, three workgroups of 512 per CU: torque 80 us where the two
+// launches took 35 + 64, gradient 74 (35 + 49), moment 65 (20 + 58); by counters the vector ALUs issue in 0.75, 0.79 and 0.71
+// of the cycles, the LDS is busy in 0.63, 0.70 and 0.65 (three eighths of that bank conflicts).
 struct CtxArgs {
   im_muscle_context c;
   const float *in;  // activation (MW_FORWARD) or grad_output (MW_GRAD)
