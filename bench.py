@@ -53,7 +53,7 @@ def algorithmic_bytes_fused(nv: int, nM: int, nefc: int, iters: int) -> int:
 
 def cpu_baseline(batch, plan_struct, gpu_x, seconds: float = 10.0):
     """The CPU oracle (a C restatement of the reference path, OpenMP over worlds) timed on this
-    host's cores on the same workload: all threads, then one thread.  As the checker it also
+    host's cores on the same workload: all threads, then one thread.  As the oracle it also
     compares what the GPU computed for the first input set of the benchmarked batch (`gpu_x`,
     (iterations, worlds, nv), every world) with its own result, bit for bit."""
     import numpy as np

@@ -18,7 +18,7 @@
 // All five are gathers over a world's row of poses (a few KB) and reuse nothing across worlds.  Their bytes would
 // pass in a tenth of the time: what bounds each is instructions or the trips within a world, and stands at its
 // kernel.  Threads are laid out output-major inside a world so that a wavefront's writes coalesce.  Arithmetic is written out operation by operation
-// (this file is compiled without floating-point contraction) and the CPU checker follows
+// (this file is compiled without floating-point contraction) and the CPU oracle follows
 // the same order.
 #include <hip/hip_runtime.h>
 

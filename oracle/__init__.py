@@ -2,7 +2,7 @@
 
 Nothing under this package is part of the shipped product.  Only ``tests/``,
 ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of ``bench.py`` may
-import it, and there only as the checker.  The product path
+import it, and there only as the oracle.  The product path
 (``instantmimic_amd``) never falls back to it.
 
 Contents

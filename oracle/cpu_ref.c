@@ -1,6 +1,6 @@
 /* CPU oracle: fp32 restatement of the reference's numeric statements for the
  * assemble + tree L'DL + solve path.  TEST INFRASTRUCTURE ONLY -- nothing in the
- * shipped library links or calls this file; it is the checker the HIP kernels
+ * shipped library links or calls this file; it is the oracle the HIP kernels
  * are compared with, and the timed "cpu_baseline" of the benchmark.
  *
  * Build: see oracle/Makefile (gcc -O2 -ffp-contract=off -fopenmp).  Every fused
