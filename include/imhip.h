@@ -679,7 +679,20 @@ int im_muscle_sparse_moment(const im_muscle_geometry *geometry,
  * what: IM_MUSCLE_TORQUE: in = activation (nworld, ld_in), passive forces where model.include_passive;
  * IM_MUSCLE_GRAD: in = grad_output; IM_MUSCLE_MOMENT: in unused.  nworld = 0 only checks the sizes:
  * IM_ERR_UNSUPPORTED if a world does not fit a workgroup (5120 packed entries; 512 muscles
- * for torque and gradient; 64 KB of LDS). */
+ * for torque and gradient; 64 KB of LDS).
+ * With ngroup > 0 the same list also comes in groups of up to three entries that share an operand, and the
+ * other tables packed, all 16-byte aligned and filled up to a multiple of 64 (null and 0: entry by entry):
+ *   waypoint_table  4 words a waypoint: local offset, 32 * body
+ *   segment_table   2 words: 12 * start waypoint | 12 * end waypoint << 16, the same of the two root bodies
+ *   length_table    a word for each of the nlength = all_segment_offsets[nmuscle] segments: 12 * its start
+ *   muscle_table    8 words: its first segment in length_table, their number, params[0 .. 2], rest, 0, 0
+ *   groups          4 words.  Torque and gradient, entries of one segment and kind: segment | dof << 16,
+ *                   dof | dof << 16, muscle | place << 16, place | place << 16.  Moment, a row's whole
+ *                   list: dof | row << 16, segment | segment << 16, segment, 0
+ *   group_kinds     per 64 groups, which are alike: kind (0, 1, 2 as in kind_count) | entries << 2; moment:
+ *                   the entries' kinds, two bits each, 3 past the last.  Fills name place nentry (moment:
+ *                   row nentry).
+ * ngroup is the number of groups with the fills. */
 enum { IM_MUSCLE_TORQUE = 0, IM_MUSCLE_GRAD = 1, IM_MUSCLE_MOMENT = 2 };
 typedef struct im_muscle_context {
   const float *xpos, *xquat, *subtree_com, *cdof;
@@ -694,6 +707,10 @@ typedef struct im_muscle_context {
   int32_t ld_params, nbody, nwaypoint, nsegment, ntorque, nmuscle, nrow, nentry, npacked;
   int32_t kind_count[3];
   im_muscle_force_model model;
+  const float *waypoint_table;
+  const uint32_t *segment_table, *length_table, *muscle_table, *groups;
+  const int32_t *group_kinds;
+  int32_t nlength, ngroup;
 } im_muscle_context;
 int im_muscle_from_context(const im_muscle_context *context, int what, const float *in, int64_t ld_in,
                            int root_dof_count, float *out, int64_t ld_out, int nworld, void *stream);

@@ -147,6 +147,8 @@ class MuscleContext(C.Structure):
         ("ld_params", C.c_int32), ("nbody", C.c_int32), ("nwaypoint", C.c_int32), ("nsegment", C.c_int32), ("ntorque", C.c_int32),
         ("nmuscle", C.c_int32), ("nrow", C.c_int32), ("nentry", C.c_int32), ("npacked", C.c_int32),
         ("kind_count", C.c_int32 * 3), ("model", MuscleForceModel),
+        ("waypoint_table", _vp), ("segment_table", _vp), ("length_table", _vp), ("muscle_table", _vp), ("groups", _vp), ("group_kinds", _vp),
+        ("nlength", C.c_int32), ("ngroup", C.c_int32),
     ]  # fmt: skip
 
 

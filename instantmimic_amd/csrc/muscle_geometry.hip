@@ -35,16 +35,16 @@ namespace {
 
 // A workgroup per world up to what the chip keeps resident at once (the workgroups walk over worlds: one that
 // does not get in starts when another has done all its worlds, and the launch takes up to twice as long).
-// Less than the runtime's answer in two ways: a CU hands out its LDS in units of 1280 bytes, and these kernels'
-// scalar registers (85 - 106) leave 24 wavefronts to a CU.  Force-velocity state of 8192 worlds by workgroups per
+// Less than the runtime's answer in two ways: a CU hands out its LDS in units of 1280 bytes, and the scalar registers
+// (85 - 106) of most of these kernels leave 24 wavefronts to a CU (`waves`; 32 with up to 96).  Force-velocity state of 8192 worlds by workgroups per
 // CU: 128 threads, 12: 20.1 us, 13: 23.3; 192 threads, 8: 25.6, 9: 32.5; 256 threads, 6: 47.1, 7: 61.1; 320
 // threads, 4: 68.8, 5: 93.3.
-int resident_grid(const void *fn, int threads, size_t lds, int nworld, unsigned *grid) {
+int resident_grid(const void *fn, int threads, size_t lds, int nworld, unsigned *grid, int waves = 24) {
   int ncu = 0, per_cu = 0;
   if (const int st = compute_units(&ncu)) return st;
   if (const int st = resident_per_cu(fn, nullptr, threads, lds, &per_cu)) return st;
   const size_t unit = 1280, granted = (std::max<size_t>(lds, 1) + unit - 1) / unit * unit;
-  per_cu = std::min({per_cu, (int)(160 * 1024 / granted), 24 * 64 / threads});
+  per_cu = std::min({per_cu, (int)(160 * 1024 / granted), waves * 64 / threads});
   *grid = (unsigned)std::min(nworld, ncu * std::max(1, per_cu));
   return IM_OK;
 }
@@ -591,7 +591,7 @@ struct MwArgs {
   int nworld;
 };
 
-constexpr int kContribPad = 4;  // floats read past the last entry by ordered_sum()
+constexpr int kContribPad = 32;  // floats read past the last entry by ordered_sum()
 constexpr int kAxis = 7;        // floats of a dof's record: its cdof and, for MW_GRAD, grad_output
 struct MwLds {
   float *segd;     // [nseg][9]: dir (0 for a degenerate segment), p0 - c0, p1 - c1
@@ -643,23 +643,30 @@ __device__ __forceinline__ float entry_contribution(const float *lds, const MwEn
   return c;
 }
 
-// Sum of contrib[e0..e1) in list order from +0.  Whole groups of 16 (LONG) and of 4 entries are
-// read with one address and added without a test (sixteen ahead of their additions: 119.6 -> 111.4 us
-// against eight with the next eight on their way, torque of 284 muscles x 8192 worlds); the last group reads up to three floats past
-// e1 (contrib is padded for that) and enters them as +0, which leaves every bit of a sum that
-// started at +0 (such a sum is never -0).
+// Sum of contrib[e0..e1) in list order from +0.  LONG: sixteen entries at a time, the next sixteen on their way while
+// these are added (torque of 284 muscles x 4096 worlds 68.2 -> 65.1 us, gradient 61.2 -> 57.3), otherwise four.  Entries
+// past e1 are read (contrib is padded for that) and enter as +0, which leaves every bit of a sum that started at +0
+// (such a sum is never -0).
 template <bool LONG>
 __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e1) {
   float total = 0.0f;
   int e = e0;
   if (LONG) {
-    for (; e + 16 <= e1; e += 16) {
-      float c[16];
+    float c[16];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
+    for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
+    for (; e + 16 <= e1; e += 16) {
+      float ahead[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) ahead[k] = contrib[e + 16 + k];
 #pragma unroll
       for (int k = 0; k < 16; ++k) total = total + c[k];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) c[k] = ahead[k];
     }
+#pragma unroll
+    for (int k = 0; k < 15; ++k) total = total + (e + k < e1 ? c[k] : 0.0f);
+    return total;
   }
   for (; e + 4 <= e1; e += 4) {
     float c[4];
@@ -863,6 +870,11 @@ bool launch_world(const MwArgs &a, int nworld, hipStream_t stream) {
 // the next world's poses.  4096 worlds of 284 muscles, three workgroups of 512 per CU: torque 80 us where the two
 // launches took 35 + 64, gradient 74 (35 + 49), moment 65 (20 + 58); by counters the vector ALUs issue in 0.75, 0.79 and 0.71
 // of the cycles, the LDS is busy in 0.63, 0.70 and 0.65 (three eighths of that bank conflicts).
+// a value every lane holds alike, as a scalar
+__device__ __forceinline__ float uniform(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
 struct CtxArgs {
   im_muscle_context c;
   const float *in;  // activation (MW_FORWARD) or grad_output (MW_GRAD)
@@ -876,20 +888,24 @@ struct CtxArgs {
 constexpr float kCtxLarge = 1.0e18f;  // two factors below it have a finite product
 constexpr int kCtxTrips = 10;     // packed entries of a thread
 constexpr int kCtxMost = kCtxTrips * 512, kCtxMuscles = 512;
+constexpr int kGroupTrips = 4, kRowTrips = 6;  // groups of a thread
 constexpr int kPose = 8;  // floats of a body's record: u, s s - u.u, 2 s, position
 struct CtxLds {
-  int contrib, segd, axis, force, com, flags, words;
+  int contrib, segd, axis, force, com, flags, dist, words;
 };
+// GROUPS: muscle_groups_kernel's, which keeps the segments' lengths too.
+template <bool GROUPS>
 __host__ __device__ inline CtxLds ctx_lds(const im_muscle_context &c, bool forces) {
   const int sums = c.nentry + kContribPad, points = 3 * c.nwaypoint, records = 9 * c.nsegment, poses = kPose * c.nbody;
   CtxLds l;
   l.contrib = 0;  // the waypoints lie here until the contributions take their place
-  l.segd = sums > points ? sums : points;  // and the bodies' records until the segments' do
+  l.segd = ((sums > points ? sums : points) + 3) & ~3;  // and the bodies' records until the segments' do
   l.axis = l.segd + (records > poses ? records : poses);
   l.force = l.axis + kAxis * c.ntorque;
   l.com = l.force + (forces ? c.nmuscle : 0);
   l.flags = l.com + 3 * c.nbody;
-  l.words = l.flags + 2;
+  l.dist = l.flags + 2;
+  l.words = l.dist + (GROUPS && forces ? c.nlength + 3 : 0);
   return l;
 }
 
@@ -903,6 +919,19 @@ __device__ __forceinline__ float one_end(const float *cd, const float *sd, const
   const V3 ang = ld3(cd), lin = ld3(cd + 3), fv = scale(f, ld3(sd));
   const float v = dot(add(lin, cross(ang, ld3(lever))), fv);
   return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ sign);
+}
+
+// A packed entry into its place by the whole expression, both levers whatever the coefficients.
+template <int MODE>
+__device__ __forceinline__ void full_contribution(float *lds, const CtxLds &l, uint2 e, bool end_only, bool start_only) {
+  const float *sd = lds + l.segd + 9 * (e.x & 0xFFFFu), *cd = lds + l.axis + kAxis * (e.x >> 16);
+  const float f = MODE == MW_MOMENT ? 1.0f : lds[l.force + (e.y >> 16)];
+  const V3 ang = ld3(cd), lin = ld3(cd + 3), fv = scale(f, ld3(sd));
+  const V3 st = add(lin, cross(ang, ld3(sd + 3))), en = add(lin, cross(ang, ld3(sd + 6)));
+  float v = dot(sub(scale(end_only ? 0.0f : 1.0f, st), scale(start_only ? 0.0f : 1.0f, en)), fv);
+  v = f == 0.0f ? 0.0f : v;
+  if (MODE == MW_GRAD) v = cd[6] * v;
+  lds[e.y & 0xFFFFu] = v;
 }
 
 // The kernel's argument block in its argument segment, through a pointer laundered once per phase: held in
@@ -932,7 +961,7 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
   {
     const CtxArgs &a = ctx_args();
     const im_muscle_context &c = a.c;
-    const CtxLds l = ctx_lds(c, FORCES);
+    const CtxLds l = ctx_lds<false>(c, FORCES);
 #pragma unroll
     for (int k = 0; k < TRIPS; ++k) {
       const int e = k * nt + tid;
@@ -953,7 +982,7 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
     {  // poses, centres, axes; activations where the forces will be
       const CtxArgs &a = ctx_args();
       const im_muscle_context &c = a.c;
-      const CtxLds l = ctx_lds(c, FORCES);
+      const CtxLds l = ctx_lds<false>(c, FORCES);
 #pragma unroll
       for (int k = 0; k < WT; ++k) {
         const int i = min(tid + k * nt, c.nwaypoint - 1);
@@ -986,7 +1015,7 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
     float par[3], rest = 0.0f;
     {
       const im_muscle_context &c = ctx_args().c;
-      const CtxLds l = ctx_lds(c, FORCES);
+      const CtxLds l = ctx_lds<false>(c, FORCES);
       if (FORCES) nseg_threads = max(nt - ((c.nmuscle + 63) & ~63), nt / 4);
 #pragma unroll
       for (int k = 0; k < ST; ++k) {
@@ -1020,7 +1049,7 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
     {
       const CtxArgs &a = ctx_args();
       const im_muscle_context &c = a.c;
-      const CtxLds l = ctx_lds(c, FORCES);
+      const CtxLds l = ctx_lds<false>(c, FORCES);
       const float *wpl = lds + l.contrib;
       if (FORCES) {
         const bool passives = MODE == MW_FORWARD && c.model.include_passive;
@@ -1085,7 +1114,7 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
       const CtxArgs &a = ctx_args();
       const int npacked = a.c.npacked, single_end = a.single_end, single = a.single;
       const char *base = (const char *)lds;
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane(((const int *)(lds + ctx_lds(a.c, FORCES).flags))[turn]) == 0, 1)) {
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(((const int *)(lds + ctx_lds<false>(a.c, FORCES).flags))[turn]) == 0, 1)) {
 #pragma unroll
         for (int k = 0; k < TRIPS; ++k) {
           const int first = k * nt + wave;  // the wavefront's entries of this trip are of one kind
@@ -1106,18 +1135,9 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
           if (k % 2) __builtin_amdgcn_sched_barrier(0);
         }
       } else {
-        const CtxLds l = ctx_lds(a.c, FORCES);
-        for (int e = tid; e < npacked; e += nt) {
-          const uint2 t = offsets_of(l, ((const uint2 *)a.c.packed)[e]);
-          const float *sd = (const float *)(base + (t.x & 0xFFFFu)), *cd = (const float *)(base + (t.x >> 16));
-          const float f = MODE == MW_MOMENT ? 1.0f : *(const float *)(base + (t.y >> 16));
-          const V3 ang = ld3(cd), lin = ld3(cd + 3), fv = scale(f, ld3(sd));
-          const V3 st = add(lin, cross(ang, ld3(sd + 3))), en = add(lin, cross(ang, ld3(sd + 6)));
-          float v = dot(sub(scale(e < single_end ? 0.0f : 1.0f, st), scale(e >= single_end && e < single ? 0.0f : 1.0f, en)), fv);
-          v = f == 0.0f ? 0.0f : v;
-          if (MODE == MW_GRAD) v = cd[6] * v;
-          *(float *)((char *)lds + (t.y & 0xFFFFu)) = v;
-        }
+        const CtxLds l = ctx_lds<false>(a.c, FORCES);
+        for (int e = tid; e < npacked; e += nt)
+          full_contribution<MODE>(lds, l, ((const uint2 *)a.c.packed)[e], e < single_end, e >= single_end && e < single);
       }
     }
     asm volatile("" : : "v"(line));
@@ -1126,18 +1146,308 @@ __global__ __launch_bounds__(NT, TRIPS > kCtxTrips ? 5 : 6) void muscle_context_
       const CtxArgs &a = ctx_args();
       for (int r = tid; r < a.c.nrow; r += nt) {
         const float sum = ordered_sum<MODE != MW_MOMENT>(lds, a.c.offsets[r], a.c.offsets[r + 1]);
-        a.out[w * a.ldo + r] = MODE == MW_GRAD && lds[ctx_lds(a.c, FORCES).force + r] == 0.0f ? 0.0f : sum;
+        a.out[w * a.ldo + r] = MODE == MW_GRAD && lds[ctx_lds<false>(a.c, FORCES).force + r] == 0.0f ? 0.0f : sum;
       }
     }
   }
 }
 
-template <int MODE, int NT, int TRIPS>
-int launch_context_on(const CtxArgs &a, hipStream_t stream) {
-  const size_t bytes = 4 * (size_t)ctx_lds(a.c, MODE != MW_MOMENT).words;
+// ---- the same with the list in groups ---------------------------------------------------------
+// What bounds the kernel above is the vector issue rate and the LDS together, and of its 7800 instructions a world (284
+// muscles, torque) the entries' own arithmetic is 2000: the others fetch and unpack each entry's two records, form
+// table addresses for every world, take a muscle's lengths on a lane that waits for the longest.  Here up to three
+// entries share what they have in common.  Torque and gradient: entries of one segment and kind (the dofs of a
+// joint; 2.6 a group), so that the segment's record is read and the force put on its direction once a group.  Moment:
+// a row's whole list on one thread, its dof's record read once and the ordered sum formed in a register.  The 64
+// groups of a wavefront are of one kind and number.  A waypoint's, a segment's and a muscle's table entries are one
+// aligned load each, from tables that are filled up to whole wavefronts; a body's record is two 16-byte reads; every
+// segment's length is taken by a lane of its own, at the price of a barrier.
+// 4096 worlds of 284 muscles, entry by entry -> in groups: torque 78.1 -> 63.1 us, gradient 68.5 -> 56.0, moment 57.9 -> 48.0; 120
+// muscles x 8192 68.1 / 63.2 / 52.2 -> 56.5 / 52.7 / 44.3; 40 x 8192 31.6 / 30.4 / 24.9 -> 29.6 / 28.2 / 24.8.  Of the
+// torque's time the entries are 21 us, waypoints, records and lengths 20, ordered sums 10, forces 6.  Not kept: the dofs'
+// and the segments' records in 8 and 12 words for 16-byte reads (more bank conflicts: 65 / 63 / 53); groups by dof ahead of
+// segment (70 / 64 / 60); eight wavefronts per SIMD for torque and gradient (64 registers, spills).
+template <int MODE, int NT, int TRIPS, int WAVES>
+__global__ __launch_bounds__(NT, WAVES) void muscle_groups_kernel(CtxArgs) {
+  extern __shared__ float lds[];
+  constexpr int nt = NT;
+  constexpr bool FORCES = MODE != MW_MOMENT;
+  int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint4 kept[TRIPS];  // LDS byte offsets, 16 bits each
+  uint64_t kinds = 0;  // six bits a trip; 63: the wavefront has no groups in it
+  float cosine = 1.0f, passive_scale = 1.0f;
+  int turn = 0;
+  {
+    const CtxArgs &a = ctx_args();
+    const im_muscle_context &c = a.c;
+    const CtxLds l = ctx_lds<true>(c, FORCES);
+    const unsigned segd = 4u * l.segd, axis = 4u * l.axis, force = 4u * l.force;
+    auto both = [](unsigned lo, unsigned hi) __attribute__((always_inline)) { return lo | hi << 16; };
+#pragma unroll
+    for (int k = 0; k < TRIPS; ++k) {
+      const int block = k * (nt / 64) + wave;
+      const bool on = 64 * block < c.ngroup;
+      kinds |= (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane(on ? c.group_kinds[on ? block : 0] & 63 : 63) << (6 * k);
+      const uint4 g = ((const uint4 *)c.groups)[(on ? 64 * block : 0) + (tid & 63)];
+      const unsigned x0 = g.x & 0xFFFFu, x1 = g.x >> 16, y0 = g.y & 0xFFFFu, y1 = g.y >> 16, z0 = g.z & 0xFFFFu, z1 = g.z >> 16;
+      if (FORCES)
+        kept[k] = {both(segd + 36 * x0, axis + 4 * kAxis * x1), both(axis + 4 * kAxis * y0, axis + 4 * kAxis * y1), both(force + 4 * z0, 4 * z1),
+                   both(4 * (g.w & 0xFFFFu), 4 * (g.w >> 16))};
+      else
+        kept[k] = {both(axis + 4 * kAxis * x0, 4 * x1), both(segd + 36 * y0, segd + 36 * y1), segd + 36 * z0, 0};
+    }
+    if (FORCES) cosine = cosf(c.params[min(tid, c.nmuscle - 1) * c.ld_params + 3]);
+    if (MODE == MW_FORWARD) passive_scale = uniform(expf(c.model.passive[1]) - 1.0f);
+    if (tid < 2) ((int *)(lds + l.flags))[tid] = 0;
+    __syncthreads();
+  }
+  // Table entries of a phase are asked for a phase ahead, behind its barrier (this many a thread; what is beyond is read
+  // where it is used).
+  constexpr int WT = 3, ST = 2;
+  for (int64_t w = blockIdx.x; w < ctx_args().nworld; w += gridDim.x, turn ^= 1) {
+    asm volatile("" : "+v"(tid));  // (no address formed from it is kept from world to world)
+    const int rid = nt - 1 - tid, rwave = nt - 64 - 64 * wave;
+    float4 wp_tab[WT];
+    {  // poses, centres, axes; activations where the forces will be
+      const CtxArgs &a = ctx_args();
+      const im_muscle_context &c = a.c;
+      const CtxLds l = ctx_lds<true>(c, FORCES);
+#pragma unroll
+      for (int k = 0; k < WT; ++k)
+        if (k * nt + 64 * wave < c.nwaypoint) wp_tab[k] = ((const float4 *)c.waypoint_table + k * nt)[(unsigned)tid];
+      const float *com = c.subtree_com + w * c.ld_subtree_com, *cdof = c.cdof + w * c.ld_cdof + 6 * a.root;
+      for (int i = rid; i < 6 * c.ntorque; i += nt) {
+        const float v = cdof[(unsigned)i];
+        lds[l.axis + i + i / 6] = v;
+        if (!(fabsf(v) < kCtxLarge)) ((int *)(lds + l.flags))[turn] = 1;
+      }
+      for (int b = rid; b < c.nbody; b += nt) {
+        const float *x = c.xpos + w * c.ld_xpos + 3 * b;
+        const BodyTurn t = body_turn(c.xquat + w * c.ld_xquat + 4 * b);
+        float *o = lds + l.segd + kPose * b;
+        *(float4 *)o = {t.u.x, t.u.y, t.u.z, t.k};
+        *(float4 *)(o + 4) = {t.s2, x[0], x[1], x[2]};
+      }
+      for (int i = rid; i < 3 * c.nbody; i += nt) lds[l.com + i] = com[(unsigned)i];
+      const float *in = a.in + w * a.ldin;
+      if (MODE == MW_FORWARD)
+        for (int m = rid; m < c.nmuscle; m += nt) lds[l.force + m] = in[(unsigned)m];
+      if (MODE == MW_GRAD)
+        for (int j = rid; j < c.ntorque; j += nt) lds[l.axis + kAxis * j + 6] = in[(unsigned)j];
+    }
+    __syncthreads();
+    uint2 seg_tab[ST];
+    unsigned len_tab[ST];
+    {
+      const im_muscle_context &c = ctx_args().c;
+      const CtxLds l = ctx_lds<true>(c, FORCES);
+#pragma unroll
+      for (int k = 0; k < ST; ++k) {
+        if (k * nt + rwave < c.nsegment) seg_tab[k] = ((const uint2 *)c.segment_table + k * nt)[(unsigned)rid];
+        if (FORCES && k * nt + 64 * wave < c.nlength) len_tab[k] = (c.length_table + k * nt)[(unsigned)tid];
+      }
+      float *wpl = lds + l.contrib;
+      auto waypoint = [&](int i, float4 t) __attribute__((always_inline)) {
+        const float *o = (const float *)((const char *)(lds + l.segd) + __builtin_bit_cast(unsigned, t.w));
+        const float4 lo = *(const float4 *)o, hi = *(const float4 *)(o + 4);
+        const V3 p = add({hi.y, hi.z, hi.w}, turned({{lo.x, lo.y, lo.z}, lo.w, hi.x}, {t.x, t.y, t.z}));
+        wpl[3 * i] = p.x, wpl[3 * i + 1] = p.y, wpl[3 * i + 2] = p.z;
+      };
+#pragma unroll
+      for (int k = 0; k < WT; ++k)
+        if (tid + k * nt < c.nwaypoint) waypoint(tid + k * nt, wp_tab[k]);
+      for (int i = tid + WT * nt; i < c.nwaypoint; i += nt) waypoint(i, ((const float4 *)c.waypoint_table)[(unsigned)i]);
+      if (tid == 0) ((int *)(lds + l.flags))[turn ^ 1] = 0;
+    }
+    __syncthreads();
+    uint4 run{};
+    float4 par{};
+    {  // segments' records, and every segment's length
+      const im_muscle_context &c = ctx_args().c;
+      const CtxLds l = ctx_lds<true>(c, FORCES);
+      if (FORCES && 64 * wave < c.nmuscle) {
+        run = ((const uint4 *)c.muscle_table)[2u * tid];
+        par = ((const float4 *)c.muscle_table)[2u * tid + 1];
+      }
+      const char *points = (const char *)(lds + l.contrib), *centres = (const char *)(lds + l.com);
+      auto point = [&](unsigned at) __attribute__((always_inline)) { return ld3((const float *)(points + at)); };
+      auto segment = [&](int sg, uint2 t) __attribute__((always_inline)) {
+        const V3 p0 = point(t.x & 0xFFFFu), p1 = point(t.x >> 16);
+        const V3 r0 = sub(p0, ld3((const float *)(centres + (t.y & 0xFFFFu)))), r1 = sub(p1, ld3((const float *)(centres + (t.y >> 16))));
+        const V3 seg = sub(p1, p0);
+        const float len = length(seg);
+        const bool ok = !(len < 1.0e-8f);  // (as in muscle_world_kernel)
+        float *o = lds + l.segd + 9 * sg;
+        o[0] = ok ? seg.x / len : 0.0f;
+        o[1] = ok ? seg.y / len : 0.0f;
+        o[2] = ok ? seg.z / len : 0.0f;
+        o[3] = r0.x, o[4] = r0.y, o[5] = r0.z;
+        o[6] = r1.x, o[7] = r1.y, o[8] = r1.z;
+        const float all = fabsf(r0.x) + fabsf(r0.y) + fabsf(r0.z) + fabsf(r1.x) + fabsf(r1.y) + fabsf(r1.z);
+        if (!(all < kCtxLarge)) ((int *)(lds + l.flags))[turn] = 1;
+      };
+      auto distance = [&](unsigned at) __attribute__((always_inline)) { return length(sub(point(at + 12), point(at))); };
+#pragma unroll
+      for (int k = 0; k < ST; ++k)
+        if (rid + k * nt < c.nsegment) segment(rid + k * nt, seg_tab[k]);
+      for (int sg = rid + ST * nt; sg < c.nsegment; sg += nt) segment(sg, ((const uint2 *)c.segment_table)[(unsigned)sg]);
+      if (FORCES) {
+#pragma unroll
+        for (int k = 0; k < ST; ++k)
+          if (tid + k * nt < c.nlength) lds[l.dist + tid + k * nt] = distance(len_tab[k]);
+        for (int i = tid + ST * nt; i < c.nlength; i += nt) lds[l.dist + i] = distance(c.length_table[(unsigned)i]);
+      }
+    }
+    __syncthreads();
+    float line = 0.0f;
+    int e0 = 0, e1 = 0;  // the list of the thread's first row
+    {  // the next world's rows are brought into the L2 beside what follows: a line each 16 floats of a row
+      const CtxArgs &a = ctx_args();
+      const im_muscle_context &c = a.c;
+      const int64_t next = w + gridDim.x < a.nworld ? w + gridDim.x : w;
+      const int nin = MODE == MW_MOMENT ? 0 : MODE == MW_FORWARD ? c.nmuscle : c.ntorque;
+      if (16 * rwave < 10 * c.nbody + 6 * c.ntorque + nin + 5 * 16) {  // (no lane of the other wavefronts has a line)
+        int i = 16 * rid;
+        auto touch = [&](const float *row, int n) __attribute__((always_inline)) {
+          if (i >= 0 && i < n) line = row[i];
+          i -= (n + 15) & ~15;
+        };
+        touch(c.xpos + next * c.ld_xpos, 3 * c.nbody);
+        touch(c.xquat + next * c.ld_xquat, 4 * c.nbody);
+        touch(c.subtree_com + next * c.ld_subtree_com, 3 * c.nbody);
+        touch(c.cdof + next * c.ld_cdof + 6 * a.root, 6 * c.ntorque);
+        if (MODE != MW_MOMENT) touch(a.in + next * a.ldin, nin);
+      }
+      if (64 * wave < c.nrow && tid < c.nrow) e0 = c.offsets[(unsigned)tid], e1 = c.offsets[(unsigned)tid + 1];
+    }
+    if constexpr (FORCES) {
+      const im_muscle_context &c = ctx_args().c;
+      const CtxLds l = ctx_lds<true>(c, FORCES);
+      const bool passives = MODE == MW_FORWARD && c.model.include_passive;
+      if (tid < c.nmuscle) {
+        const float *dist = lds + l.dist + run.x;
+        const int count = (int)run.y;
+        float len = 0.0f;
+        for (int s = 0; s < count; s += 4) {  // (up to three past the muscle's last one are read and left out)
+          float d[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) d[k] = dist[s + k];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) len = s + k < count ? len + d[k] : len;
+        }
+        const float lengths[3] = {__builtin_bit_cast(float, run.z), __builtin_bit_cast(float, run.w), par.x};
+        float unit, passive;
+        force_of_length(len, lengths, par.y, cosine, passive_scale, c.model, &unit, MODE == MW_FORWARD ? &passive : nullptr);
+        if (MODE == MW_FORWARD) {
+          unit = unit * lds[l.force + tid];
+          if (passives) unit = unit + passive;
+        }
+        lds[l.force + tid] = unit;
+      }
+      __syncthreads();
+    }
+    const bool large = __builtin_amdgcn_readfirstlane(((const int *)(lds + ctx_lds<true>(ctx_args().c, FORCES).flags))[turn]) != 0;
+    {
+      char *base = (char *)lds;
+      auto at = [&](unsigned byte) __attribute__((always_inline)) { return (const float *)(base + byte); };
+      auto vec = [&](unsigned byte) __attribute__((always_inline)) { return ld3(at(byte)); };
+      struct Dof {
+        V3 ang, lin;
+        float gout;
+      };
+      auto dof = [&](unsigned byte) __attribute__((always_inline)) {
+        return Dof{vec(byte), vec(byte + 12), MODE == MW_GRAD ? at(byte)[6] : 0.0f};
+      };
+      if (__builtin_expect(!large, 1)) {
+        asm volatile("" : "+s"(kinds));  // (nor is what follows from these)
+#pragma unroll
+        for (int k = 0; k < TRIPS; ++k) {
+          const int kind = (int)(kinds >> (6 * k)) & 63;
+          if (kind == 63) break;
+          uint4 g = kept[k];
+          asm volatile("" : "+v"(g.x), "+v"(g.y), "+v"(g.z), "+v"(g.w));  // (their parts are not kept from world to world)
+          if constexpr (FORCES) {
+            const unsigned sd = g.x & 0xFFFFu;
+            const float f = *at(g.z & 0xFFFFu);
+            const V3 fv = scale(f, vec(sd));
+            auto put = [&](unsigned place, float v, float gout) __attribute__((always_inline)) {
+              v = f == 0.0f ? 0.0f : v;
+              if (MODE == MW_GRAD) v = gout * v;
+              *(float *)(base + place) = v;
+            };
+            auto all = [&](auto one) __attribute__((always_inline)) {
+              if (kind >> 2 == 3) {
+                const Dof d0 = dof(g.x >> 16), d1 = dof(g.y & 0xFFFFu), d2 = dof(g.y >> 16);
+                put(g.z >> 16, one(d0), d0.gout), put(g.w & 0xFFFFu, one(d1), d1.gout), put(g.w >> 16, one(d2), d2.gout);
+              } else {
+                const Dof d0 = dof(g.x >> 16);
+                put(g.z >> 16, one(d0), d0.gout);
+                if (kind >> 2 == 2) {
+                  const Dof d1 = dof(g.y & 0xFFFFu);
+                  put(g.w & 0xFFFFu, one(d1), d1.gout);
+                }
+              }
+            };
+            if ((kind & 3) == 2) {
+              const V3 r0 = vec(sd + 12), r1 = vec(sd + 24);
+              all([&](const Dof &d) __attribute__((always_inline)) { return dot(sub(add(d.lin, cross(d.ang, r0)), add(d.lin, cross(d.ang, r1))), fv); });
+            } else {
+              const V3 r = vec(sd + ((kind & 3) == 0 ? 24 : 12));
+              const unsigned sign = (kind & 3) == 0 ? 0x80000000u : 0u;
+              all([&](const Dof &d) __attribute__((always_inline)) {
+                return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, dot(add(d.lin, cross(d.ang, r)), fv)) ^ sign);
+              });
+            }
+          } else {
+            const Dof d = dof(g.x & 0xFFFFu);
+            float total = 0.0f;
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+              const int one = (kind >> (2 * s)) & 3;
+              if (one == 3) break;
+              const unsigned sd = s == 0 ? g.y & 0xFFFFu : s == 1 ? g.y >> 16 : g.z;
+              const V3 dir = vec(sd);
+              float v;
+              if (one == 2) {
+                v = dot(sub(add(d.lin, cross(d.ang, vec(sd + 12))), add(d.lin, cross(d.ang, vec(sd + 24)))), dir);
+              } else {
+                v = dot(add(d.lin, cross(d.ang, vec(sd + (one == 0 ? 24 : 12)))), dir);
+                v = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ (one == 0 ? 0x80000000u : 0u));
+              }
+              total = total + v;
+            }
+            *(float *)(base + (g.x >> 16)) = total;
+          }
+        }
+      } else {
+        const CtxArgs &a = ctx_args();
+        const CtxLds l = ctx_lds<true>(a.c, FORCES);
+        for (int e = tid; e < a.c.npacked; e += nt) full_contribution<MODE>(lds, l, ((const uint2 *)a.c.packed)[e], e < a.single_end, e >= a.single_end && e < a.single);
+      }
+    }
+    asm volatile("" : : "v"(line));
+    __syncthreads();
+    {
+      const CtxArgs &a = ctx_args();
+      float *out = a.out + w * a.ldo;
+      for (int r = tid; r < a.c.nrow; r += nt) {
+        if (r != tid) e0 = a.c.offsets[r], e1 = a.c.offsets[r + 1];
+        if (MODE == MW_MOMENT)
+          out[(unsigned)r] = large ? ordered_sum<false>(lds, e0, e1) : lds[r];
+        else
+          out[(unsigned)r] = MODE == MW_GRAD && lds[ctx_lds<true>(a.c, FORCES).force + r] == 0.0f ? 0.0f : ordered_sum<true>(lds, e0, e1);
+      }
+    }
+  }
+}
+
+template <int NT>
+int launch_resident(void (*kernel)(CtxArgs), int words, const CtxArgs &a, hipStream_t stream, int waves = 24) {
+  const size_t bytes = 4 * (size_t)words;
   unsigned grid = 0;
-  if (const int st = resident_grid((const void *)muscle_context_kernel<MODE, NT, TRIPS>, NT, bytes, a.nworld, &grid)) return st;
-  hipLaunchKernelGGL((muscle_context_kernel<MODE, NT, TRIPS>), dim3(grid), dim3(NT), bytes, stream, a);
+  if (const int st = resident_grid((const void *)kernel, NT, bytes, a.nworld, &grid, waves)) return st;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), bytes, stream, a);
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
 }
@@ -1152,10 +1462,21 @@ int launch_context(const CtxArgs &a, hipStream_t stream) {
   const int packed = a.c.npacked, muscles = MODE == MW_MOMENT ? 0 : a.c.nmuscle;
   int ncu = 0;
   if (const int st = compute_units(&ncu)) return st;
-  if (packed <= kCtxTrips * 128 && muscles <= 128) return launch_context_on<MODE, 128, kCtxTrips>(a, stream);
-  if (packed <= kCtxTrips * 256 && muscles <= 256) return launch_context_on<MODE, 256, kCtxTrips>(a, stream);
-  if (packed <= 14 * 256 && muscles <= 256 && a.nworld > 6 * ncu) return launch_context_on<MODE, 256, 14>(a, stream);
-  return launch_context_on<MODE, 512, kCtxTrips>(a, stream);
+  constexpr int trips = MODE == MW_MOMENT ? kRowTrips : kGroupTrips;
+  const int groups = a.c.ngroup, with_lengths = ctx_lds<true>(a.c, MODE != MW_MOMENT).words, words = ctx_lds<false>(a.c, MODE != MW_MOMENT).words;
+  // Groups: the same, with four groups a thread (six rows for the moment), and between 1024 and 1536 groups 256 threads with
+  // six each for such batches: 200 muscles x 8192 97.1 / 84.4 -> 88.7 / 82.4 us, x 2048 28.1 / 24.8 -> 26.7 / 25.2.
+  if (groups > 0 && 4 * (size_t)with_lengths <= 64 * 1024) {
+    if (groups <= trips * 128 && muscles <= 128) return launch_resident<128>(muscle_groups_kernel<MODE, 128, trips, 6>, with_lengths, a, stream, 32);
+    if (groups <= trips * 256 && muscles <= 256) return launch_resident<256>(muscle_groups_kernel<MODE, 256, trips, 6>, with_lengths, a, stream, 32);
+    if constexpr (MODE != MW_MOMENT)
+      if (groups <= 6 * 256 && muscles <= 256 && a.nworld > 6 * ncu) return launch_resident<256>(muscle_groups_kernel<MODE, 256, 6, 5>, with_lengths, a, stream, 32);
+    if (groups <= trips * 512) return launch_resident<512>(muscle_groups_kernel<MODE, 512, trips, 6>, with_lengths, a, stream, 32);
+  }
+  if (packed <= kCtxTrips * 128 && muscles <= 128) return launch_resident<128>(muscle_context_kernel<MODE, 128, kCtxTrips>, words, a, stream);
+  if (packed <= kCtxTrips * 256 && muscles <= 256) return launch_resident<256>(muscle_context_kernel<MODE, 256, kCtxTrips>, words, a, stream);
+  if (packed <= 14 * 256 && muscles <= 256 && a.nworld > 6 * ncu) return launch_resident<256>(muscle_context_kernel<MODE, 256, 14>, words, a, stream);
+  return launch_resident<512>(muscle_context_kernel<MODE, 512, kCtxTrips>, words, a, stream);
 }
 
 bool geo_ok(const im_muscle_geometry *g) {
@@ -1511,7 +1832,7 @@ extern "C" int im_muscle_from_context(const im_muscle_context *context, int what
       c.kind_count[0] < 0 || c.kind_count[1] < 0 || c.kind_count[2] < 0 || c.kind_count[0] % 64 || c.kind_count[1] % 64 || c.ld_params < 4)
     return IM_ERR_ARG;
   if (c.npacked > kCtxMost || (what != IM_MUSCLE_MOMENT && c.nmuscle > kCtxMuscles) || 4 * (size_t)c.nentry + 16 * (size_t)c.nwaypoint + 36 * (size_t)c.nsegment + 28 * (size_t)c.ntorque + 8 * (size_t)c.nmuscle > 256 * 1024 ||
-      c.nbody > 65535 || 4 * (size_t)ctx_lds(c, true).words > 64 * 1024)
+      c.nbody > 65535 || 4 * (size_t)ctx_lds<false>(c, true).words > 64 * 1024)
     return IM_ERR_UNSUPPORTED;
   static const bool forced_off = [] {
     const char *e = std::getenv("IMHIP_MUSCLE_KERNEL");
@@ -1521,6 +1842,10 @@ extern "C" int im_muscle_from_context(const im_muscle_context *context, int what
   if (nworld == 0) return IM_OK;
   if (!c.xpos || !c.xquat || !c.subtree_com || !c.cdof || !c.waypoint_body || !c.waypoint_local || !c.start_waypoint || !c.end_waypoint ||
       !c.start_root_body || !c.end_root_body || !c.offsets || !c.packed || ((uintptr_t)c.packed & 7) || !out)
+    return IM_ERR_ARG;
+  if (c.ngroup < 0 || c.ngroup % 64 || (c.ngroup > 0 && (c.nlength < 0 || c.nlength > 256 * 1024))) return IM_ERR_ARG;
+  if (c.ngroup > 0 && (!c.waypoint_table || !c.segment_table || !c.muscle_table || !c.length_table || !c.groups || !c.group_kinds ||
+                       (((uintptr_t)c.waypoint_table | (uintptr_t)c.segment_table | (uintptr_t)c.muscle_table | (uintptr_t)c.groups) & 15)))
     return IM_ERR_ARG;
   if (what != IM_MUSCLE_MOMENT && (!c.all_segment_start || !c.all_segment_offsets || !c.params || !c.rest || !in)) return IM_ERR_ARG;
   if (c.ld_xpos < 0 || c.ld_xquat < 0 || c.ld_subtree_com < 0 || c.ld_cdof < 0 || ld_in < 0 || ld_out < c.nrow ||

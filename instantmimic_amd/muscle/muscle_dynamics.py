@@ -17,7 +17,7 @@ once on the host with NumPy.
 from __future__ import annotations
 
 import ctypes as C
-from dataclasses import dataclass, field
+from dataclasses import dataclass
 
 import numpy as np
 
@@ -185,9 +185,88 @@ def pack_context_entries(segment, torque, muscle, start_coeff, end_coeff):
     return np.concatenate(words).astype(np.uint32), counts
 
 
-@dataclass
-class _Tables:
-    keep: list = field(default_factory=list)
+def _groups_by_kind(kind, columns, fill):
+    """Groups ordered by ``kind`` (descending), each kind's filled up to whole wavefronts; (words, kind of every 64)."""
+    order = np.argsort(-kind, kind="stable")
+    counts = np.bincount(kind, minlength=1)[::-1]
+    values = np.flatnonzero(counts)
+    counts = counts[values]
+    blocks = -(-counts // 64)
+    first = 64 * (np.cumsum(blocks) - blocks) - (np.cumsum(counts) - counts)
+    at = np.arange(len(kind)) + np.repeat(first, counts)
+    out = np.empty((64 * int(blocks.sum()), 4), np.uint32)
+    for k in range(4):
+        out[:, k] = fill[k]
+        out[at, k] = columns[k][order]
+    return out, np.repeat(kind.max(initial=0) - values, blocks).astype(np.int32)
+
+
+def group_context_entries(segment, torque, muscle, start_coeff, end_coeff):
+    """The torque's or the gradient's list in groups of up to three entries of one segment and kind (of a list that
+    ``pack_context_entries`` takes): (groups (n, 4) uint32, kind | entries << 2 of every 64 groups)."""
+    segment, torque, muscle = (np.asarray(a, np.int64) for a in (segment, torque, muscle))
+    n = len(segment)
+    kind = np.where(np.asarray(start_coeff) == 0, 0, np.where(np.asarray(end_coeff) == 0, 1, 2))
+    key = (kind << 16 | segment) << 16 | torque
+    order = np.argsort(key)
+    key = key[order] >> 16
+    run = np.flatnonzero(np.concatenate([[True], key[1:] != key[:-1]]))
+    at = np.arange(n) - np.repeat(run, np.diff(np.append(run, n)))  # an entry's number in its segment and kind
+    head = np.flatnonzero(at % 3 == 0)
+    size = np.diff(np.append(head, n))
+    place, dof, key = np.append(order, [n, n]), np.append(torque[order], [0, 0]), key[head]
+    p = [place[head], np.where(size > 1, place[head + 1], n), np.where(size > 2, place[head + 2], n)]
+    d = [dof[head], np.where(size > 1, dof[head + 1], 0), np.where(size > 2, dof[head + 2], 0)]
+    columns = (key & 0xFFFF | d[0] << 16, d[1] | d[2] << 16, muscle[p[0]] | p[0] << 16, p[1] | p[2] << 16)
+    return _groups_by_kind(key >> 16 | size << 2, columns, (0, 0, n << 16, n | n << 16))
+
+
+def group_context_rows(offsets, segment, row_torque, start_coeff, end_coeff):
+    """The moment's list with a row's entries, up to three, in a group: (groups (n, 4) uint32, the kinds of every
+    64 groups), or None where a row has more or none."""
+    offsets, segment, row_torque = (np.asarray(a, np.int64) for a in (offsets, segment, row_torque))
+    a, b, n, count = np.asarray(start_coeff), np.asarray(end_coeff), len(segment), np.diff(offsets)
+    if count.min(initial=1) < 1 or count.max(initial=0) > 3:
+        return None
+    kind = np.append(np.where(a == 0, 0, np.where(b == 0, 1, 2)), [3, 3])
+    segment, e = np.append(segment, [0, 0]), offsets[:-1]
+    seg = [segment[e], np.where(count > 1, segment[e + 1], 0), np.where(count > 2, segment[e + 2], 0)]
+    kinds = kind[e] | np.where(count > 1, kind[e + 1], 3) << 2 | np.where(count > 2, kind[e + 2], 3) << 4
+    columns = (row_torque | np.arange(len(count)) << 16, seg[0] | seg[1] << 16, seg[2], np.zeros_like(count))
+    return _groups_by_kind(kinds, columns, (n << 16, 0, 0, 0))
+
+
+def _filled(words):
+    """Rows of a table up to a multiple of 64, zeros behind them."""
+    return np.concatenate([words, np.zeros((-len(words) % 64, words.shape[1]), words.dtype)]).astype(np.uint32).view(np.int32)
+
+
+class _DeviceTables:
+    """Tables of 4-byte words in one allocation on the device, copied there at once: a copy from pageable memory costs the
+    same for 100 KB as for one word (24 tables: 0.9 ms)."""
+
+    def __init__(self, device, words: int):
+        import torch
+
+        self._host, self._used = np.empty(words, np.int32), 0
+        self._device = torch.empty(words, dtype=torch.int32, device=device)
+
+    def add(self, a):
+        """The table's place on the device, filled by ``copy``."""
+        import torch
+
+        a = np.ascontiguousarray(a)
+        if self._used + a.size + 3 > len(self._host):  # (more than was asked for: a copy of its own)
+            return torch.from_numpy(a).to(self._device.device)
+        at = slice(self._used, self._used + a.size)
+        self._host[at] = a.reshape(-1).view(np.int32)
+        self._used += (a.size + 3) & ~3
+        return self._device[at].view({np.dtype(np.int32): torch.int32, np.dtype(np.float32): torch.float32}[a.dtype]).view(a.shape)
+
+    def copy(self):
+        import torch
+
+        self._device[: self._used].copy_(torch.from_numpy(self._host[: self._used]))
 
 
 def _stream(t) -> int:
@@ -280,11 +359,8 @@ class MuscleDynamicsLayer:
 
     # ------------------------------------------------------------------ device tables
     def _upload(self):
-        import torch
-
-        def up(a):
-            return torch.from_numpy(np.ascontiguousarray(a)).to(self.device)
-
+        tables = _DeviceTables(self.device, self._table_words())
+        up = tables.add
         d = self._dev
         d["seg"] = [up(a) for a in self.segments_host]
         d["tq"] = [up(a) for a in (self.torque_entries_host[i] for i in (0, 2, 3, 4, 5))]
@@ -313,6 +389,12 @@ class MuscleDynamicsLayer:
         self._muscle_entries = entries(d["ms"], self.muscle_count, self.torque_dim)
         self._moment_entries = entries(d["mom"], len(e.muscle_dof_torque_idx), self.torque_dim, other=False)
         self._upload_context(up)
+        tables.copy()
+
+    def _table_words(self) -> int:
+        """At least the words of all tables, each filled up to 16 bytes."""
+        entries, rows, t = len(self.torque_entries_host[2]), len(self.sparse_entries.muscle_dof_torque_idx), self.torque_entries_host
+        return 40 * entries + 12 * rows + 12 * self.muscle_count + 8 * self.waypoint_count + 12 * len(self.segments_host[0]) + self.muscle_params.size + 8 * len(t[0]) + 40 * 1024
 
     def _upload_context(self, up):
         """The argument blocks of im_muscle_from_context, one per output; an output whose entry list or
@@ -327,6 +409,7 @@ class MuscleDynamicsLayer:
         )
         self._context = [None, None, None]
         d["packed"] = []
+        tables = self._context_tables(up)
         for what, (offsets, nrow, entries) in enumerate(lists):
             packed = pack_context_entries(*entries)
             if packed is None:
@@ -342,9 +425,36 @@ class MuscleDynamicsLayer:
                 nentry=len(entries[0]), npacked=len(words), kind_count=(C.c_int32 * 3)(*counts), model=self._model,
             )  # fmt: skip
             c.start_waypoint, c.end_waypoint, c.start_root_body, c.end_root_body = (s.data_ptr() for s in d["seg"])
+            grouped = (
+                group_context_rows(e.muscle_dof_segment_offsets, e.segment_idx, e.muscle_dof_torque_idx, e.start_coeff, e.end_coeff)
+                if what == _MOMENT else group_context_entries(*entries)
+            )  # fmt: skip
+            keep = [t]
+            if grouped is not None and tables is not None:
+                keep += [up(grouped[0].view(np.int32)), up(grouped[1])]
+                c.groups, c.group_kinds = (x.data_ptr() for x in keep[1:])
+                c.waypoint_table, c.segment_table, c.length_table, c.muscle_table = (x.data_ptr() for x in tables)
+                c.nlength, c.ngroup = len(self.all_segment_start_idx), len(grouped[0])
             if _lib.lib().im_muscle_from_context(C.byref(c), what, None, 0, self.root_dof_count, None, nrow, 0, None) == 0:
                 self._context[what] = c
-                d["packed"].append(t)
+                d["packed"] += keep
+
+    def _context_tables(self, up):
+        """The waypoints', segments' and muscles' table entries as im_muscle_from_context loads them beside groups;
+        None where a byte offset of a waypoint does not fit 16 bits."""
+        if 12 * self.waypoint_count >= 65536 or 12 * self.body_count >= 65536:
+            return None
+        words = lambda a: np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.int64)  # noqa: E731
+        p0, p1, c0, c1 = (12 * a.astype(np.int64) for a in self.segments_host)
+        first, count = self.all_muscle_segment_offsets[:-1].astype(np.int64), np.diff(self.all_muscle_segment_offsets)
+        zero = np.zeros_like(first)
+        tables = (
+            np.concatenate([words(self.waypoints_local), 32 * self.waypoint_body[:, None].astype(np.int64)], 1),
+            np.stack([p0 | p1 << 16, c0 | c1 << 16], 1), 12 * self.all_segment_start_idx[:, None].astype(np.int64),
+            np.stack([first, count, *words(self.muscle_params[:, :3].T), words(self.muscle_rest_length), zero, zero], 1),
+        )  # fmt: skip
+        self._dev["context_tables"] = [up(_filled(a)) for a in tables]
+        return self._dev["context_tables"]
 
     def _need_gpu(self, *tensors):
         import torch

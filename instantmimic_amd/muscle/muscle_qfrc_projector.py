@@ -48,20 +48,14 @@ class MuscleDofSparseEntries:
 
 
 def _pairs(muscle_dof_offsets: np.ndarray):
-    pi, pj, pm = [], [], []
-    for muscle in range(len(muscle_dof_offsets) - 1):
-        b, e = int(muscle_dof_offsets[muscle]), int(muscle_dof_offsets[muscle + 1])
-        n = e - b
-        if n <= 0:
-            continue
-        ii, jj = np.tril_indices(n)
-        pi.append(b + ii)
-        pj.append(b + jj)
-        pm.append(np.full(ii.size, muscle))
-    if not pi:
-        z = np.zeros(0, np.int32)
-        return z, z.copy(), z.copy()
-    return (np.concatenate(a).astype(np.int32) for a in (pi, pj, pm))
+    first, count = np.asarray(muscle_dof_offsets[:-1], np.int64), np.diff(muscle_dof_offsets)
+    row = np.arange(first[0] if len(first) else 0, muscle_dof_offsets[-1])  # every entry i ...
+    start = np.repeat(first, count)
+    width = row - start + 1  # ... pairs with the muscle's entries up to itself
+    pi = np.repeat(row, width)
+    pj = np.repeat(start - np.cumsum(width) + width, width) + np.arange(int(width.sum()))
+    pm = np.repeat(np.repeat(np.arange(len(count)), count), width)
+    return (a.astype(np.int32) for a in (pi, pj, pm))
 
 
 def build_muscle_dof_sparse_entries(
