@@ -825,3 +825,90 @@ def test_gpu_groups_equal_the_list_entry_by_entry(muscles):
             c.ngroup = n
         for x, y in zip(got, want):
             assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+def test_gpu_torque_call_is_the_dispatchers_operator():
+    """``ops.muscle_torque_forward`` in eager code with a gradient to record against the operator of that name through
+    the dispatcher: values, gradients, what autograd refuses, what modes and hooks see."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from torch.utils.checkpoint import checkpoint
+
+    rig = synth.make_muscle_rig(nmuscle=12, seed=3)
+    layer = _gpu_layer(rig)
+    key, nworld = ops.warp_op_key(layer), 33
+    ctx = torch.from_numpy(synth.make_muscle_context(rig, nworld, seed=4)).cuda()
+    act = torch.rand(nworld, 12, device="cuda", requires_grad=True)
+    g = torch.randn(nworld, rig.torque_dim, device="cuda")
+    many = torch.rand(2, nworld, 12, device="cuda")
+    direct, dispatched = ops.muscle_torque_forward, torch.ops.instantmimic_muscle.torque_forward
+    assert type(direct(act, ctx, key, True).grad_fn).__name__ != type(dispatched(act, ctx, key, True).grad_fn).__name__
+
+    def outcome(f):
+        try:
+            return [t.detach().clone() for t in f()]
+        except Exception as e:  # noqa: BLE001
+            return type(e)
+
+    def same(f):
+        a, b = outcome(lambda: f(direct)), outcome(lambda: f(dispatched))
+        if isinstance(a, type) or isinstance(b, type):
+            assert a is b
+        else:
+            assert len(a) == len(b) and all(torch.equal(x, y) for x, y in zip(a, b))
+        return a
+
+    def twice(op):
+        y = op(act, ctx, key, False)
+        return [y, *torch.autograd.grad(y, act, g, retain_graph=True), *torch.autograd.grad(y, act, 2 * g)]
+
+    def second(op):
+        (ga,) = torch.autograd.grad(op(act, ctx, key, False), act, g.clone().requires_grad_(True), create_graph=True)
+        return torch.autograd.grad(ga.sum(), act)
+
+    def changed(op):
+        c = ctx.clone()
+        y = op(act, c, key, False)
+        c.add_(1.0)
+        return torch.autograd.grad(y, act, g)
+
+    def context_gradient(op):
+        c = ctx.clone().requires_grad_(True)
+        return torch.autograd.grad(op(act, c, key, False).sum(), [act, c], allow_unused=True)[:1]
+
+    assert not isinstance(same(twice), type)
+    for f in (second, changed):
+        assert issubclass(same(f), RuntimeError)
+    same(context_gradient)
+    same(lambda op: torch.autograd.grad(op(act, ctx, key, False), act, g, create_graph=True))
+    same(lambda op: [torch.func.grad(lambda a: (op(a, ctx, key, False) * g).sum())(act.detach())])
+    same(lambda op: [torch.func.vmap(lambda a: op(a, ctx, key, False))(many)])
+    same(lambda op: [torch.autograd.grad(op(act, ctx, key, False), act, torch.stack([g, g]), is_grads_batched=True)[0]])
+    same(lambda op: [torch.func.jvp(lambda a: op(a, ctx, key, False), (act.detach(),), (act.detach(),))[1]])
+    same(lambda op: torch.autograd.grad(checkpoint(lambda a: op(a, ctx, key, True), act, use_reentrant=False), act, g))
+    same(lambda op: [op(act.detach(), ctx, key, False), op(act.double(), ctx, key, False)])
+    same(lambda op: [op(act[:, :5], ctx, key, False)])
+    same(lambda op: [op(act, ctx[:, :9], key, False)])
+    same(lambda op: [op(act, ctx, 10**9, False)])
+
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        direct(act, ctx, key, False)
+    assert "instantmimic_muscle.torque_forward.default" in seen
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.cpu(), lambda t: t.cuda()):
+        y = direct(act, ctx, key, False)
+    assert packed == [ctx.shape] and torch.equal(torch.autograd.grad(y, act, g)[0], same(twice)[1])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        y = direct(act, ctx, key, False)
+        got = torch.autograd.grad(y, act, g)[0]
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got, same(twice)[1])
