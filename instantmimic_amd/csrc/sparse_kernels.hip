@@ -27,7 +27,22 @@ namespace {
 struct SparseDev {
   const int32_t *t[NHOST];
   int nv, nv_pad, nslots, nlevels;
+  // for a wavefront per world (null beyond 64 dofs)
+  const uint32_t *steps;  // the factor's, then the backward solve's
+  const uint16_t *dof_pairs;
+  int nfactor_steps, nbackward_steps;
 };
+// words of a plan's steps, the factor's first (a step more of each: the one read ahead of the last)
+__host__ __device__ inline int factor_step_words(const SparseDev &P) { return 128 * (P.nfactor_steps + 1); }
+__host__ __device__ inline int step_words(const SparseDev &P) { return factor_step_words(P) + 64 * (P.nbackward_steps + 1); }
+SparseDev sparse_dev(const im_sparse_plan &plan) {
+  SparseDev P;
+  for (int i = 0; i < NHOST; ++i) P.t[i] = plan.t[i];
+  P.nv = plan.nv, P.nv_pad = plan.nv_pad, P.nslots = plan.nslots, P.nlevels = plan.nlevels;
+  P.steps = plan.steps, P.dof_pairs = plan.dof_pairs;
+  P.nfactor_steps = plan.nfactor_steps, P.nbackward_steps = plan.nbackward_steps;
+  return P;
+}
 
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
@@ -44,17 +59,11 @@ __device__ __forceinline__ float row_shl(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N, 0xF, 0xF, true));
 }
 
-// Orders LDS writes before later reads: across the workgroup, or, when a world belongs to
-// one wavefront (WAVE), across that wavefront only.
-template <bool WAVE>
+// Orders a wavefront's LDS writes before its later reads, where a world belongs to one wavefront.
 __device__ __forceinline__ void sync_world() {
-  if (WAVE) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  } else {
-    __syncthreads();
-  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // level-scheduled numeric factor: team lanes stride an entry's terms, shuffle-down tree.
@@ -62,7 +71,7 @@ __device__ __forceinline__ void sync_world() {
 // so `block` may be any multiple of the widest team.
 // One level with the team width T as a compile-time constant: the operands of a lane's next four
 // terms then lie at constant distances, which the LDS instructions carry themselves.
-template <bool WAVE, int T>
+template <int T>
 __device__ __forceinline__ void factor_level(const SparseDev &P, float *N, float *iD, int lane, int block, int e0,
                                              int e1) {
   const int32_t *ESt = P.t[ES], *ECt = P.t[EC], *RPt = P.t[RP];
@@ -111,28 +120,26 @@ __device__ __forceinline__ void factor_level(const SparseDev &P, float *N, float
   }
 }
 
-template <bool WAVE = false>
 __device__ __forceinline__ void factor_levels(const SparseDev &P, float *N, float *iD, int lane, int block) {
   const int32_t *LPt = P.t[LP], *LTt = P.t[LT];
   for (int l = 0; l < P.nlevels; ++l) {
     const int e0 = LPt[l], e1 = LPt[l + 1];
     switch (LTt[l]) {  // team widths are powers of two
-      case 1: factor_level<WAVE, 1>(P, N, iD, lane, block, e0, e1); break;
-      case 2: factor_level<WAVE, 2>(P, N, iD, lane, block, e0, e1); break;
-      case 4: factor_level<WAVE, 4>(P, N, iD, lane, block, e0, e1); break;
-      case 8: factor_level<WAVE, 8>(P, N, iD, lane, block, e0, e1); break;
-      case 16: factor_level<WAVE, 16>(P, N, iD, lane, block, e0, e1); break;
-      case 32: factor_level<WAVE, 32>(P, N, iD, lane, block, e0, e1); break;
-      default: factor_level<WAVE, 64>(P, N, iD, lane, block, e0, e1); break;
+      case 1: factor_level<1>(P, N, iD, lane, block, e0, e1); break;
+      case 2: factor_level<2>(P, N, iD, lane, block, e0, e1); break;
+      case 4: factor_level<4>(P, N, iD, lane, block, e0, e1); break;
+      case 8: factor_level<8>(P, N, iD, lane, block, e0, e1); break;
+      case 16: factor_level<16>(P, N, iD, lane, block, e0, e1); break;
+      case 32: factor_level<32>(P, N, iD, lane, block, e0, e1); break;
+      default: factor_level<64>(P, N, iD, lane, block, e0, e1); break;
     }
-    sync_world<WAVE>();
+    __syncthreads();
   }
 }
 
 // backward pushes by level (root first), search = -x, (x.x, g.x) reduced warp then block.
 // `nthreads` lanes work on the world; the two dot products are summed as a block of `block`
 // lanes would (the plan's width: it fixes which terms a lane adds and in which order).
-template <bool WAVE = false>
 __device__ __forceinline__ void backward_sums(const SparseDev &P, float *N, const float *iD,
                                               const float *__restrict__ gw, float *__restrict__ search,
                                               float *red, float *search_dot, float *decrement, int lane,
@@ -149,7 +156,7 @@ __device__ __forceinline__ void backward_sums(const SparseDev &P, float *N, cons
         const int i = (u >> 16) & 0xFF, j = u >> 24;
         N[rhs + j] = fma_(-N[u & 0xFFFFu], N[rhs + i] * iD[i], N[rhs + j]);
       }
-      sync_world<WAVE>();
+      __syncthreads();
     }
   } else {
     for (int l = 0; l < P.nlevels; ++l) {
@@ -157,7 +164,7 @@ __device__ __forceinline__ void backward_sums(const SparseDev &P, float *N, cons
         const int i = BIt[p], j = BJt[p];
         N[rhs + j] = fma_(-N[BSt[p]], N[rhs + i] * iD[i], N[rhs + j]);
       }
-      sync_world<WAVE>();
+      __syncthreads();
     }
   }
   float s0 = 0.0f, s1 = 0.0f;
@@ -176,13 +183,120 @@ __device__ __forceinline__ void backward_sums(const SparseDev &P, float *N, cons
     red[lane >> 5] = s0;
     red[nw + (lane >> 5)] = s1;
   }
-  sync_world<WAVE>();
+  __syncthreads();
   if (lane == 0) {
     float ra = 0.0f, rb = 0.0f;
     for (int i = 0; i < nw; ++i) {
       ra = ra + red[i];
       rb = rb + red[nw + i];
     }
+    *search_dot = ra;
+    *decrement = rb;
+  }
+}
+
+// ---- the same for a wavefront per world, from the plan's steps ----------------------------------------
+// A level's teams are the same for every world and every round, so what a lane does in it is settled when the plan is
+// uploaded: a step is one word pair a lane (operands' first words and number of terms, the entry's slot and column), the
+// team's width and whether a sum starts or ends in the step alike in all lanes.  A workgroup's worlds share a copy in LDS
+// (12 KB at 35 dofs), read a step ahead.  From the tables a level waited for three LDS reads, one behind the other, before the first operand,
+// and spent two thirds of its instructions on them and their addresses; a short run's terms were read one by one.
+// Same operations in the same order.  Whole solves, from the tables -> from the steps: 35 dofs x 8192 worlds with 96 rows
+// 779 -> 661 us, x 100 with 40 rows 312 -> 252, 56 dofs x 4096 with 128 rows 892 -> 763, 62 dofs x 1000 498 -> 431.
+constexpr int kStepTerms = 4;  // terms' operands read ahead of their products
+template <int T>
+__device__ __forceinline__ float step_terms(const float *pa, const float *pb, const float *pd, int n, float v) {
+  int t = 0;
+  do {
+    float a[kStepTerms], b[kStepTerms], d[kStepTerms];
+#pragma unroll
+    for (int u = 0; u < kStepTerms; ++u) a[u] = pa[(t + u) * T], b[u] = pb[(t + u) * T], d[u] = pd[(t + u) * T];
+    asm volatile("" : "+v"(a[0]), "+v"(b[0]), "+v"(d[0]));  // (not behind a branch of the lanes that have a term)
+#pragma unroll
+    for (int u = 0; u < kStepTerms; ++u) v = t + u < n ? fma_(a[u] * b[u], d[u], v) : v;
+    t += kStepTerms;
+  } while (__ballot(t < n) != 0ull);
+  return v;
+}
+// `rec`: the plan's factor steps in LDS, one more word pair a lane behind the last
+__device__ __forceinline__ void factor_steps(const uint2 *rec, int steps, float *N, float *iD, int lane) {
+  float v = 0.0f;
+  uint2 ahead = rec[lane];
+  for (int s = 0; s < steps; ++s) {
+    const uint2 r = ahead;
+    ahead = rec[lane + 64 * (s + 1)];
+    const unsigned info = (unsigned)__builtin_amdgcn_readfirstlane((int)r.y) >> 26;
+    const float *pa = N + (r.x & 0xFFFu), *pb = N + (r.x >> 12 & 0xFFFu), *pd = iD + (r.y & 63u);
+    const int n = r.y >> 6 & 127u, slot = (int)(r.y >> 13 & 0xFFFu) - 1, col = (int)(r.x >> 24) - 1;
+    const float old = N[slot < 0 ? 0 : slot];
+    if (info & 8u) v = 0.0f;
+    float sum;
+    if ((info & 7u) == 0u) {
+      sum = v = step_terms<1>(pa, pb, pd, n, v);
+    } else {
+      switch (info & 7u) {
+        case 1: v = step_terms<2>(pa, pb, pd, n, v); break;
+        case 2: v = step_terms<4>(pa, pb, pd, n, v); break;
+        case 3: v = step_terms<8>(pa, pb, pd, n, v); break;
+        case 4: v = step_terms<16>(pa, pb, pd, n, v); break;
+        case 5: v = step_terms<32>(pa, pb, pd, n, v); break;
+        default: v = step_terms<64>(pa, pb, pd, n, v); break;
+      }
+      // the team's shuffle-down tree (as in factor_level)
+      sum = v;
+      if ((info & 7u) > 5) sum = sum + __shfl_down(sum, 32, 64);
+      if ((info & 7u) > 4) sum = sum + __shfl_down(sum, 16, 64);
+      if ((info & 7u) > 3) sum = sum + row_shl<8>(sum);
+      if ((info & 7u) > 2) sum = sum + row_shl<4>(sum);
+      if ((info & 7u) > 1) sum = sum + row_shl<2>(sum);
+      sum = sum + row_shl<1>(sum);
+    }
+    if (info & 16u) {
+      if (slot >= 0) {
+        const float wv = old - sum;
+        N[slot] = wv;
+        if (col >= 0) iD[col] = 1.0f / wv;
+      }
+      sync_world();
+    }
+  }
+}
+// `rec`: the backward solve's
+__device__ __forceinline__ void backward_steps(const uint32_t *rec, int steps, int rhs, float *N, const float *iD, int lane) {
+  uint32_t ahead = rec[lane];
+  for (int s = 0; s < steps; ++s) {
+    const uint32_t r = ahead;
+    ahead = rec[lane + 64 * (s + 1)];
+    const int i = r >> 12 & 63u, j = r >> 18 & 63u;
+    const float f = N[r & 0xFFFu], x = N[rhs + i] * iD[i], y = N[rhs + j];
+    if (r >> 31) N[rhs + j] = fma_(-f, x, y);
+    sync_world();
+  }
+}
+// The search direction and its two sums; `block` lanes add as the plan's block would.
+__device__ __forceinline__ void search_sums(int n, int rhs, const float *N, const float *iD, const int32_t *ORIGt,
+                                            const float *__restrict__ gw, float *__restrict__ search, float *search_dot,
+                                            float *decrement, int lane, int block) {
+  const int d = ORIGt[lane < n ? lane : 0], d2 = ORIGt[lane + 32 < n ? lane + 32 : 0];
+  const float g = gw[d], g2 = block == 32 ? gw[d2] : 0.0f;
+  float s0 = 0.0f, s1 = 0.0f;
+  if (lane < n && lane < block) {
+    const float v = N[rhs + lane] * iD[lane];
+    search[d] = -v;
+    s0 = fma_(v, v, s0);
+    s1 = fma_(g, v, s1);
+    if (lane + block < n) {  // (two dofs a lane in a block of 32)
+      const float u = N[rhs + lane + 32] * iD[lane + 32];
+      search[d2] = -u;
+      s0 = fma_(u, u, s0);
+      s1 = fma_(g2, u, s1);
+    }
+  }
+  search::swap_rows(s0, s1);  // both sums through one tree (as in resident::search_sums_world)
+  const float sum = search::row_sum(s0 + s1);
+  float ra = 0.0f + search::lane_of(sum, 0), rb = 0.0f + search::lane_of(sum, 16);
+  if (block > 32) ra = ra + search::lane_of(sum, 32), rb = rb + search::lane_of(sum, 48);
+  if (lane == 0) {
     *search_dot = ra;
     *decrement = rb;
   }
@@ -367,7 +481,7 @@ __global__ void sparse_init_kernel(SparseDev P, const uint8_t *__restrict__ done
 }
 
 // ---- initial factor, one wavefront per world --------------------------------------------
-// Four worlds per workgroup share one LDS copy of the factor and solve tables; each world
+// Four worlds per workgroup; each world
 // belongs to one wavefront, so its LDS traffic needs no workgroup barrier.  J'DJ is summed
 // on the matrix cores: v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one
 // after the other with a fused multiply-add each, rows ascending, which is the order and
@@ -375,19 +489,50 @@ __global__ void sparse_init_kernel(SparseDev P, const uint8_t *__restrict__ done
 // product J[r][a] * Dc[r]; the accumulators start from M.  The lower-triangle 16 x 16 tiles
 // hold every (a, b) pair, and the plan's slots pick theirs (pairs outside the pattern are
 // dropped, as in the reference, and their rows counted).
-constexpr int kStaged = 12;  // tables LP .. BJ, the ones the factor and the solves read
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct SparseWave {
   SparseDev P;
-  int staged[kStaged];        // offsets in words from the first table (the plan stores them back to back)
-  int staged_words;           // length of that stretch, a multiple of 4
   int solve[5];               // update stage only: offsets of the forward-solve tables FL .. RK from FL
-  int solve_words;            // length of that stretch, a multiple of 4 (0: not staged)
+  int solve_words;            // length of that stretch and of ORIG behind it, multiples of 4
+  int staged_steps;           // words of steps in LDS: all or none
   const int32_t *tile_index;  // [tile][4][64]: (index into M + 1) << 16 | (slot + 1), 0 = none
   int block, nM;              // the plan's block width; length of a row of M
   int staged_rows;            // update stage: changed rows of J a world keeps in LDS, 16 or 32 (more are read from memory)
 };
+
+// Steps of more than 36 KB (a chain of 47 dofs, or patterns whose entries have several runs: a step of their teams for each)
+// would leave a CU few worlds: they are read from memory, which 35 dofs x 8192 worlds, whose own are 12 KB, took 700 us
+// per solve with, 661 from LDS and 779 from the tables.
+constexpr int kStagedStepsMost = 9216;
+inline int staged_steps(const SparseDev &P) { return step_words(P) <= kStagedStepsMost ? step_words(P) : 0; }
+// The plan's factor and backward solve on one world.
+template <class Steps>
+__device__ __forceinline__ void with_steps(const SparseWave &A, const int32_t *lds, Steps &&run) {
+  if (A.staged_steps)
+    run((const uint32_t *)lds);
+  else
+    run(A.P.steps);
+}
+
+// `words` (a multiple of 4) from 16-byte aligned memory into LDS by T threads, eight loads of 16 bytes in flight a thread.
+template <int T>
+__device__ __forceinline__ void copy_words(int32_t *to, const void *from, int words, int tid) {
+  const int4 *src = (const int4 *)from;
+  const int nvec = words >> 2;
+  for (int q0 = tid; q0 < nvec; q0 += 8 * T) {
+    int4 buf[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) buf[i] = src[q0 + i * T < nvec ? q0 + i * T : nvec - 1];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (q0 + i * T < nvec) ((int4 *)to)[q0 + i * T] = buf[i];
+  }
+}
+
+// (the factor's steps read up to 3 * 64 words past an operand's last term, which they leave out)
+constexpr int kStepSlack = (kStepTerms - 1) * 64;
+__host__ __device__ inline int init_world_words(int nslots, int n) { return (nslots + n + kStepSlack + 3) & ~3; }
 
 template <int NT>
 __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
@@ -400,38 +545,17 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
   extern __shared__ float lds[];
   const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, kq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: world data is addressed from scalar registers
-  SparseDev Q = A.P;
-  int32_t *tab = (int32_t *)lds;
-  {
-    // one flat copy, every load issued before the first store (up to 32 KB)
-    const int4 *src = (const int4 *)A.P.t[0];
-    const int nvec = A.staged_words >> 2;
-    int4 buf[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int q = i * 256 + tid;
-      buf[i] = src[q < nvec ? q : nvec - 1];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int q = i * 256 + tid;
-      if (q < nvec) ((int4 *)tab)[q] = buf[i];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kStaged; ++i) Q.t[i] = tab + A.staged[i];
-  const int off = A.staged_words;
+  const SparseDev &Q = A.P;
+  copy_words<256>((int32_t *)lds, Q.steps, A.staged_steps, tid);
   __syncthreads();  // the only workgroup barrier: worlds are independent from here on
   const int w = blockIdx.x * 4 + wv;
   if (w >= nworld || (done && done[w])) return;
   const int n = Q.nv, nslots = Q.nslots, nfac = nslots - n, rhs = nfac;
-  const int nw = (A.block + 31) / 32;
-  const int njp = (njmax + 3) & ~3, factor_words = (nslots + n + 2 * nw + 3) & ~3;
+  const int njp = (njmax + 3) & ~3, factor_words = init_world_words(nslots, n);
   const int per_world = factor_words + 2 * njp;
-  float *N = lds + ((off + 3) & ~3) + wv * per_world;  // [nslots]; a row of M before the factor
-  float *iD = N + nslots;                              // [n]
-  float *red = iD + n;                                 // [2][nw]
-  float *dl = N + factor_words;                        // [njp] weights of the listed constraint rows
+  float *N = lds + A.staged_steps + wv * per_world;  // [nslots]; a row of M before the factor
+  float *iD = N + nslots;                           // [n]
+  float *dl = N + factor_words;                     // [njp] weights of the listed constraint rows
   int *rowl = (int *)(dl + njp);                       // [njp] their numbers
   float *U = U_ + (size_t)w * Q.nv_pad * Q.nv_pad;
   const float *Mw = M + (size_t)w * ldM;
@@ -508,7 +632,7 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
 #pragma unroll
   for (int c = 0; c < 16; ++c)
     if (c * 64 + lane < A.nM) N[c * 64 + lane] = mv[c];
-  sync_world<true>();
+  sync_world();
   f32x4 acc[NTILE];
 #pragma unroll
   for (int t = 0; t < NTILE; ++t)
@@ -518,7 +642,7 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
       const float m = N[mi < 0 ? 0 : mi];
       acc[t][v] = mi >= 0 ? m : 0.0f;
     }
-  sync_world<true>();
+  sync_world();
   int nbad = 0;
   for (int s0 = 0; s0 < steps; s0 += PD) {
 #pragma unroll
@@ -590,16 +714,20 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
       const int sl = (tix[t][v] & 0xFFFF) - 1;
       if (sl >= 0) N[sl] = acc[t][v];
     }
-  sync_world<true>();
+  sync_world();
   for (int s = lane; s < nfac; s += 64) U[s] = N[s];
   const int32_t *ORIGt = Q.t[ORIG];
   for (int j = lane; j < n; j += 64) N[rhs + j] = gw[ORIGt[j]];
-  sync_world<true>();
-  factor_levels<true>(Q, N, iD, lane, 64);
+  sync_world();
+  with_steps(A, (const int32_t *)lds, [&](const uint32_t *steps) __attribute__((always_inline)) {
+    factor_steps((const uint2 *)steps, Q.nfactor_steps, N, iD, lane);
+  });
   for (int s = lane; s < nfac; s += 64) U[nfac + s] = N[s];
   for (int j = lane; j < n; j += 64) U[2 * nfac + j] = iD[j];
-  backward_sums<true>(Q, N, iD, gw, search_ + (size_t)w * n, red, search_dot + w, decrement + w, lane, 64,
-                      A.block);
+  with_steps(A, (const int32_t *)lds, [&](const uint32_t *steps) __attribute__((always_inline)) {
+    backward_steps(steps + factor_step_words(Q), Q.nbackward_steps, rhs, N, iD, lane);
+  });
+  search_sums(n, rhs, N, iD, ORIGt, gw, search_ + (size_t)w * n, search_dot + w, decrement + w, lane, A.block);
   if (nbad && lane == 0) atomicAdd(U + Q.nv_pad * Q.nv_pad - 1, (float)nbad);
 }
 
@@ -612,57 +740,25 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
 // read different dofs meet in no LDS bank.  32 rows where that costs a CU no world, 16 otherwise.
 constexpr int kStagedRowsMax = 32;
 
-// The factor and solve tables of a plan into LDS, for a workgroup of T threads (a flat 16-byte copy,
-// every load issued before the first store); Q's table pointers then address the copy.
+// The steps of a plan, its forward solve's tables and its dofs' order into LDS, for a workgroup of T threads.
+__device__ __forceinline__ int orig_at(const SparseWave &A) { return A.solve_words - ((A.P.nv + 3) & ~3); }
 template <int T>
-__device__ __forceinline__ void stage_update_tables(const SparseWave &A, SparseDev &Q, float *lds, int tid) {
+__device__ __forceinline__ void stage_update_tables(const SparseWave &A, float *lds, int tid) {
   int32_t *tab = (int32_t *)lds;
-  {
-    const int4 *src = (const int4 *)A.P.t[0];
-    const int nvec = A.staged_words >> 2;
-    constexpr int NB = (2048 + T - 1) / T;  // the host admits at most 8192 words
-    int4 buf[NB];
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int q = i * T + tid;
-      buf[i] = src[q < nvec ? q : nvec - 1];
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int q = i * T + tid;
-      if (q < nvec) ((int4 *)tab)[q] = buf[i];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kStaged; ++i) Q.t[i] = tab + A.staged[i];
-  {
-    // forward-solve tables (at most 16 KB), behind the first stretch
-    const int4 *src = (const int4 *)A.P.t[FL];
-    const int nvec = A.solve_words >> 2;
-    constexpr int NB = (1024 + T - 1) / T;  // at most 4096 words
-    int4 buf[NB];
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int q = i * T + tid;
-      buf[i] = src[q < nvec ? q : 0];
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int q = i * T + tid;
-      if (q < nvec) ((int4 *)(tab + A.staged_words))[q] = buf[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 5; ++i) Q.t[FL + i] = tab + A.staged_words + A.solve[i];
-  }
+  copy_words<T>(tab, A.P.steps, A.staged_steps, tid);
+  tab += A.staged_steps;
+  const int orig = orig_at(A);
+  copy_words<T>(tab, A.P.t[FL], orig, tid);
+  if (tid < A.P.nv) tab[orig + tid] = A.P.t[ORIG][tid];
 }
-__host__ __device__ inline int update_world_words(int nslots, int n, int block, int staged_rows) {
-  const int nw = (block + 31) / 32;
-  return (nslots + n + 2 * nw + 2 * n + (staged_rows + 1) * n + staged_rows + 3) & ~3;
+__host__ __device__ inline int update_world_words(int nslots, int n, int staged_rows) {
+  const int factor = nslots + n + 2 * n + (staged_rows + 1) * n + staged_rows, reach = nslots + n + kStepSlack;
+  return ((factor > reach ? factor : reach) + 3) & ~3;
 }
 
 // The stage for one world and one wavefront (`world_lds`: update_world_words of LDS of its own).
 __device__ __forceinline__ void sparse_update_world(
-    const SparseWave &A, const SparseDev &Q, float *world_lds, const int32_t *__restrict__ changes,
+    const SparseWave &A, const int32_t *shared, float *world_lds, int count,
     const int32_t *__restrict__ ids, int ld_ids, const float *__restrict__ J, int njmax,
     const float *__restrict__ D, const int32_t *__restrict__ state, int quad, const float *__restrict__ grad, int ldg,
     float *__restrict__ U_, int32_t *__restrict__ uni_, float *__restrict__ search_, float *__restrict__ search_dot,
@@ -671,12 +767,12 @@ __device__ __forceinline__ void sparse_update_world(
   // are then worked out where a round uses them instead of each holding a register from round to round.
   int lane = lane_in;
   asm volatile("" : "+v"(lane));
+  const SparseDev &Q = A.P;
+  const int32_t *tables = shared + A.staged_steps;
   const int n = Q.nv, nslots = Q.nslots, nfac = nslots - n, rhs = nfac;
-  const int nw = (A.block + 31) / 32;
-  float *N = world_lds;  // [nslots]
+  float *N = world_lds;                              // [nslots]
   float *iD = N + nslots;                            // [n]
-  float *red = iD + n;                               // [2][nw]
-  int *ul = (int *)(red + 2 * nw);                   // [n] ascending dofs touched by the changed rows
+  int *ul = (int *)(iD + n);                         // [n] ascending dofs touched by the changed rows
   unsigned *mkl = (unsigned *)(ul + n);              // [n] per dof: bit t set where staged row t is nonzero there
   const int cap = A.staged_rows, stride = cap + 1;
   float *jr = (float *)(mkl + n);                    // [n][stride] changed rows of J, a dof's elements together
@@ -686,8 +782,7 @@ __device__ __forceinline__ void sparse_update_world(
   const float *Jw = J + (size_t)w * njmax * n;
   const float *Dw = D + (size_t)w * njmax;
   const int32_t *sw = state + (size_t)w * njmax, *idw = ids + (size_t)w * ld_ids;
-  const int32_t *ORIGt = Q.t[ORIG];
-  int count = changes[w];
+  const int32_t *ORIGt = tables + orig_at(A);
   count = count < ld_ids ? count : ld_ids;
   count = __builtin_amdgcn_readfirstlane(count);
 #ifdef IM_NEWTON_STAMPS  // development aid: time per part of the stage, summed over the rounds, left in the world's dof-union row
@@ -782,23 +877,23 @@ __device__ __forceinline__ void sparse_update_world(
 #endif
     const int32_t *PAIRt = Q.t[PAIR];
     int nbad = 0;
-    sync_world<true>();  // `ul`, `mkl` and the staged rows are read from here on
+    sync_world();  // `ul`, `mkl` and the staged rows are read from here on
     IM_SSTAMP(0);
     const int npair = nu * (nu + 1) / 2;
     for (int e0 = lane; e0 < npair; e0 += 4 * 64) {
-      int row[4], col[4], sl[4];
+      int row[4], col[4], sl[4], pairs[4];
       bool live[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         live[k] = e0 + 64 * k < npair;
-        const int e = live[k] ? e0 + 64 * k : npair - 1;
-        // e = cj (cj + 1) / 2 + ri with ri <= cj, found exactly (walking the pairs in 8 x 8 blocks
-        // of (ri, cj) instead, without this arithmetic, was measured a quarter slower)
-        int cj = (int)((sqrtf((float)(8 * e + 1)) - 1.0f) * 0.5f);
-        while ((cj + 1) * (cj + 2) / 2 <= e) ++cj;
-        while (cj * (cj + 1) / 2 > e) --cj;
-        row[k] = ul[e - cj * (cj + 1) / 2];
-        col[k] = ul[cj];
+        pairs[k] = Q.dof_pairs[(unsigned)(live[k] ? e0 + 64 * k : npair - 1)];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        // (e = c (c + 1) / 2 + r by table: worked out, with a root and two corrections, it took sixty instructions a pair)
+        const int pair = pairs[k];
+        row[k] = ul[pair & 255];
+        col[k] = ul[pair >> 8];
         sl[k] = PAIRt[row[k] * n + col[k]];
       }
 #pragma unroll
@@ -840,15 +935,19 @@ __device__ __forceinline__ void sparse_update_world(
         }
       }
     }
-    for (int o = 32; o > 0; o >>= 1) nbad += __shfl_down(nbad, o, 64);
-    if (lane == 0 && nbad) atomicAdd(U + Q.nv_pad * Q.nv_pad - 1, (float)nbad);
-    sync_world<true>();
+    if (__ballot(nbad != 0) != 0ull) {
+      for (int o = 32; o > 0; o >>= 1) nbad += __shfl_down(nbad, o, 64);
+      if (lane == 0) atomicAdd(U + Q.nv_pad * Q.nv_pad - 1, (float)nbad);
+    }
+    sync_world();
     IM_SSTAMP(1);
     for (int s = lane; s < nfac; s += 64) U[s] = N[s];
     for (int j = lane; j < n; j += 64) N[rhs + j] = gw[ORIGt[j]];
-    sync_world<true>();
+    sync_world();
     IM_SSTAMP(2);
-    factor_levels<true>(Q, N, iD, lane, 64);
+    with_steps(A, shared, [&](const uint32_t *steps) __attribute__((always_inline)) {
+      factor_steps((const uint2 *)steps, Q.nfactor_steps, N, iD, lane);
+    });
     IM_SSTAMP(3);
     for (int s = lane; s < nfac; s += 64) U[nfac + s] = N[s];
     for (int j = lane; j < n; j += 64) U[2 * nfac + j] = iD[j];
@@ -860,8 +959,8 @@ __device__ __forceinline__ void sparse_update_world(
       iD[j] = U[2 * nfac + j];
       gl[j] = gw[ORIGt[j]];
     }
-    sync_world<true>();
-    const int32_t *FLt = Q.t[FL], *FRt = Q.t[FR], *RSt = Q.t[RS], *RKPt = Q.t[RKP], *RKt = Q.t[RK];
+    sync_world();
+    const int32_t *FLt = tables + A.solve[0], *FRt = tables + A.solve[1], *RSt = tables + A.solve[2], *RKPt = tables + A.solve[3], *RKt = tables + A.solve[4];
     for (int l = 0; l < Q.nlevels; ++l) {
       for (int q = FLt[l] + lane; q < FLt[l + 1]; q += 64) {
         const int j = FRt[q];
@@ -885,12 +984,14 @@ __device__ __forceinline__ void sparse_update_world(
         }
         N[rhs + j] = v;
       }
-      sync_world<true>();
+      sync_world();
     }
     IM_SSTAMP(5);
   }
-  backward_sums<true>(Q, N, iD, gw, search_ + (size_t)w * n, red, search_dot + w, decrement + w, lane, 64,
-                      A.block);
+  with_steps(A, shared, [&](const uint32_t *steps) __attribute__((always_inline)) {
+    backward_steps(steps + factor_step_words(Q), Q.nbackward_steps, rhs, N, iD, lane);
+  });
+  search_sums(n, rhs, N, iD, ORIGt, gw, search_ + (size_t)w * n, search_dot + w, decrement + w, lane, A.block);
   IM_SSTAMP(6);
 #undef IM_SSTAMP
 }
@@ -906,13 +1007,12 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void sparse_update_wave_ker
   extern __shared__ float lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  SparseDev Q = A.P;
-  stage_update_tables<64 * WAVES>(A, Q, lds, tid);
+  stage_update_tables<64 * WAVES>(A, lds, tid);
   __syncthreads();  // the only workgroup barrier
   const int w = blockIdx.x * WAVES + wv;
   if (w >= nworld || (done && done[w]) || state_changes[w] == 0) return;
-  float *world_lds = lds + A.staged_words + A.solve_words + wv * update_world_words(Q.nslots, Q.nv, A.block, A.staged_rows);
-  sparse_update_world(A, Q, world_lds, changes, ids, ld_ids, J, njmax, D, state, quad, grad, ldg, U_, uni_, search_,
+  float *world_lds = lds + A.staged_steps + A.solve_words + wv * update_world_words(A.P.nslots, A.P.nv, A.staged_rows);
+  sparse_update_world(A, (const int32_t *)lds, world_lds, changes[w], ids, ld_ids, J, njmax, D, state, quad, grad, ldg, U_, uni_, search_,
                       search_dot, decrement, w, lane);
 }
 
@@ -920,8 +1020,8 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void sparse_update_wave_ker
 // line search to convergence, WAVES worlds per workgroup sharing one copy of the plan's tables.
 // Per wavefront in LDS: the world's row of M and the search direction, and one area that the staged
 // tile of J, the gradient's row list and the stage's factor use one after the other.
-__host__ __device__ inline int resident_area_words(int nslots, int n, int block, int njmax, int staged_rows) {
-  int words = update_world_words(nslots, n, block, staged_rows);
+__host__ __device__ inline int resident_area_words(int nslots, int n, int njmax, int staged_rows) {
+  int words = update_world_words(nslots, n, staged_rows);
   const int tile = 64 * 17, grad = 2 * njmax + n;
   words = words > tile ? words : tile;
   words = words > grad ? words : grad;
@@ -934,12 +1034,11 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
   extern __shared__ float lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  SparseDev Q = A.P;
-  stage_update_tables<64 * WAVES>(A, Q, lds, tid);
+  stage_update_tables<64 * WAVES>(A, lds, tid);
   const int nv = a.nv, njmax = a.njmax, nworld = a.nworld;
-  uint32_t *term = (uint32_t *)(lds + A.staged_words + A.solve_words);
+  uint32_t *term = (uint32_t *)(lds + A.staged_steps + A.solve_words);
   int *radr = (int *)(term + a.nterm);
-  const int area = resident_area_words(Q.nslots, nv, A.block, njmax, A.staged_rows);
+  const int area = resident_area_words(A.P.nslots, nv, njmax, A.staged_rows);
   // (M is read from memory by the round's one product with it: its row would cost a CU a third of its worlds)
   float *mine = (float *)(radr + nv + 1) + wv * (area + resident::kept_words(nv, njmax, 0));
   resident::LoopLds L;
@@ -971,7 +1070,11 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
                                     alignof(resident::NewtonArgs));
   auto stage = [&]() __attribute__((always_inline)) {
     const resident::NewtonArgs &b = resident::kernel_args(kArgsOffset);
-    sparse_update_world(A, Q, mine, b.quad_count, b.ids, b.ld_ids, b.J, b.njmax, b.D, b.state, b.quad, b.grad,
+    // the plan's block from the argument segment as well: its pointers held from round to round would be spilled
+    typedef const SparseWave __attribute__((address_space(4))) KernelSparseWave;
+    KernelSparseWave *plan = (KernelSparseWave *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(plan));
+    sparse_update_world(*(const SparseWave *)plan, (const int32_t *)lds, mine, b.quad_count[w], b.ids, b.ld_ids, b.J, b.njmax, b.D, b.state, b.quad, b.grad,
                         (int)b.ld_grad, U_, uni_, b.search, b.search_dot, b.decrement, (int)w, threadIdx.x & 63);
   };
   while (w < nworld) {
@@ -1131,6 +1234,63 @@ extern "C" {
 
 namespace im {
 
+namespace {
+// A plan's levels as the steps of a wavefront's 64 lanes (factor_steps, backward_steps).
+struct WaveSteps {
+  std::vector<uint32_t> words;  // the factor's, an empty one, the backward solve's, an empty one
+  std::vector<uint16_t> pairs;
+  int nfactor = 0, nbackward = 0;
+};
+WaveSteps wave_steps(const im_sparse_plan &pl) {
+  WaveSteps out;
+  std::vector<uint32_t> factor, backward;
+  const auto &T = pl.table;
+  for (int l = 0; l < pl.nlevels; ++l) {
+    const int width = T[LT][l], teams = 64 / width;
+    int log2 = 0;
+    while ((1 << log2) < width) ++log2;
+    for (int e0 = T[LP][l]; e0 < T[LP][l + 1]; e0 += teams) {
+      int runs = 1;
+      for (int e = e0; e < std::min(e0 + teams, T[LP][l + 1]); ++e) runs = std::max(runs, T[RP][e + 1] - T[RP][e]);
+      for (int r = 0; r < runs; ++r)
+        for (int lane = 0; lane < 64; ++lane) {
+          const int e = e0 + lane / width, tl = lane % width;
+          uint32_t x = 0, y = (uint32_t)log2 << 26 | (uint32_t)(r == 0) << 29 | (uint32_t)(r == runs - 1) << 30;
+          if (e < T[LP][l + 1]) {
+            if (r < T[RP][e + 1] - T[RP][e]) {
+              const uint32_t ab = (uint32_t)T[RAB][T[RP][e] + r], kl = (uint32_t)T[RKL][T[RP][e] + r];
+              const int terms = ((int)(kl >> 16) - tl + width - 1) / width;
+              if ((int)(kl >> 16) > tl) {
+                x = ((ab & 0xFFFFu) + tl) | ((ab >> 16) + tl) << 12;
+                y |= ((kl & 0xFFFFu) + tl) | (uint32_t)terms << 6;
+              }
+            }
+            if (r == runs - 1 && tl == 0) {
+              y |= (uint32_t)(T[ES][e] + 1) << 13;
+              x |= (uint32_t)(T[EC][e] + 1) << 24;
+            }
+          }
+          factor.push_back(x);
+          factor.push_back(y);
+        }
+    }
+    for (int p0 = T[BL][l]; p0 < T[BL][l + 1]; p0 += 64)
+      for (int lane = 0; lane < 64; ++lane) {
+        const int p = p0 + lane;
+        backward.push_back(p < T[BL][l + 1] ? (uint32_t)T[BS][p] | (uint32_t)T[BI][p] << 12 | (uint32_t)T[BJ][p] << 18 | 1u << 31 : 0u);
+      }
+  }
+  out.nfactor = (int)(factor.size() / 128), out.nbackward = (int)(backward.size() / 64);
+  factor.resize(factor.size() + 128, 0);
+  backward.resize(backward.size() + 64, 0);
+  out.words = std::move(factor);
+  out.words.insert(out.words.end(), backward.begin(), backward.end());
+  for (int c = 0; c < 64; ++c)
+    for (int r = 0; r <= c; ++r) out.pairs.push_back((uint16_t)(r | c << 8));
+  return out;
+}
+}  // namespace
+
 int sparse_plan_upload(im_sparse_plan *pl) {
   pl->device_ready = false;
   // the kernels' workgroup widths; 128 lanes only in the upstream-iteration kernel
@@ -1145,9 +1305,27 @@ int sparse_plan_upload(im_sparse_plan *pl) {
   }
   std::vector<char> host(total, 0);
   for (int i = 0; i < NHOST; ++i) memcpy(host.data() + offs[i], pl->table[i].data(), pl->table[i].size() * 4);
+  WaveSteps steps;
+  size_t steps_at[2] = {0, 0};
+  if (nv <= 64 && pl->block <= 64) {
+    steps = wave_steps(*pl);
+    const void *from[2] = {steps.words.data(), steps.pairs.data()};
+    const size_t bytes[2] = {steps.words.size() * 4, steps.pairs.size() * 2};
+    for (int i = 0; i < 2; ++i) {
+      steps_at[i] = total;
+      total += (bytes[i] + 15) / 16 * 16;
+      host.resize(total, 0);
+      memcpy(host.data() + steps_at[i], from[i], bytes[i]);
+    }
+  }
   IM_HIP_CHECK(hipMalloc(&pl->blob, total + 16));  // behind the tables: the resident Newton kernel's world counter
   IM_HIP_CHECK(hipMemcpy(pl->blob, host.data(), total, hipMemcpyHostToDevice));
   pl->next_world = (int *)((char *)pl->blob + total);
+  if (!steps.words.empty()) {
+    pl->steps = (const uint32_t *)((char *)pl->blob + steps_at[0]);
+    pl->dof_pairs = (const uint16_t *)((char *)pl->blob + steps_at[1]);
+    pl->nfactor_steps = steps.nfactor, pl->nbackward_steps = steps.nbackward;
+  }
   for (int i = 0; i < NHOST; ++i) pl->t[i] = (const int32_t *)((char *)pl->blob + offs[i]);
   if (nv <= 64 && pl->nslots < 65535 && !pl->table[SA].empty()) {
     const int32_t *sa = pl->table[SA].data(), *sb = pl->table[SB].data(), *sm = pl->table[SM].data();
@@ -1203,29 +1381,25 @@ int im_sparse_init_factor(const im_sparse_plan *plan, const uint8_t *done, const
   if (nworld == 0) return IM_OK;
   if (!nefc || !J || !D || !state || !M || !grad || !hfactor || !search || !search_dot || !decrement) return IM_ERR_ARG;
   if (ldg < plan->nv || ldM < plan->nM) return IM_ERR_STRIDE;
-  im::SparseDev P;
-  for (int i = 0; i < im::NHOST; ++i) P.t[i] = plan->t[i];
-  P.nv = plan->nv; P.nv_pad = plan->nv_pad; P.nslots = plan->nslots; P.nlevels = plan->nlevels;
+  const im::SparseDev P = im::sparse_dev(*plan);
   const int n = plan->nv, words = (n + 31) / 32, nw = (plan->block + 31) / 32;
   static const bool simple_only = [] {
     const char *e = std::getenv("IMHIP_SPARSE_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  if (plan->tile_index && !simple_only) {
+  if (plan->tile_index && plan->steps && !simple_only) {
     im::SparseWave A;
     A.P = P;
-    for (int i = 0; i < im::kStaged; ++i) A.staged[i] = (int)(plan->t[i] - plan->t[0]);
-    const size_t staged = (size_t)(plan->t[im::kStaged] - plan->t[0]);  // tables are padded to 16 bytes
-    A.staged_words = (int)staged;
     A.tile_index = plan->tile_index;
     A.staged_rows = 0;  // (the update stage's)
     A.solve_words = 0;
     A.block = plan->block;
     A.nM = plan->nM;
     // per world: the factor's arrays and the list of contributing constraint rows (weight and number)
-    const size_t per_world = (((size_t)plan->nslots + n + 2 * nw + 3) & ~(size_t)3) + 2 * (((size_t)njmax + 3) & ~(size_t)3);
-    const size_t wave_lds = 4 * (((staged + 3) & ~(size_t)3) + 4 * per_world);
-    if (wave_lds <= 64 * 1024 && staged <= 8192) {
+    const size_t per_world = (size_t)im::init_world_words(plan->nslots, n) + 2 * (((size_t)njmax + 3) & ~(size_t)3);
+    A.staged_steps = im::staged_steps(P);
+    const size_t wave_lds = 4 * (A.staged_steps + 4 * per_world);
+    if (wave_lds <= 64 * 1024) {
       const dim3 grid((unsigned)((nworld + 3) / 4)), wg(256);
       const hipStream_t st = (hipStream_t)stream;
 #define IM_SPARSE_WAVE(NT)                                                                            \
@@ -1262,33 +1436,29 @@ int im_sparse_update_factor(const im_sparse_plan *plan, const uint8_t *done, con
       !search_dot || !decrement)
     return IM_ERR_ARG;
   if (ldg < plan->nv) return IM_ERR_STRIDE;
-  im::SparseDev P;
-  for (int i = 0; i < im::NHOST; ++i) P.t[i] = plan->t[i];
-  P.nv = plan->nv; P.nv_pad = plan->nv_pad; P.nslots = plan->nslots; P.nlevels = plan->nlevels;
+  const im::SparseDev P = im::sparse_dev(*plan);
   const int n = plan->nv, nw = (plan->block + 31) / 32;
   static const bool simple_only = [] {
     const char *e = std::getenv("IMHIP_SPARSE_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  if (n <= 64 && !simple_only) {
+  if (plan->steps && !simple_only) {
     im::SparseWave A;
     A.P = P;
-    for (int i = 0; i < im::kStaged; ++i) A.staged[i] = (int)(plan->t[i] - plan->t[0]);
-    const size_t staged = (size_t)(plan->t[im::kStaged] - plan->t[0]);
-    A.staged_words = (int)staged;
     A.tile_index = nullptr;
     A.block = plan->block;
     A.nM = 0;
     const int32_t *solve_end = plan->t[im::RK] + ((plan->sizes[im::RK] + 3) & ~3);
-    const size_t solve_words = (size_t)(solve_end - plan->t[im::FL]);
+    const size_t forward_words = (size_t)(solve_end - plan->t[im::FL]), solve_words = forward_words + ((n + 3) & ~3), shared_words = im::staged_steps(P) + solve_words;
+    A.staged_steps = im::staged_steps(P);
     // 32 staged rows where a CU still holds sixteen worlds with them, else 16
     A.staged_rows =
-        4 * (staged + solve_words + 16 * (size_t)im::update_world_words(plan->nslots, n, plan->block, 32)) <= 160 * 1024 ? 32 : 16;
-    const size_t per_world = (size_t)im::update_world_words(plan->nslots, n, plan->block, A.staged_rows);
+        4 * (shared_words + 16 * (size_t)im::update_world_words(plan->nslots, n, 32)) <= 160 * 1024 ? 32 : 16;
+    const size_t per_world = (size_t)im::update_world_words(plan->nslots, n, A.staged_rows);
     for (int i = 0; i < 5; ++i) A.solve[i] = (int)(plan->t[im::FL + i] - plan->t[im::FL]);
     A.solve_words = (int)solve_words;
-    const size_t wave_lds = 4 * (staged + solve_words + 4 * per_world);
-    if (wave_lds <= 64 * 1024 && staged <= 8192 && solve_words <= 4096) {
+    const size_t wave_lds = 4 * (shared_words + 4 * per_world);
+    if (wave_lds <= 64 * 1024 && forward_words <= 4096) {
       // Worlds per workgroup: every workgroup stages the tables for itself, so larger workgroups
       // leave more of a CU's 160 KB to the worlds.  The count that keeps the most worlds on a CU
       // (at most 32 wavefronts of 57 registers) is taken, the smallest on a tie and where four
@@ -1298,12 +1468,12 @@ int im_sparse_update_factor(const im_sparse_plan *plan, const uint8_t *done, con
       int64_t best = 0;
       if (const int st = im::compute_units(&ncu)) return st;
       for (int cand = 4; cand <= 16; cand *= 2) {
-        const size_t bytes = 4 * (staged + solve_words + (size_t)cand * per_world);
+        const size_t bytes = 4 * (shared_words + (size_t)cand * per_world);
         int64_t held = (int64_t)(kCuLds / bytes) * cand;
         held = held < 32 ? held : 32;
         if (held > best && (cand == 4 || (int64_t)nworld > best * ncu)) best = held, waves = cand;
       }
-      const size_t lds_bytes = 4 * (staged + solve_words + (size_t)waves * per_world);
+      const size_t lds_bytes = 4 * (shared_words + (size_t)waves * per_world);
       const dim3 grid((unsigned)((nworld + waves - 1) / waves)), wg(64 * waves);
 #define IM_UPDATE_WAVE(W)                                                                                     \
   do {                                                                                                        \
@@ -1347,9 +1517,7 @@ int im_sparse_dense_factor(const im_sparse_plan *plan, const uint8_t *done, cons
   if (!grad || !H || !hfactor || !search || !search_dot || !decrement) return IM_ERR_ARG;
   if ((skip_unchanged && !quad_changed) || (skip_noflip && !state_changed)) return IM_ERR_ARG;
   if (ldg < plan->nv || ld_search < plan->nv || ldH < (int64_t)plan->nv_pad * plan->nv_pad) return IM_ERR_STRIDE;
-  im::SparseDev P;
-  for (int i = 0; i < im::NHOST; ++i) P.t[i] = plan->t[i];
-  P.nv = plan->nv; P.nv_pad = plan->nv_pad; P.nslots = plan->nslots; P.nlevels = plan->nlevels;
+  const im::SparseDev P = im::sparse_dev(*plan);
   const int nw = (plan->block + 31) / 32;
   // the forward solve's tables, or the backward solve's (its pushes <= nfac) in the same words
   const size_t fwd_words = 4 * (size_t)plan->nv + 2 + ((size_t)plan->nfac + 1) / 2, bwd_words = (size_t)plan->nlevels + 1 + plan->nfac;
@@ -1379,22 +1547,19 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
   if (bad != IM_OK) return bad;
   if (p->block != plan->block) return IM_ERR_ARG;
   SparseWave A;
-  for (int i = 0; i < NHOST; ++i) A.P.t[i] = plan->t[i];
-  A.P.nv = plan->nv; A.P.nv_pad = plan->nv_pad; A.P.nslots = plan->nslots; A.P.nlevels = plan->nlevels;
-  for (int i = 0; i < kStaged; ++i) A.staged[i] = (int)(plan->t[i] - plan->t[0]);
-  const size_t staged = (size_t)(plan->t[kStaged] - plan->t[0]);
-  A.staged_words = (int)staged;
+  A.P = sparse_dev(*plan);
   A.tile_index = nullptr;
   A.block = plan->block;
   A.nM = 0;
   const int32_t *solve_end = plan->t[RK] + ((plan->sizes[RK] + 3) & ~3);
-  const size_t solve_words = (size_t)(solve_end - plan->t[FL]);
+  const size_t forward_words = (size_t)(solve_end - plan->t[FL]), solve_words = forward_words + ((n + 3) & ~3);
   for (int i = 0; i < 5; ++i) A.solve[i] = (int)(plan->t[FL + i] - plan->t[FL]);
   A.solve_words = (int)solve_words;
-  if (staged > 8192 || solve_words > 4096) return IM_ERR_UNSUPPORTED;
-  const size_t shared = staged + solve_words + (size_t)p->nterm + n + 1;
+  A.staged_steps = staged_steps(A.P);
+  if (!plan->steps || forward_words > 4096) return IM_ERR_UNSUPPORTED;
+  const size_t shared = A.staged_steps + solve_words + (size_t)p->nterm + n + 1;
   auto wave_words = [&](int staged_rows) {
-    return (size_t)resident_area_words(plan->nslots, n, plan->block, njmax, staged_rows) + resident::kept_words(n, njmax, 0);
+    return (size_t)resident_area_words(plan->nslots, n, njmax, staged_rows) + resident::kept_words(n, njmax, 0);
   };
   // the most worlds per workgroup (one workgroup per CU) that 160 KB of LDS admit and whose kernel
   // keeps to registers

@@ -36,6 +36,11 @@ struct im_sparse_plan {
   // row of M and which slot it is ((M index + 1) << 16 | (slot + 1)); null when nv > 64
   int32_t *tile_index = nullptr;
   int nM = 0;
+  // for up to 64 dofs, of a wavefront's 64 lanes: the factor's steps (two words a lane), then the backward solve's (one), and the
+  // pairs r <= c of a list of dofs in order (r | c << 8); null beyond
+  const uint32_t *steps = nullptr;
+  const uint16_t *dof_pairs = nullptr;
+  int nfactor_steps = 0, nbackward_steps = 0;
   // one int on the device: the next world of a batch nobody has started (im_newton_solve_sparse)
   int *next_world = nullptr;
 };

@@ -452,3 +452,40 @@ def test_gpu_done_mask_violation_counter_and_graph_replay(device):
         g.replay()
         torch.cuda.synchronize()
         np.testing.assert_array_equal(args[8].cpu().numpy()[:, :, 0][live], got[1][live])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [32, 64])
+@pytest.mark.parametrize("nv,seed", [(1, 0), (17, 1), (33, 2), (48, 3), (57, 4), (64, 5)])
+def test_gpu_random_patterns_bitwise(device, nv, seed, block):
+    """Forests with coupled bodies: entries of several runs, teams of every width, levels of more entries than a step
+    holds, and patterns with more steps than a workgroup keeps in LDS (from 48 dofs on here)."""
+    rng = np.random.default_rng(seed)
+    m = _random_model(rng, nv)
+    nb = len(m.body_parentid)
+    groups = [sorted({int(b) for b in rng.integers(1, nb, 3)}) for _ in range(4)] if nv > 1 else []
+    plan = S.build_plan(m, groups, block, device=device)
+    runs = np.diff(plan.tables["SH_RP"]).max(initial=0)
+    assert nv < 17 or runs > 1
+    b = _batch(m, groups, 37, 40, 11)
+    ref = R.sparse_init_factor(_oracle_plan(m, groups, block), b.nefc, b.J, b.D, b.state[0], b.M, b.grad)
+    got = _run_gpu(plan, b, device)
+    n_used = 2 * plan.nfac + plan.nv
+    np.testing.assert_array_equal(got[0].reshape(37, -1)[:, :n_used], ref[0].reshape(37, -1)[:, :n_used])
+    for g, r in zip(got[1:4], ref[1:]):
+        np.testing.assert_array_equal(g, r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv", [44, 45, 46])
+def test_gpu_long_chains_bitwise(device, nv):
+    """One chain of dofs, dense: the most words a world and a step for every sixty entries of a level."""
+    m = synth.model_from_parents([-1] + list(range(nv - 1)))
+    plan = S.build_plan(m, [], S.block_width(m.nv_pad), device=device)
+    b = _batch(m, [], 21, 40, 3)
+    ref = R.sparse_init_factor(_oracle_plan(m, [], S.block_width(m.nv_pad)), b.nefc, b.J, b.D, b.state[0], b.M, b.grad)
+    got = _run_gpu(plan, b, device)
+    n_used = 2 * plan.nfac + plan.nv
+    np.testing.assert_array_equal(got[0].reshape(21, -1)[:, :n_used], ref[0].reshape(21, -1)[:, :n_used])
+    for g, r in zip(got[1:4], ref[1:]):
+        np.testing.assert_array_equal(g, r)
