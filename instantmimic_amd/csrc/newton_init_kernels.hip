@@ -18,7 +18,8 @@ namespace im {
 namespace {
 
 // LDS words of one wavefront: M's row and the tile of J, then sv, Ma, gl (nv each), Jaref, f, rowl (njmax each)
-__host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return resident::kTileWords + 3 * (size_t)nv + 3 * (size_t)njmax; }
+__host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return (resident::kTileWords + 3 * (size_t)nv + 3 * (size_t)njmax + 3) & ~(size_t)3; }
+__host__ __device__ inline int init_shared_words(int nterm, int nv) { return (nterm + nv + 1 + 3) & ~3; }
 
 // WIDE: more than 64 dofs (the product on the matrix cores, two dofs a lane in the gradient): 124 registers a lane against
 // 72.  What bounds the launch is J's trip from memory, hidden by other wavefronts, and one kernel of both forms gives every
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
   const int nv = a.nv, njmax = a.njmax;
   uint32_t *term = (uint32_t *)lds;
   int *radr = (int *)(term + a.nterm);
-  float *mine = (float *)(radr + nv + 1) + wv * init_wave_words(nv, njmax);
+  float *mine = lds + init_shared_words(a.nterm, nv) + wv * init_wave_words(nv, njmax);
   float *tile = mine, *sv = tile + resident::kTileWords, *Ma_l = sv + nv, *gl = Ma_l + nv, *Jaref_l = gl + nv, *f = Jaref_l + njmax;
   int *rowl = (int *)(f + njmax);
   for (int k = threadIdx.x; k < a.nterm; k += blockDim.x) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
@@ -63,8 +64,15 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
     if (empty && whole.active) a.qfrc_constraint[w * nv + k] = 0.0f;
     sv[k] = q;
   }
-  // Ma = M qacc, for every world
-  resident::mul_m_world_staged<false, 12>(a, term, radr, a.M + w * a.ldM, sv, a.Ma + w * nv, Ma_l, tile, lane);
+  // Ma = M qacc, for every world, and the others' J qacc
+  const float *Jw = a.J + w * (int64_t)njmax * nv;
+  resident::StagedM<false, 12, true> row;
+  resident::jv_world<WIDE ? 3 : 1>(
+      a, Jw, empty ? 0 : nefc, tile, sv, nullptr, Jaref_l, lane,
+      [&]() __attribute__((always_inline)) { row.load(a.M + w * a.ldM, a.nM, lane); },
+      [&]() __attribute__((always_inline)) {
+        row.product(a, term, radr, a.M + w * a.ldM, a.nM, sv, a.Ma + w * nv, Ma_l, tile, lane);
+      });
   if (empty) {  // what the stages leave of a done world: zero counts and the `unchanged` byte
     if (lane == 0) {
       a.quad_count[w] = 0;
@@ -73,12 +81,6 @@ __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::Newt
     }
     return;
   }
-  const float *Jw = a.J + w * (int64_t)njmax * nv;
-  resident::wave_sync();
-  if constexpr (WIDE)
-    resident::jv_world(a, Jw, nefc, sv, nullptr, Jaref_l, lane, []() {});
-  else
-    resident::jv_world_tiled<true>(a, Jw, nefc, tile, sv, nullptr, Jaref_l, lane, []() {});
   resident::wave_sync();
   // Jaref = J qacc - aref, then force and state of every row (newton_stages.py:385-444 at step 0),
   // the rows whose being quadratic differs from the state that lay there, the rows with a force
@@ -144,7 +146,7 @@ int newton_init_launch(const im_newton_args *p, const float *qacc_smooth, int64_
   const int bad = resident::convert_args(*p, nv, nM, a);
   if (bad != IM_OK) return bad;
   if (ld_qacc_smooth < nv || ld_aref < p->njmax || (whole.start && whole.ld_start < nv)) return IM_ERR_STRIDE;
-  const size_t lds = 4 * ((size_t)p->nterm + nv + 1 + 4 * init_wave_words(nv, p->njmax));
+  const size_t lds = 4 * (init_shared_words(p->nterm, nv) + 4 * init_wave_words(nv, p->njmax));
   if (lds > 160 * 1024) return IM_ERR_UNSUPPORTED;
   auto kernel = nv > 64 ? newton_init_context_kernel<true> : newton_init_context_kernel<false>;
   if (lds > 64 * 1024)

@@ -125,16 +125,20 @@ __device__ __forceinline__ void block_sync() {
 }
 
 // words of LDS of the loop's own arrays behind the factor stage's area: four flags, the row tables of M v
-// (one word per term, nv + 1 offsets), then per wavefront the world's row of M, the search
-// direction, Ma, mv, Jaref, jv, D and the friction losses, the gradient's list of rows with a force
-// (value and row number) and its copy of the gradient.  The factor stage's area must also hold four wavefronts'
+// (one word per term, nv + 1 offsets), then per wavefront the search direction, Ma, mv, qacc, Jaref, jv, D and the
+// friction losses, the gradient's list of rows with a force (value and row number) and its copy of the gradient, the
+// world's row of M.  The factor stage's area must also hold four wavefronts'
 // rows of M where those are read from memory, and their tiles of J (kTileWords each).
 // words a wavefront keeps from round to round: M, the search direction, Ma, mv, qacc; Jaref, jv, D, friction losses
 __host__ __device__ inline size_t kept_words(int nv, int njmax, int nM) { return (size_t)nM + 4 * (size_t)nv + 4 * (size_t)njmax; }
-__host__ __device__ inline size_t loop_lds_words(int nv, int njmax, int nM, int nterm) {
-  return 8 + (size_t)nterm + nv + 1 + 4 * (kept_words(nv, njmax, nM) + 2 * (size_t)njmax + nv);
+// a wavefront's own words in a cooperative kernel, a multiple of four (the search direction first)
+__host__ __device__ inline size_t coop_wave_words(int nv, int njmax, int nM) {
+  return (kept_words(nv, njmax, nM) + 2 * (size_t)njmax + nv + 3) & ~(size_t)3;
 }
-constexpr int kTileWords = 64 * 17;
+__host__ __device__ inline size_t loop_lds_words(int nv, int njmax, int nM, int nterm) {
+  return 8 + (size_t)nterm + nv + 1 + 6 + 4 * coop_wave_words(nv, njmax, nM);
+}
+constexpr int kTileWords = 64 * 17;  // (a tile of J takes 64 * 16 of them, a row of M up to all)
 constexpr size_t kStagedWords = 4 * kTileWords;
 
 // ---- M search (newton_fusion.py:171-176) -------------------------------------------------------
@@ -202,27 +206,37 @@ __device__ __forceinline__ void mul_m_world(const NewtonArgs &a, const uint32_t 
     }
   }
 }
-// The same with the world's row of M in memory: it passes through `stage` (kTileWords of LDS) where it fits,
-// LOADS a lane in flight at once.  Read term by term a free body's dofs, whose rows are nv long, waited for memory
-// once per four terms (70 dofs x 2048 worlds: 9 of the 22 us that a round's two products took).
-template <bool WALK, int LOADS>
-__device__ __forceinline__ void mul_m_world_staged(const NewtonArgs &a, const uint32_t *term, const int *radr, const float *m,
-                                                   const float *v, float *out, float *out_lds, float *stage, int lane) {
-  if (a.nM > kTileWords) {
-    wave_sync();
-    return mul_m_world<WALK>(a, term, radr, m, v, out, out_lds, lane);
+// The same with the world's row of M in memory: it passes through `stage` (kTileWords of LDS) where it fits, the
+// first LOADS words a lane asked for together, EARLY: by load() ahead of whatever else the round asks for (where the
+// registers are not what bounds a kernel's wavefronts).  Read term by term a
+// free body's dofs, whose rows are nv long, waited for memory once per four terms (70 dofs x 2048 worlds: 9 of the 22 us
+// that a round's two products took).
+template <bool WALK, int LOADS, bool EARLY>
+struct StagedM {
+  float x[LOADS];
+  __device__ __forceinline__ void load(const float *m, int nM, int lane) {
+    if constexpr (EARLY) fetch(m, nM, lane);
   }
-  for (int k0 = lane; k0 < a.nM; k0 += LOADS * 64) {
-    float x[LOADS];
+  __device__ __forceinline__ void fetch(const float *m, int nM, int lane) {
+    // (without a condition: what might be left as it was would be kept from round to round)
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u) x[u] = m[k0 + 64 * u < a.nM ? k0 + 64 * u : a.nM - 1];
+    for (int u = 0; u < LOADS; ++u) x[u] = m[(unsigned)(lane + 64 * u < nM ? lane + 64 * u : nM - 1)];
+  }
+  __device__ __forceinline__ void product(const NewtonArgs &a, const uint32_t *term, const int *radr, const float *m, int nM,
+                                          const float *v, float *out, float *out_lds, float *stage, int lane) {
+    if (nM > kTileWords) {
+      wave_sync();
+      return mul_m_world<WALK>(a, term, radr, m, v, out, out_lds, lane);
+    }
+    if constexpr (!EARLY) fetch(m, nM, lane);
 #pragma unroll
     for (int u = 0; u < LOADS; ++u)
-      if (k0 + 64 * u < a.nM) stage[k0 + 64 * u] = x[u];
+      if (lane + 64 * u < nM) stage[lane + 64 * u] = x[u];
+    for (int k = lane + 64 * LOADS; k < nM; k += 64) stage[k] = m[k];
+    wave_sync();
+    mul_m_world<WALK>(a, term, radr, stage, v, out, out_lds, lane);
   }
-  wave_sync();
-  mul_m_world<WALK>(a, term, radr, stage, v, out, out_lds, lane);
-}
+};
 
 // ---- the gradient (newton_stages.py:745-798), a lane per dof ------------------------------------
 // The world's scalars that the loop carries in registers (every lane the same values); they are
@@ -356,40 +370,47 @@ __device__ __forceinline__ void search_sums_world(const NewtonArgs &a, int64_t w
   }
 }
 
-// ---- J search (newton_stages.py:157-178) beyond 64 dofs, on the matrix cores -------------------------
-// A row's sum is a chain of multiply-adds over the dofs in order, beyond 50 dofs in parts of 20 that are
-// added up.  v_mfma_f32_16x16x4_f32 adds its four products one after the other, so sixteen rows' chains run four
-// dofs per instruction: lane (g, c) = (lane / 16, lane % 16) supplies J[row c][dof 4 q + g] and search[4 q + g]; every
-// column of the result is the rows' sums.  A step is 64 rows x 16 dofs: per sixteen rows a lane loads four neighbouring
-// dofs of a row, which four lane swaps turn into the operands of four instructions.  Four steps are on their way at
-// once (16 registers a lane each): what bounds the product is the trip to memory, J being read once per
-// round.  With the row of M staged (below), M v and J v of a round at 70 dofs x 2048 worlds: 22.4 -> 14 us.
-// `between` runs while the first steps are on their way and leaves the search direction in sv.
+// ---- J search (newton_stages.py:157-178) through a tile of 64 rows x 16 dofs in LDS -------------------
+// A row's sum is a chain of multiply-adds over the dofs in order, beyond 50 dofs in parts of 20 that are added up: a lane
+// per row, its operands by four 16-byte reads a tile, the direction's by four that every lane makes alike.  Lane (g, c) =
+// (lane / 16, lane % 16) brings dofs 4 g .. 4 g + 3 of rows c, 16 + c, .. into the tile, whose rows lie 16 words apart
+// with their quads changed round by the row (quad q of row r at q ^ (r / 4 % 4): neither the writes nor the reads meet in a
+// bank).  DEPTH tiles are on their way at once.  What bounds the product is the trips to memory and the chain.  With the
+// row of M asked for ahead (StagedM), the two products of a round of the slowest worlds, and the solve: 70 dofs x 157 rows
+// x 2048 worlds 19.2 -> 13.3 us and 800 -> 741 (the chains ran on the matrix cores there, sixteen equal columns to a result,
+// their operands turned by lane swaps); 43 dofs x 8192 worlds 9.4 -> 7.2 and 644 -> 634, 27 x 4096 247 -> 240, 14 x 64
+// 100 -> 97.5 (a tile of single words, four times the LDS instructions).  1 tile ahead up to 64 dofs, where registers bound
+// the wavefronts in flight, 3 beyond.
+// `before` runs ahead of the first request, `between` while the first tiles are on their way; it leaves the direction in
+// sv (16-byte aligned) and may use the tile.
 typedef float v4 __attribute__((ext_vector_type(4)));
 typedef v4 v4_words __attribute__((aligned(4)));
-// (the wait states written out: the compiler's builtins return one result twice when both operands hold the same value)
-__device__ __forceinline__ void turn_groups(float &r0, float &r1, float &r2, float &r3) {
-  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1\n\t"
-      "v_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
-      : "+v"(r0), "+v"(r1), "+v"(r2), "+v"(r3));
-}
-template <class Between>
-__device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, int nefc, const float *sv, float *jv,
-                                         float *jv_lds, int lane, Between &&between) {
+template <int DEPTH, class Before, class Between>
+__device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, int nefc, float *tile, const float *sv, float *jv,
+                                         float *jv_lds, int lane, Before &&before, Between &&between) {
   const int nv = a.nv, g = lane >> 4, c = lane & 15;
-  if (nefc <= 0) return between();
+  before();
+  if (nefc <= 0 || nv < 4) {  // (rows shorter than a load: from memory)
+    between();
+    for (int r = lane; r < nefc; r += 64) {
+      float p = 0.0f;
+      for (int i = 0; i < nv; ++i) p = fma_(Jw[r * nv + i], sv[i], p);
+      if (jv) jv[r] = p;
+      jv_lds[r] = p;
+    }
+    return;
+  }
   const bool split = nv > 50;
   struct Step {
     int r0, c0;
   };
-  // (not behind a branch, the last row's again past the end: a wait for one step's loads counts those of the next)
+  // (not behind a branch, the last row's again past the end: a wait for one tile's loads counts those of the next)
   auto fetch = [&](const Step &s, v4 (&v)[4]) __attribute__((always_inline)) {
     const int col = s.c0 + 4 * g, from = col < nv - 4 ? col : nv - 4;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int row = s.r0 + 16 * t + c;
-      const char *at = (const char *)Jw + 4u * (uint32_t)((row < nefc ? row : nefc - 1) * nv + from);
-      v[t] = *(const v4_words *)at;
+      v[t] = *(const v4_words *)((const char *)Jw + 4u * (uint32_t)((row < nefc ? row : nefc - 1) * nv + from));
     }
   };
   auto advance = [&](Step &s) __attribute__((always_inline)) {
@@ -397,34 +418,20 @@ __device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, i
     if (s.c0 >= nv) s.c0 = 0, s.r0 += 64;
   };
   Step now = {0, 0}, ahead = {0, 0};
-  constexpr int DEPTH = 4;
   v4 v[DEPTH][4];
 #pragma unroll
   for (int b = 0; b < DEPTH; ++b) fetch(ahead, v[b]), advance(ahead);
   between();
-  v4 p[4] = {};
-  float sum = 0.0f;  // of the row that this lane puts out: register u of group t of row 16 t + 4 g + u, the same in all
-                     // columns; lane (g, c) takes row 16 (c / 4) + 4 g + c % 4
-  auto take = [&]() __attribute__((always_inline)) {
-    float part = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) part = c == 4 * t + u ? p[t][u] : part;
-      p[t] = v4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    sum = sum + part;
-  };
+  wave_sync();
+  float *put = tile + 16 * c + 4 * (g ^ (c >> 2));
+  const float *take = tile + 16 * lane;
+  const int turn = 4 * ((lane >> 2) & 3);
+  float acc = 0.0f, p = 0.0f;
   auto work = [&](v4 (&v)[4]) __attribute__((always_inline)) {
-    const int col = now.c0 + 4 * g;
-    float x[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) x[q] = now.c0 + 4 * q + g < nv ? sv[now.c0 + 4 * q + g] : 0.0f;
     if (now.c0 + 16 > nv) {  // the row's last dofs were loaded from four before its end: moved down, zeros behind them
-      const int by = col + 4 - nv;
+      const int by = now.c0 + 4 * g + 4 - nv;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        if (t > 0 && now.r0 + 16 * t >= nefc) continue;
         v4 m = v[t];
         m = by >= 1 ? v4{m[1], m[2], m[3], 0.0f} : m;
         m = by >= 2 ? v4{m[1], m[2], 0.0f, 0.0f} : m;
@@ -432,121 +439,61 @@ __device__ __forceinline__ void jv_world(const NewtonArgs &a, const float *Jw, i
         v[t] = by >= 4 ? v4{0.0f, 0.0f, 0.0f, 0.0f} : m;
       }
     }
-    float e[4][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (t > 0 && now.r0 + 16 * t >= nefc) continue;
-      e[t][0] = v[t][0], e[t][1] = v[t][1], e[t][2] = v[t][2], e[t][3] = v[t][3];
-      turn_groups(e[t][0], e[t][1], e[t][2], e[t][3]);
-    }
+    for (int t = 0; t < 4; ++t) *(v4 *)(put + 256 * t) = v[t];
+    wave_sync();
+  };
+  auto chain = [&]() __attribute__((always_inline)) {
+    // (half a tile's operands at a time where a kernel has no registers to spare)
+    constexpr int QUADS = DEPTH > 1 ? 4 : 2;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (split && (now.c0 + 4 * q) % 20 == 0) take();
-      if (q == 0 || now.c0 + 4 * q < nv) {
+    for (int q0 = 0; q0 < 4; q0 += QUADS) {
+      v4 x[QUADS], y[QUADS];
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (t == 0 || now.r0 + 16 * t < nefc) p[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[t][q], x[q], p[t], 0, 0, 0);
+      for (int q = 0; q < QUADS; ++q) {
+        const int col = now.c0 + 4 * (q0 + q);
+        x[q] = y[q] = v4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (col >= nv) continue;
+        x[q] = *(const v4 *)(take + ((4 * (q0 + q)) ^ turn));
+        y[q] = *(const v4 *)(sv + col);
+        if (col + 4 > nv) {  // (+0 of J times -0: what a sum takes without any change, its sign as a zero too)
+          y[q][3] = -0.0f;
+          y[q][2] = col + 2 < nv ? y[q][2] : -0.0f;
+          y[q][1] = col + 1 < nv ? y[q][1] : -0.0f;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q) {
+        const int col = now.c0 + 4 * (q0 + q);
+        if (col >= nv) continue;
+        if (split && col % 20 == 0) {  // (0 + 0 at the first)
+          acc = acc + p;
+          p = 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p = fma_(x[q][u], y[q][u], p);
       }
     }
     if (now.c0 + 16 >= nv) {
-      take();
-      const int row = now.r0 + 16 * (c >> 2) + 4 * g + (c & 3);
+      const int row = now.r0 + lane;
+      const float out = split ? acc + p : p;
       if (row < nefc) {
-        if (jv) jv[row] = sum;
-        jv_lds[row] = sum;
+        if (jv) jv[row] = out;
+        jv_lds[row] = out;
       }
-      sum = 0.0f;
+      acc = p = 0.0f;
     }
     advance(now);
+    wave_sync();  // the tile is read before the next one overwrites it
   };
   for (;;) {
 #pragma unroll
     for (int b = 0; b < DEPTH; ++b) {
       work(v[b]);
-      if (now.r0 >= nefc) return;
-      fetch(ahead, v[b]);
+      if (DEPTH > 1 || ahead.r0 < nefc) fetch(ahead, v[b]);
       advance(ahead);
-    }
-  }
-}
-
-// ---- J search through a tile of 64 rows x 16 dofs (kTileWords of LDS whatever the width of J) -------
-// Up to 64 dofs, the same chains through the tile and on a lane per row: the
-// operands' way into the matrix cores takes more instructions, and where the chip is full of worlds it is the slower
-// form (27 dofs x 4096 worlds 259 us per solve against 250; 56 x 4096 768 against 740).  A lane loads 16 elements per
-// tile, four rows of 64 bytes per instruction; the next tile's elements are asked for while the current one is worked
-// on.  WIDE: a tile row's operands are read eight at a time ahead of their part of the chain (sixteen registers).
-template <bool WIDE, class Between>
-__device__ __forceinline__ void jv_world_tiled(const NewtonArgs &a, const float *Jw, int nefc, float *tile,
-                                               const float *sv, float *jv, float *jv_lds, int lane, Between &&between) {
-  const int nv = a.nv;
-  const int c = lane & 15, rq = lane >> 4;
-  const bool split = nv > 50;
-  // the 16 elements of a lane for the tile at (r0, c0); the next tile's are asked for while the
-  // current one is worked on, so the trips to memory of all but the first tile are hidden
-  auto fetch = [&](int r0, int c0, float (&v)[16]) __attribute__((always_inline)) {
-    const int rows = nefc - r0 < 64 ? nefc - r0 : 64, cw = nv - c0 < 16 ? nv - c0 : 16;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int r = rq + 4 * k;
-      v[k] = Jw[(int64_t)(r0 + (r < rows ? r : rows - 1)) * nv + c0 + (c < cw ? c : cw - 1)];
-    }
-  };
-  float v[16];
-  if (nefc > 0) fetch(0, 0, v);
-  between();
-  wave_sync();  // (a staged row of M has the tile's place until here)
-  for (int r0 = 0; r0 < nefc; r0 += 64) {
-    const int rows = nefc - r0 < 64 ? nefc - r0 : 64;
-    float acc = 0.0f, p = 0.0f;
-    for (int c0 = 0; c0 < nv; c0 += 16) {
-      const int cw = nv - c0 < 16 ? nv - c0 : 16;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) tile[(rq + 4 * k) * 17 + c] = v[k];
-      wave_sync();
-      const bool more_columns = c0 + 16 < nv;
-      const int next_r0 = more_columns ? r0 : r0 + 64, next_c0 = more_columns ? c0 + 16 : 0;
-      if (next_r0 < nefc) fetch(next_r0, next_c0, v);
-      if (lane < rows) {
-        // a tile row's operands are read eight at a time before their part of the chain (two waits
-        // per tile, not sixteen)
-        const float *row = tile + lane * 17;
-        if constexpr (!WIDE) {  // the short form, for a kernel without registers to spare
-          for (int i = 0; i < cw; ++i) {
-            if (split && (c0 + i) % 20 == 0 && c0 + i > 0) {
-              acc = acc + p;
-              p = 0.0f;
-            }
-            p = fma_(row[i], sv[c0 + i], p);
-          }
-        } else {
-          // the column, one of every four, ahead of which a part of 20 ends; and columns past the last dof, of which the
-          // products are dropped by a lane's own comparison (as scalars sixteen conditions are more than there is room for)
-          int part = split ? (c0 + 19) / 20 * 20 - c0 : 16, columns = cw;
-          part = c0 + part == 0 || part >= cw ? 16 : part;
-          asm volatile("" : "+v"(columns));
-#pragma unroll
-          for (int h = 0; h < 16; h += 8) {
-            float x[8], y[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = row[h + i], y[i] = sv[c0 + (h + i < cw ? h + i : 0)];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              if (i % 4 == 0 && part == h + i) {
-                acc = acc + p;
-                p = 0.0f;
-              }
-              p = h + i < columns ? fma_(x[i], y[i], p) : p;
-            }
-          }
-        }
-      }
-      wave_sync();  // the tile is read before the next one overwrites it
-    }
-    if (lane < rows) {
-      const float out = split ? acc + p : p;
-      if (jv) jv[r0 + lane] = out;
-      jv_lds[r0 + lane] = out;
+      chain();
+      if (now.r0 >= nefc) return;
     }
   }
 }
@@ -560,7 +507,7 @@ struct LoopLds {
   const int *radr;       // [nv + 1]
   // per wavefront, kept from round to round:
   float *m_lds;          // [nM] the world's row of M
-  float *sv;             // [nv] the search direction
+  float *sv;             // [nv] the search direction; 16-byte aligned, as rows
   float *Ma, *mv, *qacc; // [nv] each
   float *Jaref, *jv;     // [njmax] each
   float *D, *fl;         // [njmax] each: the rows' weights and friction losses (read at every step of the line search)
@@ -705,16 +652,20 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
 #pragma unroll
       for (int k = 0; k < 2; ++k) smooth[k] = a.smooth[w * nv + (lane + 64 * k < nv ? lane + 64 * k : 0)];
       if (!unchanged) {
-        auto m_search = [&]() __attribute__((always_inline)) {
-          if (MLDS && L.m_lds)
-            mul_m_world<COLS == 2>(a, L.term, L.radr, L.m_lds, L.sv, a.mv + w * nv, L.mv, lane);
-          else
-            mul_m_world_staged<COLS == 2, WIDE ? 12 : 8>(a, L.term, L.radr, a.M + w * a.ldM, L.sv, a.mv + w * nv, L.mv, L.rows, lane);
-        };
-        if constexpr (COLS == 2)
-          jv_world(a, Jw, nefc, L.sv, a.jv + w * njmax, L.jv, lane, m_search);
-        else
-          jv_world_tiled<WIDE>(a, Jw, nefc, L.rows, L.sv, a.jv + w * njmax, L.jv, lane, m_search);
+        StagedM<COLS == 2, WIDE ? 12 : 8, !MLDS> row;
+        const float *M = a.M + w * a.ldM;
+        const bool staged = !(MLDS && L.m_lds);
+        jv_world<COLS == 2 ? 3 : 1>(
+            a, Jw, nefc, L.rows, L.sv, a.jv + w * njmax, L.jv, lane,
+            [&]() __attribute__((always_inline)) {
+              if constexpr (!MLDS) row.load(M, a.nM, lane);
+            },
+            [&]() __attribute__((always_inline)) {
+              if (staged)
+                row.product(a, L.term, L.radr, M, a.nM, L.sv, a.mv + w * nv, L.mv, L.rows, lane);
+              else
+                mul_m_world<COLS == 2>(a, L.term, L.radr, L.m_lds, L.sv, a.mv + w * nv, L.mv, lane);
+            });
         wave_sync();
       }
 #pragma unroll
@@ -868,10 +819,9 @@ __device__ __forceinline__ LoopLds coop_layout(const NewtonArgs &a, float *lds) 
   L.worlds = L.votes + 4;
   uint32_t *term = (uint32_t *)(L.worlds + 4);
   int *radr = (int *)(term + a.nterm);
-  float *mine = (float *)(radr + nv + 1) + wv * (kept_words(nv, njmax, nM) + 2 * njmax + nv);
+  float *mine = lds + ((a.stage_lds_floats + 8 + a.nterm + nv + 1 + 3) & ~3) + wv * coop_wave_words(nv, njmax, nM);
   L.term = term, L.radr = radr;
-  L.m_lds = a.m_lds ? mine : nullptr;
-  L.sv = mine + nM;
+  L.sv = mine;
   L.Ma = L.sv + nv;
   L.mv = L.Ma + nv;
   L.qacc = L.mv + nv;
@@ -882,6 +832,7 @@ __device__ __forceinline__ LoopLds coop_layout(const NewtonArgs &a, float *lds) 
   L.f = L.fl + njmax;
   L.rowl = (int *)(L.f + njmax);
   L.gl = (float *)(L.rowl + njmax);
+  L.m_lds = a.m_lds ? L.gl + nv : nullptr;
   L.rows = lds + wv * kTileWords;
   for (int k = threadIdx.x; k < a.nterm; k += blockDim.x) term[k] = (uint32_t)a.mulm_col[k] | (uint32_t)a.mulm_madr[k] << 16;
   for (int k = threadIdx.x; k <= nv; k += blockDim.x) radr[k] = a.mulm_rowadr[k];

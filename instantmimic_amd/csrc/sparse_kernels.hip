@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
   int *radr = (int *)(term + a.nterm);
   const int area = resident_area_words(A.P.nslots, nv, njmax, A.staged_rows);
   // (M is read from memory by the round's one product with it: its row would cost a CU a third of its worlds)
-  float *mine = (float *)(radr + nv + 1) + wv * (area + resident::kept_words(nv, njmax, 0));
+  float *mine = lds + A.staged_steps + A.solve_words + ((a.nterm + nv + 1 + 3) & ~3) + wv * (area + resident::kept_words(nv, njmax, 0));
   resident::LoopLds L;
   L.votes = nullptr;
   L.term = term, L.radr = radr;
@@ -1557,7 +1557,7 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
   A.solve_words = (int)solve_words;
   A.staged_steps = staged_steps(A.P);
   if (!plan->steps || forward_words > 4096) return IM_ERR_UNSUPPORTED;
-  const size_t shared = A.staged_steps + solve_words + (size_t)p->nterm + n + 1;
+  const size_t shared = A.staged_steps + solve_words + (((size_t)p->nterm + n + 1 + 3) & ~(size_t)3);
   auto wave_words = [&](int staged_rows) {
     return (size_t)resident_area_words(plan->nslots, n, njmax, staged_rows) + resident::kept_words(n, njmax, 0);
   };

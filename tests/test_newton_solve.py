@@ -292,3 +292,19 @@ def test_gpu_solve_at_layout_boundaries(device, monkeypatch, nv, stage, chains, 
     assert s.done.all()
     m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=True)
     NC.compare(p, s, d, ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv", [1, 3, 4, 5, 15, 18, 50, 51, 53, 65, 66])
+def test_gpu_solve_at_the_edges_of_a_tile_of_j(device, monkeypatch, nv):
+    """J times the search direction goes through tiles of 64 rows x 16 dofs with four dofs to a load: a whole tile of
+    rows, one less and one more; rows shorter than a load, a last load that reaches back before its own dofs, and parts
+    of 20 dofs from 51 dofs on."""
+    name = f"edge{nv}"
+    shape = synth.Shape(name, _floating_chain(nv), 66, 66, (0.5, 8.0), 0.02, (-4.0, 4.0), 0.6, 1, 1300 + nv)
+    monkeypatch.setitem(synth.SHAPES, name, shape)
+    p = NC.problem(name, 401, "dense", empty_every=9)
+    assert {0, 63, 64, 65} < set(p.nefc.tolist())
+    s = NC.oracle_solve(p)
+    m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
+    NC.compare(p, s, d, ctx)
