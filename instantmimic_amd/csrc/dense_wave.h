@@ -455,42 +455,85 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
   const int count = changes_raw < 0 ? 0 : (changes_raw < ld_ids ? changes_raw : ld_ids);
   float rd[NB];
   if (refactor) {
+    // H (with its update), the identity beyond the dofs, the gradient in the last column.  The gradient passes through
+    // xl; H's tiles are asked for kAhead at a time ahead of the pairs and of one another, and what the update changed is stored
+    // behind the last of them: a store under a condition between two tiles had every tile wait for its own trip to memory
+    // (a stage of 29.2 -> 23.4 us in the slowest worlds at 70 dofs, the solve of 2048 of them 741 -> 711 us, of 8192 at 43
+    // dofs 621 -> 605; 4 and 6 tiles ahead were no faster up to 48 dofs and beyond them took registers kept in memory).
+#pragma unroll
+    for (int i0 = 0; i0 < PAD; i0 += 64) {
+      const int i = i0 + lane;
+      if (i < PAD) xl[i] = gw[i < nv ? i : nv - 1];
+    }
+    auto beyond = [&](int row, int col, float e, float grad) __attribute__((always_inline)) {
+      const bool in = col < nv && row < nv;
+      return in ? e : (c == 15 && row < nv) ? grad : row == col ? 1.0f : 0.0f;
+    };
+    // element (16 i + first, c) of a matrix: what is beyond a tile row is in the instruction's own offset (as constants of
+    // one base the rows' offsets took a pair of scalar registers each)
+    auto row_at = [&](float *base, int first, int i) __attribute__((always_inline)) {
+      unsigned at = 4u * (unsigned)(first * PAD + c);
+      asm volatile("" : "+v"(at));
+      return (char *)base + (at + 64u * PAD * i);
+    };
     if constexpr (!READY) {
+      constexpr int kAhead = 2;
+      float4v h[kAhead];
+      auto fetch = [&](auto tile_row, auto tile_col) __attribute__((always_inline)) {
+        constexpr int i = tile_row, j = tile_col, at = tile_at<NB>(i, j) % kAhead;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) h[at][v] = *(const float *)(row_at(Hw, 4 * g, i) + 4 * (v * PAD + 16 * j));
+      };
+      auto each_tile = [&](auto &&f) __attribute__((always_inline)) {
+        each<NB>([&](auto i) __attribute__((always_inline)) {
+          each<NB - i>([&](auto right) __attribute__((always_inline)) { f(i, std::integral_constant<int, i + right>{}); });
+        });
+      };
+      each_tile([&](auto i, auto j) __attribute__((always_inline)) {
+        if constexpr (tile_at<NB>(i, j) < kAhead) fetch(i, j);
+      });
       unsigned hit[NB];
       changed_pairs<NB>(t, hit, Jw, Dw, sw, idw, count, quad, nv, lane);
       write_union<NB>(uni, hit, nv, lane);
-    } else if (lane == 0) {
-      uni[nv] = 0;
-    }
-    // H (with its update), the identity beyond the dofs, the gradient in the last column
-    auto beyond = [&](int row, int col, float e) __attribute__((always_inline)) {
-      const bool in = col < nv && row < nv;
-      return in ? e : (c == 15 && row < nv) ? gw[row < nv ? row : 0] : row == col ? 1.0f : 0.0f;
-    };
+      unsigned changed = 0u;  // tiles
+      each_tile([&](auto tile_row, auto tile_col) __attribute__((always_inline)) {
+        constexpr int i = tile_row, j = tile_col, m = tile_at<NB>(i, j);
+        bool any = false;
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = i; j < NB; ++j) {
-        float4v &m = t[tile_at<NB>(i, j)];
-        const int col = 16 * j + c;
-        float h[4];
-        if constexpr (!READY) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) h[v] = Hw[(size_t)(16 * i + 4 * g + v) * PAD + col];
+        for (int v = 0; v < 4; ++v) {
+          const float d = t[m][v], e = h[m % kAhead][v];
+          any |= d != 0.0f;
+          t[m][v] = d != 0.0f ? e + d : e;
         }
+        changed |= (__ballot(any) != 0ull ? 1u : 0u) << m;
+        // (the tile kAhead further on into its place)
+        each_tile([&](auto i2, auto j2) __attribute__((always_inline)) {
+          if constexpr (tile_at<NB>(i2, j2) == m + kAhead) fetch(i2, j2);
+        });
+      });
+      each_tile([&](auto tile_row, auto tile_col) __attribute__((always_inline)) {
+        constexpr int i = tile_row, j = tile_col, m = tile_at<NB>(i, j);
+        if (!(changed >> m & 1u)) return;
+        const int col = 16 * j + c;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = 16 * i + 4 * g + v;
           const bool in = j < NB - 1 || (col < nv && (i < NB - 1 || row < nv));
-          float e = m[v];
-          if constexpr (!READY) {
-            const float d = m[v];
-            e = d != 0.0f ? h[v] + d : h[v];
-            if (d != 0.0f && in && (i < j || row <= col)) Hw[(size_t)row * PAD + col] = e;
-          }
-          m[v] = j == NB - 1 ? beyond(row, col, e) : e;
+          if (in && (i < j || row <= col)) *(float *)(row_at(Hw, 4 * g, i) + 4 * (v * PAD + 16 * j)) = t[m][v];  // (elements without a change: as they are)
         }
-      }
+      });
+    } else if (lane == 0) {
+      uni[nv] = 0;
+    }
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      float4v &m = t[tile_at<NB>(i, NB - 1)];
+      const float4v grad = *(const float4v *)(xl + 16 * i + 4 * g);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) m[v] = beyond(16 * i + 4 * g + v, 16 * (NB - 1) + c, m[v], grad[v]);
+    }
+    wave_sync();
     factor_tiles<NB>(t, rd, true, xl, nv, lane);
     // the forward-solved gradient, and the corner of the augmented column: 1e30 less its squares in order,
     // which leaves 1e30 as it is unless one of them comes near half an ulp of it (3.7e22)
@@ -522,7 +565,7 @@ __device__ __forceinline__ void dense_wave_world(float4v (&t)[kTiles<NB>], float
           float v = t[tile_at<NB>(i, j)][p];
           if (i == j) v = row <= col ? v : 0.0f;
           if (j == NB - 1 && c == 15) v = row < nv ? v : row == PAD - 1 ? corner : 0.0f;
-          Uw[(size_t)row * PAD + col] = v;
+          *(float *)(row_at(Uw, g, i) + 4 * (4 * p * PAD + 16 * j)) = v;
         }
       }
   } else {
