@@ -188,17 +188,38 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
       hc0[k] = row_quad(fr, hd[k], hf[k], hrf[k], hja[k], hv[k], hja[k]).c;
     }
   }
+  // Friction rows come first, so most trips of 32 rows have none: those form a row's point without the pieces that friction
+  // selects.  Rows read at every evaluation take three arrays instead of six there, two rows at a time, and only the trips
+  // with a friction row keep what is formed once (f / D, the cost at step 0).  A row's six loads and forty instructions were
+  // what bounded a round of the search: solves of 70 dofs x 157 rows x 2048 worlds 711 -> 695 us, 53 x 128 x 4096 (sparse)
+  // 732 -> 715, 43 x 96 x 8192 (sparse) 634 -> 624; with the rows in registers 27 x 64 x 4096 243.4 -> 241.7.
+  auto plain_rows = [&](auto point) __attribute__((always_inline)) {
+    for (int r = ne + lane + ((nf + 31) & ~31); r < nefc; r += 64) {
+      const bool second = r + 32 < nefc;
+      const int r1 = second ? r + 32 : r;
+      const float d0 = D[r], ja0 = Jaref[r], v0 = jv[r], d1 = D[r1], ja1 = Jaref[r1], v1 = jv[r1];
+      point(false, d0, 0.0f, 0.0f, ja0, v0, row_quad(false, d0, 0.0f, 0.0f, ja0, v0, ja0).c);
+      if (second) point(false, d1, 0.0f, 0.0f, ja1, v1, row_quad(false, d1, 0.0f, 0.0f, ja1, v1, ja1).c);
+    }
+  };
   // sum over this lane's rows of the rows' points at one or three step lengths
   auto rows_sum = [&](auto point) {
     if constexpr (HELD > 0) {
 #pragma unroll
       for (int k = 0; k < HELD; ++k) {
         const int r = ne + lane + 32 * k;
-        if (r < nefc) point(r < ne + nf, hd[k], hf[k], hrf[k], hja[k], hv[k], hc0[k]);
+        if (r >= nefc) continue;
+        if (k > 0 && 32 * k >= nf)
+          point(false, hd[k], 0.0f, 0.0f, hja[k], hv[k], hc0[k]);
+        else
+          point(r < ne + nf, hd[k], hf[k], hrf[k], hja[k], hv[k], hc0[k]);
       }
     } else if (wd.row_scratch0) {
-      for (int r = ne + lane; r < nefc; r += 32)
-        point(r < ne + nf, D[r], fl ? fl[r] : 0.0f, wd.row_scratch0[r], Jaref[r], jv[r], wd.row_scratch1[r]);
+      for (int base = 0; base < nf; base += 32) {
+        const int r = ne + base + lane;
+        if (r < nefc) point(r < ne + nf, D[r], fl ? fl[r] : 0.0f, wd.row_scratch0[r], Jaref[r], jv[r], wd.row_scratch1[r]);
+      }
+      plain_rows(point);
     } else {
       for (int r = ne + lane; r < nefc; r += 32) {
         const bool fr = r < ne + nf;
@@ -208,23 +229,32 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
       }
     }
   };
+  Pt z = {0.0f, 0.0f, 0.0f};
+  auto zero = [&](bool fr, float d, float f, float rf, float ja, float v, float) __attribute__((always_inline)) {
+    z = z + row_point_zero(fr, d, f, rf, ja, v);
+  };
   if (HELD == 0 && wd.row_scratch0) {
     // a lane writes and later reads its own rows only (a wavefront's two halves write the same values)
-    for (int r = ne + lane; r < nefc; r += 32) {
+    for (int base = 0; base < nf; base += 32) {
+      const int r = ne + base + lane;
+      if (r >= nefc) continue;
       const bool fr = r < ne + nf;
       const float d = D[r], f = fl ? fl[r] : 0.0f, ja = Jaref[r], v = jv[r];
       const float rf = fr ? safe_div(f, d) : 0.0f;
+      const Pt q = row_point_zero(fr, d, f, rf, ja, v);
       wd.row_scratch0[r] = rf;
-      wd.row_scratch1[r] = row_quad(fr, d, f, rf, ja, v, ja).c;
+      wd.row_scratch1[r] = q.c;
+      z = z + q;
     }
+    plain_rows(zero);
+  } else {
+    rows_sum(zero);
   }
   auto rows_at = [&](float alpha) {
     Pt s = {0.0f, 0.0f, 0.0f};
     rows_sum([&](bool fr, float d, float f, float rf, float ja, float v, float c0) { s = s + row_point_from(fr, d, f, rf, ja, v, c0, alpha); });
     return lanes_sum<SPLIT>(s);
   };
-  Pt z = {0.0f, 0.0f, 0.0f};
-  rows_sum([&](bool fr, float d, float f, float rf, float ja, float v, float) { z = z + row_point_zero(fr, d, f, rf, ja, v); });
   const Pt rows0 = lanes_sum<SPLIT>(z);
   const Pt p0 = {gauss.c + rows0.c, gauss.g + rows0.g, 2.0f * gauss.h + rows0.h};
   const Pt p0_delta = {0.0f, p0.g, p0.h};

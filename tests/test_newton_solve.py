@@ -3,6 +3,7 @@ and the force recovery (src/instantmimic/utils/mjw_step_optimized.py:2588-2683,
 src/instantmimic/utils/mjw_kernels/newton_fusion.py:330-539), started from poisoned solver state,
 captured in a graph without any read-back, against the oracle's pieces chained in the same order."""
 
+from dataclasses import replace
 from types import SimpleNamespace
 
 import numpy as np
@@ -305,6 +306,23 @@ def test_gpu_solve_at_the_edges_of_a_tile_of_j(device, monkeypatch, nv):
     monkeypatch.setitem(synth.SHAPES, name, shape)
     p = NC.problem(name, 401, "dense", empty_every=9)
     assert {0, 63, 64, 65} < set(p.nefc.tolist())
+    s = NC.oracle_solve(p)
+    m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
+    NC.compare(p, s, d, ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,stage,rows", [("g1", "sparse", 64), ("g1", "sparse", 130), ("ant", "tree", 64), ("ant", "tree", 128), ("ant", "tree", 130)])
+@pytest.mark.parametrize("ne,nf", [(0, 0), (2, 31), (1, 32), (2, 33), (3, 70)])
+def test_gpu_solve_with_friction_rows_up_to_a_trip_and_beyond(device, monkeypatch, name, stage, rows, ne, nf):
+    """The line search takes its trips of 32 rows without friction by a shorter form, with the rows in registers and
+    read at every evaluation: friction rows that end before, with and behind a trip, none at all, and more than a world has
+    rows."""
+    shape = synth.SHAPES[name]
+    monkeypatch.setitem(synth.SHAPES, name, replace(shape, nefc=rows))
+    p = NC.problem(name, 33, stage, empty_every=9)
+    p.ne = np.minimum(ne, p.nefc).astype(np.int32)
+    p.nf = np.minimum(nf, p.nefc - p.ne).astype(np.int32)
     s = NC.oracle_solve(p)
     m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
     NC.compare(p, s, d, ctx)
