@@ -236,6 +236,10 @@ __global__ __launch_bounds__(64 * WAVES, NB == 5 ? 3 : 4) void newton_dense_wave
   // as many wavefronts as the chip keeps resident; one whose world is done takes the next world
   // nobody has started (a counter in memory that only grows: every wavefront reaches the end)
   while (w < nworld) {
+    if (NB == 5) {
+      const resident::NewtonArgs &b = resident::kernel_args(0);
+      resident::row_priority(__builtin_amdgcn_readfirstlane(b.nefc ? b.nefc[w] : b.njmax), b.njmax);
+    }
     resident::newton_loop<HELD, NB == 5 ? 2 : 1, NB != 3, false, false>(0, L, w, stage);
     int next = 0;
     if ((threadIdx.x & 63) == 0) next = atomicAdd(next_world, 1);

@@ -547,6 +547,22 @@ __device__ __forceinline__ const NewtonArgs &kernel_args(int kernarg_offset) {
   return *(const NewtonArgs *)ap;
 }
 
+// The wavefront's priority among those of its SIMD: the quarter of the most rows that its world has.  A launch ends with
+// its slowest world, and rows are what is known of that beforehand (a world's time goes with its rows by 0.4 at 27 dofs,
+// 0.7 at 70): 27 dofs x 4096 worlds 242.5 -> 235.2 us, 53 x 4096 676 -> 669, 43 x 8192 623 -> 618 (tree stages), 70 x 2048
+// (dense) 693 -> 686.  The most rows of a workgroup's four worlds instead was worth half of that; on the sparse stage and
+// the dense one up to 64 dofs it made no difference either way.
+__device__ __forceinline__ void row_priority(int nefc, int njmax) {
+  if (4 * nefc > 3 * njmax)
+    __builtin_amdgcn_s_setprio(3);
+  else if (2 * nefc > njmax)
+    __builtin_amdgcn_s_setprio(2);
+  else if (4 * nefc > njmax)
+    __builtin_amdgcn_s_setprio(1);
+  else
+    __builtin_amdgcn_s_setprio(0);
+}
+
 // MLDS: the world's row of M is kept in LDS (where L.m_lds is not null); otherwise `M search` reads it from memory
 // every round, which leaves the LDS to more worlds per CU.
 template <int HELD, int COLS, bool WIDE, bool COOP, bool MLDS = true, class Stage>
@@ -582,6 +598,7 @@ __device__ __forceinline__ void newton_loop(int kernarg_offset, const LoopLds &L
     sc = Scalars{uniform(a.search_dot[w]), uniform(a.grad_dot[w]), uniform(a.decrement[w]), uniform(a.grad_scale[w]),
                  uniform(a.alpha[w]), uniform(a.improvement[w]), __builtin_amdgcn_readfirstlane(a.niter[w])};
     budget = a.maxiter;  // rounds this wavefront gives the world, whatever the data
+    if (COOP) row_priority(nefc, njmax);
     if (done) return;
     // what the loop keeps: M, Ma, Jaref into LDS (mv and jv are formed before they are read: a world
     // enters with a new search direction unless it is done) and qacc
