@@ -1459,7 +1459,7 @@ static int launch_blocked_factor(const float *M, int64_t ldM, int nM, const int3
     const char *e = std::getenv("IMHIP_BLOCKED_KERNEL");
     return e && std::strcmp(e, "simple") == 0;
   }();
-  bool wave = nv <= 128 && !simple;
+  bool wave = nv <= 128 && !simple && nM < (1 << 29);  // a row's bytes are counted in 31 bits there
   if (wave && B == 16 && nv >= 112) {
     int ncu = 0;
     if (const int st = im::compute_units(&ncu)) return st;

@@ -21,17 +21,37 @@ __device__ __forceinline__ int opaque(int i) {
   return i;
 }
 
+// n words as a buffer: a load at or past its end gives zero, a store there is dropped
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t words_of(const void *p, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, 4 * n, 0x00020000);
+}
+// the word `lane_bytes` + `bytes` from the buffer's start, the second the same for the whole wavefront
+__device__ __forceinline__ unsigned load_word(__amdgpu_buffer_rsrc_t words, int lane_bytes, int bytes) {
+  return __builtin_amdgcn_raw_buffer_load_b32(words, lane_bytes, bytes, 0);
+}
+
+// A world's right-hand side, a word or two a lane, zero where there is none; asked for ahead of the matrix, whose
+// words would otherwise be waited for first.
+template <int NB>
+constexpr int kRhs = (16 * NB + 63) / 64;
+template <int NB>
+__device__ __forceinline__ void load_rhs(float (&to)[kRhs<NB>], const float *yw, int nv, int lane) {
+#pragma unroll
+  for (int k = 0; k < kRhs<NB>; ++k) to[k] = yw && lane + 64 * k < nv ? yw[lane + 64 * k] : 0.0f;
+}
+
 // The factor, its store (rows and columns below `pad`, the tiles on and right of the block diagonal) and the
 // solution, which both kernels end with.  The tiles hold the matrix and the identity beyond
 // the dofs.  The right-hand side takes a spare last column
 // where there is one (nv < 16 NB: SPARE), and is forward-solved with the factor in either case.
 template <int NB, int B, bool SPARE>
-__device__ __forceinline__ void factor_solve_store(float4v (&t)[kTiles<NB>], float *xl, float *tt, const float *yw,
+__device__ __forceinline__ void factor_solve_store(float4v (&t)[kTiles<NB>], float *xl, float *tt, const float (&y)[kRhs<NB>],
                                                    float *xw, float *Uw, int nv, int pad, int lane) {
   const int g = lane >> 4, c = lane & 15;
-  const bool solve = yw && xw;
   float rd[NB];
-  for (int i = lane; i < 16 * NB; i += 64) xl[i] = solve && i < nv ? yw[i] : 0.0f;
+#pragma unroll
+  for (int k = 0; k < kRhs<NB>; ++k)
+    if (lane + 64 * k < 16 * NB) xl[lane + 64 * k] = y[k];
   wave_sync();
   if constexpr (SPARE) {
     if (c == 15) {
@@ -61,14 +81,16 @@ __device__ __forceinline__ void factor_solve_store(float4v (&t)[kTiles<NB>], flo
     wave_sync();
   }
   if (Uw) {
-    float *at = Uw + g * pad + c;
+    const __amdgpu_buffer_rsrc_t words = words_of(Uw, pad * pad);
+    const int at = 4 * (g * pad + c);
     auto tile = [&](int i, int j, int rows) __attribute__((always_inline)) {
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         if (4 * p >= rows) break;
         const float v = t[tile_at<NB>(i, j)][p];
         // (blocks of 8: a diagonal tile's lower left block lies below the block diagonal)
-        if (!(B == 8 && i == j && p > 1) || c >= 8) at[(16 * i + 4 * p) * pad + 16 * j] = i == j && 4 * p + g > c ? 0.0f : v;
+        if (!(B == 8 && i == j && p > 1) || c >= 8)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, i == j && 4 * p + g > c ? 0.0f : v), words, at, 4 * ((16 * i + 4 * p) * pad + 16 * j), 0);
       }
     };
     each<NB>([&](auto tile_row) __attribute__((always_inline)) {
@@ -85,7 +107,7 @@ __device__ __forceinline__ void factor_solve_store(float4v (&t)[kTiles<NB>], flo
         tile(i, NB - 1, B == 8 && i == NB - 1 ? edge : 16);
       });
   }
-  if (!solve) return;
+  if (!xw) return;
   backward_tiles<NB, B>(t, rd, xl, tt, nv, lane);
   for (int i = lane; i < nv; i += 64) xw[i] = xl[i];
 }
@@ -96,6 +118,12 @@ __device__ __forceinline__ void factor_solve_store(float4v (&t)[kTiles<NB>], flo
 // wavefront four (below, with B = 8 up to 40, in LDS): 8192 worlds of 35 / 64 dofs took 39.5 / 159 us with B = 8 and
 // 78 / 129 us with B = 16, 2048 of 128 dofs 225 and 127; here 37.7 / 77, 36.8 / 71, 107 and 92.  500 worlds of 35 dofs, one
 // wavefront each instead of a quarter: 24.3 -> 9.4 us.
+// The matrix, the table and the factor go through buffer descriptors: what lies past a world's words reads as zero without a
+// test, and a tile's place is a scalar, so that an element takes its two loads and three vector instructions where it took
+// twelve, and a store none beside its value.  The right-hand side, which the first panel needs, is asked for ahead of the
+// matrix.  B = 8 / B = 16, before and after: 35 dofs x 100 worlds 9.15 / 8.72 -> 8.88 / 8.62 us, x 8192 38.0 / 36.6 -> 36.0 / 34.2;
+// 64 x 1000 16.7 / 15.8 -> 15.9 / 15.0; 101 x 8192 233 / 220 -> 204 / 172 (registers that addresses held); 128 x 8192
+// 328 / 293 -> 281 / 256.  Priorities by a workgroup's place in the grid made no difference.
 // Element (r, c) of tile (i, j) is M[block_idx[tile][r][c]], zero at or past nM, with 1 on the padded diagonal;
 // of a diagonal block the lower triangle counts, as in the workgroup-per-world kernel.
 template <int NB, int B, bool SPARE>
@@ -108,26 +136,30 @@ __global__ __launch_bounds__(256, NB <= 4 ? 4 : NB <= 6 ? 3 : 2) void blocked_so
   const int64_t w = (int64_t)blockIdx.x * 4 + wv;
   if (w >= nworld || (active && active[w] == 0)) return;
   float *xl = lds + wv * wave_stage_words<NB>(), *tt = xl + 16 * NB;
+  const bool solve = y && x;
+  float rhs[kRhs<NB>];
+  load_rhs<NB>(rhs, solve ? y + w * ldy : nullptr, nv, lane);
   const int nblk = pad / B, edge = pad - 16 * (NB - 1);
-  const float *Mw = M + w * ldM;
-  // the lane's first element in the table, and where a diagonal block's upper triangle is found below it
-  const int at = ((4 * g / B) * nblk + c / B) * B * B + (4 * g % B) * B + c % B;
-  const int across = ((4 * g / B) * nblk + c / B) * B * B + (c % B) * B + 4 * g % B;
-  const bool same = 4 * g / B == c / B;
+  const __amdgpu_buffer_rsrc_t Mw = words_of(M + w * ldM, nM), table = words_of(block_idx, pad * pad);
+  // the lane's first element in the table, and where a diagonal block's upper triangle is found below it, in bytes; with blocks
+  // of 8 the last tile row and column may hold one block, whose place the lanes beyond it read instead
+  const int brow = 4 * g / B, bcol = c / B, here = 4 * (brow * nblk + bcol) * B * B;
+  const int at = here + 4 * ((4 * g % B) * B + c % B), across = here + 4 * ((c % B) * B + 4 * g % B);
+  const bool in_last = B == 16 || c < edge, in_corner = B == 16 || (c < edge && 4 * g < edge);
+  const int back = in_last ? 0 : 4 * bcol * B * B, corner_back = in_corner ? 0 : 4 * ((4 * g < edge ? 0 : brow * nblk) + (in_last ? 0 : bcol)) * B * B;
+  int upper[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) upper[v] = brow == bcol && 4 * g + v < c ? across + 4 * v : at + 4 * v * B;
   float4v t[kTiles<NB>];
-  int idx[kTiles<NB>][4];
+  unsigned idx[kTiles<NB>][4];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = i; j < NB; ++j) {
-      const int tile = (16 / B) * B * B * (i * nblk + j);
-      const bool in = B == 16 || j < NB - 1 || (c < edge && (i < NB - 1 || 4 * g < edge));
+      const int tile = 4 * (16 / B) * B * B * (i * nblk + j);
+      const int less = j < NB - 1 ? 0 : i < NB - 1 ? back : corner_back;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int e = i == j && same && 4 * g + v < c ? across + v : at + v * B;
-        const int id = block_idx[opaque(in ? tile + e : 0)];
-        idx[tile_at<NB>(i, j)][v] = in ? id : nM;
-      }
+      for (int v = 0; v < 4; ++v) idx[tile_at<NB>(i, j)][v] = load_word(table, (i == j ? upper[v] : at + 4 * v * B) - less, tile);
     }
 #pragma unroll
   for (int i = 0; i < NB; ++i)
@@ -135,12 +167,15 @@ __global__ __launch_bounds__(256, NB <= 4 ? 4 : NB <= 6 ? 3 : 2) void blocked_so
     for (int j = i; j < NB; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int e = idx[tile_at<NB>(i, j)][v];
-        const float m = Mw[opaque(e < nM ? e : 0)];
-        t[tile_at<NB>(i, j)][v] = (e < nM ? m : 0.0f) + (i == NB - 1 && 4 * g + v == c && 16 * i + c >= nv ? 1.0f : 0.0f);
+        unsigned e = idx[tile_at<NB>(i, j)][v];
+        e = e < (unsigned)nM ? e : (unsigned)nM;
+        if (B == 8 && j == NB - 1) e = (i == NB - 1 ? in_corner : in_last) ? e : (unsigned)nM;
+        float m = __builtin_bit_cast(float, load_word(Mw, (int)(4 * e), 0));
+        if (i == NB - 1) m += 4 * g + v == c && 16 * i + c >= nv ? 1.0f : 0.0f;
+        t[tile_at<NB>(i, j)][v] = m;
       }
-  factor_solve_store<NB, B, SPARE>(t, xl, tt, y ? y + w * ldy : nullptr, x ? x + w * ldx : nullptr,
-                            U ? U + w * (int64_t)pad * pad : nullptr, nv, pad, lane);
+  factor_solve_store<NB, B, SPARE>(t, xl, tt, rhs, solve ? x + w * ldx : nullptr, U ? U + w * (int64_t)pad * pad : nullptr, nv,
+                                   pad, lane);
 }
 
 // H's upper tiles into both triangles (a diagonal tile's upper half counts); ld a multiple of four and Hw on 16
@@ -198,6 +233,9 @@ __global__ __launch_bounds__(256, NB <= 4 ? 4 : NB <= 6 ? 3 : 2) void jtdj_solve
   const int32_t *sw = state + w * (int64_t)njmax;
   int nefc = nefc_p ? nefc_p[w] : njmax;
   nefc = __builtin_amdgcn_readfirstlane(nefc < njmax ? nefc : njmax);
+  const bool solve = y && x;
+  float rhs[kRhs<NB>];
+  load_rhs<NB>(rhs, solve ? y + w * ldy : nullptr, nv, lane);
   float4v t[kTiles<NB>];
   // M first: its trips to memory pass under the listing
 #pragma unroll
@@ -283,8 +321,8 @@ __global__ __launch_bounds__(256, NB <= 4 ? 4 : NB <= 6 ? 3 : 2) void jtdj_solve
       const bool out = c >= tail || (i == NB - 1 && 4 * g + v >= tail);
       if (out) t[tile_at<NB>(i, NB - 1)][v] = i == NB - 1 && 4 * g + v == c ? 1.0f : 0.0f;
     }
-  factor_solve_store<NB, 16, SPARE>(t, xl, tt, y ? y + w * ldy : nullptr, x ? x + w * ldx : nullptr,
-                             U ? U + w * (int64_t)pad * pad : nullptr, nv, pad, lane);
+  factor_solve_store<NB, 16, SPARE>(t, xl, tt, rhs, solve ? x + w * ldx : nullptr, U ? U + w * (int64_t)pad * pad : nullptr, nv,
+                                    pad, lane);
 }
 
 template <int NB, int B>

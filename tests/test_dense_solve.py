@@ -37,6 +37,39 @@ def test_gpu_blocked_solve_at_block_edges(device, nv, B):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B", [8, 16])
+@pytest.mark.parametrize("nv", [7, 24, 35, 56, 101, 128])
+def test_gpu_blocked_solve_of_a_sparse_matrix(device, nv, B):
+    """Elements whose id is past the matrix's (by one, by many, by more than a byte count of 32 bits holds) are zero; the values lie
+    in another order, in rows of a wider array whose other words are poison."""
+    import torch
+
+    rng, nworld, wide = np.random.default_rng(nv), 5, 3
+    A = rng.standard_normal((nworld, nv, nv)).astype(np.float32) / np.float32(nv)
+    A = A + A.transpose(0, 2, 1) + 4 * np.eye(nv, dtype=np.float32)
+    drop = np.triu(rng.random((nv, nv)) < 0.3, 1)
+    drop |= drop.T
+    A[:, drop] = 0.0
+    keep = np.argwhere(~drop)
+    keep = keep[rng.permutation(len(keep))]
+    nM = len(keep)
+    elemid = rng.choice(np.array([nM, nM + 9, 1 << 30, 2**31 - 1], np.int32), (nv, nv))
+    elemid[keep[:, 0], keep[:, 1]] = np.arange(nM)
+    M = np.full((nworld, nM + wide), np.nan, np.float32)
+    M[:, :nM] = A[:, keep[:, 0], keep[:, 1]]
+    y = rng.standard_normal((nworld, nv)).astype(np.float32)
+    pad, layout, _ = BD.block_index_layout(elemid, nv, nM, B)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    Md, yd, idx, x, U = t(M), t(y), t(layout), torch.full((nworld, nv), np.nan, device=device), torch.zeros((nworld, pad, pad), device=device)
+    st = _lib.lib().im_blocked_factor_solve(Md.data_ptr(), nM + wide, nM, idx.data_ptr(), B, nv, pad, yd.data_ptr(), nv, U.data_ptr(), x.data_ptr(), nv, nworld, None)
+    assert st == 0
+    torch.cuda.synchronize()
+    x_ref, U_ref = R.blocked_factor_solve(M[:, :nM], layout, nv, pad, B, y)
+    np.testing.assert_array_equal(U.cpu().numpy(), U_ref)
+    np.testing.assert_array_equal(x.cpu().numpy(), x_ref)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nv", [1, 15, 16, 17, 33, 48, 64, 79, 80, 96, 112, 127, 128])
 def test_gpu_dense_hessian_solve_at_block_edges(device, nv):
     import torch
