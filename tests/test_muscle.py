@@ -165,15 +165,15 @@ def test_gpu_projection_with_more_entries_than_one_staging_trip(device):
     assert (got[:, : mb.root_dof_count] == 7.0).all()
 
 
-def _fv_case(nworld, seed=4, active_type=1.0, nmuscle=37):
+def _fv_case(nworld, seed=4, active_type=1.0, nmuscle=37, points=(2, 6), dofs=(1, 4)):
     """Random muscles over random waypoints: every branch of the force-velocity curve is hit."""
     rng = np.random.default_rng(seed)
     nv, root = 30, 6
-    counts = rng.integers(2, 6, nmuscle)
+    counts = rng.integers(*points, nmuscle)
     wp_start = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
     nwp = int(wp_start[-1])
     waypoints = rng.normal(size=(nworld, nwp, 3)).astype(np.float32)
-    ndof = rng.integers(1, 4, nmuscle)
+    ndof = rng.integers(*dofs, nmuscle)
     dof_offsets = np.concatenate([[0], np.cumsum(ndof)]).astype(np.int32)
     dof_torque = np.concatenate([np.sort(rng.choice(nv - root, n, replace=False)) for n in ndof]).astype(np.int32)
     params = np.stack([rng.uniform(100, 3000, nmuscle), rng.uniform(0.5, 1.5, nmuscle), rng.uniform(0.0, 0.5, nmuscle), rng.uniform(0, 0.5, nmuscle)], 1).astype(np.float32)
@@ -294,6 +294,30 @@ def test_gpu_force_velocity_state_on_every_workgroup_size(device, nmuscle, n):
     import torch
 
     c = _fv_case(n, active_type=1.0, nmuscle=nmuscle)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    outs = [torch.full((n, nmuscle), float("nan"), device=device) for _ in range(5)]
+    Q.eval_muscle_force_velocity_state(
+        t(c["waypoints"]), t(c["wp_start"]), t(c["params"]), t(c["rest"]), t(c["length_scale"]), t(c["act"]), t(c["qvel"]),
+        t(c["moment"]), t(c["dof_offsets"]), t(c["dof_torque"]), c["root"], muscle_force_scale=float(c["model"][0]),
+        muscle_length_norm_min=float(c["model"][1]), muscle_length_norm_max=float(c["model"][2]), vmax=1.5, fvmax=1.4,
+        clamp_activation=True, include_active=True, active_force_model_params=c["model"][3:6],
+        muscle_length=outs[0], effective_activation=outs[1], length_velocity=outs[2], force_velocity_multiplier=outs[3],
+        force_velocity_slope=outs[4],
+    )  # fmt: skip
+    want = R.muscle_force_velocity_state(**c)
+    for k in range(4):
+        np.testing.assert_array_equal(outs[k].cpu().numpy(), want[k])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nmuscle, points, n", [(60, 18, 3), (60, 18, 1500), (200, 10, 1500), (350, 18, 1100)])
+def test_gpu_force_velocity_state_of_short_and_long_muscles(device, nmuscle, points, n):
+    """Muscles of no, one and up to sixteen distances and entries (both sums go four terms at a time with the next four
+    asked for ahead), with the next world's rows held in registers and with muscles beyond the threads: bit for bit."""
+    import torch
+
+    c = _fv_case(n, seed=nmuscle, nmuscle=nmuscle, points=(1, points), dofs=(0, 17))
+    assert {1, 2, 5, 6, 9} <= set(np.diff(c["wp_start"])) and {0, 1, 4, 5} <= set(np.diff(c["dof_offsets"]))
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
     outs = [torch.full((n, nmuscle), float("nan"), device=device) for _ in range(5)]
     Q.eval_muscle_force_velocity_state(
