@@ -13,6 +13,7 @@
 #include <cstdint>
 
 #include "common.h"
+#include "newton_solve.h"
 
 namespace im {
 namespace {
@@ -104,74 +105,138 @@ struct QhGain {
   int nu;
 };
 
+// LDS written by some of a world's threads, then read by others
+template <int NT>
+__device__ __forceinline__ void world_sync() {
+  if constexpr (NT == 64) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
+// NT threads per world, 256 / NT worlds per workgroup.  What bounds it is trips to memory behind one another (tables, values,
+// three more of both kinds in each term) and barriers between phases of a few hundred words: a workgroup per world had
+// three of its four wavefronts idle in most of them, and two thousand of them fill the chip.  A wavefront per world has no
+// barrier and four times as many worlds under way; twelve of M's elements and two of a term's are in flight per lane, and no
+// load waits for a test.  qH and its solve, 62 dofs x 4096 worlds 31.4 -> 24.9 us, x 8192 54.8 -> 39.6, x 64 11.8 -> 11.1.
+template <int NT>
 __global__ __launch_bounds__(256) void implicit_qh_kernel(const float *__restrict__ M, int64_t ldM, int nM,
                                                           const int32_t *__restrict__ elem_dof,
                                                           const float *__restrict__ damping, int64_t ld_damping,
                                                           float timestep, QhGain g, im_row_pair_term ta,
-                                                          im_row_pair_term tt, int max_entries,
-                                                          float *__restrict__ out, int64_t ldo) {
+                                                          im_row_pair_term tt, int max_entries, int world_words,
+                                                          float *__restrict__ out, int64_t ldo, int nworld) {
   extern __shared__ float lds[];
-  float *q = lds;                           // [nM]
+  const int part = NT == 256 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+  const int tid = threadIdx.x % NT;
+  const int64_t w = (int64_t)blockIdx.x * (256 / NT) + part;
+  if (w >= nworld) return;  // a whole wavefront; with NT = 256 there is none
+  float *q = lds + part * world_words;      // [nM]
   float *gain = q + nM;                     // [nu]
   float *m = gain + g.nu;                   // [max_entries + 1]
   float *weighted = m + max_entries + 1;    // [max_entries + 1]
   float *partial = weighted + max_entries + 1;  // [max chunk count]
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int64_t w = blockIdx.x;
   const float *Mw = M + w * ldM, *dw = damping + w * ld_damping;
-  for (int e = tid; e < nM; e += nt) {
-    const int d = elem_dof[e];
-    const float v = Mw[e];
-    q[e] = d >= 0 ? __builtin_fmaf(timestep, dw[d], v) : v;
-  }
-  for (int a = tid; a < g.nu; a += nt) {
-    float v = 0.0f;
-    if (g.biastype[a] == 1) v = g.biasprm[a * g.ldprm + 2];
-    if (g.gaintype[a] == 1) v = __builtin_fmaf(g.gainprm[a * g.ldprm + 2], g.input[w * g.ld_input + a], v);
-    if (g.forcelimited && g.forcelimited[a] && g.force) {
-      const float f = g.force[w * g.ld_force + a];
-      if (f <= g.forcerange[2 * a] || f >= g.forcerange[2 * a + 1]) v = 0.0f;
+  constexpr int U = NT == 64 ? 12 : 3, UT = NT == 64 ? 2 : 1;  // elements, and a term's entries, chunks and sums, in flight per thread
+  for (int e0 = tid; e0 < nM; e0 += U * NT) {
+    int d[U];
+    float v[U], b[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int e = e0 + k * NT < nM ? e0 + k * NT : nM - 1;
+      d[k] = elem_dof[e];
+      v[k] = Mw[e];
     }
+#pragma unroll
+    for (int k = 0; k < U; ++k) b[k] = dw[d[k] >= 0 ? d[k] : 0];
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (e0 + k * NT < nM) q[e0 + k * NT] = d[k] >= 0 ? __builtin_fmaf(timestep, b[k], v[k]) : v[k];
+  }
+  // (every load ahead of every test: a test between two of them is a trip to memory of its own)
+  for (int a = tid; a < g.nu; a += NT) {
+    const int bias_affine = g.biastype[a], gain_affine = g.gaintype[a];
+    const float bias = g.biasprm[a * g.ldprm + 2], slope = g.gainprm[a * g.ldprm + 2], in = g.input[w * g.ld_input + a];
+    bool limited = false;
+    float f = 0.0f, low = 0.0f, high = 0.0f;
+    if (g.forcelimited && g.force) {  // the same for the whole grid
+      limited = g.forcelimited[a] != 0;
+      f = g.force[w * g.ld_force + a], low = g.forcerange[2 * a], high = g.forcerange[2 * a + 1];
+    }
+    float v = bias_affine == 1 ? bias : 0.0f;
+    if (gain_affine == 1) v = __builtin_fmaf(slope, in, v);
+    if (limited && (f <= low || f >= high)) v = 0.0f;
     gain[a] = v;
     if (g.gain) g.gain[w * g.ld_gain + a] = v;
   }
-  __syncthreads();
+  world_sync<NT>();
   for (int which = 0; which < 2; ++which) {
     const im_row_pair_term &t = which == 0 ? ta : tt;
     if (t.nentry <= 0 || t.nelem <= 0) continue;  // the same for the whole workgroup
-    for (int e = tid; e < t.nentry; e += nt) {
-      const float v = t.values[w * t.ld_values + (t.entry_source ? t.entry_source[e] : e)];
-      const int row = t.entry_row[e];
-      const float wt = t.weight ? t.weight[w * t.ld_weight + row] : gain[row];
-      m[e] = v;
-      weighted[e] = wt * v;
+    for (int e0 = tid; e0 < t.nentry; e0 += UT * NT) {
+      int from[UT], row[UT];
+      float v[UT], wt[UT];
+#pragma unroll
+      for (int k = 0; k < UT; ++k) {
+        const int e = e0 + k * NT < t.nentry ? e0 + k * NT : t.nentry - 1;
+        from[k] = t.entry_source ? t.entry_source[e] : e;
+        row[k] = t.entry_row[e];
+      }
+#pragma unroll
+      for (int k = 0; k < UT; ++k) {
+        v[k] = t.values[w * t.ld_values + from[k]];
+        wt[k] = t.weight ? t.weight[w * t.ld_weight + row[k]] : gain[row[k]];
+      }
+#pragma unroll
+      for (int k = 0; k < UT; ++k)
+        if (e0 + k * NT < t.nentry) {
+          m[e0 + k * NT] = v[k];
+          weighted[e0 + k * NT] = wt[k] * v[k];
+        }
     }
     if (tid == 0) {
       m[t.nentry] = 0.0f;
       weighted[t.nentry] = 0.0f;
     }
-    __syncthreads();
-    for (int c = tid; c < t.chunk_count; c += nt) {
-      float total = 0.0f;
+    world_sync<NT>();
+    for (int c0 = tid; c0 < t.chunk_count; c0 += UT * NT) {
+      int packed[UT][16];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int packed = t.chunk_pairs[(size_t)k * t.chunk_count + c];
-        total = __builtin_fmaf(weighted[packed & 0xFFFF], m[packed >> 16], total);
+      for (int u = 0; u < UT; ++u) {
+        const int c = c0 + u * NT < t.chunk_count ? c0 + u * NT : t.chunk_count - 1;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) packed[u][k] = t.chunk_pairs[(size_t)k * t.chunk_count + c];
       }
-      partial[c] = total;
+#pragma unroll
+      for (int u = 0; u < UT; ++u) {
+        float total = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) total = __builtin_fmaf(weighted[packed[u][k] & 0xFFFF], m[packed[u][k] >> 16], total);
+        if (c0 + u * NT < t.chunk_count) partial[c0 + u * NT] = total;
+      }
     }
-    __syncthreads();
-    for (int slot = tid; slot < t.nelem; slot += nt) {
-      float acc = 0.0f;
-      const int c1 = t.chunk_offsets[slot + 1];
-      for (int c = t.chunk_offsets[slot]; c < c1; ++c) acc = acc + partial[c];
-      const int e = t.elem_ids[slot];
-      q[e] = __builtin_fmaf(t.scale, acc, q[e]);
+    world_sync<NT>();
+    for (int s0 = tid; s0 < t.nelem; s0 += UT * NT) {
+      int first[UT], end[UT], at[UT];
+#pragma unroll
+      for (int u = 0; u < UT; ++u) {
+        const int slot = s0 + u * NT < t.nelem ? s0 + u * NT : t.nelem - 1;
+        first[u] = t.chunk_offsets[slot], end[u] = t.chunk_offsets[slot + 1], at[u] = t.elem_ids[slot];
+      }
+#pragma unroll
+      for (int u = 0; u < UT; ++u) {
+        float acc = 0.0f;
+        for (int c = first[u]; c < end[u]; ++c) acc = acc + partial[c];
+        if (s0 + u * NT < t.nelem) q[at[u]] = __builtin_fmaf(t.scale, acc, q[at[u]]);
+      }
     }
-    __syncthreads();
+    world_sync<NT>();
   }
   float *ow = out + w * ldo;
-  for (int e = tid; e < nM; e += nt) ow[e] = q[e];
+  for (int e = tid; e < nM; e += NT) ow[e] = q[e];
 }
 
 }  // namespace
@@ -263,8 +328,16 @@ int im_implicit_qh(const float *M, int64_t ldM, int nM, const int32_t *elem_dof,
   if (lds_bytes > 64 * 1024) return IM_ERR_UNSUPPORTED;
   const im::QhGain g{gaintype, biastype, gainprm, biasprm, ld_prm, forcelimited, forcerange, input, ld_input,
                      force, ld_force, gain, ld_gain, nu};
-  hipLaunchKernelGGL(im::implicit_qh_kernel, dim3((unsigned)nworld), dim3(256), lds_bytes, (hipStream_t)stream, M, ldM,
-                     nM, elem_dof, dof_damping, ld_damping, timestep, g, ta, tt, max_entries, qH, ld_qH);
+  // A wavefront per world for batches that a workgroup per world would take in several rounds, as far as four worlds' rows
+  // share 64 KB: qH and its solve at 62 dofs, workgroups / wavefronts, us: x 64 11.1 / 13.2, x 1000 13.1 / 14.0, x 1500
+  // 15.6 / 15.9, x 2000 16.9 / 16.5, x 3000 24.4 / 19.9, x 8192 48.9 / 39.6 (256 compute units).
+  int ncu = 0;
+  if (const int st = im::compute_units(&ncu)) return st;
+  const bool wave = nworld > 7 * ncu && 4 * lds_bytes <= 64 * 1024;
+  const int worlds = wave ? 4 : 1;
+  hipLaunchKernelGGL(wave ? im::implicit_qh_kernel<64> : im::implicit_qh_kernel<256>, dim3((unsigned)((nworld + worlds - 1) / worlds)), dim3(256),
+                     worlds * lds_bytes, (hipStream_t)stream, M, ldM, nM, elem_dof, dof_damping, ld_damping, timestep, g, ta, tt, max_entries,
+                     (int)(lds_bytes / sizeof(float)), qH, ld_qH, nworld);
   IM_HIP_CHECK(hipGetLastError());
   return IM_OK;
 }

@@ -213,3 +213,39 @@ def test_gpu_qh_with_polynomial_dampers(device):
     m.has_fluid = True
     with pytest.raises(NotImplementedError):
         Q.create_implicit_qh_scratch(m, dd, device)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("actuators, tendons", [(True, True), (True, False), (False, True), (False, False)])
+def test_gpu_qh_of_large_batches(device, actuators, tendons):
+    """Batches on a wavefront per world, whole workgroups of four and remainders of one to three, and the last one on a
+    workgroup per world; with both terms, one and none: every world as in a small batch, bit for bit."""
+    import torch
+
+    host = 61
+    m, d, st, _ = _model(host)
+    if not actuators:
+        m.nactuator = 0
+    if not tendons:
+        m.ntendon = 0
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+
+    def qh(rows, fused=True):
+        dd = SimpleNamespace(nworld=len(rows), M=t(d.M[rows]), moment_rownnz=d.moment_rownnz, moment_rowadr=d.moment_rowadr, moment_colind=d.moment_colind,
+                             actuator_moment=t(d.actuator_moment[rows]), ten_J=t(d.ten_J[rows]), ctrl=t(d.ctrl[rows]),
+                             actuator_force=t(d.actuator_force[rows]))  # fmt: skip
+        scratch = Q.create_implicit_qh_scratch(m, dd, device)
+        scratch.implicit_qderiv.fill_(float("nan"))
+        Q.deriv_smooth_vel(m, dd, scratch.implicit_qderiv, scratch, fused=fused)
+        return scratch.implicit_qderiv.cpu().numpy(), None if scratch.actuator_gain is None else scratch.actuator_gain.cpu().numpy()
+
+    want, gain = qh(np.arange(host), fused=False)
+    if actuators and tendons:
+        np.testing.assert_array_equal(want, _oracle_qh(m, d, st)[0])
+    waves = 7 * torch.cuda.get_device_properties(device).multi_processor_count
+    for n in (waves, waves + 1, waves + 2, waves + 3, waves + 4, 2 * waves + 1):
+        rows = (np.arange(n) * 7 + n) % host
+        got, got_gain = qh(rows)
+        np.testing.assert_array_equal(got, want[rows])
+        if actuators:
+            np.testing.assert_array_equal(got_gain, gain[rows])
