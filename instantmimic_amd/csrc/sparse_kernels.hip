@@ -20,6 +20,7 @@
 #include "newton_solve.h"
 #include "newton_wave.h"
 #include "sparse_plan.h"
+#include "sparse_steps.h"
 
 namespace im {
 namespace {
@@ -42,6 +43,11 @@ SparseDev sparse_dev(const im_sparse_plan &plan) {
   P.steps = plan.steps, P.dof_pairs = plan.dof_pairs;
   P.nfactor_steps = plan.nfactor_steps, P.nbackward_steps = plan.nbackward_steps;
   return P;
+}
+
+inline SparseSizes sparse_sizes(const im_sparse_plan &plan) {
+  const int32_t *solve_end = plan.t[RK] + ((plan.sizes[RK] + 3) & ~3);
+  return {plan.nv, plan.nslots, plan.steps ? step_words(sparse_dev(plan)) : 0, (int)(solve_end - plan.t[FL]) + ((plan.nv + 3) & ~3)};
 }
 
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -198,12 +204,11 @@ __device__ __forceinline__ void backward_sums(const SparseDev &P, float *N, cons
 // ---- the same for a wavefront per world, from the plan's steps ----------------------------------------
 // A level's teams are the same for every world and every round, so what a lane does in it is settled when the plan is
 // uploaded: a step is one word pair a lane (operands' first words and number of terms, the entry's slot and column), the
-// team's width and whether a sum starts or ends in the step alike in all lanes.  A workgroup's worlds share a copy in LDS
-// (12 KB at 35 dofs), read a step ahead.  From the tables a level waited for three LDS reads, one behind the other, before the first operand,
+// team's width and whether a sum starts or ends in the step alike in all lanes.  They are read a step ahead, from memory or,
+// in the resident loop, from a copy in LDS that a workgroup's worlds share (12 KB at 35 dofs).  From the tables a level waited for three LDS reads, one behind the other, before the first operand,
 // and spent two thirds of its instructions on them and their addresses; a short run's terms were read one by one.
 // Same operations in the same order.  Whole solves, from the tables -> from the steps: 35 dofs x 8192 worlds with 96 rows
 // 779 -> 661 us, x 100 with 40 rows 312 -> 252, 56 dofs x 4096 with 128 rows 892 -> 763, 62 dofs x 1000 498 -> 431.
-constexpr int kStepTerms = 4;  // terms' operands read ahead of their products
 template <int T>
 __device__ __forceinline__ float step_terms(const float *pa, const float *pb, const float *pd, int n, float v) {
   int t = 0;
@@ -218,7 +223,7 @@ __device__ __forceinline__ float step_terms(const float *pa, const float *pb, co
   } while (__ballot(t < n) != 0ull);
   return v;
 }
-// `rec`: the plan's factor steps in LDS, one more word pair a lane behind the last
+// `rec`: the plan's factor steps, in LDS or in memory, one more word pair a lane behind the last
 __device__ __forceinline__ void factor_steps(const uint2 *rec, int steps, float *N, float *iD, int lane) {
   float v = 0.0f;
   uint2 ahead = rec[lane];
@@ -481,8 +486,10 @@ __global__ void sparse_init_kernel(SparseDev P, const uint8_t *__restrict__ done
 }
 
 // ---- initial factor, one wavefront per world --------------------------------------------
-// Four worlds per workgroup; each world
-// belongs to one wavefront, so its LDS traffic needs no workgroup barrier.  J'DJ is summed
+// Four worlds per workgroup; each world belongs to one wavefront, so its LDS traffic needs no workgroup barrier, and the
+// plan's steps are read from memory a step ahead.  A copy of them in LDS is staged for one pass and costs a CU worlds where it is
+// large: forest of 57 dofs, 34 KB of steps, 40 rows x 8192 worlds 107.1 us with the copy, 89.0 without, 49 dofs (34 KB), 96 rows
+// x 4096 78.9 / 60.0, 35 dofs (12 KB) 40 rows x 8192 56.5 / 55.8, 56 dofs (19 KB) x 100 25.1 / 25.0.  J'DJ is summed
 // on the matrix cores: v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one
 // after the other with a fused multiply-add each, rows ascending, which is the order and
 // rounding of `v = fmaf(J[r][a] * Dc[r], J[r][b], v)` when one operand is the rounded
@@ -495,25 +502,11 @@ struct SparseWave {
   SparseDev P;
   int solve[5];               // update stage only: offsets of the forward-solve tables FL .. RK from FL
   int solve_words;            // length of that stretch and of ORIG behind it, multiples of 4
-  int staged_steps;           // words of steps in LDS: all or none
+  int staged_steps;           // resident loop only: words of steps in LDS, all or none
   const int32_t *tile_index;  // [tile][4][64]: (index into M + 1) << 16 | (slot + 1), 0 = none
   int block, nM;              // the plan's block width; length of a row of M
   int staged_rows;            // update stage: changed rows of J a world keeps in LDS, 16 or 32 (more are read from memory)
 };
-
-// Steps of more than 36 KB (a chain of 47 dofs, or patterns whose entries have several runs: a step of their teams for each)
-// would leave a CU few worlds: they are read from memory, which 35 dofs x 8192 worlds, whose own are 12 KB, took 700 us
-// per solve with, 661 from LDS and 779 from the tables.
-constexpr int kStagedStepsMost = 9216;
-inline int staged_steps(const SparseDev &P) { return step_words(P) <= kStagedStepsMost ? step_words(P) : 0; }
-// The plan's factor and backward solve on one world.
-template <class Steps>
-__device__ __forceinline__ void with_steps(const SparseWave &A, const int32_t *lds, Steps &&run) {
-  if (A.staged_steps)
-    run((const uint32_t *)lds);
-  else
-    run(A.P.steps);
-}
 
 // `words` (a multiple of 4) from 16-byte aligned memory into LDS by T threads, eight loads of 16 bytes in flight a thread.
 template <int T>
@@ -530,10 +523,6 @@ __device__ __forceinline__ void copy_words(int32_t *to, const void *from, int wo
   }
 }
 
-// (the factor's steps read up to 3 * 64 words past an operand's last term, which they leave out)
-constexpr int kStepSlack = (kStepTerms - 1) * 64;
-__host__ __device__ inline int init_world_words(int nslots, int n) { return (nslots + n + kStepSlack + 3) & ~3; }
-
 template <int NT>
 __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
     SparseWave A, const uint8_t *__restrict__ done, const int32_t *__restrict__ nefc_p,
@@ -546,17 +535,14 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
   const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, kq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: world data is addressed from scalar registers
   const SparseDev &Q = A.P;
-  copy_words<256>((int32_t *)lds, Q.steps, A.staged_steps, tid);
-  __syncthreads();  // the only workgroup barrier: worlds are independent from here on
   const int w = blockIdx.x * 4 + wv;
   if (w >= nworld || (done && done[w])) return;
   const int n = Q.nv, nslots = Q.nslots, nfac = nslots - n, rhs = nfac;
-  const int njp = (njmax + 3) & ~3, factor_words = init_world_words(nslots, n);
-  const int per_world = factor_words + 2 * njp;
-  float *N = lds + A.staged_steps + wv * per_world;  // [nslots]; a row of M before the factor
-  float *iD = N + nslots;                           // [n]
-  float *dl = N + factor_words;                     // [njp] weights of the listed constraint rows
-  int *rowl = (int *)(dl + njp);                       // [njp] their numbers
+  const int njp = (njmax + 3) & ~3;
+  float *N = lds + wv * init_world_words(nslots, n, njmax);  // [nslots]; a row of M before the factor
+  float *iD = N + nslots;                                  // [n]
+  float *dl = N + ((nslots + n + 3) & ~3);                 // [njp] weights of the listed constraint rows
+  int *rowl = (int *)(dl + njp);                           // [njp] their numbers
   float *U = U_ + (size_t)w * Q.nv_pad * Q.nv_pad;
   const float *Mw = M + (size_t)w * ldM;
   const float *gw = grad + (size_t)w * ldg;
@@ -719,14 +705,10 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
   const int32_t *ORIGt = Q.t[ORIG];
   for (int j = lane; j < n; j += 64) N[rhs + j] = gw[ORIGt[j]];
   sync_world();
-  with_steps(A, (const int32_t *)lds, [&](const uint32_t *steps) __attribute__((always_inline)) {
-    factor_steps((const uint2 *)steps, Q.nfactor_steps, N, iD, lane);
-  });
+  factor_steps((const uint2 *)Q.steps, Q.nfactor_steps, N, iD, lane);
   for (int s = lane; s < nfac; s += 64) U[nfac + s] = N[s];
   for (int j = lane; j < n; j += 64) U[2 * nfac + j] = iD[j];
-  with_steps(A, (const int32_t *)lds, [&](const uint32_t *steps) __attribute__((always_inline)) {
-    backward_steps(steps + factor_step_words(Q), Q.nbackward_steps, rhs, N, iD, lane);
-  });
+  backward_steps(Q.steps + factor_step_words(Q), Q.nbackward_steps, rhs, N, iD, lane);
   search_sums(n, rhs, N, iD, ORIGt, gw, search_ + (size_t)w * n, search_dot + w, decrement + w, lane, A.block);
   if (nbad && lane == 0) atomicAdd(U + Q.nv_pad * Q.nv_pad - 1, (float)nbad);
 }
@@ -740,7 +722,8 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
 // read different dofs meet in no LDS bank.  32 rows where that costs a CU no world, 16 otherwise.
 constexpr int kStagedRowsMax = 32;
 
-// The steps of a plan, its forward solve's tables and its dofs' order into LDS, for a workgroup of T threads.
+// The steps of a plan (where A.staged_steps says so), its forward solve's tables and its dofs' order into LDS, for a
+// workgroup of T threads.
 __device__ __forceinline__ int orig_at(const SparseWave &A) { return A.solve_words - ((A.P.nv + 3) & ~3); }
 template <int T>
 __device__ __forceinline__ void stage_update_tables(const SparseWave &A, float *lds, int tid) {
@@ -751,12 +734,10 @@ __device__ __forceinline__ void stage_update_tables(const SparseWave &A, float *
   copy_words<T>(tab, A.P.t[FL], orig, tid);
   if (tid < A.P.nv) tab[orig + tid] = A.P.t[ORIG][tid];
 }
-__host__ __device__ inline int update_world_words(int nslots, int n, int staged_rows) {
-  const int factor = nslots + n + 2 * n + (staged_rows + 1) * n + staged_rows, reach = nslots + n + kStepSlack;
-  return ((factor > reach ? factor : reach) + 3) & ~3;
-}
-
-// The stage for one world and one wavefront (`world_lds`: update_world_words of LDS of its own).
+// The stage for one world and one wavefront (`world_lds`: update_world_words of LDS of its own).  STAGED: the steps may lie in
+// `shared`.  The kernel of a single pass reads them from memory (as the first factor; 57 dofs x 8192 worlds with four of 40 rows
+// changed 75.0 us with a copy in LDS, 74.9 without, 56 dofs 71.6 / 68.3, 35 dofs 48.7 / 47.5).
+template <bool STAGED>
 __device__ __forceinline__ void sparse_update_world(
     const SparseWave &A, const int32_t *shared, float *world_lds, int count,
     const int32_t *__restrict__ ids, int ld_ids, const float *__restrict__ J, int njmax,
@@ -768,7 +749,13 @@ __device__ __forceinline__ void sparse_update_world(
   int lane = lane_in;
   asm volatile("" : "+v"(lane));
   const SparseDev &Q = A.P;
-  const int32_t *tables = shared + A.staged_steps;
+  const int32_t *tables = STAGED ? shared + A.staged_steps : shared;
+  auto with_steps = [&](auto &&run) __attribute__((always_inline)) {
+    if (STAGED && A.staged_steps)
+      run((const uint32_t *)shared);
+    else
+      run(Q.steps);
+  };
   const int n = Q.nv, nslots = Q.nslots, nfac = nslots - n, rhs = nfac;
   float *N = world_lds;                              // [nslots]
   float *iD = N + nslots;                            // [n]
@@ -945,7 +932,7 @@ __device__ __forceinline__ void sparse_update_world(
     for (int j = lane; j < n; j += 64) N[rhs + j] = gw[ORIGt[j]];
     sync_world();
     IM_SSTAMP(2);
-    with_steps(A, shared, [&](const uint32_t *steps) __attribute__((always_inline)) {
+    with_steps([&](const uint32_t *steps) __attribute__((always_inline)) {
       factor_steps((const uint2 *)steps, Q.nfactor_steps, N, iD, lane);
     });
     IM_SSTAMP(3);
@@ -988,7 +975,7 @@ __device__ __forceinline__ void sparse_update_world(
     }
     IM_SSTAMP(5);
   }
-  with_steps(A, shared, [&](const uint32_t *steps) __attribute__((always_inline)) {
+  with_steps([&](const uint32_t *steps) __attribute__((always_inline)) {
     backward_steps(steps + factor_step_words(Q), Q.nbackward_steps, rhs, N, iD, lane);
   });
   search_sums(n, rhs, N, iD, ORIGt, gw, search_ + (size_t)w * n, search_dot + w, decrement + w, lane, A.block);
@@ -1011,8 +998,8 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void sparse_update_wave_ker
   __syncthreads();  // the only workgroup barrier
   const int w = blockIdx.x * WAVES + wv;
   if (w >= nworld || (done && done[w]) || state_changes[w] == 0) return;
-  float *world_lds = lds + A.staged_steps + A.solve_words + wv * update_world_words(A.P.nslots, A.P.nv, A.staged_rows);
-  sparse_update_world(A, (const int32_t *)lds, world_lds, changes[w], ids, ld_ids, J, njmax, D, state, quad, grad, ldg, U_, uni_, search_,
+  float *world_lds = lds + A.solve_words + wv * update_world_words(A.P.nslots, A.P.nv, A.staged_rows);
+  sparse_update_world<false>(A, (const int32_t *)lds, world_lds, changes[w], ids, ld_ids, J, njmax, D, state, quad, grad, ldg, U_, uni_, search_,
                       search_dot, decrement, w, lane);
 }
 
@@ -1020,13 +1007,6 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void sparse_update_wave_ker
 // line search to convergence, WAVES worlds per workgroup sharing one copy of the plan's tables.
 // Per wavefront in LDS: the world's row of M and the search direction, and one area that the staged
 // tile of J, the gradient's row list and the stage's factor use one after the other.
-__host__ __device__ inline int resident_area_words(int nslots, int n, int njmax, int staged_rows) {
-  int words = update_world_words(nslots, n, staged_rows);
-  const int tile = 64 * 17, grad = 2 * njmax + n;
-  words = words > tile ? words : tile;
-  words = words > grad ? words : grad;
-  return (words + 3) & ~3;
-}
 template <int WAVES, int HELD>
 __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident_kernel(
     SparseWave A, resident::NewtonArgs a, float *__restrict__ U_, int32_t *__restrict__ uni_,
@@ -1074,7 +1054,7 @@ __global__ __launch_bounds__(64 * WAVES, 16 / WAVES) void newton_sparse_resident
     typedef const SparseWave __attribute__((address_space(4))) KernelSparseWave;
     KernelSparseWave *plan = (KernelSparseWave *)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(plan));
-    sparse_update_world(*(const SparseWave *)plan, (const int32_t *)lds, mine, b.quad_count[w], b.ids, b.ld_ids, b.J, b.njmax, b.D, b.state, b.quad, b.grad,
+    sparse_update_world<true>(*(const SparseWave *)plan, (const int32_t *)lds, mine, b.quad_count[w], b.ids, b.ld_ids, b.J, b.njmax, b.D, b.state, b.quad, b.grad,
                         (int)b.ld_grad, U_, uni_, b.search, b.search_dot, b.decrement, (int)w, threadIdx.x & 63);
   };
   while (w < nworld) {
@@ -1234,63 +1214,6 @@ extern "C" {
 
 namespace im {
 
-namespace {
-// A plan's levels as the steps of a wavefront's 64 lanes (factor_steps, backward_steps).
-struct WaveSteps {
-  std::vector<uint32_t> words;  // the factor's, an empty one, the backward solve's, an empty one
-  std::vector<uint16_t> pairs;
-  int nfactor = 0, nbackward = 0;
-};
-WaveSteps wave_steps(const im_sparse_plan &pl) {
-  WaveSteps out;
-  std::vector<uint32_t> factor, backward;
-  const auto &T = pl.table;
-  for (int l = 0; l < pl.nlevels; ++l) {
-    const int width = T[LT][l], teams = 64 / width;
-    int log2 = 0;
-    while ((1 << log2) < width) ++log2;
-    for (int e0 = T[LP][l]; e0 < T[LP][l + 1]; e0 += teams) {
-      int runs = 1;
-      for (int e = e0; e < std::min(e0 + teams, T[LP][l + 1]); ++e) runs = std::max(runs, T[RP][e + 1] - T[RP][e]);
-      for (int r = 0; r < runs; ++r)
-        for (int lane = 0; lane < 64; ++lane) {
-          const int e = e0 + lane / width, tl = lane % width;
-          uint32_t x = 0, y = (uint32_t)log2 << 26 | (uint32_t)(r == 0) << 29 | (uint32_t)(r == runs - 1) << 30;
-          if (e < T[LP][l + 1]) {
-            if (r < T[RP][e + 1] - T[RP][e]) {
-              const uint32_t ab = (uint32_t)T[RAB][T[RP][e] + r], kl = (uint32_t)T[RKL][T[RP][e] + r];
-              const int terms = ((int)(kl >> 16) - tl + width - 1) / width;
-              if ((int)(kl >> 16) > tl) {
-                x = ((ab & 0xFFFFu) + tl) | ((ab >> 16) + tl) << 12;
-                y |= ((kl & 0xFFFFu) + tl) | (uint32_t)terms << 6;
-              }
-            }
-            if (r == runs - 1 && tl == 0) {
-              y |= (uint32_t)(T[ES][e] + 1) << 13;
-              x |= (uint32_t)(T[EC][e] + 1) << 24;
-            }
-          }
-          factor.push_back(x);
-          factor.push_back(y);
-        }
-    }
-    for (int p0 = T[BL][l]; p0 < T[BL][l + 1]; p0 += 64)
-      for (int lane = 0; lane < 64; ++lane) {
-        const int p = p0 + lane;
-        backward.push_back(p < T[BL][l + 1] ? (uint32_t)T[BS][p] | (uint32_t)T[BI][p] << 12 | (uint32_t)T[BJ][p] << 18 | 1u << 31 : 0u);
-      }
-  }
-  out.nfactor = (int)(factor.size() / 128), out.nbackward = (int)(backward.size() / 64);
-  factor.resize(factor.size() + 128, 0);
-  backward.resize(backward.size() + 64, 0);
-  out.words = std::move(factor);
-  out.words.insert(out.words.end(), backward.begin(), backward.end());
-  for (int c = 0; c < 64; ++c)
-    for (int r = 0; r <= c; ++r) out.pairs.push_back((uint16_t)(r | c << 8));
-  return out;
-}
-}  // namespace
-
 int sparse_plan_upload(im_sparse_plan *pl) {
   pl->device_ready = false;
   // the kernels' workgroup widths; 128 lanes only in the upstream-iteration kernel
@@ -1395,10 +1318,8 @@ int im_sparse_init_factor(const im_sparse_plan *plan, const uint8_t *done, const
     A.solve_words = 0;
     A.block = plan->block;
     A.nM = plan->nM;
-    // per world: the factor's arrays and the list of contributing constraint rows (weight and number)
-    const size_t per_world = (size_t)im::init_world_words(plan->nslots, n) + 2 * (((size_t)njmax + 3) & ~(size_t)3);
-    A.staged_steps = im::staged_steps(P);
-    const size_t wave_lds = 4 * (A.staged_steps + 4 * per_world);
+    A.staged_steps = 0;
+    const size_t wave_lds = im::init_lds_bytes(im::sparse_sizes(*plan), njmax);
     if (wave_lds <= 64 * 1024) {
       const dim3 grid((unsigned)((nworld + 3) / 4)), wg(256);
       const hipStream_t st = (hipStream_t)stream;
@@ -1448,32 +1369,17 @@ int im_sparse_update_factor(const im_sparse_plan *plan, const uint8_t *done, con
     A.tile_index = nullptr;
     A.block = plan->block;
     A.nM = 0;
-    const int32_t *solve_end = plan->t[im::RK] + ((plan->sizes[im::RK] + 3) & ~3);
-    const size_t forward_words = (size_t)(solve_end - plan->t[im::FL]), solve_words = forward_words + ((n + 3) & ~3), shared_words = im::staged_steps(P) + solve_words;
-    A.staged_steps = im::staged_steps(P);
-    // 32 staged rows where a CU still holds sixteen worlds with them, else 16
-    A.staged_rows =
-        4 * (shared_words + 16 * (size_t)im::update_world_words(plan->nslots, n, 32)) <= 160 * 1024 ? 32 : 16;
-    const size_t per_world = (size_t)im::update_world_words(plan->nslots, n, A.staged_rows);
     for (int i = 0; i < 5; ++i) A.solve[i] = (int)(plan->t[im::FL + i] - plan->t[im::FL]);
-    A.solve_words = (int)solve_words;
-    const size_t wave_lds = 4 * (shared_words + 4 * per_world);
-    if (wave_lds <= 64 * 1024 && forward_words <= 4096) {
-      // Worlds per workgroup: every workgroup stages the tables for itself, so larger workgroups
-      // leave more of a CU's 160 KB to the worlds.  The count that keeps the most worlds on a CU
-      // (at most 32 wavefronts of 57 registers) is taken, the smallest on a tie and where four
-      // per workgroup already hold the whole batch.
-      constexpr size_t kCuLds = 160 * 1024;
-      int waves = 4, ncu = 0;
-      int64_t best = 0;
-      if (const int st = im::compute_units(&ncu)) return st;
-      for (int cand = 4; cand <= 16; cand *= 2) {
-        const size_t bytes = 4 * (shared_words + (size_t)cand * per_world);
-        int64_t held = (int64_t)(kCuLds / bytes) * cand;
-        held = held < 32 ? held : 32;
-        if (held > best && (cand == 4 || (int64_t)nworld > best * ncu)) best = held, waves = cand;
-      }
-      const size_t lds_bytes = 4 * (shared_words + (size_t)waves * per_world);
+    const im::SparseSizes sizes = im::sparse_sizes(*plan);
+    int ncu = 0;
+    if (const int st = im::compute_units(&ncu)) return st;
+    const im::SparseUpdate u = im::sparse_update_layout(sizes, nworld, ncu);
+    A.solve_words = sizes.shared_words;
+    A.staged_steps = 0;
+    A.staged_rows = u.staged_rows;
+    if (u.waves) {
+      const int waves = u.waves;
+      const size_t lds_bytes = u.lds;
       const dim3 grid((unsigned)((nworld + waves - 1) / waves)), wg(64 * waves);
 #define IM_UPDATE_WAVE(W)                                                                                     \
   do {                                                                                                        \
@@ -1551,18 +1457,10 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
   A.tile_index = nullptr;
   A.block = plan->block;
   A.nM = 0;
-  const int32_t *solve_end = plan->t[RK] + ((plan->sizes[RK] + 3) & ~3);
-  const size_t forward_words = (size_t)(solve_end - plan->t[FL]), solve_words = forward_words + ((n + 3) & ~3);
   for (int i = 0; i < 5; ++i) A.solve[i] = (int)(plan->t[FL + i] - plan->t[FL]);
-  A.solve_words = (int)solve_words;
-  A.staged_steps = staged_steps(A.P);
-  if (!plan->steps || forward_words > 4096) return IM_ERR_UNSUPPORTED;
-  const size_t shared = A.staged_steps + solve_words + (((size_t)p->nterm + n + 1 + 3) & ~(size_t)3);
-  auto wave_words = [&](int staged_rows) {
-    return (size_t)resident_area_words(plan->nslots, n, njmax, staged_rows) + resident::kept_words(n, njmax, 0);
-  };
-  // the most worlds per workgroup (one workgroup per CU) that 160 KB of LDS admit and whose kernel
-  // keeps to registers
+  const SparseSizes sizes = sparse_sizes(*plan);
+  A.solve_words = sizes.shared_words;
+  if (!plan->steps) return IM_ERR_UNSUPPORTED;
   struct Variant {
     int waves, held;
     const void *fn;
@@ -1581,32 +1479,29 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
   static Kept<int, std::array<bool, kVariants>> probed;
   std::array<bool, kVariants> usable;
   if (const int st = usable_variants(probed, variants, &usable)) return st;
-  for (int i = 0; i < kVariants; ++i) {
-    if (!usable[i] || variants[i].held != (njmax <= 64 ? 2 : 0)) continue;
-    // 32 staged rows where the workgroup still fits with them (they cost a CU no world then), else 16
-    // (snu: 32 rows with eight worlds per CU instead of twelve was measured slower, 1344 against 1283 us per loop)
-    A.staged_rows = 4 * (shared + (size_t)variants[i].waves * wave_words(32)) <= 158 * 1024 ? 32 : 16;
-    const size_t lds = 4 * (shared + (size_t)variants[i].waves * wave_words(A.staged_rows));
-    if (lds > 158 * 1024) continue;
-    const int waves = variants[i].waves;
-    // as many workgroups as stay resident at once (LDS, and sixteen wavefronts of up to 128 registers
-    // per CU); the others' worlds are taken up by the wavefronts that finish
-    int ncu = 0;
-    if (const int st = compute_units(&ncu)) return st;
-    const int per_cu = std::max(1, std::min((int)(160 * 1024 / lds), 16 / waves));
-    const int grid = resident_worlds_grid(p->nworld, waves, ncu, per_cu, false, &a.group_worlds);
-    int *counter = plan->next_world;
-    if (before) {
-      a.final_force = 1;
-      if (const int st = (*before)(counter, grid * waves)) return st;
-    } else {
-      set_counter(counter, grid * waves, stream);
-    }
-    void *args[] = {&A, &a, &hfactor, &dof_union, &counter};
-    IM_HIP_CHECK(hipLaunchKernel(variants[i].fn, dim3((unsigned)grid), dim3(64 * waves), args, lds, stream));
-    return IM_OK;
+  const int held = njmax <= 64 ? 2 : 0;
+  std::vector<int> admitted;
+  for (int i = 0; i < kVariants; ++i)
+    if (usable[i] && variants[i].held == held) admitted.push_back(variants[i].waves);
+  int ncu = 0;
+  if (const int st = compute_units(&ncu)) return st;
+  const SparseResident r = sparse_resident_layout(sizes, njmax, ((p->nterm + n + 1 + 3) & ~3), resident::kept_words(n, njmax, 0), admitted, p->nworld, ncu);
+  if (r.waves == 0) return IM_ERR_UNSUPPORTED;
+  A.staged_rows = r.staged_rows;
+  A.staged_steps = r.step_words;
+  // as many workgroups as stay resident at once; the others' worlds are taken up by the wavefronts that finish
+  const int grid = resident_worlds_grid(p->nworld, r.waves, ncu, r.per_cu, false, &a.group_worlds);
+  int *counter = plan->next_world;
+  if (before) {
+    a.final_force = 1;
+    if (const int st = (*before)(counter, grid * r.waves)) return st;
+  } else {
+    set_counter(counter, grid * r.waves, stream);
   }
-  return IM_ERR_UNSUPPORTED;
+  void *args[] = {&A, &a, &hfactor, &dof_union, &counter};
+  for (const Variant &v : variants)
+    if (v.held == held && v.waves == r.waves) IM_HIP_CHECK(hipLaunchKernel(v.fn, dim3((unsigned)grid), dim3(64 * r.waves), args, r.lds, stream));
+  return IM_OK;
 }
 
 }  // namespace im
