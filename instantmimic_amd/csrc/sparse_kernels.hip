@@ -207,6 +207,10 @@ __device__ __forceinline__ void backward_sums(const SparseDev &P, float *N, cons
 // team's width and whether a sum starts or ends in the step alike in all lanes.  They are read a step ahead, from memory or,
 // in the resident loop, from a copy in LDS that a workgroup's worlds share (12 KB at 35 dofs).  From the tables a level waited for three LDS reads, one behind the other, before the first operand,
 // and spent two thirds of its instructions on them and their addresses; a short run's terms were read one by one.
+// A forest's entries have several runs of a term or two each, a step to a run: steps in which no lane has more than one term, or two,
+// read those alone (four are read otherwise, whatever there are), and a team's sum is formed behind its last run.  Forests of 54 and 57
+// dofs, from the tables / four terms a step / now: first factor x 8192 worlds 79 / 80 / 70 and 80 / 89 / 72 us, update stage 66 / 64 /
+// 52 and 68 / 75 / 55, solve 642 / 551 / 475 and 687 / 642 / 539; trees with one run an entry as before (35 dofs x 8192 441 / 433).
 // Same operations in the same order.  Whole solves, from the tables -> from the steps: 35 dofs x 8192 worlds with 96 rows
 // 779 -> 661 us, x 100 with 40 rows 312 -> 252, 56 dofs x 4096 with 128 rows 892 -> 763, 62 dofs x 1000 498 -> 431.
 template <int T>
@@ -230,16 +234,26 @@ __device__ __forceinline__ void factor_steps(const uint2 *rec, int steps, float 
   for (int s = 0; s < steps; ++s) {
     const uint2 r = ahead;
     ahead = rec[lane + 64 * (s + 1)];
-    const unsigned info = (unsigned)__builtin_amdgcn_readfirstlane((int)r.y) >> 26;
+    const unsigned info = (unsigned)__builtin_amdgcn_readfirstlane((int)r.y) >> 25;
+    const unsigned log2 = info >> 1 & 7u;
     const float *pa = N + (r.x & 0xFFFu), *pb = N + (r.x >> 12 & 0xFFFu), *pd = iD + (r.y & 63u);
     const int n = r.y >> 6 & 127u, slot = (int)(r.y >> 13 & 0xFFFu) - 1, col = (int)(r.x >> 24) - 1;
     const float old = N[slot < 0 ? 0 : slot];
-    if (info & 8u) v = 0.0f;
-    float sum;
-    if ((info & 7u) == 0u) {
-      sum = v = step_terms<1>(pa, pb, pd, n, v);
+    if (info & 16u) v = 0.0f;
+    if (info & 65u) {  // no lane has more than one term, or than two
+      const float a = *pa, b = *pb, d = *pd;
+      if (info & 1u) {
+        v = n > 0 ? fma_(a * b, d, v) : v;
+      } else {
+        const int next = 1 << log2;
+        const float a1 = pa[next], b1 = pb[next], d1 = pd[next];
+        v = n > 0 ? fma_(a * b, d, v) : v;
+        v = n > 1 ? fma_(a1 * b1, d1, v) : v;
+      }
+    } else if (log2 == 0u) {
+      v = step_terms<1>(pa, pb, pd, n, v);
     } else {
-      switch (info & 7u) {
+      switch (log2) {
         case 1: v = step_terms<2>(pa, pb, pd, n, v); break;
         case 2: v = step_terms<4>(pa, pb, pd, n, v); break;
         case 3: v = step_terms<8>(pa, pb, pd, n, v); break;
@@ -247,16 +261,17 @@ __device__ __forceinline__ void factor_steps(const uint2 *rec, int steps, float 
         case 5: v = step_terms<32>(pa, pb, pd, n, v); break;
         default: v = step_terms<64>(pa, pb, pd, n, v); break;
       }
-      // the team's shuffle-down tree (as in factor_level)
-      sum = v;
-      if ((info & 7u) > 5) sum = sum + __shfl_down(sum, 32, 64);
-      if ((info & 7u) > 4) sum = sum + __shfl_down(sum, 16, 64);
-      if ((info & 7u) > 3) sum = sum + row_shl<8>(sum);
-      if ((info & 7u) > 2) sum = sum + row_shl<4>(sum);
-      if ((info & 7u) > 1) sum = sum + row_shl<2>(sum);
-      sum = sum + row_shl<1>(sum);
     }
-    if (info & 16u) {
+    if (info & 32u) {
+      float sum = v;
+      if (log2) {  // the team's shuffle-down tree (as in factor_level)
+        if (log2 > 5) sum = sum + __shfl_down(sum, 32, 64);
+        if (log2 > 4) sum = sum + __shfl_down(sum, 16, 64);
+        if (log2 > 3) sum = sum + row_shl<8>(sum);
+        if (log2 > 2) sum = sum + row_shl<4>(sum);
+        if (log2 > 1) sum = sum + row_shl<2>(sum);
+        sum = sum + row_shl<1>(sum);
+      }
       if (slot >= 0) {
         const float wv = old - sum;
         N[slot] = wv;

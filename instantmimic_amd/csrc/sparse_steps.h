@@ -38,10 +38,13 @@ inline WaveSteps wave_steps(const im_sparse_plan &pl) {
     for (int e0 = T[LP][l]; e0 < T[LP][l + 1]; e0 += teams) {
       int runs = 1;
       for (int e = e0; e < std::min(e0 + teams, T[LP][l + 1]); ++e) runs = std::max(runs, T[RP][e + 1] - T[RP][e]);
-      for (int r = 0; r < runs; ++r)
+      for (int r = 0; r < runs; ++r) {
+        int most = 0;  // terms of a lane
+        for (int e = e0; e < std::min(e0 + teams, T[LP][l + 1]); ++e)
+          if (r < T[RP][e + 1] - T[RP][e]) most = std::max(most, (int)(((uint32_t)T[RKL][T[RP][e] + r] >> 16) + width - 1) / width);
         for (int lane = 0; lane < 64; ++lane) {
           const int e = e0 + lane / width, tl = lane % width;
-          uint32_t x = 0, y = (uint32_t)log2 << 26 | (uint32_t)(r == 0) << 29 | (uint32_t)(r == runs - 1) << 30;
+          uint32_t x = 0, y = (uint32_t)(most < 2) << 25 | (uint32_t)log2 << 26 | (uint32_t)(r == 0) << 29 | (uint32_t)(r == runs - 1) << 30 | (uint32_t)(most == 2) << 31;
           if (e < T[LP][l + 1]) {
             if (r < T[RP][e + 1] - T[RP][e]) {
               const uint32_t ab = (uint32_t)T[RAB][T[RP][e] + r], kl = (uint32_t)T[RKL][T[RP][e] + r];
@@ -59,6 +62,7 @@ inline WaveSteps wave_steps(const im_sparse_plan &pl) {
           factor.push_back(x);
           factor.push_back(y);
         }
+      }
     }
     for (int p0 = T[BL][l]; p0 < T[BL][l + 1]; p0 += 64)
       for (int lane = 0; lane < 64; ++lane) {

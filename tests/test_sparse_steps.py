@@ -58,7 +58,9 @@ def test_steps_factor_and_solve(name):
     assert not steps[-1].any()
     v = np.zeros(64)
     for x, y in (s.T for s in steps[:-1]):
-        assert len(set((y >> 26) & 31)) == 1
+        assert len(set(y >> 25)) == 1
+        most = int((y >> 6 & 127).max())
+        assert (y[0] >> 25 & 1, y[0] >> 31) == (most < 2, most == 2)
         width = 1 << int(y[0] >> 26 & 7)
         if y[0] >> 29 & 1:
             v[:] = 0.0
