@@ -912,3 +912,80 @@ def test_gpu_torque_call_is_the_dispatchers_operator():
         got = torch.autograd.grad(y, act, g)[0]
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(got, same(twice)[1])
+
+
+def _in_a_process_of_its_own(script: str) -> None:
+    """What is registered with an operator, or taken from torch, stays so for the process."""
+    import subprocess
+    import sys
+
+    from conftest import ROOT
+
+    done = subprocess.run([sys.executable, "-c", script], cwd=ROOT, capture_output=True, text=True, timeout=110)
+    assert done.returncode == 0, done.stdout + done.stderr
+
+
+@pytest.mark.parametrize("take", ["del torch._C._dispatch_keys", "del torch._C._functorch.peek_interpreter_stack", "del torch.autograd.forward_ad._current_level",
+                                  "torch._C._dispatch_has_kernel_for_any_dispatch_key = lambda name: False"])  # fmt: skip
+def test_torque_operator_without_a_private_name_of_torch(take):
+    _in_a_process_of_its_own(f"""
+import torch
+{take}
+from instantmimic_amd.muscle import warp_custom_ops as ops
+assert ops._EAGER is None
+assert type(ops.muscle_torque_forward) is type(ops.muscle_torque_backward) is torch.library.CustomOpDef
+""")
+
+
+def test_torque_operator_notices_what_is_registered_with_it():
+    _in_a_process_of_its_own("""
+import torch
+from instantmimic_amd.muscle import warp_custom_ops as ops
+forward, backward = ops.muscle_torque_forward, ops.muscle_torque_backward
+assert ops._is_as_defined(forward) and ops._is_as_defined(backward)
+for key in ("CUDA", "AutocastCUDA", "AutogradCUDA"):
+    lib = torch.library.Library(ops.NAMESPACE, "IMPL")
+    lib.impl("torque_forward", lambda *a: None, key)
+    assert not ops._is_as_defined(forward) and ops._is_as_defined(backward)
+    lib._destroy()
+    assert ops._is_as_defined(forward)
+torch.library.register_autocast("instantmimic_muscle::torque_backward", "cuda", torch.float16)
+assert not ops._is_as_defined(backward) and ops._is_as_defined(forward)
+forward.register_autocast("cuda", torch.float16)
+assert not ops._is_as_defined(forward)
+""")
+    for register in ('register_kernel("cuda", lambda *a: None)', 'register_kernel(None, lambda *a: None)', "register_autograd(lambda ctx, g: g)"):
+        _in_a_process_of_its_own(f"""
+from instantmimic_amd.muscle import warp_custom_ops as ops
+ops.muscle_torque_forward.{register}
+assert not ops._is_as_defined(ops.muscle_torque_forward)
+""")
+
+
+@pytest.mark.gpu
+def test_gpu_torque_call_under_a_registered_cast():
+    """With a gradient to record as without, and in the backward."""
+    _in_a_process_of_its_own("""
+import torch
+from instantmimic_amd import synth
+from instantmimic_amd.muscle import warp_custom_ops as ops
+from instantmimic_amd.muscle.muscle_dynamics import MuscleDynamicsLayer
+rig = synth.make_muscle_rig(nmuscle=12, seed=3)
+layer = MuscleDynamicsLayer(rig.topology, **rig.dims(), device="cuda")
+key, ctx = ops.warp_op_key(layer), torch.from_numpy(synth.make_muscle_context(rig, 33, seed=4)).cuda()
+act, g = torch.rand(33, 12, device="cuda", requires_grad=True), torch.randn(33, rig.torque_dim, device="cuda")
+direct, dispatched = ops.muscle_torque_forward, torch.ops.instantmimic_muscle.torque_forward
+def both(op):
+    with torch.autocast("cuda", torch.float16):
+        y = op(act, ctx, key, False)
+        return y.detach(), torch.autograd.grad(y, act, g)[0]
+def same(a, b):
+    return all(x.dtype == y.dtype and torch.equal(x, y) for x, y in zip(a, b))
+plain = both(direct)
+assert same(plain, both(dispatched))
+ops.muscle_torque_backward.register_autocast("cuda", torch.float16)
+assert same(both(direct), both(dispatched))
+direct.register_autocast("cuda", torch.float16)
+cast = both(direct)
+assert same(cast, both(dispatched)) and not torch.equal(cast[0], plain[0])
+""")
