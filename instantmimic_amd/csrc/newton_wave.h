@@ -232,7 +232,14 @@ struct StagedM {
 #pragma unroll
     for (int u = 0; u < LOADS; ++u)
       if (lane + 64 * u < nM) stage[lane + 64 * u] = x[u];
-    for (int k = lane + 64 * LOADS; k < nM; k += 64) stage[k] = m[k];
+    for (int k = lane + 64 * LOADS; k < nM; k += 64 * 4) {  // a longer row's other words
+      float y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) y[u] = m[(unsigned)(k + 64 * u < nM ? k + 64 * u : nM - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (k + 64 * u < nM) stage[k + 64 * u] = y[u];
+    }
     wave_sync();
     mul_m_world<WALK>(a, term, radr, stage, v, out, out_lds, lane);
   }
