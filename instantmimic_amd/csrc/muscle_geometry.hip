@@ -635,7 +635,7 @@ struct MwArgs {
   int nworld;
 };
 
-constexpr int kContribPad = 32;  // floats read past the last entry by ordered_sum()
+constexpr int kContribPad = 4;  // floats read past the last entry by ordered_sum()
 constexpr int kAxis = 7;        // floats of a dof's record: its cdof and, for MW_GRAD, grad_output
 struct MwLds {
   float *segd;     // [nseg][9]: dir (0 for a degenerate segment), p0 - c0, p1 - c1
@@ -687,30 +687,22 @@ __device__ __forceinline__ float entry_contribution(const float *lds, const MwEn
   return c;
 }
 
-// Sum of contrib[e0..e1) in list order from +0.  LONG: sixteen entries at a time, the next sixteen on their way while
-// these are added (torque of 284 muscles x 4096 worlds 68.2 -> 65.1 us, gradient 61.2 -> 57.3), otherwise four.  Entries
-// past e1 are read (contrib is padded for that) and enter as +0, which leaves every bit of a sum that started at +0
-// (such a sum is never -0).
+// Sum of contrib[e0..e1) in list order from +0.  Whole groups of 16 (LONG) and of 4 entries are
+// read with one address and added without a test; the last group reads up to three floats past
+// e1 (contrib is padded for that) and enters them as +0, which leaves every bit of a sum that
+// started at +0 (such a sum is never -0).
 template <bool LONG>
 __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e1) {
   float total = 0.0f;
   int e = e0;
   if (LONG) {
-    float c[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
     for (; e + 16 <= e1; e += 16) {
-      float ahead[16];
+      float c[16];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) ahead[k] = contrib[e + 16 + k];
+      for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
 #pragma unroll
       for (int k = 0; k < 16; ++k) total = total + c[k];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) c[k] = ahead[k];
     }
-#pragma unroll
-    for (int k = 0; k < 15; ++k) total = total + (e + k < e1 ? c[k] : 0.0f);
-    return total;
   }
   for (; e + 4 <= e1; e += 4) {
     float c[4];
@@ -726,6 +718,29 @@ __device__ __forceinline__ float ordered_sum(const float *contrib, int e0, int e
 #pragma unroll
     for (int k = 0; k < 3; ++k) total = total + (e + k < e1 ? c[k] : 0.0f);
   }
+  return total;
+}
+
+// The same with the next sixteen entries on their way while sixteen are added, for a kernel with the registers for them (torque of 284 muscles x 4096 worlds
+// 68.2 -> 65.1 us in groups, gradient 61.2 -> 57.3; muscle_world_kernel with kept entries spilled: 90 muscles x 4096 41.3 -> 43.7 us).
+// Words up to kSumAhead past the last entry are read and left out.
+constexpr int kSumAhead = 16;
+__device__ __forceinline__ float ordered_sum_ahead(const float *contrib, int e0, int e1) {
+  float total = 0.0f, c[16];
+  int e = e0;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) c[k] = contrib[e + k];
+  for (; e + 16 <= e1; e += 16) {
+    float ahead[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) ahead[k] = contrib[e + 16 + k];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) total = total + c[k];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) c[k] = ahead[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 15; ++k) total = total + (e + k < e1 ? c[k] : 0.0f);
   return total;
 }
 
@@ -943,13 +958,15 @@ __host__ __device__ inline CtxLds ctx_lds(const im_muscle_context &c, bool force
   const int sums = c.nentry + kContribPad, points = 3 * c.nwaypoint, records = 9 * c.nsegment, poses = kPose * c.nbody;
   CtxLds l;
   l.contrib = 0;  // the waypoints lie here until the contributions take their place
-  l.segd = ((sums > points ? sums : points) + 3) & ~3;  // and the bodies' records until the segments' do
+  l.segd = sums > points ? sums : points;  // and the bodies' records until the segments' do
+  if (GROUPS) l.segd = (l.segd + 3) & ~3;
   l.axis = l.segd + (records > poses ? records : poses);
   l.force = l.axis + kAxis * c.ntorque;
   l.com = l.force + (forces ? c.nmuscle : 0);
   l.flags = l.com + 3 * c.nbody;
   l.dist = l.flags + 2;
   l.words = l.dist + (GROUPS && forces ? c.nlength + 3 : 0);
+  if (GROUPS && l.words < c.nentry + kSumAhead) l.words = c.nentry + kSumAhead;
   return l;
 }
 
@@ -1480,7 +1497,7 @@ __global__ __launch_bounds__(NT, WAVES) void muscle_groups_kernel(CtxArgs) {
         if (MODE == MW_MOMENT)
           out[(unsigned)r] = large ? ordered_sum<false>(lds, e0, e1) : lds[r];
         else
-          out[(unsigned)r] = MODE == MW_GRAD && lds[ctx_lds<true>(a.c, FORCES).force + r] == 0.0f ? 0.0f : ordered_sum<true>(lds, e0, e1);
+          out[(unsigned)r] = MODE == MW_GRAD && lds[ctx_lds<true>(a.c, FORCES).force + r] == 0.0f ? 0.0f : ordered_sum_ahead(lds, e0, e1);
       }
     }
   }

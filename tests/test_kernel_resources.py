@@ -61,3 +61,10 @@ def test_resident_loops_stay_within_the_private_memory_they_are_admitted_with(ke
         limit = int(re.search(r"kResidentPrivate = (\d+);", f.read())[1])
     private = {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if re.search(r"newton_(sparse|dense_tile|dense_wave)_resident_kernel", n)}
     assert len(private) == 22 and max(private.values()) <= limit <= 2 * max(private.values())
+
+
+def test_kept_muscle_entries_stay_in_registers(kernels):
+    """Up to four kept entries a thread (with six, six values are parked); sums that read ahead of their additions took
+    twelve to twenty bytes of private memory a lane."""
+    kept = [k for n, k in kernels.items() if re.search(r"muscle_world_kernelILi\dELi\d+ELi[24]E", n)]
+    assert len(kept) == 12 and all(k[".private_segment_fixed_size"] == 0 for k in kept)

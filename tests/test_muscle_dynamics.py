@@ -801,6 +801,24 @@ def test_groups_are_the_list_in_another_order(muscles, swap):
     assert group_context_rows(longer, np.append(seg, [0] * 4), e.muscle_dof_torque_idx, np.append(e.start_coeff, [1.0] * 4), np.append(e.end_coeff, [1.0] * 4)) is None
 
 
+@pytest.mark.parametrize("what", [0, 1, 2])
+def test_a_world_that_fills_64_kb_goes_from_its_context(what):
+    """The words of a world, entries with four behind them, segments, axes, forces, centres and two flags, up to the limit
+    and one past it (nworld = 0 only checks the sizes)."""
+    import ctypes as C
+
+    from instantmimic_amd import _lib
+
+    sizes = dict(nbody=23, nwaypoint=900, nsegment=1160, ntorque=61, nmuscle=500)
+    rest = 9 * sizes["nsegment"] + 7 * sizes["ntorque"] + sizes["nmuscle"] + 3 * sizes["nbody"] + 2
+    for over in (0, 1):
+        n = 16384 + over - rest - 4
+        c = _lib.MuscleContext(ld_params=4, nrow=60, nentry=n, npacked=n, kind_count=(C.c_int32 * 3)(0, 0, n), **sizes)
+        assert n <= 5120
+        status = _lib.lib().im_muscle_from_context(C.byref(c), what, None, 0, 6, None, 60, 0, None)
+        assert status == (_lib.IM_ERR_UNSUPPORTED if over else 0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("muscles", [1, 57, 58, 64, 148, 149, 310, 314])
 def test_gpu_groups_equal_the_list_entry_by_entry(muscles):
