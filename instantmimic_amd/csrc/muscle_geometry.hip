@@ -1525,18 +1525,29 @@ int launch_context(const CtxArgs &a, hipStream_t stream) {
   if (const int st = compute_units(&ncu)) return st;
   constexpr int trips = MODE == MW_MOMENT ? kRowTrips : kGroupTrips;
   const int groups = a.c.ngroup, with_lengths = ctx_lds<true>(a.c, MODE != MW_MOMENT).words, words = ctx_lds<false>(a.c, MODE != MW_MOMENT).words;
-  // Groups: the same, with four groups a thread (six rows for the moment), and between 1024 and 1536 groups 256 threads with
-  // six each for such batches: 200 muscles x 8192 97.1 / 84.4 -> 88.7 / 82.4 us, x 2048 28.1 / 24.8 -> 26.7 / 25.2.
-  if (groups > 0 && 4 * (size_t)with_lengths <= 64 * 1024) {
+  // Groups: the same, with four groups a thread (six rows for the moment); for batches beyond six workgroups a CU also
+  // 128 threads with five each (75 muscles x 8192 42.5 / 41.2 us with 256 of four, 38.3 / 38.2; with six each 90 muscles x 8192 gained, x 4096
+  // lost) and 256 with six: 200 muscles x 8192 97.1 / 84.4 -> 88.7 / 82.4, x 2048 28.1 / 24.8 -> 26.7 / 25.2.
+  // Where 128 threads take the entries one by one, groups are not always less: their fills make up whole wavefronts of each kind, and
+  // a moment's rows cost more before the first world.  Entry by entry / in groups, us: torque of 60 muscles (977 entries, 576 groups) x
+  // 4096 19.1 / 19.7, of 65 (1082, 576) 21.1 / 20.9, of 57 (931, 512) 19.9 / 17.7; moment of 10 muscles (198, 384) x 8192 16.5 / 18.2,
+  // of 40 (657, 576) x 8192 22.5 / 23.1, of 57 (931, 640) x 1100 8.6 / 9.0, x 2000 10.6 / 10.2, of 75 (1276, 896) x 8192 31.9 / 34.9.
+  const bool many = a.nworld > 6 * ncu, few_entries = packed <= kCtxTrips * 128 && muscles <= 128;
+  bool grouped = groups > 0 && 4 * (size_t)with_lengths <= 64 * 1024;
+  if (MODE == MW_MOMENT && few_entries) grouped = grouped && a.nworld > 7 * ncu && groups <= trips * 128 && 5 * groups <= 4 * packed;
+  if (MODE != MW_MOMENT && few_entries && many && groups > trips * 128 && packed <= 8 * 128) grouped = false;
+  if (grouped) {
     if (groups <= trips * 128 && muscles <= 128) return launch_resident<128>(muscle_groups_kernel<MODE, 128, trips, 6>, with_lengths, a, stream, 32);
+    if constexpr (MODE != MW_MOMENT)
+      if (groups <= 5 * 128 && muscles <= 128 && many) return launch_resident<128>(muscle_groups_kernel<MODE, 128, 5, 5>, with_lengths, a, stream, 32);
     if (groups <= trips * 256 && muscles <= 256) return launch_resident<256>(muscle_groups_kernel<MODE, 256, trips, 6>, with_lengths, a, stream, 32);
     if constexpr (MODE != MW_MOMENT)
-      if (groups <= 6 * 256 && muscles <= 256 && a.nworld > 6 * ncu) return launch_resident<256>(muscle_groups_kernel<MODE, 256, 6, 5>, with_lengths, a, stream, 32);
+      if (groups <= 6 * 256 && muscles <= 256 && many) return launch_resident<256>(muscle_groups_kernel<MODE, 256, 6, 5>, with_lengths, a, stream, 32);
     if (groups <= trips * 512) return launch_resident<512>(muscle_groups_kernel<MODE, 512, trips, 6>, with_lengths, a, stream, 32);
   }
   if (packed <= kCtxTrips * 128 && muscles <= 128) return launch_resident<128>(muscle_context_kernel<MODE, 128, kCtxTrips>, words, a, stream);
   if (packed <= kCtxTrips * 256 && muscles <= 256) return launch_resident<256>(muscle_context_kernel<MODE, 256, kCtxTrips>, words, a, stream);
-  if (packed <= 14 * 256 && muscles <= 256 && a.nworld > 6 * ncu) return launch_resident<256>(muscle_context_kernel<MODE, 256, 14>, words, a, stream);
+  if (packed <= 14 * 256 && muscles <= 256 && many) return launch_resident<256>(muscle_context_kernel<MODE, 256, 14>, words, a, stream);
   return launch_resident<512>(muscle_context_kernel<MODE, 512, kCtxTrips>, words, a, stream);
 }
 

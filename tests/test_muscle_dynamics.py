@@ -846,6 +846,30 @@ def test_gpu_groups_equal_the_list_entry_by_entry(muscles):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("muscles", [30, 40, 57, 58, 60, 65, 80, 90, 91, 128, 230, 231])
+def test_gpu_groups_of_large_batches_equal_the_list_entry_by_entry(muscles):
+    """Batches of a workgroup more than six, and than seven, for every compute unit: the rules between entries and groups, and
+    five and six groups a thread up to their last size and beyond it; the same bits."""
+    rig = synth.make_muscle_rig(nmuscle=muscles, seed=1003)
+    layer = _gpu_layer(rig)
+    stated = [c.ngroup for c in layer._context]
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    for nworld in (6 * ncu, 6 * ncu + 1, 7 * ncu + 1):
+        ctx = torch.from_numpy(synth.make_muscle_context(rig, 67, seed=8)).cuda()[torch.arange(nworld, device="cuda") % 67].contiguous()
+        act, g = torch.rand(nworld, muscles, device="cuda"), torch.randn(nworld, rig.torque_dim, device="cuda")
+        run = lambda: [layer._torque_from_context(act, ctx, True), layer._warp_muscle_dynamics_from_activation_backward(ctx, g),  # noqa: E731
+                       layer.eval_muscle_sparse_moment(ctx)]  # fmt: skip
+        got = run()
+        for c in layer._context:
+            c.ngroup = 0
+        want = run()
+        for c, n in zip(layer._context, stated):
+            c.ngroup = n
+        for x, y in zip(got, want):
+            assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
 def test_gpu_torque_call_is_the_dispatchers_operator():
     """``ops.muscle_torque_forward`` in eager code with a gradient to record against the operator of that name through
     the dispatcher: values, gradients, what autograd refuses, what modes and hooks see."""
