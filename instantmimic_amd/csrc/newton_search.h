@@ -192,7 +192,8 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
   // selects.  Rows read at every evaluation take three arrays instead of six there, two rows at a time, and only the trips
   // with a friction row keep what is formed once (f / D, the cost at step 0).  A row's six loads and forty instructions were
   // what bounded a round of the search: solves of 70 dofs x 157 rows x 2048 worlds 711 -> 695 us, 53 x 128 x 4096 (sparse)
-  // 732 -> 715, 43 x 96 x 8192 (sparse) 634 -> 624; with the rows in registers 27 x 64 x 4096 243.4 -> 241.7.
+  // 732 -> 715, 43 x 96 x 8192 (sparse) 634 -> 624.  With eight rows a lane in registers both forms took a wavefront's registers
+  // (131 against 125; a search of 35 dofs x 200 rows x 4096 worlds 32.0 us against 29.6): one form there.
   auto plain_rows = [&](auto point) __attribute__((always_inline)) {
     for (int r = ne + lane + ((nf + 31) & ~31); r < nefc; r += 64) {
       const bool second = r + 32 < nefc;
@@ -209,7 +210,7 @@ __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane)
       for (int k = 0; k < HELD; ++k) {
         const int r = ne + lane + 32 * k;
         if (r >= nefc) continue;
-        if (k > 0 && 32 * k >= nf)
+        if (HELD <= 4 && k > 0 && 32 * k >= nf)
           point(false, hd[k], 0.0f, 0.0f, hja[k], hv[k], hc0[k]);
         else
           point(r < ne + nf, hd[k], hf[k], hrf[k], hja[k], hv[k], hc0[k]);

@@ -68,3 +68,9 @@ def test_kept_muscle_entries_stay_in_registers(kernels):
     twelve to twenty bytes of private memory a lane."""
     kept = [k for n, k in kernels.items() if re.search(r"muscle_world_kernelILi\dELi\d+ELi[24]E", n)]
     assert len(kept) == 12 and all(k[".private_segment_fixed_size"] == 0 for k in kept)
+
+
+def test_line_search_with_eight_rows_a_lane_keeps_four_wavefronts(kernels):
+    """Up to 256 rows: 128 registers a lane; a shorter form for the rows without friction beside the other took 131."""
+    (search,) = [k for n, k in kernels.items() if "newton_linesearch_kernelILi8E" in n]
+    assert _wavefronts(search) >= 4 and search[".private_segment_fixed_size"] == 0
