@@ -1495,12 +1495,12 @@ int newton_solve_sparse(const im_sparse_plan *plan, const im_newton_args *p, flo
   std::array<bool, kVariants> usable;
   if (const int st = usable_variants(probed, variants, &usable)) return st;
   const int held = njmax <= 64 ? 2 : 0;
-  std::vector<int> admitted;
+  int admitted[kVariants], nadmitted = 0;
   for (int i = 0; i < kVariants; ++i)
-    if (usable[i] && variants[i].held == held) admitted.push_back(variants[i].waves);
+    if (usable[i] && variants[i].held == held) admitted[nadmitted++] = variants[i].waves;
   int ncu = 0;
   if (const int st = compute_units(&ncu)) return st;
-  const SparseResident r = sparse_resident_layout(sizes, njmax, ((p->nterm + n + 1 + 3) & ~3), resident::kept_words(n, njmax, 0), admitted, p->nworld, ncu);
+  const SparseResident r = sparse_resident_layout(sizes, njmax, ((p->nterm + n + 1 + 3) & ~3), resident::kept_words(n, njmax, 0), admitted, nadmitted, p->nworld, ncu);
   if (r.waves == 0) return IM_ERR_UNSUPPORTED;
   A.staged_rows = r.staged_rows;
   A.staged_steps = r.step_words;

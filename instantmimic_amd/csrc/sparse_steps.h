@@ -138,21 +138,22 @@ struct SparseResident {
   size_t lds = 0;
   int per_cu = 0;  // workgroups that a CU holds: by LDS, and sixteen wavefronts of up to 128 registers
 };
-// `waves`: the worlds per workgroup that there are kernels for, most first; `table_words`: of the loop's shared row tables;
+// `waves` (nwaves): the worlds per workgroup that there are kernels for, most first; `table_words`: of the loop's shared row tables;
 // `kept_words`: what a world keeps beside the area.
 // The most worlds per workgroup (one workgroup per CU) that 158 KB of LDS admit, with 32 staged rows where they still
 // fit (they cost a CU no world then; snu: 32 rows with eight worlds per CU instead of twelve was measured slower, 1344
-// against 1283 us per loop), else 16.  The steps lie in LDS unless they cost a CU worlds, or a world half of its staged rows, and the
-// batch does not fit the chip at once with them there.  Whole solves, us, steps in LDS / in memory: a forest of 57 dofs
-// with 34 KB of steps, 96 rows, where memory leaves room for 16 worlds instead of 12, x 4096 632 / 596, x 1000 478 / 490; one of 40
-// dofs (31 KB, 32 staged rows instead of 16) x 8192 580 / 564, x 1000 446 / 454; 35 dofs (12 KB, as many worlds and rows in both) x
-// 8192 442 / 453, x 1000 300 / 307.
-inline SparseResident sparse_resident_layout(const SparseSizes &s, int njmax, int table_words, size_t kept_words, const std::vector<int> &waves,
+// against 1283 us per loop), else 16.  The steps lie in LDS unless they cost a CU worlds and the batch does not fit the
+// chip at once with them there.  Whole solves, us, steps in LDS / in memory: 16 worlds instead of 12 in memory: a forest of 54
+// dofs (29 KB of steps), 96 rows x 4096 worlds 503 / 463, x 1000 376 / 378, one of 57 (34 KB) 522 / 496 and 393 / 394; as many worlds:
+// 35 dofs (13 KB) x 8192 436 / 445, x 1000 296 / 302, a forest of 40 dofs (31 KB; 32 staged rows instead of 16 in memory) x 8192
+// 468 / 483.
+inline SparseResident sparse_resident_layout(const SparseSizes &s, int njmax, int table_words, size_t kept_words, const int *waves, int nwaves,
                                              int nworld, int ncu) {
   auto layout = [&](int step_words) {
     SparseResident r;
     const size_t shared = (size_t)step_words + s.shared_words + table_words;
-    for (const int w : waves) {
+    for (int i = 0; i < nwaves; ++i) {
+      const int w = waves[i];
       auto bytes = [&](int rows) { return 4 * (shared + w * (resident_area_words(s.nslots, s.nv, njmax, rows) + kept_words)); };
       const int rows = bytes(32) <= 158 * 1024 ? 32 : 16;
       if (bytes(rows) > 158 * 1024) continue;
@@ -164,9 +165,8 @@ inline SparseResident sparse_resident_layout(const SparseSizes &s, int njmax, in
   };
   const SparseResident near = layout(s.step_words), far = layout(0);
   if (near.waves == 0) return far;
-  const int held = near.waves * near.per_cu, held_far = far.waves * far.per_cu;
-  const bool better = held_far > held || (held_far == held && far.staged_rows > near.staged_rows);
-  return better && (int64_t)nworld > (int64_t)held * ncu ? far : near;
+  const int held = near.waves * near.per_cu;
+  return far.waves * far.per_cu > held && (int64_t)nworld > (int64_t)held * ncu ? far : near;
 }
 
 }  // namespace im

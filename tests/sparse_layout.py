@@ -34,7 +34,8 @@ void update(const int *s, int nworld, int ncu, long *out) {
   out[0] = u.waves, out[1] = u.staged_rows, out[2] = (long)u.lds;
 }
 void resident(const int *s, int njmax, int tables, int kept, int nworld, int ncu, long *out) {
-  const SparseResident r = sparse_resident_layout({s[0], s[1], s[2], s[3]}, njmax, tables, kept, {16, 12, 8, 4}, nworld, ncu);
+  const int waves[] = {16, 12, 8, 4};
+  const SparseResident r = sparse_resident_layout({s[0], s[1], s[2], s[3]}, njmax, tables, kept, waves, 4, nworld, ncu);
   out[0] = r.waves, out[1] = r.staged_rows, out[2] = r.step_words, out[3] = (long)r.lds, out[4] = r.per_cu;
 }
 }
