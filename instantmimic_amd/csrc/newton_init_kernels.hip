@@ -21,8 +21,8 @@ namespace {
 __host__ __device__ inline size_t init_wave_words(int nv, int njmax) { return (resident::kTileWords + 3 * (size_t)nv + 3 * (size_t)njmax + 3) & ~(size_t)3; }
 __host__ __device__ inline int init_shared_words(int nterm, int nv) { return (nterm + nv + 1 + 3) & ~3; }
 
-// WIDE: more than 64 dofs (the product on the matrix cores, two dofs a lane in the gradient): 124 registers a lane against
-// 72.  What bounds the launch is J's trip from memory, hidden by other wavefronts, and one kernel of both forms gives every
+// WIDE: more than 64 dofs (three tiles of J on their way instead of one, two dofs a lane in the gradient): 119 registers a lane
+// against 76.  What bounds the launch is J's trip from memory, hidden by other wavefronts, and one kernel of both forms gives every
 // model the wide form's four per SIMD: 27 dofs x 8192 worlds with 64 rows 33.1 -> 29.9 us, 35 x 8192 with 96 rows 47.9 -> 43.1.
 template <bool WIDE>
 __global__ __launch_bounds__(256) void newton_init_context_kernel(resident::NewtonArgs a, const float *__restrict__ qacc_smooth,

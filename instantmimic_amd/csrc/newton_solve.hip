@@ -51,7 +51,7 @@ int compute_units(int *ncu) {
 }
 
 // Bytes of private memory a lane of a resident kernel may have: four values parked from the prologue to the next world.
-// The kernels of this library have 8 at most; one beyond the limit spills within a round and is left out.
+// The kernels of this library have 12 at most; one beyond the limit spills within a round and is left out.
 constexpr size_t kResidentPrivate = 16;
 bool usable_resident(const void *fn) {
   hipFuncAttributes fa{};

@@ -729,7 +729,7 @@ __global__ __launch_bounds__(256, 4) void sparse_init_mfma_kernel(
 }
 
 // Per-iteration factor stage, one wavefront per world (WAVES worlds per workgroup share the LDS
-// copy of the factor and solve tables: four, eight or sixteen, chosen by the launcher).  Same arithmetic as
+// copy of the forward solve's tables: four, eight or sixteen, chosen by the launcher).  Same arithmetic as
 // sparse_update_kernel below; the changed constraint rows are staged in LDS (up to A.staged_rows
 // of them, else they are read from memory), packed H is updated in LDS and written back whole,
 // and a lane keeps four pairs' table look-ups in flight.

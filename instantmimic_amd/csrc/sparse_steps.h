@@ -114,7 +114,7 @@ inline SparseUpdate sparse_update_layout(const SparseSizes &s, int nworld, int n
   if (bytes(4) > 64 * 1024) return u;
   // Worlds per workgroup: every workgroup stages the tables for itself, so larger workgroups
   // leave more of a CU's 160 KB to the worlds.  The count that keeps the most worlds on a CU
-  // (at most 32 wavefronts of 57 registers) is taken, the smallest on a tie and where four
+  // (at most 32 wavefronts) is taken, the smallest on a tie and where four
   // per workgroup already hold the whole batch.
   int64_t best = 0;
   for (int cand = 4; cand <= 16; cand *= 2) {

@@ -316,8 +316,8 @@ def test_gpu_solve_at_the_edges_of_a_tile_of_j(device, monkeypatch, nv):
 @pytest.mark.parametrize("ne,nf", [(0, 0), (2, 31), (1, 32), (2, 33), (3, 70)])
 def test_gpu_solve_with_friction_rows_up_to_a_trip_and_beyond(device, monkeypatch, name, stage, rows, ne, nf):
     """The line search takes its trips of 32 rows without friction by a shorter form, with the rows in registers and
-    read at every evaluation: friction rows that end before, with and behind a trip, none at all, and more than a world has
-    rows."""
+    read at every evaluation: friction rows that end before, with and behind a trip, none at all, and all of a world's rows
+    behind its equalities."""
     shape = synth.SHAPES[name]
     monkeypatch.setitem(synth.SHAPES, name, replace(shape, nefc=rows))
     p = NC.problem(name, 33, stage, empty_every=9)
