@@ -326,3 +326,17 @@ def test_gpu_solve_with_friction_rows_up_to_a_trip_and_beyond(device, monkeypatc
     s = NC.oracle_solve(p)
     m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
     NC.compare(p, s, d, ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nf", [-1, -40, -(1 << 30), 1 << 20, 1 << 30])
+def test_gpu_solve_with_a_friction_count_that_no_world_has(device, monkeypatch, nf):
+    """Below zero: no friction rows; past the rows: all of them behind the equalities.  The line search counts its trips of
+    rows read at every evaluation by that number."""
+    monkeypatch.setitem(synth.SHAPES, "g1", replace(synth.SHAPES["g1"], nefc=130))
+    p = NC.problem("g1", 33, "sparse", empty_every=9)
+    p.ne = np.minimum(2, p.nefc).astype(np.int32)
+    p.nf = np.full_like(p.nefc, nf, dtype=np.int32)
+    s = NC.oracle_solve(p)
+    m, d, ctx, nsolving = _solve_on_gpu(p, device, graph=False)
+    NC.compare(p, s, d, ctx)
