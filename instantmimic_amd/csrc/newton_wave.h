@@ -383,11 +383,11 @@ __device__ __forceinline__ void search_sums_world(const NewtonArgs &a, int64_t w
 // (lane / 16, lane % 16) brings dofs 4 g .. 4 g + 3 of rows c, 16 + c, .. into the tile, whose rows lie 16 words apart
 // with their quads changed round by the row (quad q of row r at q ^ (r / 4 % 4): neither the writes nor the reads meet in a
 // bank).  DEPTH tiles are on their way at once.  What bounds the product is the trips to memory and the chain.  With the
-// row of M asked for ahead (StagedM), the two products of a round of the slowest worlds, and the solve: 70 dofs x 157 rows
-// x 2048 worlds 19.2 -> 13.3 us and 800 -> 741 (the chains ran on the matrix cores there, sixteen equal columns to a result,
-// their operands turned by lane swaps); 43 dofs x 8192 worlds 9.4 -> 7.2 and 644 -> 634, 27 x 4096 247 -> 240, 14 x 64
-// 100 -> 97.5 (a tile of single words, four times the LDS instructions).  1 tile ahead up to 64 dofs, where registers bound
-// the wavefronts in flight, 3 beyond.
+// row of M asked for ahead (StagedM), the two products of a round of the slowest worlds: 70 dofs x 157 rows x 2048 worlds
+// 19.2 -> 13.3 us, 43 x 96 x 8192 9.4 -> 7.2; the solves, three runs in turn within 0.3 %: 70 x 2048 797 -> 738 (the chains ran on the
+// matrix cores there, sixteen equal columns to a result, their operands turned by lane swaps), 53 x 4096 715 -> 679, 43 x 8192
+// 651 -> 621, 27 x 4096 249 -> 242, 14 x 64 106.8 -> 104.3 (a tile of single words, four times the LDS instructions).  1 tile ahead
+// up to 64 dofs, where registers bound the wavefronts in flight, 3 beyond.
 // `before` runs ahead of the first request, `between` while the first tiles are on their way; it leaves the direction in
 // sv (16-byte aligned) and may use the tile.
 typedef float v4 __attribute__((ext_vector_type(4)));
@@ -556,9 +556,10 @@ __device__ __forceinline__ const NewtonArgs &kernel_args(int kernarg_offset) {
 
 // The wavefront's priority among those of its SIMD: the quarter of the most rows that its world has.  A launch ends with
 // its slowest world, and rows are what is known of that beforehand (a world's time goes with its rows by 0.4 at 27 dofs,
-// 0.7 at 70): 27 dofs x 4096 worlds 242.5 -> 235.2 us, 53 x 4096 676 -> 669, 43 x 8192 623 -> 618 (tree stages), 70 x 2048
-// (dense) 693 -> 686.  The most rows of a workgroup's four worlds instead was worth half of that; on the sparse stage and
-// the dense one up to 64 dofs it made no difference either way.
+// 0.7 at 70).  Without / with it, us, medians of three runs in turn whose medians lie within 0.4 %: 27 dofs x 4096 worlds 241.9 / 239.3, 53 x 4096
+// 676.6 / 670.2, 43 x 8192 618.3 / 616.6 (tree stages), 70 x 2048 688.5 / 681.8, 78 x 2048 722.2 / 710.3, 70 x 6000 1364 / 1340 (dense); 14 x 64,
+// where a SIMD has one wavefront, 103.9 / 105.0.  The most rows of a workgroup's four worlds instead was worth half of that; on the
+// sparse stage and the dense one up to 64 dofs it made no difference either way.
 __device__ __forceinline__ void row_priority(int nefc, int njmax) {
   if (4 * nefc > 3 * njmax)
     __builtin_amdgcn_s_setprio(3);
