@@ -153,7 +153,7 @@ struct LsResult {
 template <int HELD, bool SPLIT = false>
 __device__ __forceinline__ LsResult linesearch_rows(const LsWorld &wd, int lane) {
   const int nv = wd.nv, ne = wd.ne, nefc = wd.nefc;
-  const int nf = wd.nf < 0 ? 0 : wd.nf < nefc ? wd.nf : nefc;  // (trips are counted by it)
+  const int nf = HELD > 0 ? wd.nf : wd.nf < 0 ? 0 : wd.nf < nefc ? wd.nf : nefc;  // (trips of rows that are not held are counted by it)
   const float *D = wd.D, *fl = wd.frictionloss, *Jaref = wd.Jaref, *jv = wd.jv;
   const float tolerance = wd.tolerance, ls_tolerance = wd.ls_tolerance;
   const float snorm = sqrtf(wd.search_dot);
