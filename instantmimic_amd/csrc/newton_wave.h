@@ -228,17 +228,28 @@ struct StagedM {
       wave_sync();
       return mul_m_world<WALK>(a, term, radr, m, v, out, out_lds, lane);
     }
-    if constexpr (!EARLY) fetch(m, nM, lane);
+    if constexpr (EARLY) {
 #pragma unroll
-    for (int u = 0; u < LOADS; ++u)
-      if (lane + 64 * u < nM) stage[lane + 64 * u] = x[u];
-    for (int k = lane + 64 * LOADS; k < nM; k += 64 * 4) {  // a longer row's other words
-      float y[4];
+      for (int u = 0; u < LOADS; ++u)
+        if (lane + 64 * u < nM) stage[lane + 64 * u] = x[u];
+      // a longer row's other words, four a lane at once (as many as the first took the start's kernel from 77 registers to 83,
+      // past a wavefront)
+      for (int k = lane + 64 * LOADS; k < nM; k += 64 * 4) {
+        float y[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) y[u] = m[(unsigned)(k + 64 * u < nM ? k + 64 * u : nM - 1)];
+        for (int u = 0; u < 4; ++u) y[u] = m[(unsigned)(k + 64 * u < nM ? k + 64 * u : nM - 1)];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (k + 64 * u < nM) stage[k + 64 * u] = y[u];
+        for (int u = 0; u < 4; ++u)
+          if (k + 64 * u < nM) stage[k + 64 * u] = y[u];
+      }
+    } else {
+      // (a loop of its own behind the first words, though never run, cost 14 dofs x 64 worlds 0.8 of 93 us)
+      for (int k0 = 0; k0 < nM; k0 += 64 * LOADS) {
+        fetch(m + k0, nM - k0, lane);
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u)
+          if (k0 + lane + 64 * u < nM) stage[k0 + lane + 64 * u] = x[u];
+      }
     }
     wave_sync();
     mul_m_world<WALK>(a, term, radr, stage, v, out, out_lds, lane);
